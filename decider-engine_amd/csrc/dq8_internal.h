@@ -146,6 +146,9 @@ hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, 
 hipError_t launch_quantize_raw(const void* x, int dtype, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
                                uint32_t* nonfinite, hipStream_t s);
 hipError_t launch_repack(const uint8_t* values, const float* scales, int n, int k, Weights* w, hipStream_t s);
+// Data::quantize of stored elements x [n][k] (type dtype, kDtype*) into w; a
+// non-finite element stores 1 to *nonfinite.
+hipError_t launch_quantize_weights(const void* x, int dtype, int n, int k, Weights* w, uint32_t* nonfinite, hipStream_t s);
 hipError_t launch_export(const Weights* w, uint8_t* values, float* scales, hipStream_t s);
 hipError_t launch_pad_rows(const int8_t* q, int rows, int k, int8_t* dst, int ldq, hipStream_t s);
 hipError_t launch_pad_scales(const float* xs, int rows, int g, float* dst, int ld, hipStream_t s);

@@ -41,9 +41,9 @@
  *     and dq8_linear_f32in) cannot be captured: on a capturing stream they
  *     return DQ8_ERR_CAPTURE and enqueue nothing.
  *   - The library starts no threads.
- *   - Weight loads keep their device buffers (stored elements, and values and
- *     scales before the repack) in the context, grown to the largest tensor
- *     loaded so far and freed by dq8_destroy.
+ *   - Weight loads from host memory keep their device buffer (the stored
+ *     elements) in the context, grown to the largest tensor loaded so far and
+ *     freed by dq8_destroy.
  *
  * Layouts (M tokens, K input width, N outputs, G = ceil(K/64)):
  *   activations x  fp32 [M][K] row-major        (tensor.rs:315)

@@ -158,3 +158,23 @@ def test_load_weights_rejects_non_projection_shapes_and_dtypes(ctx, tmp_path):
             with pytest.raises(dq8.Dq8Error) as e:
                 st.load_weights(ctx, name)
             assert e.value.status == status
+
+
+# The fused load kernel's edges: rows past the last 32-row block, a partial last
+# group, widths below one 16-byte piece, more tiles than the grid has waves, and
+# data that starts at an odd element (the loads are 16 bytes wide).
+@pytest.mark.parametrize("dtype", ["F32", "BF16", "F16"])
+@pytest.mark.parametrize("n,k", [(1, 1), (31, 15), (32, 64), (33, 65), (257, 79), (95, 1000), (4200, 2113)])
+def test_quantize_weights_edges_and_alignment(ctx, n, k, dtype):
+    raw = random_raw(np.random.default_rng(7 * n + k), n, k, dtype)
+    store = torch.empty(n * k + 1, dtype=torch.float32 if dtype == "F32" else torch.int16, device="cuda")
+    store[1:] = torch.from_numpy(raw.view(np.float32 if dtype == "F32" else np.int16)).cuda().reshape(-1)
+    data = store[1:].view(n, k)
+    if dtype != "F32":
+        data = data.view(torch.bfloat16 if dtype == "BF16" else torch.float16)
+    assert_same(ctx.weights_from_raw(data), raw, dtype)
+    bad = store.clone()
+    bad[-1] = float("inf") if dtype == "F32" else (0x7F80 if dtype == "BF16" else 0x7C00)
+    data = bad[1:].view(n, k)
+    with pytest.raises(dq8.NonFinite):
+        ctx.weights_from_raw(data if dtype == "F32" else data.view(torch.uint16), None if dtype == "F32" else DTYPE[dtype])
