@@ -10,7 +10,7 @@
 #include <string.h>
 #include <vector>
 
-// Scratch of dq8_apply_noalloc: its non-finite flag (first 256 bytes), then
+// Scratch of dq8_apply_noalloc: its chain state (first 256 bytes), then
 // the quantized inputs and their scales.  Each device holds its own copy for
 // the life of the process; host code uses only the per-device address that
 // hipGetSymbolAddress returns (dq8_create looks it up once per device).
@@ -29,6 +29,7 @@ struct dq8_ctx {
   void* chain = nullptr;
   size_t chain_bytes = 0;
   uint32_t* flag = nullptr;  // non-finite flag for synchronous checks
+  dq8::Chain* chain_state = nullptr;  // the same for calls that choose on the device (beside flag)
   // Two pinned host buffers through which weight loads stream to the device,
   // and the events of the copies out of them (created on first use).
   void* staging[2] = {nullptr, nullptr};
@@ -230,12 +231,15 @@ void fill_proj(dq8::Proj& p, const dq8::Weights& w, const int8_t* q, int ldq, co
   p.hq = nullptr;
   p.hs = nullptr;
   p.hflag = nullptr;
+  p.hchain = nullptr;
   p.pair = 0;
   p.lmid2 = nullptr;
   p.lb2 = nullptr;
   p.lora2 = 0;
   p.rank2 = 0;
   p.lscale2 = 0.0f;
+  p.fx = nullptr;
+  p.fk = 0;
 }
 
 // Wide kernel: split the tile grid into gm x gn regions, gm * gn = 8, one per
@@ -446,16 +450,49 @@ struct QOut {
   int8_t* q;
   float* scales;
   uint32_t* nonfinite;
+  dq8::Chain* chain;
 };
+
+// The FP32 path beside an int8 projection: its fp32 inputs [m][k] and the
+// chain that says which of the two runs on the device.
+struct Fallback {
+  dq8::Chain* chain;
+  const float* x;
+};
+
+// The FP32 path of a projection (k_linear_fp32) over x [m][w.k].
+dq8::FProj make_fproj(const dq8::Weights& w, const float* x, size_t m, const float* bias, const dq8_lora* lora,
+                      float* out, int layout, int epilogue, dq8::Chain* chain) {
+  dq8::FProj p;
+  p.x = x;
+  p.wt = w.values;
+  p.wst = w.scales;
+  p.bias = bias;
+  p.lora = lora != nullptr;
+  p.rank = lora ? (int)lora->rank : 0;
+  p.lscale = lora ? lora->scale : 0.0f;
+  p.lmid = lora ? lora->mid : nullptr;
+  p.lb = lora ? lora->b : nullptr;
+  p.out = out;
+  p.m = (int)m;
+  p.k = w.k;
+  p.g = w.g;
+  p.n = w.n;
+  p.np = w.np;
+  p.epilogue = epilogue;
+  p.layout = layout;
+  p.chain = chain;
+  return p;
+}
 
 // Split items by kernel kind and launch.  Items with m == 0 do nothing (tensor.rs:152-154).
 // qout (one item only): the item's stored result is then quantized by k_quantize.
 // (Only the SwiGLU pair launch, run_pair, quantizes its result in its own
 // epilogue; the step's other quantized inputs come from outside the projections.)
-// unless: the launches do nothing on the device if *unless != 0 (the inputs
-// were not finite; the caller runs the FP32 kernel for these items).
+// fb (one item only): if the chain says that the inputs were not finite, the
+// FP32 path computes the item's outputs instead, and the call ends the chain's.
 dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, int32_t* dots, hipStream_t s,
-                      const QOut* qout = nullptr, const uint32_t* unless = nullptr) {
+                      const QOut* qout = nullptr, const Fallback* fb = nullptr) {
   size_t need = 0;
   for (size_t i = 0; i < count; ++i) {
     if (!items[i].m) continue;
@@ -470,7 +507,8 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
   dq8::Batch batch[dq8::kKinds];
   for (dq8::Batch& b : batch) {
     b.count = b.total_waves = b.any_lora = 0;
-    b.unless = unless;
+    b.chain = fb ? fb->chain : nullptr;
+    b.fallback = 0;
   }
   const bool small = small_call(items, count, [](const dq8_linear_item& it) -> const dq8::Weights& { return it.w->w; });
   // one-wave strips each skinny launch would have (see kSkinnyFewStrips)
@@ -541,6 +579,11 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
         p.lmid += r0 * p.rank;
         b.any_lora = 1;
       }
+      if (fb) {
+        p.fx = fb->x + r0 * w.k;
+        p.fk = w.k;
+        b.fallback = kind != 0;  // the skinny kernels hold the FP32 path themselves
+      }
       place_proj(p, kind, b, strips[kind] < kSkinnyFewStrips, units[kind], has_long[kind]);
     }
   }
@@ -549,10 +592,16 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
     hipError_t e = dq8::launch_linear(batch[kind], kind, dots != nullptr, s);
     if (e != hipSuccess) return from_hip(e);
   }
+  if (fb && batch[0].count) {
+    const dq8_linear_item& it = items[0];
+    hipError_t e = dq8::launch_linear_fp32(
+        make_fproj(it.w->w, fb->x, it.m, it.bias, it.lora, it.out, it.layout, it.epilogue, fb->chain), s);
+    if (e != hipSuccess) return from_hip(e);
+  }
   if (qout && count == 1 && items[0].m > 0) {
     const dq8::Weights& w = items[0].w->w;
     hipError_t e = dq8::launch_quantize(items[0].out, (int)items[0].m, w.n, qout->q, w.n, qout->scales,
-                                        (w.n + kGroup - 1) / kGroup, qout->nonfinite, s);
+                                        (w.n + kGroup - 1) / kGroup, qout->nonfinite, qout->chain, s);
     if (e != hipSuccess) return from_hip(e);
   }
   return DQ8_OK;
@@ -574,7 +623,8 @@ dq8_status run_pair(dq8_ctx* ctx, const dq8::Weights& g, const dq8::Weights& u, 
   b.count = 1;
   b.total_waves = 0;
   b.any_lora = gate_lora != nullptr || up_lora != nullptr;
-  b.unless = nullptr;
+  b.chain = nullptr;
+  b.fallback = 0;
   dq8::Proj& p = b.p[0];
   fill_proj(p, g, q, g.k, xs, g.g, m, gate_bias, h, nullptr, DQ8_ROWS, DQ8_WRITE, gate_lora);
   p.wt2 = u.values;
@@ -589,6 +639,7 @@ dq8_status run_pair(dq8_ctx* ctx, const dq8::Weights& g, const dq8::Weights& u, 
     p.hq = qout->q;
     p.hs = qout->scales;
     p.hflag = qout->nonfinite;
+    p.hchain = qout->chain;
   }
   p.pair = 1;
   place_proj(p, 0, b, false, 0, false);
@@ -642,23 +693,12 @@ WorkInputs inputs_at(const dq8::Weights& w, size_t m, void* base) {
   return in;
 }
 
-// QuantizedInputs::new of x [m][w.k] into `in`.  *flag is cleared first (by a
-// kernel, so the call can be graph-captured) and ends up non-zero if x holds
-// a non-finite value.
-dq8_status quantize_into(const dq8::Weights& w, const float* x, size_t m, const WorkInputs& in, uint32_t* flag,
-                         hipStream_t s) {
-  hipError_t e = dq8::launch_fill_u32(flag, 0, s);
-  if (e == hipSuccess) e = dq8::launch_quantize(x, (int)m, w.k, in.q, in.ldq, in.xs, in.ldxs, flag, s);
-  return from_hip(e);
-}
-
-// The same into the context workspace, with ctx->flag.
-dq8_status quantize_to_work(dq8_ctx* ctx, const dq8::Weights& w, const float* x, size_t m, hipStream_t s,
-                            WorkInputs& in) {
+// Room for QuantizedInputs::new of x [m][w.k] in the context workspace.
+dq8_status work_inputs(dq8_ctx* ctx, const dq8::Weights& w, size_t m, hipStream_t s, WorkInputs& in) {
   dq8_status st = ensure_work(ctx, work_q_bytes(w, m) + xs_pad_bytes(w, m), s);
   if (st != DQ8_OK) return st;
   in = inputs_at(w, m, ctx->work);
-  return quantize_into(w, x, m, in, ctx->flag, s);
+  return DQ8_OK;
 }
 
 // Waits for the stream and reports ctx->flag as DQ8_ERR_NONFINITE.
@@ -670,14 +710,13 @@ dq8_status finish_nonfinite(dq8_ctx* ctx, hipStream_t s) {
   return host ? DQ8_ERR_NONFINITE : DQ8_OK;
 }
 
-// The int8 kernels for one projection over workspace inputs.
+// The int8 kernels for one projection over workspace inputs; with fb, the FP32
+// path instead if the chain says that the inputs were not finite (run_linear).
 dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, const float* bias, const dq8_lora* lora,
-                      float* out, int layout, int epilogue, const uint32_t* unless, hipStream_t s) {
+                      float* out, int layout, int epilogue, const Fallback* fb, hipStream_t s) {
   dq8::Batch b;
-  b.count = 1;
   b.total_waves = 0;
   b.any_lora = lora != nullptr;
-  b.unless = unless;
   // (row chunks as in run_linear; at most 512 rows make at most 16 chunks)
   struct One {
     size_t m;
@@ -688,50 +727,36 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
   const int kind = nch > 1 ? 2 : kind_of(w, m);
   const size_t half = (m + nch - 1) / nch;
   b.count = 0;
+  b.chain = fb ? fb->chain : nullptr;
+  b.fallback = fb && kind != 0;
   for (size_t r0 = 0; r0 < m; r0 += half) {
     dq8::Proj& p = b.p[b.count++];
     fill_proj(p, w, in.q + r0 * in.ldq, in.ldq, in.xs + r0 * in.ldxs, in.ldxs, std::min(half, m - r0), bias,
               out + r0 * w.n, nullptr, layout, epilogue, lora);
     if (p.lora) p.lmid += r0 * p.rank;
+    if (fb) {
+      p.fx = fb->x + r0 * w.k;
+      p.fk = w.k;
+    }
     place_proj(p, kind, b, (long)nch * short_strips(w) < kSkinnyFewStrips, (long)nch * short_units(w), w.g > 32);
   }
-  return from_hip(dq8::launch_linear(b, kind, false, s));
+  hipError_t e = dq8::launch_linear(b, kind, false, s);
+  if (e == hipSuccess && fb && kind == 0)
+    e = dq8::launch_linear_fp32(make_fproj(w, fb->x, m, bias, lora, out, layout, epilogue, fb->chain), s);
+  return from_hip(e);
 }
 
-// The FP32 path of a projection (k_linear_fp32) over x [m][w.k].
-dq8::FProj make_fproj(const dq8::Weights& w, const float* x, size_t m, const float* bias, const dq8_lora* lora,
-                      float* out, int layout, int epilogue, const uint32_t* when) {
-  dq8::FProj p;
-  p.x = x;
-  p.wt = w.values;
-  p.wst = w.scales;
-  p.bias = bias;
-  p.lora = lora != nullptr;
-  p.rank = lora ? (int)lora->rank : 0;
-  p.lscale = lora ? lora->scale : 0.0f;
-  p.lmid = lora ? lora->mid : nullptr;
-  p.lb = lora ? lora->b : nullptr;
-  p.out = out;
-  p.m = (int)m;
-  p.k = w.k;
-  p.g = w.g;
-  p.n = w.n;
-  p.np = w.np;
-  p.epilogue = epilogue;
-  p.layout = layout;
-  p.when = when;
-  return p;
-}
-
-// Projection::apply_quantized after the quantization of x into `in` with its
-// non-finite flag: both paths are queued and the flag lets exactly one of them
-// run on the device (tensor.rs:190-201), with no synchronization.
-dq8_status apply_paths(const dq8::Weights& w, const float* x, size_t m, const float* bias, const dq8_lora* lora,
-                       float* out, int layout, int epilogue, const WorkInputs& in, const uint32_t* flag,
-                       hipStream_t s) {
-  dq8_status st = launch_one(w, in, m, bias, lora, out, layout, epilogue, flag, s);
+// Projection::apply_quantized of x [m][w.k] (tensor.rs:190-201) through `in`:
+// the quantizer, then the int8 kernels or the FP32 path, as the chain says on
+// the device, with no synchronization.
+dq8_status apply_through(const dq8::Weights& w, const float* x, size_t m, const float* bias, const dq8_lora* lora,
+                         float* out, int layout, int epilogue, const WorkInputs& in, dq8::Chain* chain, hipStream_t s) {
+  dq8_status st = from_hip(dq8::launch_quantize(x, (int)m, w.k, in.q, in.ldq, in.xs, in.ldxs, nullptr, chain, s));
   if (st != DQ8_OK) return st;
-  return from_hip(dq8::launch_linear_fp32(make_fproj(w, x, m, bias, lora, out, layout, epilogue, flag), s));
+  const Fallback fb = {chain, x};
+  st = launch_one(w, in, m, bias, lora, out, layout, epilogue, &fb, s);
+  if (st != DQ8_OK) (void)dq8::launch_chain_reset(chain, s);
+  return st;
 }
 
 // ------------------------------------------------------------- weight loads
@@ -846,10 +871,14 @@ dq8_status dq8_create(int device, dq8_ctx** out) {
   dq8_ctx* ctx = new (std::nothrow) dq8_ctx();
   if (!ctx) return DQ8_ERR_NOMEM;
   ctx->device = device;
-  hipError_t e = hipMalloc(&ctx->flag, sizeof(uint32_t));
+  // the chain state, then the flag
+  hipError_t e = hipMalloc(&ctx->chain_state, sizeof(dq8::Chain) + sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMemset(ctx->chain_state, 0, sizeof(dq8::Chain) + sizeof(uint32_t));
+  if (e == hipSuccess) e = hipDeviceSynchronize();  // zero before any stream's first call
+  ctx->flag = reinterpret_cast<uint32_t*>(ctx->chain_state + 1);
   if (e == hipSuccess) e = hipHostMalloc(&ctx->host_flag, sizeof(uint32_t), hipHostMallocDefault);
   if (e != hipSuccess) {
-    (void)hipFree(ctx->flag);
+    (void)hipFree(ctx->chain_state);
     delete ctx;
     return from_hip(e);
   }
@@ -864,7 +893,7 @@ dq8_status dq8_destroy(dq8_ctx* ctx) {
   (void)hipDeviceSynchronize();
   (void)hipFree(ctx->work);
   (void)hipFree(ctx->chain);
-  (void)hipFree(ctx->flag);
+  (void)hipFree(ctx->chain_state);
   for (int b = 0; b < 2; ++b) {
     if (ctx->staged[b]) (void)hipEventDestroy(ctx->staged[b]);
     if (ctx->staging[b]) (void)hipHostFree(ctx->staging[b]);
@@ -993,7 +1022,7 @@ dq8_status dq8_quantize(dq8_ctx* ctx, const float* x, size_t m, size_t k, int8_t
   uint32_t* flag = nonfinite ? nonfinite : ctx->flag;
   hipError_t e = hipSuccess;
   if (!nonfinite) e = dq8::launch_fill_u32(ctx->flag, 0, s);
-  if (e == hipSuccess) e = dq8::launch_quantize(x, (int)m, (int)k, q, (int)k, scales, (int)groups_of(k), flag, s);
+  if (e == hipSuccess) e = dq8::launch_quantize(x, (int)m, (int)k, q, (int)k, scales, (int)groups_of(k), flag, nullptr, s);
   if (e != hipSuccess) return from_hip(e);
   if (nonfinite) return DQ8_OK;
   uint32_t host = 0;
@@ -1160,7 +1189,7 @@ dq8_status dq8_ffn_gate_up_lora(dq8_ctx* ctx, const dq8_weights* gate, const dq8
     hipError_t e = dq8::launch_fill_u32(ctx->flag, 0, s);
     if (e != hipSuccess) return from_hip(e);
   }
-  QOut qo = {h_q, h_scales, nonfinite ? nonfinite : ctx->flag};
+  QOut qo = {h_q, h_scales, nonfinite ? nonfinite : ctx->flag, nullptr};
   st = gate_up(ctx, gate, up, q, scales, m, gate_bias, up_bias, gate_lora, up_lora, h, &qo, s);
   if (st != DQ8_OK || nonfinite) return st;
   return finish_nonfinite(ctx, s);
@@ -1181,8 +1210,12 @@ dq8_status dq8_linear_f32in(dq8_ctx* ctx, const dq8_weights* w, const float* x, 
   hipStream_t s = (hipStream_t)stream;
   if (capturing(s)) return DQ8_ERR_CAPTURE;  // it synchronizes
   WorkInputs in;
-  st = quantize_to_work(ctx, w->w, x, m, s, in);
+  st = work_inputs(ctx, w->w, m, s, in);
   if (st != DQ8_OK) return st;
+  hipError_t e = dq8::launch_fill_u32(ctx->flag, 0, s);
+  if (e == hipSuccess)
+    e = dq8::launch_quantize(x, (int)m, w->w.k, in.q, in.ldq, in.xs, in.ldxs, ctx->flag, nullptr, s);
+  if (e != hipSuccess) return from_hip(e);
   st = finish_nonfinite(ctx, s);
   if (st != DQ8_OK) return st;
   return launch_one(w->w, in, m, bias, nullptr, out, layout, epilogue, nullptr, s);
@@ -1204,9 +1237,9 @@ dq8_status dq8_apply(dq8_ctx* ctx, const dq8_weights* w, const float* x, size_t 
   DeviceGuard guard(ctx->device);
   hipStream_t s = (hipStream_t)stream;
   WorkInputs in;
-  st = quantize_to_work(ctx, w->w, x, m, s, in);
+  st = work_inputs(ctx, w->w, m, s, in);
   if (st != DQ8_OK) return st;
-  return apply_paths(w->w, x, m, bias, lora, out, layout, epilogue, in, ctx->flag, s);
+  return apply_through(w->w, x, m, bias, lora, out, layout, epilogue, in, ctx->chain_state, s);
 }
 
 dq8_status dq8_apply_noalloc(dq8_ctx* ctx, const dq8_weights* w, const float* x, size_t m, const float* bias,
@@ -1218,11 +1251,10 @@ dq8_status dq8_apply_noalloc(dq8_ctx* ctx, const dq8_weights* w, const float* x,
   if (!ctx->scratch) return DQ8_ERR_DEVICE;
   DeviceGuard guard(ctx->device);
   hipStream_t s = (hipStream_t)stream;
-  uint32_t* flag = reinterpret_cast<uint32_t*>(ctx->scratch);
+  dq8::Chain* chain = reinterpret_cast<dq8::Chain*>(ctx->scratch);
+  static_assert(sizeof(dq8::Chain) <= kScratchFlagBytes, "scratch head");
   const WorkInputs in = inputs_at(w->w, m, ctx->scratch + kScratchFlagBytes);
-  st = quantize_into(w->w, x, m, in, flag, s);
-  if (st != DQ8_OK) return st;
-  return apply_paths(w->w, x, m, bias, lora, out, layout, epilogue, in, flag, s);
+  return apply_through(w->w, x, m, bias, lora, out, layout, epilogue, in, chain, s);
 }
 
 dq8_status dq8_linear_q(dq8_ctx* ctx, const dq8_weights* w, const int8_t* q, const float* scales, size_t m,
@@ -1242,7 +1274,7 @@ dq8_status dq8_linear_q(dq8_ctx* ctx, const dq8_weights* w, const int8_t* q, con
     hipError_t e = dq8::launch_fill_u32(ctx->flag, 0, s);
     if (e != hipSuccess) return from_hip(e);
   }
-  QOut qo = {q_out, scales_out, nonfinite ? nonfinite : ctx->flag};
+  QOut qo = {q_out, scales_out, nonfinite ? nonfinite : ctx->flag, nullptr};
   dq8_linear_item it = {w, q, scales, m, bias, out, DQ8_ROWS, epilogue, lora};
   st = run_linear(ctx, &it, 1, nullptr, s, &qo);
   if (st != DQ8_OK || nonfinite) return st;
@@ -1274,33 +1306,31 @@ dq8_status dq8_ffn(dq8_ctx* ctx, const dq8_ffn_weights* f, const int8_t* q, cons
   int8_t* qh = (int8_t*)ctx->chain;
   float* sh = (float*)((char*)ctx->chain + qbytes);
   float* mid = (float*)((char*)ctx->chain + qbytes + sbytes);
-  hipError_t e = dq8::launch_fill_u32(ctx->flag, 0, s);
-  if (e != hipSuccess) return from_hip(e);
   // gate: Write into h (qwen.rs:489); up: SwiGlu into h (qwen.rs:490); h is
   // then quantized for down (qwen.rs:491).  Without adapters, on the wide
   // kernel, both projections run in one launch that stores h directly.
-  QOut qo = {qh, sh, ctx->flag};
+  dq8::Chain* chain = ctx->chain_state;
+  QOut qo = {qh, sh, nonfinite, chain};
   st = gate_up(ctx, f->gate, f->up, q, scales, m, f->gate_bias, f->up_bias, f->gate_lora, f->up_lora, h, &qo, s);
-  if (st != DQ8_OK) return st;
-  if (nonfinite) {
-    e = dq8::launch_or_u32(nonfinite, ctx->flag, s);
-    if (e != hipSuccess) return from_hip(e);
+  if (st != DQ8_OK) {
+    (void)dq8::launch_chain_reset(chain, s);
+    return st;
   }
   // down: Add into the residual (qwen.rs:492), its adapter's middle product from h.
   // If h holds a non-finite value, QuantizedInputs::new(h) is None and the crate
-  // takes the FP32 path on h (tensor.rs:197-201): both are queued and the flag
-  // lets exactly one of them run on the device.
+  // takes the FP32 path on h (tensor.rs:197-201), as the chain says on the device.
   dq8_lora dl = {mid, f->down_lora_b, rank, f->down_lora_scale};
-  if (rank > 0) {
-    e = dq8::launch_lora_mid(h, (int)m, (int)inter, f->down_lora_a, (int)rank, mid, s);
-    if (e != hipSuccess) return from_hip(e);
+  hipError_t e = hipSuccess;
+  if (rank > 0) e = dq8::launch_lora_mid(h, (int)m, (int)inter, f->down_lora_a, (int)rank, mid, s);
+  st = from_hip(e);
+  if (st == DQ8_OK) {
+    const dq8_lora* dlp = f->down_lora_a ? &dl : nullptr;
+    dq8_linear_item di = {f->down, qh, sh, m, f->down_bias, residual, DQ8_ROWS, DQ8_ADD, dlp};
+    const Fallback fb = {chain, h};
+    st = run_linear(ctx, &di, 1, nullptr, s, nullptr, &fb);
   }
-  const dq8_lora* dlp = f->down_lora_a ? &dl : nullptr;
-  dq8_linear_item di = {f->down, qh, sh, m, f->down_bias, residual, DQ8_ROWS, DQ8_ADD, dlp};
-  st = run_linear(ctx, &di, 1, nullptr, s, nullptr, ctx->flag);
-  if (st != DQ8_OK) return st;
-  return from_hip(
-      dq8::launch_linear_fp32(make_fproj(d, h, m, f->down_bias, dlp, residual, DQ8_ROWS, DQ8_ADD, ctx->flag), s));
+  if (st != DQ8_OK) (void)dq8::launch_chain_reset(chain, s);
+  return st;
 }
 
 dq8_status dq8_group_dots(dq8_ctx* ctx, const dq8_weights* w, const int8_t* q, size_t m, int32_t* dots,

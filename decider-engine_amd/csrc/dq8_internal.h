@@ -42,6 +42,17 @@ struct Divider {
   __host__ __device__ int div(uint32_t n) const { return (int)(((uint64_t)n * mul) >> shift); }
 };
 
+// Whether the inputs of a call were finite, decided on the device with no
+// clearing launch and no synchronization.  A call's quantizer stores next into
+// cur (its first block) and next + 1 into hit if it sees a non-finite value;
+// the launches after it compare hit with cur + 1, and the call's last launch
+// stores cur + 1 into next (its first block).  No launch reads a word that it
+// writes, so calls in stream order, and graph replays of them, each see their
+// own answer.  All zero at first.
+struct Chain {
+  uint64_t next, cur, hit;
+};
+
 // One projection of a launch.  q is [M][ldq] bytes with ldq % 16 == 0 and
 // every byte up to G*64 of each row readable (zero past K).
 struct Proj {
@@ -78,13 +89,15 @@ struct Proj {
   // wt2/wst2/bias2 the up weights of the same shape; the launch stores
   // h = silu(gate(x) + bias) * (up(x) + bias2) into out [M][N].  With hq
   // set it also quantizes h as k_quantize does: hq [M][N] int8, hs [M][G_h]
-  // scales (G_h = ceil(N / 64)), 1 ORed into *hflag if h is not finite.
+  // scales (G_h = ceil(N / 64)); if h is not finite, 1 is ORed into *hflag
+  // (when set) and *hchain (when set) is marked.
   const uint8_t* wt2;
   const float* wst2;
   const float* bias2;
   int8_t* hq;
   float* hs;
   uint32_t* hflag;
+  Chain* hchain;
   int pair;
   // The up projection's LoRA adapter in a pair launch (lmid/lb/rank/lscale of
   // the fields above are the gate's).
@@ -93,6 +106,9 @@ struct Proj {
   int lora2;
   int rank2;
   float lscale2;
+  // FP32 inputs [M][fk] of the projection (launches with Batch::fallback).
+  const float* fx;
+  int fk;
 };
 
 struct Batch {
@@ -101,9 +117,12 @@ struct Batch {
   int count;
   int total_waves;  // blocks of the launch
   int any_lora;     // some projection has a LoRA adapter (selects the kernels with the LoRA epilogue)
-  // When set, the launch does nothing if *unless != 0: the inputs were not
-  // finite and the FP32 kernel (k_linear_fp32) computes these outputs instead.
-  const uint32_t* unless;
+  // When set, and the chain says that the inputs were not finite: with
+  // `fallback` (skinny kernels) the blocks compute the FP32 path of their
+  // outputs from Proj::fx, and the launch ends the chain's call; without it the
+  // launch does nothing and k_linear_fp32 computes these outputs instead.
+  Chain* chain;
+  int fallback;
 };
 
 // LoRA middle products of several (x, A) pairs in one launch of the few-rows
@@ -135,16 +154,14 @@ struct FProj {
   float* out;
   int m, k, g, n, np;
   int epilogue, layout;
-  const uint32_t* when;  // if set, the launch does nothing unless *when != 0
+  Chain* chain;  // if set, the launch computes only if the chain's inputs were not finite, and ends its call
 };
 
 // Kernel launchers (dq8_kernels.hip).  All return hipError_t of the launch.
-// scales row stride lds >= G = ceil(k / 64)
+// scales row stride lds >= G = ceil(k / 64).  A non-finite element ORs 1 into
+// *nonfinite (when set) and marks *chain (when set), whose call this opens.
 hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
-                           uint32_t* nonfinite, hipStream_t s);
-// The same over raw stored elements of type dtype (kDtype*), decoded exactly.
-hipError_t launch_quantize_raw(const void* x, int dtype, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
-                               uint32_t* nonfinite, hipStream_t s);
+                           uint32_t* nonfinite, Chain* chain, hipStream_t s);
 hipError_t launch_repack(const uint8_t* values, const float* scales, int n, int k, Weights* w, hipStream_t s);
 // Data::quantize of stored elements x [n][k] (type dtype, kDtype*) into w; a
 // non-finite element stores 1 to *nonfinite.
@@ -154,8 +171,8 @@ hipError_t launch_pad_rows(const int8_t* q, int rows, int k, int8_t* dst, int ld
 hipError_t launch_pad_scales(const float* xs, int rows, int g, float* dst, int ld, hipStream_t s);
 // *p = v, as a kernel (graph-capturable, unlike a memset node).
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, hipStream_t s);
-// *dst |= *src on the device.
-hipError_t launch_or_u32(uint32_t* dst, const uint32_t* src, hipStream_t s);
+// chain->hit = 0 (a call that failed between its launches).
+hipError_t launch_chain_reset(Chain* chain, hipStream_t s);
 // The FP32 path of a projection (see FProj).
 hipError_t launch_linear_fp32(const FProj& p, hipStream_t s);
 // LoRA middle product mid [m][rank] = dot_scores(x_r, a_j) + 0.0 (x [m][k], a [rank][k]).

@@ -411,21 +411,30 @@ __device__ __forceinline__ float decode(const void* base, size_t i) {
 #ifndef DQ8_QUANT_NTS
 #define DQ8_QUANT_NTS 1
 #endif
-template <int DT>
-__device__ __forceinline__ void decode4(const void* base, size_t i, float (&v)[4]) {
-  if constexpr (DT == kDtypeF32) {
+__device__ __forceinline__ void load4(const float* p, float (&v)[4]) {
 #if DQ8_QUANT_NT
-    const v4f t4 = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(static_cast<const float*>(base) + i));
-    v[0] = t4[0]; v[1] = t4[1]; v[2] = t4[2]; v[3] = t4[3];
+  const v4f t = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p));
 #else
-    const float4 t = *reinterpret_cast<const float4*>(static_cast<const float*>(base) + i);
-    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+  const v4f t = *reinterpret_cast<const v4f*>(p);
 #endif
-  } else {
-    const uint2 t = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + i);
-    const uint16_t h[4] = {(uint16_t)t.x, (uint16_t)(t.x >> 16), (uint16_t)t.y, (uint16_t)(t.y >> 16)};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = decode<DT>(h, j);
+  for (int j = 0; j < 4; ++j) v[j] = t[j];
+}
+
+// Chain (dq8_internal.h): whether the call's inputs were not finite; its two ends.
+__device__ __forceinline__ bool chain_hit(const Chain* c) { return c->hit == c->cur + 1; }
+__device__ __forceinline__ void chain_open(Chain* c) {  // by the quantizer's first block
+  if (blockIdx.x == 0 && threadIdx.x == 0) c->cur = c->next;
+}
+__device__ __forceinline__ void chain_close(Chain* c) {  // by the last launch's first block
+  if (blockIdx.x == 0 && threadIdx.x == 0) c->next = c->cur + 1;
+}
+// One report per wave with a lane that saw a non-finite element.
+__device__ __forceinline__ void report_nonfinite(bool bad, uint32_t* flag, Chain* chain) {
+  const unsigned long long b = __ballot(bad);
+  if (b != 0 && (int)(threadIdx.x & 63) == __builtin_ffsll((long long)b) - 1) {
+    if (flag) atomicOr(flag, 1u);
+    if (chain) chain->hit = chain->next + 1;  // every reporter stores the same value
   }
 }
 
@@ -523,17 +532,17 @@ __device__ __forceinline__ void quant_pack(const float (&v)[N], float scale, uin
 // chunk); every chunk's load is issued before the first is used, so a wave
 // keeps PER KB (fp32) in flight.  A group's absmax is a max-reduction over its
 // 16 lanes; quant_pack rounds the elements (the IEEE quotient by the scale,
-// half away from zero, as f32::round).  x holds DT elements; a non-finite one ORs 1 into
-// *nonfinite (Data::read rejects it for weights, QuantizedInputs::new returns
-// None for inputs).  The host guarantees rows * ceil(chunks / PER) < 2^31 and
+// half away from zero, as f32::round).  A non-finite element (for which
+// QuantizedInputs::new returns None) is reported in *nonfinite and *chain.  The host guarantees rows * ceil(chunks / PER) < 2^31 and
 // passes wdiv, the divider by the waves per row (wave / wpr without a division).
 #ifndef DQ8_QUANT_WPB
 #define DQ8_QUANT_WPB 4
 #endif
-template <int DT, int PER>
-__global__ __launch_bounds__(64 * DQ8_QUANT_WPB) void k_quantize(const void* __restrict__ x, int rows, int k, int8_t* __restrict__ q,
+template <int PER>
+__global__ __launch_bounds__(64 * DQ8_QUANT_WPB) void k_quantize(const float* __restrict__ x, int rows, int k, int8_t* __restrict__ q,
                                                   int ldq, float* __restrict__ scales, int lds, uint32_t* nonfinite,
-                                                  Divider wdiv) {
+                                                  Chain* chain, Divider wdiv) {
+  if (chain) chain_open(chain);
   const int lane = threadIdx.x & 63;
   const int chunks = (k + 255) >> 8;
   const int wpr = (chunks + PER - 1) / PER;  // waves per row
@@ -541,7 +550,7 @@ __global__ __launch_bounds__(64 * DQ8_QUANT_WPB) void k_quantize(const void* __r
   const int row = wdiv.div((uint32_t)wave);
   if (row >= rows) return;  // wave-uniform
   const int c0 = (wave - row * wpr) * PER;
-  const bool vec = (k & 3) == 0 && ((uintptr_t)x & (DT == kDtypeF32 ? 15 : 7)) == 0;
+  const bool vec = (k & 3) == 0 && ((uintptr_t)x & 15) == 0;
   const size_t r0 = (size_t)row * k;
   int8_t* qr = q + (size_t)row * ldq;
   const bool qvec = (ldq & 3) == 0 && ((uintptr_t)q & 3) == 0;
@@ -597,7 +606,7 @@ __global__ __launch_bounds__(64 * DQ8_QUANT_WPB) void k_quantize(const void* __r
     // waits for its own load only (loads under a lane-divergent branch make
     // the compiler wait for all of them where the paths join).
 #pragma unroll
-    for (int p = 0; p < PER; ++p) decode4<DT>(x, r0 + (c0 + p) * 256 + lane * 4, v[p]);
+    for (int p = 0; p < PER; ++p) load4(x + r0 + (c0 + p) * 256 + lane * 4, v[p]);
     asm volatile("" ::: "memory");
     bad = finish(v, std::true_type{});
   } else {
@@ -605,18 +614,15 @@ __global__ __launch_bounds__(64 * DQ8_QUANT_WPB) void k_quantize(const void* __r
     for (int p = 0; p < PER; ++p) {
       const int k0 = (c0 + p) * 256 + lane * 4;  // chunks past the row's end: k0 >= k, all zeros, not stored
       if (vec && k0 + 3 < k) {
-        decode4<DT>(x, r0 + k0, v[p]);
+        load4(x + r0 + k0, v[p]);
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[p][i] = (k0 + i < k) ? decode<DT>(x, r0 + k0 + i) : 0.0f;
+        for (int i = 0; i < 4; ++i) v[p][i] = (k0 + i < k) ? x[r0 + k0 + i] : 0.0f;
       }
     }
     bad = finish(v, std::false_type{});
   }
-  if (nonfinite) {  // one atomic per wave that saw a non-finite element
-    const unsigned long long b = __ballot(bad);
-    if (b != 0 && lane == __builtin_ffsll((long long)b) - 1) atomicOr(nonfinite, 1u);
-  }
+  report_nonfinite(bad, nonfinite, chain);
 }
 
 // The fp32 quantizer for rows of whole chunks (k % 256 == 0, 16-byte aligned x,
@@ -649,14 +655,15 @@ constexpr int kQuantLoopBlocks = DQ8_QUANT_LOOP_BLOCKS;
 template <int D>
 __global__ __launch_bounds__(64 * DQ8_QUANT_LOOP_WPB) void k_quantize_loop(const float* __restrict__ x, int k, int total,
                                                        int8_t* __restrict__ q, int ldq, float* __restrict__ scales,
-                                                       int lds, uint32_t* nonfinite, Divider cdiv) {
+                                                       int lds, uint32_t* nonfinite, Chain* chain, Divider cdiv) {
+  if (chain) chain_open(chain);
   const int lane = threadIdx.x & 63;
   const int W = (int)gridDim.x * DQ8_QUANT_LOOP_WPB;
   const int w = (int)blockIdx.x * DQ8_QUANT_LOOP_WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cpr = k >> 8;
   auto load = [&](int c, float (&v)[4]) {
     const int row = cdiv.div((uint32_t)c);
-    decode4<kDtypeF32>(x, (size_t)row * k + (size_t)(c - row * cpr) * 256 + lane * 4, v);
+    load4(x + (size_t)row * k + (size_t)(c - row * cpr) * 256 + lane * 4, v);
   };
   float v[D][4];
 #pragma unroll
@@ -718,10 +725,7 @@ __global__ __launch_bounds__(64 * DQ8_QUANT_LOOP_WPB) void k_quantize_loop(const
 #endif
     }
   }
-  if (nonfinite) {  // one atomic per wave that saw a non-finite element
-    const unsigned long long b = __ballot(bad);
-    if (b != 0 && lane == __builtin_ffsll((long long)b) - 1) atomicOr(nonfinite, 1u);
-  }
+  report_nonfinite(bad, nonfinite, chain);
 }
 
 // Sixteen consecutive stored elements as loaded: 16-byte loads at element
@@ -1117,7 +1121,7 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
   };
   __shared__ __attribute__((aligned(16))) Ring ring;
   __shared__ __attribute__((aligned(16))) XChunk xc[DOTS ? 1 : 2];
-  // Non-finite inputs (*b.unless != 0): the FP32 kernel runs instead.  The
+  // Non-finite inputs (b.chain): the FP32 kernel runs instead.  The
   // flag is read once a tile's first loads are out.
 
   // One tile (block index blk of the launch's tile list).
@@ -1252,7 +1256,7 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
     issue_b(ring.b[i], i);
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (b.unless && *b.unless) {  // uniform: the block leaves once its loads into LDS have landed
+  if (b.chain && chain_hit(b.chain)) {  // uniform: the block leaves once its loads into LDS have landed
     wait_vmcnt<0>();
     return;
   }
@@ -1448,8 +1452,7 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
           }
           if ((t & 3) == 0) P.hs[(size_t)row * ((P.n + kGroup - 1) / kGroup) + nt] = scale;
         }
-        const unsigned long long bb = __ballot(bad && row < P.m);
-        if (bb != 0 && lane == __builtin_ffsll((long long)bb) - 1) atomicOr(P.hflag, 1u);
+        report_nonfinite(bad && row < P.m, P.hflag, P.hchain);
       }
       return;
     }
@@ -1635,6 +1638,9 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
     __syncthreads();
   }
 #else
+  // (a batch that quantizes h holds the one pair)
+  if constexpr (!DOTS && wide_pair_shape(WN, RT, CT))
+    if (b.p[0].hq != nullptr && b.p[0].hchain != nullptr) chain_open(b.p[0].hchain);
   run_tile(blockIdx.x);
 #endif
 }
@@ -1836,11 +1842,12 @@ __device__ __forceinline__ void skinny_group(const Proj& P, int c0, int lane, bo
 #define DQ8_SKINNY_NT_SHORT 1
 #endif
 // Short K (G <= 32): one wave streams the 16*CT columns from c0 over all
-// groups, 2 groups per step.  The block's 4 waves first load its activation
+// groups, 2 groups per step.  Returns true, with nothing computed, if the
+// inputs were not finite (so does skinny_long).  The block's 4 waves first load its activation
 // together; a wave with no columns (live false) only helps with that.
 template <int RT, int CT, int DB, bool DOTS, bool LORA>
-__device__ __forceinline__ void skinny_short(const Proj& P, int c0, bool live, int wid, int lane, uint8_t* lds,
-                                             const uint32_t* unless) {
+__device__ __forceinline__ bool skinny_short(const Proj& P, int c0, bool live, int wid, int lane, uint8_t* lds,
+                                             const Chain* chain) {
   constexpr int ROWS = 16 * RT;
   constexpr int STEP_A = RT * 2 * kFragBytes;  // activation bytes of one step (8-row units)
   constexpr int OPS = 2 * CT * (DOTS ? 1 : 2);  // ring loads per step
@@ -1896,11 +1903,11 @@ __device__ __forceinline__ void skinny_short(const Proj& P, int c0, bool live, i
   }
   // the non-finite flag is read while the first loads are in flight; the
   // whole block leaves on it (after they land: they write this block's LDS)
-  const bool skip = unless != nullptr && *unless != 0;
+  const bool skip = chain != nullptr && chain_hit(chain);
   wait_vmcnt<0>();
-  if (skip) return;
+  if (skip) return true;
   lds_barrier();
-  if (!live) return;  // no later barrier in this path
+  if (!live) return false;  // no later barrier in this path
 
   int aoff[RT][2];  // [row tile][group parity]: row 16rt + l%16, chunk 4*parity + l/16
 #pragma unroll
@@ -1958,13 +1965,14 @@ __device__ __forceinline__ void skinny_short(const Proj& P, int c0, bool live, i
   wait_vmcnt<0>();  // the clamped loads past the end
   if constexpr (!DOTS)
     if (live) skinny_store<RT, CT, LORA>(P, c0, lane, s);
+  return false;
 }
 
 // Long K (G > 32): one strip per block (TPB = 4/NSEG = 1), its 16*RT rows from row
 // r0, NSEG waves, one group per wave and step.
 template <int RT, int CT, int DB, int NSEG, bool DOTS, bool LORA>
-__device__ __forceinline__ void skinny_long(const Proj& P, int local, int wid, int lane, uint8_t* lds, int r0,
-                                            const uint32_t* unless) {
+__device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, int lane, uint8_t* lds, int r0,
+                                            const Chain* chain) {
   constexpr int ROWS = 16 * RT, NT = RT * CT, TPB = 4 / NSEG;
   constexpr int XP = 2 * NSEG;                 // x pieces per row of a chunk of 8 steps (8*NSEG groups)
   constexpr int XBYTES = ROWS * XP * 16;
@@ -2036,9 +2044,9 @@ __device__ __forceinline__ void skinny_long(const Proj& P, int local, int wid, i
   }
   // the non-finite flag, read while the first loads are in flight (the block
   // leaves after they land: the x chunk writes this block's LDS)
-  if (unless != nullptr && *unless != 0) {
+  if (chain != nullptr && chain_hit(chain)) {
     wait_vmcnt<0>();
-    return;
+    return true;
   }
   // Step j from ring slot d (a constant after unrolling); as in the short-K
   // loop, every slot is consumed on every path and the ring loop has no early
@@ -2095,18 +2103,175 @@ __device__ __forceinline__ void skinny_long(const Proj& P, int local, int wid, i
   wait_vmcnt<0>();  // the clamped loads past the end
   if constexpr (!DOTS)
     if (live && sidx == 0) skinny_store<RT, CT, LORA>(P, c0, lane, s, r0);
+  return false;
+}
+
+// dot_scores (tensor.rs:6-25, the x86-64 order) of a[0..len) and b[0..len)
+// from plain memory: eight lane sums over the full chunks of 8, added in
+// order from -0.0, then the tail elements one by one; no fused multiply-add.
+__device__ __forceinline__ float dot_scores_rows(const float* a, const float* b, int len) {
+  const int chunks = len >> 3;
+  float lanes[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  for (int c = 0; c < chunks; ++c)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) lanes[q] = lanes[q] + a[8 * c + q] * b[8 * c + q];
+  float sum = -0.0f;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) sum = sum + lanes[q];
+  for (int t = 8 * chunks; t < len; ++t) sum = sum + a[t] * b[t];
+  return sum;
+}
+
+// Weight element (n, t) of the repacked layout, dequantized as Data::row does
+// for 8-bit Quantized data (weights.rs:47-78): (float)(int8)q * scale.
+__device__ __forceinline__ float dequant(const FProj& P, int n, int t) {
+  const int g = t >> 6, off = t & 63, h = off >> 5, part = (off >> 4) & 1;
+  const int8_t q = (int8_t)P.wt[((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16 +
+                                (off & 15)];
+  return (float)q * P.wst[(size_t)g * P.np + n];
+}
+
+// The FP32 path of a projection, Projection::columns_tiled (tensor.rs:206-269),
+// which the crate takes when the inputs are not finite (tensor.rs:197-201):
+//   y = dot_scores(x_r, w_n) + (bias[n] or 0.0)     w_n dequantized (dequant)
+//   y = y + scale * (dot_scores(mid_r, B_n) + 0.0)   with an adapter (Adapter::combine)
+// stored through the epilogue.  The dot products run in dot_scores' order, so
+// NaN and infinity propagate as in the crate.  fp32_tile: a block of 256
+// threads computes 16*RPT rows x 64 columns from (m0, n0) and stores those in rows
+// [m0, mhi) x columns [nlo, nhi); for RPT = 2 thread (tr, tc) owns rows 2tr, 2tr+1 and columns tc + 16j (j < 4)
+// with eight lane sums each.  Per group of 64 inputs the block stages x and
+// the dequantized weights in LDS (rows padded to 68 floats: the 16 columns a
+// wave reads per step fall in distinct banks).
+constexpr int kF32Rows = 32, kF32Cols = 64, kF32Pad = 68;
+struct F32Lds {
+  float xs[kF32Rows][kF32Pad], ws[kF32Cols][kF32Pad];
+};
+template <int RPT>
+__device__ __forceinline__ void fp32_tile(const FProj& P, int m0, int n0, int mhi, int nlo, int nhi, F32Lds& L) {
+  auto &xs = L.xs;
+  auto &ws = L.ws;
+  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
+  const int chunks = P.k >> 3;  // full chunks of 8 go to the lane sums
+  float acc[RPT][4][8];
+#pragma unroll
+  for (int i = 0; i < RPT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[i][j][q] = 0.0f;
+  for (int g = 0; 8 * g < chunks; ++g) {
+    const int nfull = min(8, chunks - 8 * g);  // uniform over the block
+    __syncthreads();                           // the previous group's reads are done
+    {
+      // x: thread t stages 4*RPT inputs of one row (zero past m or k)
+      constexpr int SEG = 4 * RPT, SPR = kGroup / SEG;
+      const int r = tid / SPR, seg = tid % SPR, row = m0 + r, kk = 64 * g + SEG * seg;
+#pragma unroll
+      for (int u = 0; u < SEG; ++u)
+        xs[r][SEG * seg + u] = (row < P.m && kk + u < P.k) ? P.x[(size_t)row * P.k + kk + u] : 0.0f;
+    }
+    {
+      // w: thread t stages column t/4, 16 inputs from one fragment lane (the
+      // repacked layout is zero past n and k, and n0 + 63 < np)
+      const int c = tid >> 2, h = (tid >> 1) & 1, part = tid & 1, n = n0 + c;
+      const uint4 raw = *reinterpret_cast<const uint4*>(
+          P.wt + ((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16);
+      const float sc = P.wst[(size_t)g * P.np + n];
+      const uint32_t word[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+      for (int u = 0; u < 16; ++u) ws[c][32 * h + 16 * part + u] = (float)(int8_t)(word[u >> 2] >> (8 * (u & 3))) * sc;
+    }
+    __syncthreads();
+    for (int cc = 0; cc < nfull; ++cc) {
+      float xv[RPT][8], wv[4][8];
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) {
+        const float4 a = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc]);
+        const float4 b = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc + 4]);
+        xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w;
+        xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 a = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc]);
+        const float4 b = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc + 4]);
+        wv[j][0] = a.x; wv[j][1] = a.y; wv[j][2] = a.z; wv[j][3] = a.w;
+        wv[j][4] = b.x; wv[j][5] = b.y; wv[j][6] = b.z; wv[j][7] = b.w;
+      }
+#pragma unroll
+      for (int i = 0; i < RPT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int q = 0; q < 8; ++q) acc[i][j][q] = acc[i][j][q] + xv[i][q] * wv[j][q];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int row = m0 + RPT * tr + i;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = n0 + tc + 16 * j;
+      if (row >= mhi || n < nlo || n >= nhi) continue;
+      float y = -0.0f;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) y = y + acc[i][j][q];
+      for (int t = 8 * chunks; t < P.k; ++t) y = y + P.x[(size_t)row * P.k + t] * dequant(P, n, t);
+      y = y + (P.bias ? P.bias[n] : 0.0f);
+      if (P.lora) {
+        const float delta =
+            (P.rank > 0 ? dot_scores_rows(P.lmid + (size_t)row * P.rank, P.lb + (size_t)n * P.rank, P.rank) : -0.0f) +
+            0.0f;
+        const float scaled = P.lscale * delta;
+        y = y + scaled;
+      }
+      float* dst = P.layout == 1 ? P.out + (size_t)n * P.m + row : P.out + (size_t)row * P.n + n;
+      if (P.epilogue == 0 || P.layout == 1) *dst = y;
+      else if (P.epilogue == 1) *dst = *dst + y;
+      else *dst = silu(*dst) * y;
+    }
+  }
+}
+// The FP32 path of a whole projection: the blocks walk its tiles.  After int8
+// launches (P.chain) the grid is small, since its blocks mostly only leave.
+__global__ __launch_bounds__(256) void k_linear_fp32(FProj P) {
+  __shared__ __attribute__((aligned(16))) F32Lds L;
+  if (P.chain) {
+    const bool hit = chain_hit(P.chain);
+    chain_close(P.chain);
+    if (!hit) return;  // the inputs were finite: the int8 kernels ran
+  }
+  const int col_tiles = (P.n + kF32Cols - 1) / kF32Cols;
+  const int tiles = ((P.m + kF32Rows - 1) / kF32Rows) * col_tiles;
+  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const int m0 = t / col_tiles * kF32Rows, n0 = t % col_tiles * kF32Cols;
+    fp32_tile<2>(P, m0, n0, P.m, 0, P.n, L);
+  }
+}
+// The FP32 path of a skinny block's outputs: rows [m0, mhi) (at most 16*RPT), columns [nlo, nhi).
+template <int RPT>
+__device__ __forceinline__ void fp32_block(const Proj& S, int m0, int mhi, int nlo, int nhi, uint8_t* lds) {
+  const FProj P = {S.fx, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, S.fk, S.g, S.n, S.np,
+                   S.epilogue, S.layout, nullptr};
+  __syncthreads();  // every wave's loads into this LDS have landed
+  for (int n0 = nlo / kF32Cols * kF32Cols; n0 < nhi; n0 += kF32Cols)
+    fp32_tile<RPT>(P, m0, n0, mhi, nlo, nhi, *reinterpret_cast<F32Lds*>(lds));
 }
 
 template <int RT, int CT, int CTL, int DBS, int DBL, bool DOTS, bool LORA>
 __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[skinny_lds_bytes(RT, CTL)];
-  // non-finite inputs (*b.unless != 0): the FP32 kernel runs instead; each
-  // path checks the flag once its first loads are out
+  static_assert(DOTS || skinny_lds_bytes(RT, CTL) >= (int)sizeof(F32Lds), "the FP32 tile fits");
   const int pidx = find_proj<true>(b, blockIdx.x);
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Proj P = b.p[pidx];  // by value: its fields load in one batch
   const int local = blockIdx.x - P.wave_begin;
+  // non-finite inputs (b.chain): each path checks for them once its first loads
+  // are out and computes nothing; the block's outputs, rows [m0, mhi) and
+  // columns [nlo, nhi), then take the FP32 path
+  bool skip;
+  int m0 = 0, mhi = P.m, nlo, nhi;
   if (P.nseg == 1) {
     static_assert(CT == 2, "short-K waves take at most two 16-column units");
     const int H = P.waves_n;  // units of 16 columns
@@ -2115,6 +2280,8 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
       // 4 strips of two units per block, one per wave, from unit 8*local
       u0 = 2 * (4 * local + wid);
       cnt = u0 < H ? 2 : 0;
+      nlo = 128 * local;
+      nhi = nlo + 128;
     } else {
       // The units are dealt to B = ceil(H / units) blocks, deal_q to each and
       // one more to the first deal_r (at most 7; the host divides), so blocks
@@ -2124,25 +2291,39 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
       const int h0 = local * P.deal_q + min(local, P.deal_r), c = P.deal_q + (local < P.deal_r ? 1 : 0);
       u0 = h0 + wid * c / 4;
       cnt = h0 + (wid + 1) * c / 4 - u0;
+      nlo = 16 * h0;
+      nhi = nlo + 16 * c;
     }
     if (cnt == 2)
-      skinny_short<RT, 2, DBS, DOTS, LORA>(P, 16 * u0, true, wid, lane, lds, b.unless);
+      skip = skinny_short<RT, 2, DBS, DOTS, LORA>(P, 16 * u0, true, wid, lane, lds, b.chain);
     else
-      skinny_short<RT, 1, DBS, DOTS, LORA>(P, 16 * u0, cnt == 1, wid, lane, lds, b.unless);
-  } else if (RT == 1) {
-    skinny_long<1, CTL, DBL, 4, DOTS, LORA>(P, local, wid, lane, lds, 0, b.unless);
+      skip = skinny_short<RT, 1, DBS, DOTS, LORA>(P, 16 * u0, cnt == 1, wid, lane, lds, b.chain);
   } else {
-    // One 16-row tile per block: 17-32 rows take two blocks per strip.  The
-    // two blocks of a strip are 8 apart (blocks are dealt to the 8 XCDs in
-    // turn), so both run on one XCD and the second read of the strip's weights
-    // is served by that XCD's L2: in each run of 16 blocks, blocks 0-7 take
-    // the first row tile of 8 strips and blocks 8-15 the second.  A last run
-    // of R < 8 strips pairs blocks R apart.
-    const int run = local >> 4, in = local & 15;
-    const int left = P.waves_n - 8 * run;  // strips from this run on
-    const int r = left >= 8 ? 8 : left;
-    const int t = r == 8 ? in >> 3 : in / r;  // the row tile (a division only in the last run)
-    skinny_long<1, CTL, DBL, 4, DOTS, LORA>(P, 8 * run + in - t * r, wid, lane, lds, 16 * t, b.unless);
+    int strip = local;
+    if (RT == 2) {
+      // One 16-row tile per block: 17-32 rows take two blocks per strip.  The
+      // two blocks of a strip are 8 apart (blocks are dealt to the 8 XCDs in
+      // turn), so both run on one XCD and the second read of the strip's weights
+      // is served by that XCD's L2: in each run of 16 blocks, blocks 0-7 take
+      // the first row tile of 8 strips and blocks 8-15 the second.  A last run
+      // of R < 8 strips pairs blocks R apart.
+      const int run = local >> 4, in = local & 15;
+      const int left = P.waves_n - 8 * run;  // strips from this run on
+      const int r = left >= 8 ? 8 : left;
+      const int t = r == 8 ? in >> 3 : in / r;  // the row tile (a division only in the last run)
+      strip = 8 * run + in - t * r;
+      m0 = 16 * t;
+      mhi = min(mhi, m0 + 16);
+    }
+    nlo = 16 * CTL * strip;
+    nhi = nlo + 16 * CTL;
+    skip = skinny_long<1, CTL, DBL, 4, DOTS, LORA>(P, strip, wid, lane, lds, m0, b.chain);
+  }
+  if constexpr (!DOTS) {
+    if (b.fallback) {  // uniform over the launch
+      chain_close(b.chain);
+      if (skip) fp32_block<RT>(P, m0, mhi, nlo, min(nhi, P.n), lds);
+    }
   }
 }
 // LoRA middle product (weights.rs:480, 495): mid[r][j] = dot_scores(x_r, a_j)
@@ -2490,152 +2671,31 @@ __global__ __launch_bounds__(256) void k_lora_mid_small_batch(MidBatch bt) {
   lora_mid_small<kSmallR, kSmallJ, kSmallKR>(I.x, I.m, I.k, I.a, I.rank, I.mid, b - I.block_begin, lds);
 }
 
-// dot_scores (tensor.rs:6-25, the x86-64 order) of a[0..len) and b[0..len)
-// from plain memory: eight lane sums over the full chunks of 8, added in
-// order from -0.0, then the tail elements one by one; no fused multiply-add.
-__device__ __forceinline__ float dot_scores_rows(const float* a, const float* b, int len) {
-  const int chunks = len >> 3;
-  float lanes[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-  for (int c = 0; c < chunks; ++c)
-#pragma unroll
-    for (int q = 0; q < 8; ++q) lanes[q] = lanes[q] + a[8 * c + q] * b[8 * c + q];
-  float sum = -0.0f;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) sum = sum + lanes[q];
-  for (int t = 8 * chunks; t < len; ++t) sum = sum + a[t] * b[t];
-  return sum;
-}
-
-// Weight element (n, t) of the repacked layout, dequantized as Data::row does
-// for 8-bit Quantized data (weights.rs:47-78): (float)(int8)q * scale.
-__device__ __forceinline__ float dequant(const FProj& P, int n, int t) {
-  const int g = t >> 6, off = t & 63, h = off >> 5, part = (off >> 4) & 1;
-  const int8_t q = (int8_t)P.wt[((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16 +
-                                (off & 15)];
-  return (float)q * P.wst[(size_t)g * P.np + n];
-}
-
-// The FP32 path of a projection, Projection::columns_tiled (tensor.rs:206-269),
-// which the crate takes when the inputs are not finite (tensor.rs:197-201):
-//   y = dot_scores(x_r, w_n) + (bias[n] or 0.0)     w_n dequantized (dequant)
-//   y = y + scale * (dot_scores(mid_r, B_n) + 0.0)   with an adapter (Adapter::combine)
-// stored through the epilogue.  The dot products run in dot_scores' order, so
-// NaN and infinity propagate as in the crate.  A block computes 32 rows x 64
-// columns; thread (tr, tc) owns rows 2tr, 2tr+1 and columns tc + 16j (j < 4)
-// with eight lane sums each.  Per group of 64 inputs the block stages x and
-// the dequantized weights in LDS (rows padded to 68 floats: the 16 columns a
-// wave reads per step fall in distinct banks).
-constexpr int kF32Rows = 32, kF32Cols = 64, kF32Pad = 68;
-__global__ __launch_bounds__(256) void k_linear_fp32(FProj P) {
-  __shared__ __attribute__((aligned(16))) float xs[kF32Rows][kF32Pad];
-  __shared__ __attribute__((aligned(16))) float ws[kF32Cols][kF32Pad];
-  if (P.when && *P.when == 0) return;  // the inputs were finite: the int8 kernels ran
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  const int col_tiles = (P.n + kF32Cols - 1) / kF32Cols;
-  const int m0 = (int)(blockIdx.x / col_tiles) * kF32Rows, n0 = (int)(blockIdx.x % col_tiles) * kF32Cols;
-  const int chunks = P.k >> 3;  // full chunks of 8 go to the lane sums
-  float acc[2][4][8];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int q = 0; q < 8; ++q) acc[i][j][q] = 0.0f;
-  for (int g = 0; 8 * g < chunks; ++g) {
-    const int nfull = min(8, chunks - 8 * g);  // uniform over the block
-    __syncthreads();                           // the previous group's reads are done
-    {
-      // x: thread t stages row t/8, inputs 64g + 8(t%8) .. +8 (zero past m or k)
-      const int r = tid >> 3, seg = tid & 7, row = m0 + r, kk = 64 * g + 8 * seg;
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        xs[r][8 * seg + u] = (row < P.m && kk + u < P.k) ? P.x[(size_t)row * P.k + kk + u] : 0.0f;
-    }
-    {
-      // w: thread t stages column t/4, 16 inputs from one fragment lane (the
-      // repacked layout is zero past n and k, and n0 + 63 < np)
-      const int c = tid >> 2, h = (tid >> 1) & 1, part = tid & 1, n = n0 + c;
-      const uint4 raw = *reinterpret_cast<const uint4*>(
-          P.wt + ((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16);
-      const float sc = P.wst[(size_t)g * P.np + n];
-      const uint32_t word[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-      for (int u = 0; u < 16; ++u) ws[c][32 * h + 16 * part + u] = (float)(int8_t)(word[u >> 2] >> (8 * (u & 3))) * sc;
-    }
-    __syncthreads();
-    for (int cc = 0; cc < nfull; ++cc) {
-      float xv[2][8], wv[4][8];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const float4 a = *reinterpret_cast<const float4*>(&xs[2 * tr + i][8 * cc]);
-        const float4 b = *reinterpret_cast<const float4*>(&xs[2 * tr + i][8 * cc + 4]);
-        xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w;
-        xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float4 a = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc]);
-        const float4 b = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc + 4]);
-        wv[j][0] = a.x; wv[j][1] = a.y; wv[j][2] = a.z; wv[j][3] = a.w;
-        wv[j][4] = b.x; wv[j][5] = b.y; wv[j][6] = b.z; wv[j][7] = b.w;
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int q = 0; q < 8; ++q) acc[i][j][q] = acc[i][j][q] + xv[i][q] * wv[j][q];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = m0 + 2 * tr + i;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tc + 16 * j;
-      if (row >= P.m || n >= P.n) continue;
-      float y = -0.0f;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) y = y + acc[i][j][q];
-      for (int t = 8 * chunks; t < P.k; ++t) y = y + P.x[(size_t)row * P.k + t] * dequant(P, n, t);
-      y = y + (P.bias ? P.bias[n] : 0.0f);
-      if (P.lora) {
-        const float delta =
-            (P.rank > 0 ? dot_scores_rows(P.lmid + (size_t)row * P.rank, P.lb + (size_t)n * P.rank, P.rank) : -0.0f) +
-            0.0f;
-        const float scaled = P.lscale * delta;
-        y = y + scaled;
-      }
-      float* dst = P.layout == 1 ? P.out + (size_t)n * P.m + row : P.out + (size_t)row * P.n + n;
-      if (P.epilogue == 0 || P.layout == 1) *dst = y;
-      else if (P.epilogue == 1) *dst = *dst + y;
-      else *dst = silu(*dst) * y;
-    }
-  }
-}
-
 }  // namespace
 
 static unsigned blocks_for(long n, int per) { return (unsigned)((n + per - 1) / per); }
 
 __global__ void k_fill_u32(uint32_t* p, uint32_t v) { *p = v; }
-__global__ void k_or_u32(uint32_t* dst, const uint32_t* src) {
-  if (*src) atomicOr(dst, *src);
-}
+__global__ void k_chain_reset(Chain* c) { c->hit = 0; }
 
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, hipStream_t s) {
   k_fill_u32<<<1, 1, 0, s>>>(p, v);
   return hipGetLastError();
 }
 
-hipError_t launch_or_u32(uint32_t* dst, const uint32_t* src, hipStream_t s) {
-  k_or_u32<<<1, 1, 0, s>>>(dst, src);
+hipError_t launch_chain_reset(Chain* chain, hipStream_t s) {
+  k_chain_reset<<<1, 1, 0, s>>>(chain);
   return hipGetLastError();
 }
 
+// Blocks of a k_linear_fp32 launch behind int8 launches, which nearly always
+// find finite inputs: a grid of one block per tile took 3.7-5 us to leave
+// (2048 blocks), KF32_TIME at this size.
+constexpr long kF32ChainBlocks = 512;
 hipError_t launch_linear_fp32(const FProj& p, hipStream_t s) {
   if (p.m == 0 || p.n == 0) return hipSuccess;
-  const long blocks = (long)((p.m + kF32Rows - 1) / kF32Rows) * ((p.n + kF32Cols - 1) / kF32Cols);
+  const long tiles = (long)((p.m + kF32Rows - 1) / kF32Rows) * ((p.n + kF32Cols - 1) / kF32Cols);
+  const long blocks = p.chain ? std::min(tiles, kF32ChainBlocks) : std::min(tiles, 1L << 23);  // a grid under 2^32 threads
   k_linear_fp32<<<(unsigned)blocks, 256, 0, s>>>(p);
   return hipGetLastError();
 }
@@ -2682,17 +2742,17 @@ hipError_t launch_lora_mid(const float* x, int m, int k, const float* a, int ran
 }
 
 
-hipError_t launch_quantize_raw(const void* x, int dtype, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
-                               uint32_t* nonfinite, hipStream_t s) {
+hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
+                           uint32_t* nonfinite, Chain* chain, hipStream_t s) {
 #if DQ8_QUANT_LOOP > 0
-  if (dtype == kDtypeF32 && k % 256 == 0 && ((uintptr_t)x & 15) == 0 && ldq % 4 == 0 && ((uintptr_t)q & 3) == 0) {
+  if (k % 256 == 0 && ((uintptr_t)x & 15) == 0 && ldq % 4 == 0 && ((uintptr_t)q & 3) == 0) {
     const long total = (long)rows * (k / 256);
     if (total == 0) return hipSuccess;
     // the waves' chunk indices run to total + (DQ8_QUANT_LOOP + 1) * W (W <= 4 * kQuantLoopBlocks) in int
     if (total < (1L << 31) - (DQ8_QUANT_LOOP + 1) * (long)DQ8_QUANT_LOOP_WPB * kQuantLoopBlocks) {
       const int blocks = (int)std::min<long>(kQuantLoopBlocks, (total + DQ8_QUANT_LOOP_WPB - 1) / DQ8_QUANT_LOOP_WPB);
-      k_quantize_loop<DQ8_QUANT_LOOP><<<blocks, 64 * DQ8_QUANT_LOOP_WPB, 0, s>>>(static_cast<const float*>(x), k, (int)total, q, ldq,
-                                                             scales, lds, nonfinite, Divider::of((uint32_t)(k / 256)));
+      k_quantize_loop<DQ8_QUANT_LOOP><<<blocks, 64 * DQ8_QUANT_LOOP_WPB, 0, s>>>(
+          x, k, (int)total, q, ldq, scales, lds, nonfinite, chain, Divider::of((uint32_t)(k / 256)));
       return hipGetLastError();
     }
   }
@@ -2701,20 +2761,10 @@ hipError_t launch_quantize_raw(const void* x, int dtype, int rows, int k, int8_t
   const long waves = (long)rows * (((k + 255) / 256 + PER - 1) / PER);
   if (waves == 0) return hipSuccess;
   if (waves >= (1L << 31) - 4) return hipErrorInvalidValue;
-  const int blocks = blocks_for(waves, DQ8_QUANT_WPB);
   const Divider wdiv = Divider::of((uint32_t)(((k + 255) / 256 + PER - 1) / PER));
-  if (dtype == kDtypeBF16)
-    k_quantize<kDtypeBF16, PER><<<blocks, 64 * DQ8_QUANT_WPB, 0, s>>>(x, rows, k, q, ldq, scales, lds, nonfinite, wdiv);
-  else if (dtype == kDtypeF16)
-    k_quantize<kDtypeF16, PER><<<blocks, 64 * DQ8_QUANT_WPB, 0, s>>>(x, rows, k, q, ldq, scales, lds, nonfinite, wdiv);
-  else
-    k_quantize<kDtypeF32, PER><<<blocks, 64 * DQ8_QUANT_WPB, 0, s>>>(x, rows, k, q, ldq, scales, lds, nonfinite, wdiv);
+  k_quantize<PER><<<blocks_for(waves, DQ8_QUANT_WPB), 64 * DQ8_QUANT_WPB, 0, s>>>(x, rows, k, q, ldq, scales, lds,
+                                                                                 nonfinite, chain, wdiv);
   return hipGetLastError();
-}
-
-hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
-                           uint32_t* nonfinite, hipStream_t s) {
-  return launch_quantize_raw(x, kDtypeF32, rows, k, q, ldq, scales, lds, nonfinite, s);
 }
 
 hipError_t launch_repack(const uint8_t* values, const float* scales, int n, int k, Weights* w, hipStream_t s) {
