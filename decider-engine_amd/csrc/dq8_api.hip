@@ -394,7 +394,7 @@ void place_proj(dq8::Proj& p, int kind, dq8::Batch& b, bool few_strips, long lau
     p.nseg = dq8::skinny_segments(p.g, few_strips);
     if (p.nseg == 1) {
       // short K: 16-column units dealt to blocks, units_per_block at a time
-      p.waves_n = (p.n + 15) / 16;
+      p.waves_n = p.pair ? (p.n + 7) / 8 : (p.n + 15) / 16;  // a pair's unit holds 8 outputs of each projection
       p.units = units_per_block(launch_units, launch_has_long);
       const int blocks = (p.waves_n + p.units - 1) / p.units;
       p.deal_q = p.waves_n / blocks;
@@ -402,7 +402,7 @@ void place_proj(dq8::Proj& p, int kind, dq8::Batch& b, bool few_strips, long lau
       b.total_waves += blocks;
     } else {
       // long K: one 16-row tile of a strip per block (kind 2: two per strip)
-      p.waves_n = (p.n + dq8::skinny_cols(p.nseg) - 1) / dq8::skinny_cols(p.nseg);
+      p.waves_n = ((p.pair ? 2 : 1) * p.n + dq8::skinny_cols(p.nseg) - 1) / dq8::skinny_cols(p.nseg);
       b.total_waves += p.waves_n * (kind == 2 ? 2 : 1);
     }
   }
@@ -607,43 +607,54 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
   return DQ8_OK;
 }
 
-// One layer's gate and up projections (same shape, shared quantized input)
-// in one wide launch that stores h = silu(gate + bias + adapter) * (up + bias2
-// + adapter2) into h [m][n] and, as qout asks, quantizes h in the same launch
-// (q [m][n], scales [m][ceil(n/64)], the non-finite flag).  The results equal
-// the separate Write and SwiGlu launches and k_quantize bit for bit: each
-// output's arithmetic is unchanged, only the two tiles of one output sit in
-// one wave, and a block holds whole 64-column groups of h.  gate_lora and
-// up_lora are NULL or pass pair_lora_ok.
-dq8_status run_pair(dq8_ctx* ctx, const dq8::Weights& g, const dq8::Weights& u, const int8_t* q, const float* xs,
-                    size_t m, const float* gate_bias, const float* up_bias, const dq8_lora* gate_lora,
-                    const dq8_lora* up_lora, float* h, const QOut* qout, hipStream_t s) {
-  (void)ctx;
+// One layer's gate and up projections (same shape, shared quantized input) in
+// one launch that stores h = silu(gate + bias + adapter) * (up + bias2 +
+// adapter2) into h [m][n] and, as qout asks, quantizes h (q [m][n], scales
+// [m][ceil(n/64)], the non-finite report): in the wide launch itself, whose
+// blocks hold whole 64-column groups of h, or behind the skinny one.  The
+// results equal the separate Write and SwiGlu launches and k_quantize bit for
+// bit: each output's arithmetic is unchanged, only its gate and up values meet
+// in one wave.  kind as pair_kind gives it.
+dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* q, const float* xs, size_t m,
+                    const float* gate_bias, const float* up_bias, const dq8_lora* gate_lora, const dq8_lora* up_lora,
+                    float* h, const QOut* qout, int kind, hipStream_t s) {
   dq8::Batch b;
-  b.count = 1;
+  b.count = 0;
   b.total_waves = 0;
   b.any_lora = gate_lora != nullptr || up_lora != nullptr;
   b.chain = nullptr;
   b.fallback = 0;
-  dq8::Proj& p = b.p[0];
-  fill_proj(p, g, q, g.k, xs, g.g, m, gate_bias, h, nullptr, DQ8_ROWS, DQ8_WRITE, gate_lora);
-  p.wt2 = u.values;
-  p.wst2 = u.scales;
-  p.bias2 = up_bias;
-  p.lmid2 = up_lora ? up_lora->mid : nullptr;
-  p.lb2 = up_lora ? up_lora->b : nullptr;
-  p.lora2 = up_lora != nullptr;
-  p.rank2 = up_lora ? (int)up_lora->rank : 0;
-  p.lscale2 = up_lora ? up_lora->scale : 0.0f;
-  if (qout) {
-    p.hq = qout->q;
-    p.hs = qout->scales;
-    p.hflag = qout->nonfinite;
-    p.hchain = qout->chain;
+  // skinny: row chunks of at most 32 (run_linear)
+  const size_t nch = kind == 0 ? 1 : (m + 31) / 32, rows = (m + nch - 1) / nch;
+  const long units = (long)nch * ((g.n + 7) / 8);
+  for (size_t r0 = 0; r0 < m; r0 += rows) {
+    dq8::Proj& p = b.p[b.count++];
+    fill_proj(p, g, q + r0 * g.k, g.k, xs + r0 * g.g, g.g, std::min(rows, m - r0), gate_bias, h + r0 * g.n, nullptr,
+              DQ8_ROWS, DQ8_WRITE, gate_lora);
+    p.wt2 = u.values;
+    p.wst2 = u.scales;
+    p.bias2 = up_bias;
+    p.lmid2 = up_lora ? up_lora->mid : nullptr;
+    p.lb2 = up_lora ? up_lora->b : nullptr;
+    p.lora2 = up_lora != nullptr;
+    p.rank2 = up_lora ? (int)up_lora->rank : 0;
+    p.lscale2 = up_lora ? up_lora->scale : 0.0f;
+    if (p.lora) p.lmid += r0 * p.rank;
+    if (p.lora2) p.lmid2 += r0 * p.rank2;
+    if (qout && kind == 0) {
+      p.hq = qout->q;
+      p.hs = qout->scales;
+      p.hflag = qout->nonfinite;
+      p.hchain = qout->chain;
+    }
+    p.pair = 1;
+    place_proj(p, kind, b, units / 2 < kSkinnyFewStrips, units, g.g > 32);
   }
-  p.pair = 1;
-  place_proj(p, 0, b, false, 0, false);
-  return from_hip(dq8::launch_linear(b, 0, false, s));
+  hipError_t e = dq8::launch_linear(b, kind, false, s);
+  if (e == hipSuccess && qout && kind != 0)
+    e = dq8::launch_quantize(h, (int)m, g.n, qout->q, g.n, qout->scales, (int)groups_of(g.n), qout->nonfinite,
+                             qout->chain, s);
+  return from_hip(e);
 }
 
 // ------------------------------------------------------- fp32-input paths
@@ -1070,26 +1081,29 @@ dq8_status check_mid(const float* x, size_t m, size_t k, const float* a, size_t 
     return DQ8_ERR_SHAPE;  // the last bound keeps the grid under 2^32 work-items
   return DQ8_OK;
 }
-// Whether the gate and up projections of an FFN can run as one SwiGLU pair
-// launch: a wide-kernel build whose tile shape has the pair mode, the wide
-// kernel (more than 64 rows), inputs the kernel reads as they are.
-bool pair_ok(const dq8::Weights& g, const int8_t* q, const float* xs, size_t m) {
-  return dq8::wide_can_pair() && kind_of(g, m) == 0 && m > 64 && !needs_pad(g, q) && !needs_xs_pad(g, xs);
-}
-// Adapters the pair launch's epilogue takes: rank 0, or rank 16 with 16-byte
-// aligned mid and b (the rank of the reference's checkpoints); any other goes
-// to the separate gate and up launches.
-bool pair_lora_ok(const dq8_lora* l) {
-  return !l || l->rank == 0 ||
-         (l->rank == 16 && ((uintptr_t)l->mid & 15) == 0 && ((uintptr_t)l->b & 15) == 0);
+// Kernel kind (launch_linear) of the gate and up projections of an FFN as one
+// SwiGLU pair launch, or -1 if they run as two: inputs the kernels read as they
+// are; above 64 rows the wide kernel, in a build whose tile shape has the pair
+// mode, with adapters of rank 0 or of rank 16 with 16-byte aligned mid and b
+// (the rank of the reference's checkpoints); up to 64 rows the skinny kernels,
+// with no adapter or two of one rank.
+int pair_kind(const dq8::Weights& g, const int8_t* q, const float* xs, size_t m, const dq8_lora* a, const dq8_lora* b) {
+  if (needs_pad(g, q) || needs_xs_pad(g, xs)) return -1;
+  if (m <= 64) return !a == !b && (!a || a->rank == b->rank) ? (m > 16 ? 2 : 1) : -1;
+  auto lora_ok = [](const dq8_lora* l) {
+    return !l || l->rank == 0 ||
+           (l->rank == 16 && ((uintptr_t)l->mid & 15) == 0 && ((uintptr_t)l->b & 15) == 0);
+  };
+  return dq8::wide_can_pair() && lora_ok(a) && lora_ok(b) ? 0 : -1;
 }
 
-// gate Write into h, then up SwiGlu into h; one launch when pair_ok.
+// gate Write into h, then up SwiGlu into h; one launch where pair_kind has one.
 dq8_status gate_up(dq8_ctx* ctx, const dq8_weights* gate, const dq8_weights* up, const int8_t* q, const float* xs,
                    size_t m, const float* gate_bias, const float* up_bias, const dq8_lora* gate_lora,
                    const dq8_lora* up_lora, float* h, const QOut* qout, hipStream_t s) {
-  if (pair_ok(gate->w, q, xs, m) && pair_lora_ok(gate_lora) && pair_lora_ok(up_lora))
-    return run_pair(ctx, gate->w, up->w, q, xs, m, gate_bias, up_bias, gate_lora, up_lora, h, qout, s);
+  const int kind = pair_kind(gate->w, q, xs, m, gate_lora, up_lora);
+  if (kind >= 0)
+    return run_pair(gate->w, up->w, q, xs, m, gate_bias, up_bias, gate_lora, up_lora, h, qout, kind, s);
   dq8_linear_item gi = {gate, q, xs, m, gate_bias, h, DQ8_ROWS, DQ8_WRITE, gate_lora};
   dq8_status st = run_linear(ctx, &gi, 1, nullptr, s);
   if (st != DQ8_OK) return st;

@@ -85,10 +85,10 @@ struct Proj {
   int xcd_rm, xcd_rn, xcd_gn_shift;
   Divider d_cols, d_band, d_chunk, d_sr;
   int nseg;           // skinny: waves per strip (1 or 4)
-  // Fused SwiGLU pair (wide kernel only): wt/wst/bias are the gate weights,
+  // Fused SwiGLU pair: wt/wst/bias are the gate weights,
   // wt2/wst2/bias2 the up weights of the same shape; the launch stores
   // h = silu(gate(x) + bias) * (up(x) + bias2) into out [M][N].  With hq
-  // set it also quantizes h as k_quantize does: hq [M][N] int8, hs [M][G_h]
+  // set (wide kernel only) it also quantizes h as k_quantize does: hq [M][N] int8, hs [M][G_h]
   // scales (G_h = ceil(N / 64)); if h is not finite, 1 is ORed into *hflag
   // (when set) and *hchain (when set) is marked.
   const uint8_t* wt2;

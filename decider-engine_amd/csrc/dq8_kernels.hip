@@ -1724,14 +1724,21 @@ __device__ __forceinline__ void issue_x_chunk(const Proj& P, int c, int wid, uin
 // (tensor.rs:438, 109-117) when the projection has an adapter, stored by the
 // epilogue.  LoRA products: K=1 MFMA with A lane a = mid of row 4*(a/16) + a%4
 // and B lane l = b of column l%16, the x/w scale convention of the group loop.
+// In a SwiGLU pair each lane takes the bias and adapter of its projection (the
+// host pairs adapters of one rank only; a block of 4 lanes, which forms its own
+// products, never mixes the two), then the gate lanes store h = silu(gate) * up
+// (tensor.rs:96-99, qwen.rs:489-490) with up from 8 lanes on.
 template <int RT, int CT, bool LORA>
 __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4f (&s)[RT * CT], int r0 = 0) {
   constexpr int E = 4 * RT * CT;
   const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  const bool up = P.pair && (lane & 8);
+  auto col_of = [&](int ct) { return P.pair ? ((c0 + 16 * ct) >> 1) + (lane & 7) : c0 + 16 * ct + (lane & 15); };
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
-    const int col = c0 + 16 * ct + (lane & 15);
-    const float bias = P.bias != nullptr && col < P.n ? P.bias[col] : 0.0f;
+    const int col = col_of(ct);
+    const float* bp = up ? P.bias2 : P.bias;
+    const float bias = bp != nullptr && col < P.n ? bp[col] : 0.0f;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) s[rt * CT + ct] = s[rt * CT + ct] + bias;
   }
@@ -1740,14 +1747,16 @@ __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4
     const float* lbc[CT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
-      lm[rt] = P.lmid + (size_t)min(r0 + 16 * rt + 4 * (lane >> 4) + (lane & 3), P.m - 1) * P.rank;
+      lm[rt] = (up ? P.lmid2 : P.lmid) + (size_t)min(r0 + 16 * rt + 4 * (lane >> 4) + (lane & 3), P.m - 1) * P.rank;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) lbc[ct] = P.lb + (size_t)min(c0 + 16 * ct + (lane & 15), P.n - 1) * P.rank;
+    for (int ct = 0; ct < CT; ++ct) lbc[ct] = (up ? P.lb2 : P.lb) + (size_t)min(col_of(ct), P.n - 1) * P.rank;
+    const float lscale = up ? P.lscale2 : P.lscale;
     if (P.rank <= 16) {
       // every operand of the strip loaded up front (one memory latency), as
       // 16-byte loads when rank is 16 and the rows are 16-byte aligned
       float am[RT][16], bm[CT][16];
-      if (P.rank == 16 && ((size_t)P.lmid & 15) == 0 && ((size_t)P.lb & 15) == 0) {
+      if (P.rank == 16 && ((size_t)P.lmid & 15) == 0 && ((size_t)P.lb & 15) == 0 &&
+          (!P.pair || (((size_t)P.lmid2 & 15) == 0 && ((size_t)P.lb2 & 15) == 0))) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -1776,16 +1785,33 @@ __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
-          s[rt * CT + ct] = lora_term16(s[rt * CT + ct], zero4, P.rank, P.lscale,
+          s[rt * CT + ct] = lora_term16(s[rt * CT + ct], zero4, P.rank, lscale,
                                         [&](int i) { return mfma_k1_4(am[rt][i], bm[ct][i], zero4); });
     } else {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
-          s[rt * CT + ct] = lora_term(s[rt * CT + ct], zero4, P.rank, P.lscale,
+          s[rt * CT + ct] = lora_term(s[rt * CT + ct], zero4, P.rank, lscale,
                                       [&](int i) { return mfma_k1_4(lm[rt][i], lbc[ct][i], zero4); });
     }
+  }
+  if (P.pair) {
+    const ExpTab T = exp_table(lane);
+#pragma unroll
+    for (int k = 0; k < RT * CT; ++k) {
+      const int ct = k % CT, rt = k / CT, col = col_of(ct);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float y = s[k][v];
+        const float yu = __builtin_bit_cast(float, dpp<0x128>(__builtin_bit_cast(uint32_t, y)));  // lane l + 8 of 16
+        const float h = silu_wave(y, T) * yu;
+        const int row = r0 + 16 * rt + 4 * (lane >> 4) + v;
+        if (!up && row < P.m && col < P.n) st_out(P.out + (size_t)row * P.n + col, h);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the f64 temporaries of 4 values at a time
+    }
+    return;
   }
   int rows[E], cols[E];
   float y[E];
@@ -1801,6 +1827,25 @@ __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4
         y[e] = s[rt * CT + ct][v];
       }
   store_tile(P, rows, cols, y);
+}
+
+// This lane's first weight fragment bytes and w scale of a tile's column: tile
+// column l%16 is output column c0 + l%16, or, in a SwiGLU pair, column
+// c0/2 + l%8 of the gate (l%16 < 8) or the up projection.  A pair's tile thus
+// reads 128-byte runs of both projections' fragments, and the gate and up
+// values of one output sit 8 lanes apart.
+template <bool DOTS>
+__device__ __forceinline__ void skinny_weights(const Proj& P, int c0, int lane, const uint8_t*& pb, const float*& pw) {
+  int col = c0 + (lane & 15);
+  const uint8_t* wt = P.wt;
+  const float* wst = P.wst;
+  if (!DOTS && P.pair) {  // uniform
+    col = (c0 >> 1) + (lane & 7);
+    wt = lane & 8 ? P.wt2 : wt;
+    wst = lane & 8 ? P.wst2 : wst;
+  }
+  pb = wt + ((size_t)(col >> 5) * P.g * 2 + (lane >> 5)) * kFragBytes + ((col & 31) + 32 * ((lane >> 4) & 1)) * 16;
+  pw = wst + col;
 }
 
 // One group of a wave's tiles: dots (exported when DOTS) or t = dot * p.
@@ -1859,12 +1904,7 @@ __device__ __forceinline__ bool skinny_short(const Proj& P, int c0, bool live, i
   const uint8_t* pb[CT];
   const float* pw[CT];
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const int cc = c0 + 16 * ct;
-    pb[ct] = P.wt + ((size_t)(cc >> 5) * G * 2 + (lane >> 5)) * kFragBytes +
-             ((cc & 31) + (lane & 15) + 32 * ((lane >> 4) & 1)) * 16;
-    pw[ct] = P.wst + cc + (lane & 15);
-  }
+  for (int ct = 0; ct < CT; ++ct) skinny_weights<DOTS>(P, c0 + 16 * ct, lane, pb[ct], pw[ct]);
   v4i bq[DB][2][CT];
   float wq[DB][2][CT];
   auto issue = [&](v4i (&bs)[2][CT], float (&ws)[2][CT], int j) {
@@ -1995,12 +2035,7 @@ __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, i
   const uint8_t* pb[CT];
   const float* pw[CT];
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const int cc = c0 + 16 * ct;
-    pb[ct] = P.wt + ((size_t)(cc >> 5) * G * 2 + (lane >> 5)) * kFragBytes +
-             ((cc & 31) + (lane & 15) + 32 * ((lane >> 4) & 1)) * 16;
-    pw[ct] = P.wst + cc + (lane & 15);
-  }
+  for (int ct = 0; ct < CT; ++ct) skinny_weights<DOTS>(P, c0 + 16 * ct, lane, pb[ct], pw[ct]);
   v4i aq[DB][RT], bq[DB][CT];
   float wq[DB][CT];
   auto issue = [&](v4i (&as)[RT], v4i (&bs)[CT], float (&ws)[CT], int j) {

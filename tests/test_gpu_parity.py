@@ -929,8 +929,8 @@ def test_ffn_chain_matches_the_reference_sequence(ctx, m, hidden, inter, lora):
 def test_ffn_gate_up_equals_write_then_swiglu(ctx, m, hidden, inter):
     # dq8_ffn_gate_up stores what the crate's gate Write and up SwiGlu apply
     # calls store (qwen.rs:489-490): the same bits as two dq8_linear calls and as
-    # the oracle, with and without biases; more than 64 rows take the one-launch
-    # pair path, fewer the two launches.  With quantize=True, h is also
+    # the oracle, with and without biases; more than 64 rows take the wide pair
+    # launch, fewer the skinny one.  With quantize=True, h is also
     # quantized (qwen.rs:491): the same bytes and scales as dq8_quantize(h) and
     # as the oracle's QuantizedInputs::new(h), for widths that end in a partial
     # group and widths that are not a multiple of 16 (byte stores).
@@ -1188,6 +1188,22 @@ def test_ffn_gate_up_with_adapters(ctx, m, hidden, inter, gl, ul):
     assert bits_equal(host(hf), want_h)
     oq, os_ = dq8o.quantize_inputs(want_h, threads=8)
     assert np.array_equal(host(hq), oq) and bits_equal(host(hs), os_)
+
+
+# The skinny pair launch (up to 64 rows), whose 16-column tiles hold 8 gate and
+# 8 up columns: one and two row tiles and chunks, widths that end inside a unit,
+# the one-wave path (160 or more strips) and the 4-wave paths for few strips and
+# for long K, adapters of one rank, and the two-launch form they exclude.
+SKINNY_PAIR_CASES = [(1, 256, 5, None, None), (16, 256, 264, (16, "aligned"), (16, "aligned")),
+                     (17, 2304, 72, (16, "aligned"), (16, "offset")), (24, 512, 2571, None, None),
+                     (24, 256, 2560, (16, "aligned"), (16, "aligned")), (33, 256, 100, (13, "aligned"), (13, "aligned")),
+                     (48, 2304, 260, None, None), (64, 256, 1300, (20, "aligned"), (20, "aligned")),
+                     (20, 256, 96, (0, "aligned"), (0, "aligned")), (12, 512, 2600, (16, "aligned"), None)]
+
+
+@pytest.mark.parametrize("m,hidden,inter,gl,ul", SKINNY_PAIR_CASES)
+def test_skinny_ffn_gate_up(ctx, m, hidden, inter, gl, ul):
+    test_ffn_gate_up_with_adapters(ctx, m, hidden, inter, gl, ul)
 
 
 # 65-512 rows whose wide launch would be small run as 32-row chunks on the
