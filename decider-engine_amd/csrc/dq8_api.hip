@@ -231,15 +231,12 @@ void fill_proj(dq8::Proj& p, const dq8::Weights& w, const int8_t* q, int ldq, co
   p.hq = nullptr;
   p.hs = nullptr;
   p.hflag = nullptr;
-  p.hchain = nullptr;
   p.pair = 0;
   p.lmid2 = nullptr;
   p.lb2 = nullptr;
   p.lora2 = 0;
   p.rank2 = 0;
   p.lscale2 = 0.0f;
-  p.fx = nullptr;
-  p.fk = 0;
 }
 
 // Wide kernel: split the tile grid into gm x gn regions, gm * gn = 8, one per
@@ -580,8 +577,8 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
         b.any_lora = 1;
       }
       if (fb) {
-        p.fx = fb->x + r0 * w.k;
-        p.fk = w.k;
+        b.fx[b.count - 1] = fb->x + r0 * w.k;
+        b.fk = w.k;
         b.fallback = kind != 0;  // the skinny kernels hold the FP32 path themselves
       }
       place_proj(p, kind, b, strips[kind] < kSkinnyFewStrips, units[kind], has_long[kind]);
@@ -622,7 +619,7 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
   b.count = 0;
   b.total_waves = 0;
   b.any_lora = gate_lora != nullptr || up_lora != nullptr;
-  b.chain = nullptr;
+  b.chain = b.hchain = nullptr;
   b.fallback = 0;
   // skinny: row chunks of at most 32 (run_linear)
   const size_t nch = kind == 0 ? 1 : (m + 31) / 32, rows = (m + nch - 1) / nch;
@@ -645,7 +642,7 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
       p.hq = qout->q;
       p.hs = qout->scales;
       p.hflag = qout->nonfinite;
-      p.hchain = qout->chain;
+      b.hchain = qout->chain;
     }
     p.pair = 1;
     place_proj(p, kind, b, units / 2 < kSkinnyFewStrips, units, g.g > 32);
@@ -746,8 +743,8 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
               out + r0 * w.n, nullptr, layout, epilogue, lora);
     if (p.lora) p.lmid += r0 * p.rank;
     if (fb) {
-      p.fx = fb->x + r0 * w.k;
-      p.fk = w.k;
+      b.fx[b.count - 1] = fb->x + r0 * w.k;
+      b.fk = w.k;
     }
     place_proj(p, kind, b, (long)nch * short_strips(w) < kSkinnyFewStrips, (long)nch * short_units(w), w.g > 32);
   }

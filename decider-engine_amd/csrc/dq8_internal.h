@@ -90,14 +90,13 @@ struct Proj {
   // h = silu(gate(x) + bias) * (up(x) + bias2) into out [M][N].  With hq
   // set (wide kernel only) it also quantizes h as k_quantize does: hq [M][N] int8, hs [M][G_h]
   // scales (G_h = ceil(N / 64)); if h is not finite, 1 is ORed into *hflag
-  // (when set) and *hchain (when set) is marked.
+  // (when set) and Batch::hchain (when set) is marked.
   const uint8_t* wt2;
   const float* wst2;
   const float* bias2;
   int8_t* hq;
   float* hs;
   uint32_t* hflag;
-  Chain* hchain;
   int pair;
   // The up projection's LoRA adapter in a pair launch (lmid/lb/rank/lscale of
   // the fields above are the gate's).
@@ -106,9 +105,6 @@ struct Proj {
   int lora2;
   int rank2;
   float lscale2;
-  // FP32 inputs [M][fk] of the projection (launches with Batch::fallback).
-  const float* fx;
-  int fk;
 };
 
 struct Batch {
@@ -123,6 +119,9 @@ struct Batch {
   // launch does nothing and k_linear_fp32 computes these outputs instead.
   Chain* chain;
   int fallback;
+  int fk;                       // with fallback: fx[i] [M][fk], the FP32 inputs of p[i]
+  const float* fx[kMaxBatch];
+  Chain* hchain;                // with Proj::hq: marked if h is not finite
 };
 
 // LoRA middle products of several (x, A) pairs in one launch of the few-rows

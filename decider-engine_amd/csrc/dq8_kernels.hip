@@ -1452,7 +1452,8 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
           }
           if ((t & 3) == 0) P.hs[(size_t)row * ((P.n + kGroup - 1) / kGroup) + nt] = scale;
         }
-        report_nonfinite(bad && row < P.m, P.hflag, P.hchain);
+        report_nonfinite(bad && row < P.m, P.hflag, b.hchain);
+        if (b.hchain) chain_open(b.hchain);  // (the launch holds this one pair; at its start this would delay the first loads)
       }
       return;
     }
@@ -1638,9 +1639,6 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
     __syncthreads();
   }
 #else
-  // (a batch that quantizes h holds the one pair)
-  if constexpr (!DOTS && wide_pair_shape(WN, RT, CT))
-    if (b.p[0].hq != nullptr && b.p[0].hchain != nullptr) chain_open(b.p[0].hchain);
   run_tile(blockIdx.x);
 #endif
 }
@@ -2285,8 +2283,8 @@ __global__ __launch_bounds__(256) void k_linear_fp32(FProj P) {
 }
 // The FP32 path of a skinny block's outputs: rows [m0, mhi) (at most 16*RPT), columns [nlo, nhi).
 template <int RPT>
-__device__ __forceinline__ void fp32_block(const Proj& S, int m0, int mhi, int nlo, int nhi, uint8_t* lds) {
-  const FProj P = {S.fx, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, S.fk, S.g, S.n, S.np,
+__device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k, int m0, int mhi, int nlo, int nhi, uint8_t* lds) {
+  const FProj P = {x, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, k, S.g, S.n, S.np,
                    S.epilogue, S.layout, nullptr};
   __syncthreads();  // every wave's loads into this LDS have landed
   for (int n0 = nlo / kF32Cols * kF32Cols; n0 < nhi; n0 += kF32Cols)
@@ -2357,7 +2355,7 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   if constexpr (!DOTS) {
     if (b.fallback) {  // uniform over the launch
       chain_close(b.chain);
-      if (skip) fp32_block<RT>(P, m0, mhi, nlo, min(nhi, P.n), lds);
+      if (skip) fp32_block<RT>(P, b.fx[pidx], b.fk, m0, mhi, nlo, min(nhi, P.n), lds);
     }
   }
 }
