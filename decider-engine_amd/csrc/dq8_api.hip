@@ -268,12 +268,12 @@ int xcd_rows_split(int row_tiles, int col_tiles, size_t a_bytes, size_t b_bytes)
 // once; pick the sr (a divisor of the region's row tiles) whose chunk touches
 // the fewest operand bytes: sr row tiles of activations plus sc column tiles
 // of weights (a column tile of a SwiGLU pair holds both projections' rows).
-void xcd_chunks(dq8::Proj& p, int row_tiles) {
+void xcd_chunks(dq8::Proj& p, int kind, int row_tiles) {
   p.xcd_sr = 1;
   p.xcd_sc = 1;
   if (p.xcd_gm == 0) return;
   const int rm = row_tiles / p.xcd_gm, rn = p.waves_n / (8 / p.xcd_gm);
-  const double a_tile = (double)dq8::wide_block_rows(), b_tile = (double)dq8::wide_block_cols();
+  const double a_tile = dq8::block_rows(kind, p.pair), b_tile = (p.pair ? 2 : 1) * dq8::block_cols(kind, p.pair);
   double best = -1.0;
   for (int sr = 1; sr <= rm; ++sr) {
     if (rm % sr) continue;
@@ -317,49 +317,69 @@ int units_per_block(long units, bool /*has_long*/) {
   return (int)std::min((long)DQ8_SKINNY_UNITS_MAX, std::max(2L, (units + 255) / 256));
 }
 
-// Row chunks for the skinny kernel.  Up to 64 rows (rows layout) always run as
-// chunks of at most 32 rows on the skinny kernel.  65-512 rows do when the
-// call's wide launch would be small: at most kSplitWideBlocks blocks (under one
-// block per CU, so every block would run alone on its CU and wait out each
-// group's dependency chain), at most kSplitBytes of weights read by all the
-// chunks (the first read comes from HBM, the rest mostly from cache), and no
-// projection's weights above kSplitWeightBytes (larger ones are re-read from
-// the MALL rather than L2).  Rows are independent, so the results are the same
-// bits either way.  Measured (graph-replayed launches, wide -> chunks):
-// 128 x 2048 -> 2048 17.5 -> 10.2 us, 128 x 2048 -> 6144 18.1 -> 10.9 us,
-// 192 x 2048 -> 6144 18.4 -> 14.7 us, 192 x 6144 -> 2048 Add 48.1 -> 38.1 us,
-// 512 x 2048 -> 2048 18.3 -> 12.6 us.  The chunks lost for 128 x 2048 -> 8224
-// (18.7 -> 20.1 us), 256 x 6144 -> 2048 Add (48.3 -> 50.3 us) and 384 x 2048
-// -> 6144 (23.6 -> 24.1 us).
-constexpr long kSplitWideBlocks = 192;
-constexpr double kSplitBytes = 96e6;
-constexpr double kSplitWeightBytes = 16e6;
+// How a call's items of more than 32 rows run (measured graph-replayed, 24
+// launches over rotating weights):
+//  * small: items of at most 512 rows (rows layout) as chunks of at most 32
+//    rows on the skinny kernel, if all the call's chunks together read at most
+//    chunk_bytes of weights (the first read comes from HBM, the rest mostly
+//    from cache).  Against the mid kernel: 128 x 2048 -> 2048 7.8 and 9.6 us,
+//    256 x 2048 -> 2048 (36 MB) 8.1 and 9.9, 64 x 2048 -> 6144 (27 MB) 7.9 and
+//    9.9, 96 x 6144 -> 2048 (40 MB) 18.9 and 20.9; beyond the limit 96 x 2048 ->
+//    6144 (40 MB) 11.2 and 10.3, 256 x 6144 -> 1024 (53 MB) 22.0 and 21.1, 64 x
+//    6144 -> 8224 (107 MB) 45 and 21.5, 512 x 512 -> 2048 (18 MB) 8.1 and 5.7.
+//    A chunk's time is its bytes, the mid kernel's its K.
+//  * mid: the others on the mid kernel if the wide grid would leave its blocks
+//    alone on their CUs: at most kMidBlocks blocks (64 x 128; one round of the
+//    mid kernel's 64 x 64 blocks, two per CU).  Against the wide kernel: 512 x
+//    6144 -> 2048 (128 blocks) 22.3 and 39.0 us, 1000 x 2048 -> 2048 (256) 14.4
+//    and 16.3; beyond it 400 x 2048 -> 6144 (336) 20.2 and 19.9, 2048 x 2048 ->
+//    2048 (512) 25.0 and 21.1.  In a call that mixes long and short K the wide
+//    kernel's long blocks trail, up to kMidMixedBlocks: a layer set of 9
+//    projections at 77 rows (466) 29.5 and 42.3 us, 192 (699) 42.6 and 49.4;
+//    384 (1404) 77.9 and 66.6.
+//  * the wide kernel otherwise.
+// Rows are independent, so the results are the same bits either way.
+constexpr long kMidBlocks = 256, kMidMixedBlocks = 768;
+double chunk_bytes(size_t k) { return std::min(17.5e3 * (double)k, 45e6); }
 double weight_bytes(const dq8::Weights& w) { return (double)w.n * w.k + 4.0 * w.n * w.g; }
 bool may_split(const dq8::Weights& w, size_t m, int layout) {
-  return kind_of(w, m) == 0 && layout == DQ8_ROWS && (m <= 64 || (m <= 512 && weight_bytes(w) <= kSplitWeightBytes));
+  return kind_of(w, m) == 0 && layout == DQ8_ROWS && m <= 512;
 }
 long wide_blocks(const dq8::Weights& w, size_t m) {
-  return (long)((m + dq8::wide_block_rows() - 1) / dq8::wide_block_rows()) * (w.np / dq8::wide_block_cols());
+  return (long)((m + dq8::block_rows(0, false) - 1) / dq8::block_rows(0, false)) * (w.np / dq8::block_cols(0, false));
 }
-size_t row_chunks(const dq8::Weights& w, size_t m, int layout, bool small_call) {
-  if (!may_split(w, m, layout) || (m > 64 && !small_call)) return 1;
-  return (m + 31) / 32;
+size_t row_chunks(const dq8::Weights& w, size_t m, int layout, bool small) {
+  return may_split(w, m, layout) && small ? (m + 31) / 32 : 1;
 }
-// Whether a call's 65-512-row items run as skinny row chunks (see row_chunks).
+struct CallPlan {
+  bool small, mid;
+};
 template <class Item, class W>
-bool small_call(const Item* items, size_t count, W weights_of) {
-  long blocks = 0;
+CallPlan call_plan(const Item* items, size_t count, W weights_of) {
+  long blocks = 0, fixed = 0;  // wide blocks of the items that may run as chunks, and of the others
   double bytes = 0;
+  size_t longest = 0;
+  bool has_long = false, has_short = false;
   for (size_t i = 0; i < count; ++i) {
     const dq8::Weights& w = weights_of(items[i]);
     const size_t m = items[i].m;
     if (m == 0 || kind_of(w, m) != 0) continue;
     const bool can = may_split(w, m, items[i].layout);
-    if (can && m <= 64) continue;  // split whatever the call
-    blocks += wide_blocks(w, m);
-    if (can) bytes += (double)((m + 31) / 32) * weight_bytes(w);
+    (can ? blocks : fixed) += wide_blocks(w, m);
+    if (can) {
+      bytes += (double)((m + 31) / 32) * weight_bytes(w);
+      longest = std::max(longest, (size_t)w.k);
+    }
+    (w.g > 32 ? has_long : has_short) = true;
   }
-  return blocks <= kSplitWideBlocks && bytes <= kSplitBytes;
+  const bool small = bytes <= chunk_bytes(longest);
+  const long left = fixed + (small ? 0 : blocks);
+  return {small, left <= (has_long && has_short ? kMidMixedBlocks : kMidBlocks)};
+}
+// Kernel kind of an item in nch row chunks.
+int item_kind(const dq8::Weights& w, size_t m, size_t nch, const CallPlan& plan) {
+  const int kind = nch > 1 ? 2 : kind_of(w, m);
+  return kind == 0 && plan.mid ? 3 : kind;
 }
 
 // Place a filled projection in a launch of the given kernel kind: its first
@@ -369,13 +389,12 @@ void place_proj(dq8::Proj& p, int kind, dq8::Batch& b, bool few_strips, long lau
   b.wave_begin[&p - b.p] = p.wave_begin;
   p.xcd_gm = 0;
   p.nseg = 1;
-  if (kind == 0) {
-    // a SwiGLU pair's block covers half as many outputs of each projection
-    p.waves_n = p.pair ? (p.n + dq8::wide_block_cols() / 2 - 1) / (dq8::wide_block_cols() / 2)
-                       : p.np / dq8::wide_block_cols();
-    const int row_tiles = (p.m + dq8::wide_block_rows() - 1) / dq8::wide_block_rows();
+  if (kind == 0 || kind == 3) {
+    const int cols = dq8::block_cols(kind, p.pair), rows = dq8::block_rows(kind, p.pair);
+    p.waves_n = p.pair || kind == 3 ? (p.n + cols - 1) / cols : p.np / cols;
+    const int row_tiles = (p.m + rows - 1) / rows;
     p.xcd_gm = xcd_rows_split(row_tiles, p.waves_n, (size_t)p.m * p.g, (size_t)(p.pair ? 2 : 1) * p.n * p.g);
-    xcd_chunks(p, row_tiles);
+    xcd_chunks(p, kind, row_tiles);
     p.d_cols = dq8::Divider::of((uint32_t)std::max(1, p.waves_n));
     if (p.xcd_gm) {
       const int gn = 8 / p.xcd_gm;
@@ -507,15 +526,16 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
     b.chain = fb ? fb->chain : nullptr;
     b.fallback = 0;
   }
-  const bool small = small_call(items, count, [](const dq8_linear_item& it) -> const dq8::Weights& { return it.w->w; });
+  CallPlan plan = call_plan(items, count, [](const dq8_linear_item& it) -> const dq8::Weights& { return it.w->w; });
+  if (dots) plan.mid = false;
   // one-wave strips each skinny launch would have (see kSkinnyFewStrips)
   long strips[dq8::kKinds] = {}, units[dq8::kKinds] = {};
   bool has_long[dq8::kKinds] = {};
   for (size_t i = 0; i < count; ++i) {
     const dq8_linear_item& it = items[i];
     if (it.m == 0) continue;
-    const size_t nch = row_chunks(it.w->w, it.m, it.layout, small);
-    const int kind = nch > 1 ? 2 : kind_of(it.w->w, it.m);
+    const size_t nch = row_chunks(it.w->w, it.m, it.layout, plan.small);
+    const int kind = item_kind(it.w->w, it.m, nch, plan);
     strips[kind] += (long)nch * short_strips(it.w->w);
     units[kind] += (long)nch * short_units(it.w->w);
     has_long[kind] = has_long[kind] || it.w->w.g > 32;
@@ -554,8 +574,8 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
     // once from HBM), which beats a wide launch of half-empty row tiles whose
     // long-K blocks trail (measured 44 against 52 us for 48 rows of a layer's
     // projection set).  Rows are independent, so the results are the same bits.
-    const size_t nch = row_chunks(w, it.m, it.layout, small);
-    const int kind = nch > 1 ? 2 : kind_of(w, it.m);
+    const size_t nch = row_chunks(w, it.m, it.layout, plan.small);
+    const int kind = item_kind(w, it.m, nch, plan);
     const size_t half = (it.m + nch - 1) / nch;
     for (size_t r0 = 0; r0 < it.m; r0 += half) {
       const size_t rows = std::min(half, it.m - r0);
@@ -579,7 +599,7 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
       if (fb) {
         b.fx[b.count - 1] = fb->x + r0 * w.k;
         b.fk = w.k;
-        b.fallback = kind != 0;  // the skinny kernels hold the FP32 path themselves
+        b.fallback = kind != 0;  // the other kernels hold the FP32 path themselves
       }
       place_proj(p, kind, b, strips[kind] < kSkinnyFewStrips, units[kind], has_long[kind]);
     }
@@ -607,8 +627,8 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
 // One layer's gate and up projections (same shape, shared quantized input) in
 // one launch that stores h = silu(gate + bias + adapter) * (up + bias2 +
 // adapter2) into h [m][n] and, as qout asks, quantizes h (q [m][n], scales
-// [m][ceil(n/64)], the non-finite report): in the wide launch itself, whose
-// blocks hold whole 64-column groups of h, or behind the skinny one.  The
+// [m][ceil(n/64)], the non-finite report): in the wide or mid launch itself,
+// whose blocks hold whole 64-column groups of h, or behind the skinny one.  The
 // results equal the separate Write and SwiGlu launches and k_quantize bit for
 // bit: each output's arithmetic is unchanged, only its gate and up values meet
 // in one wave.  kind as pair_kind gives it.
@@ -622,7 +642,7 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
   b.chain = b.hchain = nullptr;
   b.fallback = 0;
   // skinny: row chunks of at most 32 (run_linear)
-  const size_t nch = kind == 0 ? 1 : (m + 31) / 32, rows = (m + nch - 1) / nch;
+  const size_t nch = kind == 0 || kind == 3 ? 1 : (m + 31) / 32, rows = (m + nch - 1) / nch;
   const long units = (long)nch * ((g.n + 7) / 8);
   for (size_t r0 = 0; r0 < m; r0 += rows) {
     dq8::Proj& p = b.p[b.count++];
@@ -638,7 +658,7 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
     p.lscale2 = up_lora ? up_lora->scale : 0.0f;
     if (p.lora) p.lmid += r0 * p.rank;
     if (p.lora2) p.lmid2 += r0 * p.rank2;
-    if (qout && kind == 0) {
+    if (qout && nch == 1 && (kind == 0 || kind == 3)) {
       p.hq = qout->q;
       p.hs = qout->scales;
       p.hflag = qout->nonfinite;
@@ -648,7 +668,7 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
     place_proj(p, kind, b, units / 2 < kSkinnyFewStrips, units, g.g > 32);
   }
   hipError_t e = dq8::launch_linear(b, kind, false, s);
-  if (e == hipSuccess && qout && kind != 0)
+  if (e == hipSuccess && qout && (kind == 1 || kind == 2))
     e = dq8::launch_quantize(h, (int)m, g.n, qout->q, g.n, qout->scales, (int)groups_of(g.n), qout->nonfinite,
                              qout->chain, s);
   return from_hip(e);
@@ -730,9 +750,10 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
     size_t m;
     int layout;
   } one = {m, layout};
-  const size_t nch = row_chunks(w, m, layout, small_call(&one, 1, [&](const One&) -> const dq8::Weights& { return w; }));
+  const CallPlan plan = call_plan(&one, 1, [&](const One&) -> const dq8::Weights& { return w; });
+  const size_t nch = row_chunks(w, m, layout, plan.small);
   static_assert(dq8::kMaxBatch >= 16, "512 rows in chunks of 32");
-  const int kind = nch > 1 ? 2 : kind_of(w, m);
+  const int kind = item_kind(w, m, nch, plan);
   const size_t half = (m + nch - 1) / nch;
   b.count = 0;
   b.chain = fb ? fb->chain : nullptr;
@@ -749,7 +770,7 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
     place_proj(p, kind, b, (long)nch * short_strips(w) < kSkinnyFewStrips, (long)nch * short_units(w), w.g > 32);
   }
   hipError_t e = dq8::launch_linear(b, kind, false, s);
-  if (e == hipSuccess && fb && kind == 0)
+  if (e == hipSuccess && fb && !b.fallback)
     e = dq8::launch_linear_fp32(make_fproj(w, fb->x, m, bias, lora, out, layout, epilogue, fb->chain), s);
   return from_hip(e);
 }
@@ -1080,13 +1101,26 @@ dq8_status check_mid(const float* x, size_t m, size_t k, const float* a, size_t 
 }
 // Kernel kind (launch_linear) of the gate and up projections of an FFN as one
 // SwiGLU pair launch, or -1 if they run as two: inputs the kernels read as they
-// are; above 64 rows the wide kernel, in a build whose tile shape has the pair
-// mode, with adapters of rank 0 or of rank 16 with 16-byte aligned mid and b
-// (the rank of the reference's checkpoints); up to 64 rows the skinny kernels,
-// with no adapter or two of one rank.
+// are, and
+//  * the skinny kernels up to 32 rows, and as row chunks by call_plan's rule for
+//    both weights (with h's quantization behind them, which the others hold: 64
+//    x 2048 -> 2 x 6144, 53 MB, 15.8 us against 12.4), with no adapter or two of
+//    one rank;
+//  * the mid kernel up to 512 blocks of its own (32 x 64 outputs; one round),
+//    any adapters: 128 x 2048 -> 2 x 6144 (384 of them) 16.2 us against 18.5 on
+//    the wide kernel, 150 rows (480) 16.3 and 22.8, 192 rows (576) 24.1 and 22.8;
+//  * the wide kernel, in a build whose tile shape has the pair mode, with
+//    adapters of rank 0 or of rank 16 with 16-byte aligned mid and b (the rank
+//    of the reference's checkpoints).
+constexpr long kMidPairBlocks = 512;
 int pair_kind(const dq8::Weights& g, const int8_t* q, const float* xs, size_t m, const dq8_lora* a, const dq8_lora* b) {
   if (needs_pad(g, q) || needs_xs_pad(g, xs)) return -1;
-  if (m <= 64) return !a == !b && (!a || a->rank == b->rank) ? (m > 16 ? 2 : 1) : -1;
+  const bool skinny = m <= 32 || (m <= 512 && 2.0 * (double)((m + 31) / 32) * weight_bytes(g) <= chunk_bytes(g.k));
+  if (skinny && !a == !b && (!a || a->rank == b->rank)) return m > 16 ? 2 : 1;
+  if (m <= 32) return -1;
+  const long tiles = (long)((m + dq8::block_rows(3, true) - 1) / dq8::block_rows(3, true)) *
+                     ((g.n + dq8::block_cols(3, true) - 1) / dq8::block_cols(3, true));
+  if (tiles <= kMidPairBlocks) return 3;
   auto lora_ok = [](const dq8_lora* l) {
     return !l || l->rank == 0 ||
            (l->rank == 16 && ((uintptr_t)l->mid & 15) == 0 && ((uintptr_t)l->b & 15) == 0);

@@ -181,9 +181,9 @@ long lora_mid_small_blocks(int m, int rank);
 bool lora_mid_tiled_ok(const float* x, int k, const float* a);  // otherwise the LDS-tiled kernel, if this holds
 long lora_mid_tiled_blocks(int m, int rank);
 hipError_t launch_lora_mid_batch(const MidBatch& b, long blocks, bool tiled, hipStream_t s);
-// Kind: 0 wide (M > 32), 1 skinny (M <= 16), 2 skinny (16 < M <= 32).  dots
-// selects the debug kernel.
-constexpr int kKinds = 3;
+// Kind: 0 wide (M > 32), 1 skinny (M <= 16), 2 skinny (16 < M <= 32), 3 mid (M >
+// 32, few blocks).  dots selects the debug kernel (not for kind 3).
+constexpr int kKinds = 4;
 hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s);
 // Columns of a skinny strip for g groups (all rows), and the waves that share
 // a strip's groups (1 or 4).
@@ -191,9 +191,10 @@ hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s);
 // 4 (a strip's groups split over 4 waves; long K, or launches with few strips).
 int skinny_segments(int g, bool few_strips);
 int skinny_cols(int nseg);  // strip width of a path
-// Block tile of the wide kernel (rows, columns); kColPad is a multiple of the columns.
-int wide_block_rows();
-int wide_block_cols();
+// Rows and output columns of a block of the wide or mid kernel (kColPad is a
+// multiple of the columns); a SwiGLU pair's block holds both projections.
+int block_rows(int kind, bool pair);
+int block_cols(int kind, bool pair);
 // Whether this build's wide-kernel tile shape has the SwiGLU pair mode (the
 // kernel ignores Proj::pair otherwise).
 bool wide_can_pair();

@@ -422,7 +422,13 @@ __device__ __forceinline__ void load4(const float* p, float (&v)[4]) {
 }
 
 // Chain (dq8_internal.h): whether the call's inputs were not finite; its two ends.
-__device__ __forceinline__ bool chain_hit(const Chain* c) { return c->hit == c->cur + 1; }
+// (Read through the scalar cache: no launch writes the words that it reads, and
+// a vector load would wait for the direct loads issued before it.)
+__device__ __forceinline__ bool chain_hit(const Chain* c) {
+  typedef const __attribute__((address_space(4))) Chain* scalar_chain;
+  const scalar_chain sc = (scalar_chain)(uintptr_t)c;
+  return sc->hit == sc->cur + 1;
+}
 __device__ __forceinline__ void chain_open(Chain* c) {  // by the quantizer's first block
   if (blockIdx.x == 0 && threadIdx.x == 0) c->cur = c->next;
 }
@@ -1643,6 +1649,501 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
 #endif
 }
 
+// dot_scores (tensor.rs:6-25, the x86-64 order) of a[0..len) and b[0..len)
+// from plain memory: eight lane sums over the full chunks of 8, added in
+// order from -0.0, then the tail elements one by one; no fused multiply-add.
+__device__ __forceinline__ float dot_scores_rows(const float* a, const float* b, int len) {
+  const int chunks = len >> 3;
+  float lanes[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  for (int c = 0; c < chunks; ++c)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) lanes[q] = lanes[q] + a[8 * c + q] * b[8 * c + q];
+  float sum = -0.0f;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) sum = sum + lanes[q];
+  for (int t = 8 * chunks; t < len; ++t) sum = sum + a[t] * b[t];
+  return sum;
+}
+
+// Weight element (n, t) of the repacked layout, dequantized as Data::row does
+// for 8-bit Quantized data (weights.rs:47-78): (float)(int8)q * scale.
+__device__ __forceinline__ float dequant(const FProj& P, int n, int t) {
+  const int g = t >> 6, off = t & 63, h = off >> 5, part = (off >> 4) & 1;
+  const int8_t q = (int8_t)P.wt[((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16 +
+                                (off & 15)];
+  return (float)q * P.wst[(size_t)g * P.np + n];
+}
+
+// The FP32 path of a projection, Projection::columns_tiled (tensor.rs:206-269),
+// which the crate takes when the inputs are not finite (tensor.rs:197-201):
+//   y = dot_scores(x_r, w_n) + (bias[n] or 0.0)     w_n dequantized (dequant)
+//   y = y + scale * (dot_scores(mid_r, B_n) + 0.0)   with an adapter (Adapter::combine)
+// stored through the epilogue.  The dot products run in dot_scores' order, so
+// NaN and infinity propagate as in the crate.  fp32_tile: a block of 256
+// threads computes 16*RPT rows x 64 columns from (m0, n0) and stores those in rows
+// [m0, mhi) x columns [nlo, nhi); for RPT = 2 thread (tr, tc) owns rows 2tr, 2tr+1 and columns tc + 16j (j < 4)
+// with eight lane sums each.  Per group of 64 inputs the block stages x and
+// the dequantized weights in LDS (rows padded to 68 floats: the 16 columns a
+// wave reads per step fall in distinct banks).
+constexpr int kF32Rows = 32, kF32Cols = 64, kF32Pad = 68;
+struct F32Lds {
+  float xs[kF32Rows][kF32Pad], ws[kF32Cols][kF32Pad];
+};
+template <int RPT>
+__device__ __forceinline__ void fp32_tile(const FProj& P, int m0, int n0, int mhi, int nlo, int nhi, F32Lds& L) {
+  auto &xs = L.xs;
+  auto &ws = L.ws;
+  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
+  const int chunks = P.k >> 3;  // full chunks of 8 go to the lane sums
+  float acc[RPT][4][8];
+#pragma unroll
+  for (int i = 0; i < RPT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[i][j][q] = 0.0f;
+  for (int g = 0; 8 * g < chunks; ++g) {
+    const int nfull = min(8, chunks - 8 * g);  // uniform over the block
+    __syncthreads();                           // the previous group's reads are done
+    {
+      // x: thread t stages 4*RPT inputs of one row (zero past m or k)
+      constexpr int SEG = 4 * RPT, SPR = kGroup / SEG;
+      const int r = tid / SPR, seg = tid % SPR, row = m0 + r, kk = 64 * g + SEG * seg;
+#pragma unroll
+      for (int u = 0; u < SEG; ++u)
+        xs[r][SEG * seg + u] = (row < P.m && kk + u < P.k) ? P.x[(size_t)row * P.k + kk + u] : 0.0f;
+    }
+    {
+      // w: thread t stages column t/4, 16 inputs from one fragment lane (the
+      // repacked layout is zero past n and k, and n0 + 63 < np)
+      const int c = tid >> 2, h = (tid >> 1) & 1, part = tid & 1, n = n0 + c;
+      const uint4 raw = *reinterpret_cast<const uint4*>(
+          P.wt + ((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16);
+      const float sc = P.wst[(size_t)g * P.np + n];
+      const uint32_t word[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+      for (int u = 0; u < 16; ++u) ws[c][32 * h + 16 * part + u] = (float)(int8_t)(word[u >> 2] >> (8 * (u & 3))) * sc;
+    }
+    __syncthreads();
+    for (int cc = 0; cc < nfull; ++cc) {
+      float xv[RPT][8], wv[4][8];
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) {
+        const float4 a = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc]);
+        const float4 b = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc + 4]);
+        xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w;
+        xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 a = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc]);
+        const float4 b = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc + 4]);
+        wv[j][0] = a.x; wv[j][1] = a.y; wv[j][2] = a.z; wv[j][3] = a.w;
+        wv[j][4] = b.x; wv[j][5] = b.y; wv[j][6] = b.z; wv[j][7] = b.w;
+      }
+#pragma unroll
+      for (int i = 0; i < RPT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int q = 0; q < 8; ++q) acc[i][j][q] = acc[i][j][q] + xv[i][q] * wv[j][q];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int row = m0 + RPT * tr + i;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = n0 + tc + 16 * j;
+      if (row >= mhi || n < nlo || n >= nhi) continue;
+      float y = -0.0f;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) y = y + acc[i][j][q];
+      for (int t = 8 * chunks; t < P.k; ++t) y = y + P.x[(size_t)row * P.k + t] * dequant(P, n, t);
+      y = y + (P.bias ? P.bias[n] : 0.0f);
+      if (P.lora) {
+        const float delta =
+            (P.rank > 0 ? dot_scores_rows(P.lmid + (size_t)row * P.rank, P.lb + (size_t)n * P.rank, P.rank) : -0.0f) +
+            0.0f;
+        const float scaled = P.lscale * delta;
+        y = y + scaled;
+      }
+      float* dst = P.layout == 1 ? P.out + (size_t)n * P.m + row : P.out + (size_t)row * P.n + n;
+      if (P.epilogue == 0 || P.layout == 1) *dst = y;
+      else if (P.epilogue == 1) *dst = *dst + y;
+      else *dst = silu(*dst) * y;
+    }
+  }
+}
+// The FP32 path of a whole projection: the blocks walk its tiles.  Behind a wide
+// launch (P.chain) they mostly only leave, which takes ~4.6 us by rocprof whether
+// the grid is 512 or 2048 blocks.
+__global__ __launch_bounds__(256) void k_linear_fp32(FProj P) {
+  __shared__ __attribute__((aligned(16))) F32Lds L;
+  if (P.chain) {
+    const bool hit = chain_hit(P.chain);
+    chain_close(P.chain);
+    if (!hit) return;  // the inputs were finite: the int8 kernels ran
+  }
+  const int col_tiles = (P.n + kF32Cols - 1) / kF32Cols;
+  const int tiles = ((P.m + kF32Rows - 1) / kF32Rows) * col_tiles;
+  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const int m0 = t / col_tiles * kF32Rows, n0 = t % col_tiles * kF32Cols;
+    fp32_tile<2>(P, m0, n0, P.m, 0, P.n, L);
+  }
+}
+// The FP32 path of an int8 block's outputs: rows [m0, mhi) (at most 16*RPT), columns [nlo, nhi).
+template <int RPT>
+__device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k, int m0, int mhi, int nlo, int nhi, uint8_t* lds) {
+  const FProj P = {x, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, k, S.g, S.n, S.np,
+                   S.epilogue, S.layout, nullptr};
+  __syncthreads();  // every wave's loads into this LDS have landed
+  for (int n0 = nlo / kF32Cols * kF32Cols; n0 < nhi; n0 += kF32Cols)
+    fp32_tile<RPT>(P, m0, n0, mhi, nlo, nhi, *reinterpret_cast<F32Lds*>(lds));
+}
+
+// ---------------------------------------------------------------------------
+// Projection kernel for launches that leave the wide kernel's blocks alone on
+// their CUs.  There every wave waits out each group's whole chain (LDS reads,
+// two dependent i8 MFMAs, conversion and product, 64 VALU instructions: ~1000
+// cycles), so this kernel halves the wave's tile (32 x 32, twice the waves),
+// takes two groups per step, and overlaps the steps: a step's dots are formed
+// while the step before is rescaled.  The two groups share the K=1 MFMAs as the
+// wide kernel's two column tiles do: blocks 0 and 1 of
+// v_mfma_f32_32x32x1_2b_f32 are groups 2j and 2j + 1 of the one tile, A lane l
+// = x of row l%32 and B lane l = w of column l%32, both of group 2j + l/32; the
+// two t's are then added in group order.
+//
+// A block of 4 waves owns (32*WM) x (32*WN) outputs.  Per step, operands reach
+// LDS by direct loads into a ring of S steps:
+//  * A: 8 rows x 128 bytes (8 whole cache lines) per 1 KB load; lane l fetches
+//    row l/8, 16-byte chunk (l%8) ^ (l/8), as in the skinny kernel's preload;
+//  * B: a column block's 4 fragments (2 groups), contiguous in the repacked
+//    layout, and the w scales of both groups;
+//  * x scales as in the wide kernel, 16 groups (8 steps) at a time.
+// An odd last group is computed beside a clamped copy whose t's are zeros.
+// A step is ~140-170 instructions per wave; alone on its SIMD a wave takes ~800
+// cycles for it (two waves per SIMD ~720 each: by then the CU's LDS, 48 KB in
+// and out per block and step, and the load path share the cost).  Measured
+// graph-replayed against the wide kernel: 512 x 6144 -> 2048 39.0 -> 22.2 us,
+// 128 x 2048 -> 2048 14.9 -> 9.6, 1000 x 6144 -> 2048 39.1 -> 33.0, pair 128 x
+// 2048 -> 2 x 6144 18.5 -> 16.2.  Also measured: without the overlap of steps 26.6
+// us for the first; a ring of 4 steps 22.1 (and one block per CU for the pair:
+// 22.2 for the last); one MFMA per 8 VALU instructions forced by
+// sched_group_barrier 23.2.
+// PAIR: a SwiGLU pair block owns 32 rows x 64 outputs, waves 0 and 1 the gate
+// projection's two column tiles, waves 2 and 3 the up projection's; the tiles
+// meet in LDS after the loop, where 8 threads take one row's group of h.
+constexpr int kMidRing = 3;
+template <int WM, int WN, int S, bool LORA, bool PAIR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_linear_mid(Batch b) {
+  constexpr int NW = 4, BM = 32 * WM, BN = 32 * WN, XCH = 16;
+  constexpr int AS = BM / 8, BF = 4 * WN;       // 1 KB loads per step: A units, B fragments
+  constexpr int KA = AS / NW, KB = BF / NW;     // ... per wave
+  constexpr int WSD = 2 * BN / 64;              // w-scale loads per step
+  constexpr int LOADS = KA + KB + 1;            // loads per wave and step (with one w-scale load)
+  constexpr int XD = BM / 16;                   // x-scale loads per chunk (16 rows of 16 groups)
+  static_assert(WM * WN == NW && AS % NW == 0 && BF % NW == 0 && WSD <= NW && XD <= NW, "loads split over the waves");
+  static_assert(!PAIR || (WM == 1 && WN == 4), "a pair block holds whole groups of h");
+  static_assert((S - 1) * LOADS + 1 <= 63, "ring depth");
+  struct Step {
+    uint8_t a[AS][kFragBytes], bf[BF][kFragBytes];
+    float ws[2][BN];
+  };
+  __shared__ __attribute__((aligned(16))) Step ring[S];
+  __shared__ __attribute__((aligned(16))) uint8_t xc[2][XD][kFragBytes];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pidx = find_proj<true>(b, blockIdx.x);
+  const Proj P = b.p[pidx];
+  int mt, nt;
+  tile_of(P, blockIdx.x - P.wave_begin, mt, nt);
+  const int m0 = mt * BM, n0 = nt * (PAIR ? BN / 2 : BN);
+  const int G = P.g, steps = (G + 1) >> 1;
+  const int wm = wid / WN, wn = wid - wm * WN;
+
+  const uint8_t* abase[KA];
+  uint32_t aoff[KA];
+#pragma unroll
+  for (int k = 0; k < KA; ++k) {
+    const int r0 = min(m0 + 8 * (k * NW + wid), P.m - 1), row = min(m0 + 8 * (k * NW + wid) + (lane >> 3), P.m - 1);
+    abase[k] = reinterpret_cast<const uint8_t*>(P.q) + (size_t)r0 * P.ldq;
+    aoff[k] = (uint32_t)((row - r0) * P.ldq + 16 * ((lane & 7) ^ (lane >> 3)));
+  }
+  const uint32_t atail = ((lane & 7) ^ (lane >> 3)) >= 4 ? 64u : 0u;  // an odd last group's copy
+  // B load k of this wave: fragment k*NW + wid, of column block (k*NW + wid)/4,
+  // group parity and half (k*NW + wid)%4
+  const uint8_t* bbase[KB];
+#pragma unroll
+  for (int k = 0; k < KB; ++k) {
+    const int cb = (k * NW + wid) >> 2;
+    const uint8_t* wt = PAIR && cb >= 2 ? P.wt2 : P.wt;
+    bbase[k] = wt + ((size_t)(n0 / 32 + (PAIR ? cb & 1 : cb)) * G * 2 + (wid & 1)) * kFragBytes;
+  }
+  const int bpar = (wid >> 1) & 1;  // NW = 4 fragments per column block: the group parity is the wave's
+  // w scales: load wid % WSD covers group parity wi / (BN/64), columns 64 (wi % (BN/64)) ..
+  const int wi = wid % WSD, wpar = wi / (BN / 64), wpart = wi % (BN / 64);
+  const float* wsbase = PAIR ? (wpart ? P.wst2 : P.wst) + n0 : P.wst + n0 + 64 * wpart;
+  const uint32_t wsrow = 4u * (uint32_t)P.np;
+
+  auto issue = [&](Step& T, int j) {
+    const int jc = min(j, steps - 1);
+    const bool odd = 2 * jc + 1 >= G;  // uniform
+#pragma unroll
+    for (int k = 0; k < KA; ++k)
+      dma16s(abase[k] + (uint32_t)jc * 128u, odd ? aoff[k] - atail : aoff[k], &T.a[k * NW + wid][0]);
+    const uint32_t gb = (uint32_t)min(2 * jc + bpar, G - 1);
+#pragma unroll
+    for (int k = 0; k < KB; ++k)
+      dma16s(bbase[k] + gb * (uint32_t)(2 * kFragBytes), (uint32_t)lane * 16, &T.bf[k * NW + wid][0]);
+    dma4s(reinterpret_cast<const char*>(wsbase) + (uint32_t)min(2 * j + wpar, G) * wsrow, (uint32_t)lane * 4,
+          &T.ws[wpar][64 * wpart]);
+  };
+  auto issue_x = [&](int c) {
+    int ln;  // lane id, read here so that nothing derived from it stays live across the loop
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+    if (wid < XD) {  // wave-uniform
+      const int xr = ln >> 2, xp = (ln & 3) ^ (xr & 3), g0 = XCH * c + 4 * xp;
+      const int r0 = min(m0 + 16 * wid, P.m - 1);
+      const uint32_t row = (uint32_t)((min(m0 + 16 * wid + xr, P.m - 1) - r0) * P.ldxs * 4);
+      dma16s(P.xs + (size_t)r0 * P.ldxs, row + 4u * (uint32_t)(g0 < G ? g0 : 0), &xc[c & 1][wid][0]);
+    }
+  };
+
+  // A operand: lane reads row R = 32*wm + lane%32, chunk 4*parity + 2h + lane/32
+  const int R = 32 * wm + (lane & 31);
+  int ard[2][2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) ard[p][h] = (R >> 3) * kFragBytes + 16 * (8 * (R & 7) + ((4 * p + 2 * h + (lane >> 5)) ^ (R & 7)));
+  const int xbx = (R >> 4) * kFragBytes + 16 * (4 * (R & 15) + (R & 3));  // x piece 0, swizzled by row
+
+  v16i cinit;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) cinit[i] = kMagicBits;
+  v32f zero32;
+#pragma unroll
+  for (int i = 0; i < 32; ++i) zero32[i] = 0.0f;
+  v16f s;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+
+  // Operands of one step in registers, its scales (the x scale of a clamped
+  // odd group is zero: its t's are then zeros, and s is never -0, so adding
+  // them changes nothing), and its dots.
+  struct Ops {
+    v4i a[2][2], b[2][2];
+    float x, w;
+  };
+  auto operands = [&](Ops& o, const Step& T, int j) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        o.a[p][h] = *reinterpret_cast<const v4i*>(&T.a[0][0] + ard[p][h]);
+        o.b[p][h] = *reinterpret_cast<const v4i*>(&T.bf[4 * wn + 2 * p + h][0] + 16 * lane);
+      }
+    const int gg = (2 * j) % XCH;
+    o.x = *reinterpret_cast<const float*>(&xc[(2 * j / XCH) & 1][0][0] + ((xbx ^ (16 * (gg >> 2))) + 4 * (gg & 3)) +
+                                          4 * (lane >> 5));
+    o.w = T.ws[lane >> 5][32 * wn + (lane & 31)];
+  };
+  auto dots = [&](v16i (&d)[2], const Ops& o) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) d[p] = mfma_i8(o.a[p][0], o.b[p][0], cinit);
+    asm volatile("" : "+v"(cinit));
+#pragma unroll
+    for (int p = 0; p < 2; ++p) d[p] = mfma_i8(o.a[p][1], o.b[p][1], d[p]);
+  };
+
+  issue_x(0);
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    issue(ring[i], i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (!PAIR && b.chain) {  // uniform; non-finite inputs take the FP32 path, once the loads into LDS have landed
+    const bool hit = chain_hit(b.chain);
+    chain_close(b.chain);
+    if (hit) {
+      wait_vmcnt<0>();
+      // (the fields are read again here, so that they do not stay in registers)
+      int pi = __builtin_amdgcn_readfirstlane(pidx);
+      asm volatile("" : "+s"(pi));
+      for (int r = m0; r < min(m0 + BM, P.m); r += 32)
+        fp32_block<2>(b.p[pi], b.fx[pi], b.fk, r, min(r + 32, P.m), n0, min(n0 + BN, P.n), reinterpret_cast<uint8_t*>(&ring));
+      return;
+    }
+  }
+  wait_vmcnt<(S - 1) * LOADS>();
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  v16i dt[2][2];  // the dots of even and odd steps
+  float xv, wv;
+  {
+    Ops o;
+    operands(o, ring[0], 0);
+    dots(dt[0], o);
+    xv = (lane >> 5) < G ? o.x : 0.0f;
+    wv = o.w;
+  }
+  // Step j, with d = j modulo the unroll (a constant): the ring slot and which
+  // set of dots.
+  auto step = [&](int j, int d) __attribute__((always_inline)) {
+    // step j's dots are in flight.  Step j + 1's loads have landed for this
+    // wave (those of j + 2 .. j + S - 1 may remain); after the barrier, for
+    // every wave, and every wave has read step j.  (Past the last step all of
+    // this runs on clamped copies.)
+    wait_vmcnt<(S - 2) * LOADS>();
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    Ops o;
+    operands(o, ring[(d + 1) % S], j + 1);
+    const v32f dv = mfma_k1(-kMagic, 1.0f, concat(dt[d & 1][0], dt[d & 1][1]));
+    const v32f pv = mfma_k1(xv, wv, zero32);
+    __builtin_amdgcn_sched_barrier(0);
+    if ((2 * (j + S)) % XCH == 0 && j + S < steps) issue_x(2 * (j + S) / XCH);
+    issue(ring[d % S], j + S);
+    __builtin_amdgcn_sched_barrier(0);
+    // step j + 1's dots between step j's t = dot * p and s = s + t (group 2j,
+    // then 2j + 1)
+    dots(dt[(d + 1) & 1], o);
+    v16f t0, t1;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      t0[v] = dv[v] * pv[v];
+      t1[v] = dv[16 + v] * pv[16 + v];
+    }
+    s = s + t0;
+    s = s + t1;
+    asm volatile("" : "+v"(s));  // keeps the compiler from sinking the sums of several steps behind the branches
+    xv = 2 * j + 2 + (lane >> 5) < G ? o.x : 0.0f;
+    wv = o.w;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int U = S % 2 == 0 ? S : 2 * S;  // an even unroll: the two sets of dots keep their registers
+  int j0 = 0;
+  for (; j0 + U <= steps; j0 += U) {
+#pragma unroll
+    for (int d = 0; d < U; ++d) step(j0 + d, d);
+  }
+#pragma unroll
+  for (int d = 0; d < U - 1; ++d)
+    if (j0 + d < steps) step(j0 + d, d);  // uniform over the block
+  wait_vmcnt<0>();  // the clamped loads past the end
+
+  // y = s + bias[col], or s + 0.0f without a bias (tensor.rs:437), then the
+  // adapter term (438, 109-117)
+  const bool up = PAIR && wn >= 2;  // wave-uniform
+  const int mw = m0 + 32 * wm, nw = n0 + 32 * (PAIR ? wn & 1 : wn), col = nw + (lane & 31);
+  const float* bp = up ? P.bias2 : P.bias;
+  const float bias = bp != nullptr && col < P.n ? bp[col] : 0.0f;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) s[v] = s[v] + bias;
+  if constexpr (LORA) {
+    const bool has = up ? P.lora2 : P.lora;
+    const float *lm = up ? P.lmid2 : P.lmid, *lb = up ? P.lb2 : P.lb;
+    const int rank = up ? P.rank2 : P.rank;
+    const float ls = up ? P.lscale2 : P.lscale;
+    lds_barrier();  // every wave is done reading the ring
+    if (has) {      // wave-uniform
+      if (rank == 0 || (rank == 16 && ((uintptr_t)lm & 15) == 0 && ((uintptr_t)lb & 15) == 0)) {
+        static_assert(sizeof(ring) >= NW * kLoraStage, "adapter staging fits the ring");
+        s = lora_block32(s, lm, lb, rank, ls, P.m, P.n, mw, nw, lane,
+                         reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(&ring) + wid * kLoraStage));
+      } else {
+        v16f zero16;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) zero16[i] = 0.0f;
+        const bool k0 = lane < 32;  // products from a K=2 MFMA whose k=1 operands are zero, as in the wide kernel
+        const float* lmr = lm + (size_t)min(mw + (lane & 31), P.m - 1) * rank;
+        const float* lbc = lb + (size_t)min(col, P.n - 1) * rank;
+        s = lora_term(s, zero16, rank, ls, [&](int i) { return mfma_k2(k0 ? lmr[i] : 0.0f, k0 ? lbc[i] : 0.0f, zero16); });
+      }
+    }
+  }
+  if constexpr (PAIR) {
+    // h = silu(gate) * up (tensor.rs:96-99, qwen.rs:489-490) and its
+    // quantization (qwen.rs:491, QuantizedInputs::new, tensor.rs:321-339): 8
+    // threads take one row's group of 64, 8 columns each.
+    constexpr int HP = 72;
+    float* ty = reinterpret_cast<float*>(&ring);  // [2][32][HP]: gate, up
+    static_assert(sizeof(ring) >= 2 * 32 * HP * 4, "both tiles fit the ring");
+    lds_barrier();  // every wave is done with the ring
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      ty[((up ? 32 : 0) + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * HP + 32 * (wn & 1) + (lane & 31)] = s[v];
+    lds_barrier();
+    const int t = threadIdx.x, rl = t >> 3, c0 = 8 * (t & 7);
+    const int row = m0 + rl, cb = n0 + c0;
+    const ExpTab T = exp_table(lane);
+    float e[8];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const v4f g4 = *reinterpret_cast<const v4f*>(ty + rl * HP + c0 + 4 * q);
+      const v4f u4 = *reinterpret_cast<const v4f*>(ty + (32 + rl) * HP + c0 + 4 * q);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[4 * q + i] = silu_wave(g4[i], T) * u4[i];
+      __builtin_amdgcn_sched_barrier(0);  // the f64 temporaries of 4 values at a time
+    }
+    if (row < P.m) {
+      float* hr = P.out + (size_t)row * P.n + cb;
+      if ((P.n & 3) == 0 && ((uintptr_t)P.out & 15) == 0 && cb + 8 <= P.n) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const v4f h4 = {e[4 * q], e[4 * q + 1], e[4 * q + 2], e[4 * q + 3]};
+          __builtin_nontemporal_store(h4, reinterpret_cast<v4f*>(hr + 4 * q));
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (cb + i < P.n) st_out(hr + i, e[i]);
+      }
+    }
+    if (P.hq != nullptr) {  // uniform over the launch
+#pragma unroll
+      for (int i = 0; i < 8; ++i) e[i] = cb + i < P.n ? e[i] : 0.0f;  // columns past n count as zero
+      uint32_t mb = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mb = max(mb, __builtin_bit_cast(uint32_t, e[i]) & 0x7fffffffu);
+      const bool bad = mb >= 0x7f800000u;
+      mb = __builtin_bit_cast(uint32_t, max_quad(__builtin_bit_cast(float, mb)));
+      mb = max(mb, (uint32_t)__shfl_xor((int)mb, 4));  // the group's 8 threads are lanes 8j .. 8j+7
+      const float scale = quant_scale_fma(__builtin_bit_cast(float, mb));
+      uint32_t w2[2];
+      quant_pack<8, true>(e, scale, w2);
+      if (row < P.m) {
+        int8_t* qr = P.hq + (size_t)row * P.n + cb;
+        if ((P.n & 7) == 0 && ((uintptr_t)P.hq & 7) == 0) {
+          if (cb < P.n) *reinterpret_cast<uint2*>(qr) = make_uint2(w2[0], w2[1]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            if (cb + i < P.n) qr[i] = (int8_t)(w2[i >> 2] >> (8 * (i & 3)));
+        }
+        if ((t & 7) == 0) P.hs[(size_t)row * ((P.n + kGroup - 1) / kGroup) + nt] = scale;
+      }
+      report_nonfinite(bad && row < P.m, P.hflag, b.hchain);
+      if (b.hchain) chain_open(b.hchain);  // (the launch holds this one pair)
+    }
+    return;
+  }
+  int rows[16], cols[16];
+  float y[16];
+  const bool full = P.layout == 0 && mw + 32 <= P.m && nw + 32 <= P.n;  // as in the wide kernel
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    rows[v] = mw + 8 * (v >> 2) + (v & 3) + (full ? 0 : 4 * (lane >> 5));
+    cols[v] = nw + (full ? 0 : (lane & 31));
+    y[v] = s[v];
+  }
+  if (full)
+    store_tile_full(P, rows, cols, (uint32_t)(4 * (lane >> 5) * P.n + (lane & 31)) * 4u, y);
+  else
+    store_tile(P, rows, cols, y);
+}
+
 // ---------------------------------------------------------------------------
 // Skinny projection kernel (M <= 32).  Per group and 16 x 16 tile:
 //   v_mfma_i32_16x16x64_i8 gives the group's dots (lane l, element v: row
@@ -2139,158 +2640,6 @@ __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, i
   return false;
 }
 
-// dot_scores (tensor.rs:6-25, the x86-64 order) of a[0..len) and b[0..len)
-// from plain memory: eight lane sums over the full chunks of 8, added in
-// order from -0.0, then the tail elements one by one; no fused multiply-add.
-__device__ __forceinline__ float dot_scores_rows(const float* a, const float* b, int len) {
-  const int chunks = len >> 3;
-  float lanes[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-  for (int c = 0; c < chunks; ++c)
-#pragma unroll
-    for (int q = 0; q < 8; ++q) lanes[q] = lanes[q] + a[8 * c + q] * b[8 * c + q];
-  float sum = -0.0f;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) sum = sum + lanes[q];
-  for (int t = 8 * chunks; t < len; ++t) sum = sum + a[t] * b[t];
-  return sum;
-}
-
-// Weight element (n, t) of the repacked layout, dequantized as Data::row does
-// for 8-bit Quantized data (weights.rs:47-78): (float)(int8)q * scale.
-__device__ __forceinline__ float dequant(const FProj& P, int n, int t) {
-  const int g = t >> 6, off = t & 63, h = off >> 5, part = (off >> 4) & 1;
-  const int8_t q = (int8_t)P.wt[((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16 +
-                                (off & 15)];
-  return (float)q * P.wst[(size_t)g * P.np + n];
-}
-
-// The FP32 path of a projection, Projection::columns_tiled (tensor.rs:206-269),
-// which the crate takes when the inputs are not finite (tensor.rs:197-201):
-//   y = dot_scores(x_r, w_n) + (bias[n] or 0.0)     w_n dequantized (dequant)
-//   y = y + scale * (dot_scores(mid_r, B_n) + 0.0)   with an adapter (Adapter::combine)
-// stored through the epilogue.  The dot products run in dot_scores' order, so
-// NaN and infinity propagate as in the crate.  fp32_tile: a block of 256
-// threads computes 16*RPT rows x 64 columns from (m0, n0) and stores those in rows
-// [m0, mhi) x columns [nlo, nhi); for RPT = 2 thread (tr, tc) owns rows 2tr, 2tr+1 and columns tc + 16j (j < 4)
-// with eight lane sums each.  Per group of 64 inputs the block stages x and
-// the dequantized weights in LDS (rows padded to 68 floats: the 16 columns a
-// wave reads per step fall in distinct banks).
-constexpr int kF32Rows = 32, kF32Cols = 64, kF32Pad = 68;
-struct F32Lds {
-  float xs[kF32Rows][kF32Pad], ws[kF32Cols][kF32Pad];
-};
-template <int RPT>
-__device__ __forceinline__ void fp32_tile(const FProj& P, int m0, int n0, int mhi, int nlo, int nhi, F32Lds& L) {
-  auto &xs = L.xs;
-  auto &ws = L.ws;
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  const int chunks = P.k >> 3;  // full chunks of 8 go to the lane sums
-  float acc[RPT][4][8];
-#pragma unroll
-  for (int i = 0; i < RPT; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int q = 0; q < 8; ++q) acc[i][j][q] = 0.0f;
-  for (int g = 0; 8 * g < chunks; ++g) {
-    const int nfull = min(8, chunks - 8 * g);  // uniform over the block
-    __syncthreads();                           // the previous group's reads are done
-    {
-      // x: thread t stages 4*RPT inputs of one row (zero past m or k)
-      constexpr int SEG = 4 * RPT, SPR = kGroup / SEG;
-      const int r = tid / SPR, seg = tid % SPR, row = m0 + r, kk = 64 * g + SEG * seg;
-#pragma unroll
-      for (int u = 0; u < SEG; ++u)
-        xs[r][SEG * seg + u] = (row < P.m && kk + u < P.k) ? P.x[(size_t)row * P.k + kk + u] : 0.0f;
-    }
-    {
-      // w: thread t stages column t/4, 16 inputs from one fragment lane (the
-      // repacked layout is zero past n and k, and n0 + 63 < np)
-      const int c = tid >> 2, h = (tid >> 1) & 1, part = tid & 1, n = n0 + c;
-      const uint4 raw = *reinterpret_cast<const uint4*>(
-          P.wt + ((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16);
-      const float sc = P.wst[(size_t)g * P.np + n];
-      const uint32_t word[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-      for (int u = 0; u < 16; ++u) ws[c][32 * h + 16 * part + u] = (float)(int8_t)(word[u >> 2] >> (8 * (u & 3))) * sc;
-    }
-    __syncthreads();
-    for (int cc = 0; cc < nfull; ++cc) {
-      float xv[RPT][8], wv[4][8];
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const float4 a = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc]);
-        const float4 b = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc + 4]);
-        xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w;
-        xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float4 a = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc]);
-        const float4 b = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc + 4]);
-        wv[j][0] = a.x; wv[j][1] = a.y; wv[j][2] = a.z; wv[j][3] = a.w;
-        wv[j][4] = b.x; wv[j][5] = b.y; wv[j][6] = b.z; wv[j][7] = b.w;
-      }
-#pragma unroll
-      for (int i = 0; i < RPT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int q = 0; q < 8; ++q) acc[i][j][q] = acc[i][j][q] + xv[i][q] * wv[j][q];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int row = m0 + RPT * tr + i;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tc + 16 * j;
-      if (row >= mhi || n < nlo || n >= nhi) continue;
-      float y = -0.0f;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) y = y + acc[i][j][q];
-      for (int t = 8 * chunks; t < P.k; ++t) y = y + P.x[(size_t)row * P.k + t] * dequant(P, n, t);
-      y = y + (P.bias ? P.bias[n] : 0.0f);
-      if (P.lora) {
-        const float delta =
-            (P.rank > 0 ? dot_scores_rows(P.lmid + (size_t)row * P.rank, P.lb + (size_t)n * P.rank, P.rank) : -0.0f) +
-            0.0f;
-        const float scaled = P.lscale * delta;
-        y = y + scaled;
-      }
-      float* dst = P.layout == 1 ? P.out + (size_t)n * P.m + row : P.out + (size_t)row * P.n + n;
-      if (P.epilogue == 0 || P.layout == 1) *dst = y;
-      else if (P.epilogue == 1) *dst = *dst + y;
-      else *dst = silu(*dst) * y;
-    }
-  }
-}
-// The FP32 path of a whole projection: the blocks walk its tiles.  After int8
-// launches (P.chain) the grid is small, since its blocks mostly only leave.
-__global__ __launch_bounds__(256) void k_linear_fp32(FProj P) {
-  __shared__ __attribute__((aligned(16))) F32Lds L;
-  if (P.chain) {
-    const bool hit = chain_hit(P.chain);
-    chain_close(P.chain);
-    if (!hit) return;  // the inputs were finite: the int8 kernels ran
-  }
-  const int col_tiles = (P.n + kF32Cols - 1) / kF32Cols;
-  const int tiles = ((P.m + kF32Rows - 1) / kF32Rows) * col_tiles;
-  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const int m0 = t / col_tiles * kF32Rows, n0 = t % col_tiles * kF32Cols;
-    fp32_tile<2>(P, m0, n0, P.m, 0, P.n, L);
-  }
-}
-// The FP32 path of a skinny block's outputs: rows [m0, mhi) (at most 16*RPT), columns [nlo, nhi).
-template <int RPT>
-__device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k, int m0, int mhi, int nlo, int nhi, uint8_t* lds) {
-  const FProj P = {x, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, k, S.g, S.n, S.np,
-                   S.epilogue, S.layout, nullptr};
-  __syncthreads();  // every wave's loads into this LDS have landed
-  for (int n0 = nlo / kF32Cols * kF32Cols; n0 < nhi; n0 += kF32Cols)
-    fp32_tile<RPT>(P, m0, n0, mhi, nlo, nhi, *reinterpret_cast<F32Lds*>(lds));
-}
-
 template <int RT, int CT, int CTL, int DBS, int DBL, bool DOTS, bool LORA>
 __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[skinny_lds_bytes(RT, CTL)];
@@ -2721,14 +3070,10 @@ hipError_t launch_chain_reset(Chain* chain, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Blocks of a k_linear_fp32 launch behind int8 launches, which nearly always
-// find finite inputs: a grid of one block per tile took 3.7-5 us to leave
-// (2048 blocks), KF32_TIME at this size.
-constexpr long kF32ChainBlocks = 512;
 hipError_t launch_linear_fp32(const FProj& p, hipStream_t s) {
   if (p.m == 0 || p.n == 0) return hipSuccess;
   const long tiles = (long)((p.m + kF32Rows - 1) / kF32Rows) * ((p.n + kF32Cols - 1) / kF32Cols);
-  const long blocks = p.chain ? std::min(tiles, kF32ChainBlocks) : std::min(tiles, 1L << 23);  // a grid under 2^32 threads
+  const long blocks = std::min(tiles, 1L << 23);  // a grid under 2^32 threads
   k_linear_fp32<<<(unsigned)blocks, 256, 0, s>>>(p);
   return hipGetLastError();
 }
@@ -2870,8 +3215,10 @@ hipError_t launch_pad_rows(const int8_t* q, int rows, int k, int8_t* dst, int ld
 #endif
 int skinny_segments(int g, bool few_strips) { return g <= DQ8_SKINNY_SHORT_MAX_G && !few_strips ? 1 : 4; }
 int skinny_cols(int nseg) { return 16 * (nseg == 1 ? DQ8_SKINNY_CT : DQ8_SKINNY_CTL); }
-int wide_block_rows() { return 32 * DQ8_WIDE_RT * DQ8_WIDE_WM; }
-int wide_block_cols() { return 32 * DQ8_WIDE_CT * DQ8_WIDE_WN; }
+int block_rows(int kind, bool pair) { return kind == 0 ? 32 * DQ8_WIDE_RT * DQ8_WIDE_WM : pair ? 32 : 64; }
+int block_cols(int kind, bool pair) {
+  return kind == 0 ? 32 * DQ8_WIDE_CT * DQ8_WIDE_WN / (pair ? 2 : 1) : 64;
+}
 bool wide_can_pair() { return wide_pair_shape(DQ8_WIDE_WN, DQ8_WIDE_RT, DQ8_WIDE_CT); }
 
 hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s) {
@@ -2921,6 +3268,17 @@ hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s) {
     else DQ8_WIDE(2, 3, 8, false, false);
 #endif
 #undef DQ8_WIDE
+    return hipGetLastError();
+  }
+  if (kind == 3) {
+    bool pair = false;
+    for (int i = 0; i < b.count; ++i) pair |= b.p[i].pair != 0;
+    if (pair)
+      lora ? k_linear_mid<1, 4, kMidRing, true, true><<<b.total_waves, 256, 0, s>>>(b)
+           : k_linear_mid<1, 4, kMidRing, false, true><<<b.total_waves, 256, 0, s>>>(b);
+    else
+      lora ? k_linear_mid<2, 2, kMidRing, true, false><<<b.total_waves, 256, 0, s>>>(b)
+           : k_linear_mid<2, 2, kMidRing, false, false><<<b.total_waves, 256, 0, s>>>(b);
     return hipGetLastError();
   }
   // total_waves counts blocks of 4 waves for the skinny kernel; kind 1: M <= 16, kind 2: M <= 32

@@ -1255,3 +1255,73 @@ def test_small_call_with_adapter_and_group(ctx, m):
     ctx.linear_batch([dq8.Item(h, q, s, o1), dq8.Item(h2, q, s, o2)])
     assert bits_equal(host(o1), dq8o.linear(x, wv, ws, threads=8))
     assert bits_equal(host(o2), dq8o.linear(x, w2v, w2s, threads=8))
+
+
+# The mid kernel (more than 32 rows whose wide grid is at most 256 blocks, here
+# past the 512 rows that run as chunks, or in the columns layout): one row and
+# one column past a tile, widths of one input, of one and several groups, an odd
+# group count (the last group is paired with a clamped copy) and long K; and the
+# wide kernel's own ragged edges, in grids just past that limit.
+MID_CASES = [(513, 1, 1, None), (513, 64, 65, 16), (577, 100, 63, None), (600, 192, 200, 5), (540, 1088, 130, 16),
+             (520, 2112, 64, 20), (520, 6200, 70, 0), (1100, 100, 2050, None), (1090, 320, 2100, 16),
+             (1100, 192, 2050, 5)]
+
+
+@pytest.mark.parametrize("m,k,n,rank", MID_CASES)
+def test_mid_and_wide_kernel_edges(ctx, m, k, n, rank):
+    rng = np.random.default_rng(m + 3 * k + n)
+    x = make_x(rng, m, k, "outliers")
+    wv, ws = dq8o.quantize_weights(make_w(rng, n, k))
+    bias = rng.standard_normal(n).astype(np.float32)
+    h = ctx.weights_from_quantized(dev(wv), dev(ws))
+    q, s = ctx.quantize(dev(x))
+    base = rng.standard_normal((m, n)).astype(np.float32)
+    a = b = lora = None
+    if rank is not None:
+        a = (rng.standard_normal((rank, k)) * 0.05).astype(np.float32)
+        b = (rng.standard_normal((n, rank)) * 0.05).astype(np.float32)
+        mid = ctx.lora_mid(dev(x), dev(a)) if rank else torch.zeros((m, 0), dtype=torch.float32, device="cuda")
+        lora = dq8.Lora(mid, dev(b), -0.75)
+    for ep in (dq8.WRITE, dq8.ADD, dq8.SWIGLU):
+        if rank is None:
+            want = dq8o.linear(x, wv, ws, bias=bias, result=base, epilogue=ep, threads=8)
+            got = ctx.linear(h, q, s, out=dev(base.copy()), bias=dev(bias), epilogue=ep)
+        else:
+            want = dq8o.linear_lora(x, wv, ws, a, b, -0.75, bias=bias, result=base, epilogue=ep, threads=8)
+            got = ctx.linear_lora(h, q, s, lora, out=dev(base.copy()), bias=dev(bias), epilogue=ep)
+        assert bits_equal(host(got), want)
+    if rank is None:  # columns, from 33 rows up
+        for rows in (33, m):
+            got = host(ctx.linear(h, q[:rows], s[:rows], layout=dq8.COLUMNS))
+            assert bits_equal(got, np.ascontiguousarray(dq8o.linear(x[:rows], wv, ws, threads=8).T))
+
+
+# The FP32 path inside the mid kernel's blocks (64 x 64, partial ones included)
+# and behind the wide kernel, and finite calls after it.
+@pytest.mark.parametrize("m,k,n", [(530, 100, 70), (560, 1088, 65), (1100, 70, 2050)])
+def test_apply_non_finite_on_the_mid_and_wide_kernels(ctx, m, k, n):
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    v, s = dq8o.quantize_weights(make_w(rng, n, k))
+    h = ctx.weights_from_quantized(dev(v), dev(s))
+    base = rng.standard_normal((m, n)).astype(np.float32)
+    bad = x.copy()
+    bad[m - 1, k // 2] = np.inf
+    for inp in (x, bad, x, bad, bad, x):
+        got = host(ctx.apply(h, dev(inp), out=dev(base.copy()), epilogue=dq8.ADD))
+        want, fp32 = dq8o.apply(inp, v, s, result=base, epilogue=1, threads=8)
+        assert fp32 == (inp is bad)
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got), nan) and got[~nan].tobytes() == want[~nan].tobytes()
+
+
+# The mid kernel's SwiGLU pair (at most 512 blocks of 32 x 64 outputs): partial
+# row and column blocks, long K, adapters of any two ranks or on one projection only; and the wide pair's
+# ragged edges just past that limit.
+@pytest.mark.parametrize("m,hidden,inter,gl,ul",
+                         [(100, 2304, 1000, None, None), (65, 6400, 136, (16, "aligned"), (5, "aligned")),
+                          (97, 2048, 1300, (16, "offset"), (16, "aligned")), (130, 2048, 1001, None, (16, "aligned")),
+                          (600, 256, 1100, (0, "aligned"), (20, "aligned")), (300, 256, 3300, None, None),
+                          (330, 256, 3100, (16, "aligned"), (16, "aligned"))])
+def test_mid_and_wide_ffn_gate_up(ctx, m, hidden, inter, gl, ul):
+    test_ffn_gate_up_with_adapters(ctx, m, hidden, inter, gl, ul)
