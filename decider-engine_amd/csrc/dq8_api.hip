@@ -467,7 +467,22 @@ struct QOut {
   float* scales;
   uint32_t* nonfinite;
   dq8::Chain* chain;
+  // The stored result's middle product mid [m][rank] with an adapter's a
+  // [rank][n], wanted with the quantization (rank 0: none).
+  const float* a;
+  size_t rank;
+  float* mid;
 };
+// The stored result [m][n] quantized as qo asks, and its middle product.
+hipError_t quantize_result(const float* result, size_t m, int n, const QOut& qo, hipStream_t s) {
+  if (qo.rank && dq8::quantize_mid_ok(result, (int)m, n, qo.q, qo.a, (int)qo.rank))
+    return dq8::launch_quantize_mid(result, (int)m, n, qo.q, qo.scales, qo.nonfinite, qo.chain, qo.a, (int)qo.rank, qo.mid, s);
+  hipError_t e = dq8::launch_quantize(result, (int)m, n, qo.q, n, qo.scales, (n + kGroup - 1) / kGroup, qo.nonfinite,
+                                      qo.chain, s);
+  if (e == hipSuccess && qo.rank)
+    e = dq8::launch_lora_mid(result, (int)m, n, qo.a, (int)qo.rank, qo.mid, s);
+  return e;
+}
 
 // The FP32 path beside an int8 projection: its fp32 inputs [m][k] and the
 // chain that says which of the two runs on the device.
@@ -617,8 +632,7 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
   }
   if (qout && count == 1 && items[0].m > 0) {
     const dq8::Weights& w = items[0].w->w;
-    hipError_t e = dq8::launch_quantize(items[0].out, (int)items[0].m, w.n, qout->q, w.n, qout->scales,
-                                        (w.n + kGroup - 1) / kGroup, qout->nonfinite, qout->chain, s);
+    hipError_t e = quantize_result(items[0].out, items[0].m, w.n, *qout, s);
     if (e != hipSuccess) return from_hip(e);
   }
   return DQ8_OK;
@@ -668,9 +682,10 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
     place_proj(p, kind, b, units / 2 < kSkinnyFewStrips, units, g.g > 32);
   }
   hipError_t e = dq8::launch_linear(b, kind, false, s);
-  if (e == hipSuccess && qout && (kind == 1 || kind == 2))
-    e = dq8::launch_quantize(h, (int)m, g.n, qout->q, g.n, qout->scales, (int)groups_of(g.n), qout->nonfinite,
-                             qout->chain, s);
+  if (e == hipSuccess && qout) {
+    if (kind == 1 || kind == 2) e = quantize_result(h, m, g.n, *qout, s);
+    else if (qout->rank) e = dq8::launch_lora_mid(h, (int)m, g.n, qout->a, (int)qout->rank, qout->mid, s);
+  }
   return from_hip(e);
 }
 
@@ -1234,7 +1249,7 @@ dq8_status dq8_ffn_gate_up_lora(dq8_ctx* ctx, const dq8_weights* gate, const dq8
     hipError_t e = dq8::launch_fill_u32(ctx->flag, 0, s);
     if (e != hipSuccess) return from_hip(e);
   }
-  QOut qo = {h_q, h_scales, nonfinite ? nonfinite : ctx->flag, nullptr};
+  QOut qo = {h_q, h_scales, nonfinite ? nonfinite : ctx->flag, nullptr, nullptr, 0, nullptr};
   st = gate_up(ctx, gate, up, q, scales, m, gate_bias, up_bias, gate_lora, up_lora, h, &qo, s);
   if (st != DQ8_OK || nonfinite) return st;
   return finish_nonfinite(ctx, s);
@@ -1319,7 +1334,7 @@ dq8_status dq8_linear_q(dq8_ctx* ctx, const dq8_weights* w, const int8_t* q, con
     hipError_t e = dq8::launch_fill_u32(ctx->flag, 0, s);
     if (e != hipSuccess) return from_hip(e);
   }
-  QOut qo = {q_out, scales_out, nonfinite ? nonfinite : ctx->flag, nullptr};
+  QOut qo = {q_out, scales_out, nonfinite ? nonfinite : ctx->flag, nullptr, nullptr, 0, nullptr};
   dq8_linear_item it = {w, q, scales, m, bias, out, DQ8_ROWS, epilogue, lora};
   st = run_linear(ctx, &it, 1, nullptr, s, &qo);
   if (st != DQ8_OK || nonfinite) return st;
@@ -1355,25 +1370,20 @@ dq8_status dq8_ffn(dq8_ctx* ctx, const dq8_ffn_weights* f, const int8_t* q, cons
   // then quantized for down (qwen.rs:491).  Without adapters, on the wide
   // kernel, both projections run in one launch that stores h directly.
   dq8::Chain* chain = ctx->chain_state;
-  QOut qo = {qh, sh, nonfinite, chain};
+  QOut qo = {qh, sh, nonfinite, chain, f->down_lora_a, rank, mid};  // (down's middle product from h)
   st = gate_up(ctx, f->gate, f->up, q, scales, m, f->gate_bias, f->up_bias, f->gate_lora, f->up_lora, h, &qo, s);
   if (st != DQ8_OK) {
     (void)dq8::launch_chain_reset(chain, s);
     return st;
   }
-  // down: Add into the residual (qwen.rs:492), its adapter's middle product from h.
+  // down: Add into the residual (qwen.rs:492).
   // If h holds a non-finite value, QuantizedInputs::new(h) is None and the crate
   // takes the FP32 path on h (tensor.rs:197-201), as the chain says on the device.
   dq8_lora dl = {mid, f->down_lora_b, rank, f->down_lora_scale};
-  hipError_t e = hipSuccess;
-  if (rank > 0) e = dq8::launch_lora_mid(h, (int)m, (int)inter, f->down_lora_a, (int)rank, mid, s);
-  st = from_hip(e);
-  if (st == DQ8_OK) {
-    const dq8_lora* dlp = f->down_lora_a ? &dl : nullptr;
-    dq8_linear_item di = {f->down, qh, sh, m, f->down_bias, residual, DQ8_ROWS, DQ8_ADD, dlp};
-    const Fallback fb = {chain, h};
-    st = run_linear(ctx, &di, 1, nullptr, s, nullptr, &fb);
-  }
+  const dq8_lora* dlp = f->down_lora_a ? &dl : nullptr;
+  dq8_linear_item di = {f->down, qh, sh, m, f->down_bias, residual, DQ8_ROWS, DQ8_ADD, dlp};
+  const Fallback fb = {chain, h};
+  st = run_linear(ctx, &di, 1, nullptr, s, nullptr, &fb);
   if (st != DQ8_OK) (void)dq8::launch_chain_reset(chain, s);
   return st;
 }

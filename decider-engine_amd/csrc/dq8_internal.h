@@ -161,6 +161,11 @@ struct FProj {
 // *nonfinite (when set) and marks *chain (when set), whose call this opens.
 hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
                            uint32_t* nonfinite, Chain* chain, hipStream_t s);
+// launch_quantize (q [m][k], scales [m][k/64]) and the middle product of x and a
+// [rank][k] in one launch, where quantize_mid_ok: few rows (m <= 32).
+bool quantize_mid_ok(const float* x, int m, int k, const int8_t* q, const float* a, int rank);
+hipError_t launch_quantize_mid(const float* x, int m, int k, int8_t* q, float* scales, uint32_t* nonfinite, Chain* chain,
+                               const float* a, int rank, float* mid, hipStream_t s);
 hipError_t launch_repack(const uint8_t* values, const float* scales, int n, int k, Weights* w, hipStream_t s);
 // Data::quantize of stored elements x [n][k] (type dtype, kDtype*) into w; a
 // non-finite element stores 1 to *nonfinite.

@@ -659,13 +659,10 @@ constexpr int kQuantLoopBlocks = DQ8_QUANT_LOOP_BLOCKS;
 #define DQ8_QUANT_LOOP_WPB 4
 #endif
 template <int D>
-__global__ __launch_bounds__(64 * DQ8_QUANT_LOOP_WPB) void k_quantize_loop(const float* __restrict__ x, int k, int total,
-                                                       int8_t* __restrict__ q, int ldq, float* __restrict__ scales,
-                                                       int lds, uint32_t* nonfinite, Chain* chain, Divider cdiv) {
-  if (chain) chain_open(chain);
+__device__ __forceinline__ void quantize_chunks(const float* __restrict__ x, int k, int total, int8_t* __restrict__ q,
+                                                int ldq, float* __restrict__ scales, int lds, uint32_t* nonfinite,
+                                                Chain* chain, const Divider& cdiv, int w, int W) {
   const int lane = threadIdx.x & 63;
-  const int W = (int)gridDim.x * DQ8_QUANT_LOOP_WPB;
-  const int w = (int)blockIdx.x * DQ8_QUANT_LOOP_WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cpr = k >> 8;
   auto load = [&](int c, float (&v)[4]) {
     const int row = cdiv.div((uint32_t)c);
@@ -732,6 +729,15 @@ __global__ __launch_bounds__(64 * DQ8_QUANT_LOOP_WPB) void k_quantize_loop(const
     }
   }
   report_nonfinite(bad, nonfinite, chain);
+}
+template <int D>
+__global__ __launch_bounds__(64 * DQ8_QUANT_LOOP_WPB) void k_quantize_loop(const float* __restrict__ x, int k, int total,
+                                                       int8_t* __restrict__ q, int ldq, float* __restrict__ scales,
+                                                       int lds, uint32_t* nonfinite, Chain* chain, Divider cdiv) {
+  if (chain) chain_open(chain);
+  quantize_chunks<D>(x, k, total, q, ldq, scales, lds, nonfinite, chain, cdiv,
+                     (int)blockIdx.x * DQ8_QUANT_LOOP_WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
+                     (int)gridDim.x * DQ8_QUANT_LOOP_WPB);
 }
 
 // Sixteen consecutive stored elements as loaded: 16-byte loads at element
@@ -2972,85 +2978,168 @@ __global__ __launch_bounds__(256) void k_lora_mid_dma_batch(MidBatch bt) {
   lora_mid_tiled(I.x, I.m, I.k, I.a, I.rank, I.mid, b - I.block_begin, lds);
 }
 
-// k_lora_mid_small<R, J>: few rows (m <= 32).  A block holds R whole rows of x
-// and J whole adapter rows in LDS, fetched by one round of direct global->LDS
-// loads (1 KB each; the block's 4 waves issue every 4th, at most 39 each), so
-// the memory latency is paid once; then the first R * J * 8 threads compute.  Lane l works on row r0 + (l/8)/J, adapter row j0 + (l/8)%J and lane
-// sum i = l%8: the chunks are summed in order on the VALU (one rounded product
-// and one rounded add each), then the 8 lane sums of a pair, in consecutive
-// lanes, are added in order from -0.0, then the tail elements.  Loads past a
-// row's end are clamped to its last 16 bytes and land in the row padding.
-// Requires k % 4 == 0, 16-byte aligned x and a, and roundup(k, 256) <= KR.
-constexpr int kSmallR = 4, kSmallJ = 2, kSmallKR = 6656;  // the one configuration in use
-constexpr int kSmallRS = kSmallKR + 8;                     // row stride: the 8 rows of a step in distinct banks
-template <int R, int J, int KR>
+// k_lora_mid_small: few rows (m <= 32).  A block covers 4 rows of x and 2
+// adapter rows: 64 lane sums, one per lane of wave 0, which only adds.  The
+// time is that chain (K/8 dependent adds of ~9.5 cycles), so everything else is
+// kept off it: waves 1-6 load 512-input tiles of the 6 rows into a ring by
+// direct global->LDS loads (a row each), form a tile's rounded products and
+// post them as [step][lane sum]; wave 0 reads a tile's 64 products per lane one
+// tile ahead of the adds, its reads between them.  One barrier per tile: in
+// iteration t the producers post tile t while wave 0 reads tile t - 1 and adds
+// tile t - 2.  The 8 lane sums of a pair, in consecutive lanes, are then added
+// in order from -0.0, then the tail elements.  Loads past a row's end are
+// clamped to its last 16 bytes; their products are never added.
+// Requires k % 4 == 0 and 16-byte aligned x and a.  24 rows, rank 16, by
+// rocprof: MIDS_FIG (one wave reading
+// both operands, multiplying and adding, after whole rows had landed: 5.4 us at
+// K = 2048, 11.4 at 6144).
+constexpr int kSmallR = 4, kSmallJ = 2, kSmallSlots = 8, kSmallKT = 512, kSmallSteps = kSmallKT / 8;
+constexpr int kSmallWaves = 1 + kSmallR + kSmallJ;
+struct SmallLds {
+  float ring[kSmallSlots][kSmallR + kSmallJ][kSmallKT + 8];  // rows padded by 8 floats: distinct banks
+  float prod[2][kSmallSteps][64];
+};
+// Waits for this wave's 2 loads of a tile, when those of `newer` later tiles may remain.
+template <int N>
+__device__ __forceinline__ void wait_tile(int newer) {
+  if constexpr (N > 0) {
+    if (newer < N) return wait_tile<N - 1>(newer);
+  }
+  wait_vmcnt<2 * N>();
+}
 __device__ __forceinline__ void lora_mid_small(const float* __restrict__ x, int m, int k, const float* __restrict__ a,
-                                               int rank, float* __restrict__ mid, int block, float* lds) {
-  constexpr int NT = R * J * 8, NW = 4, RS = KR + 8;
-  static_assert(NT % 64 == 0 && NT <= 256, "whole waves of one block");
-  static_assert((R + J) * ((KR + 255) / 256) <= 48 * NW, "at most 48 loads in flight per wave");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+                                               int rank, float* __restrict__ mid, int block, SmallLds& L) {
+  constexpr int R = kSmallR, J = kSmallJ, NS = kSmallSlots, KT = kSmallKT, ST = kSmallSteps;
+  static_assert(R == 4 && J == 2, "64 lane sums; 16 items over 6 producing waves");
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int jblocks = (rank + J - 1) / J;
   const int r0 = (block / jblocks) * R, j0 = (block % jblocks) * J;
-  const int segs = (k + 255) >> 8;  // 1 KB pieces per row
-  for (int t = w; t < (R + J) * segs; t += NW) {  // wave-uniform
-    const int row = t / segs, seg = t - row * segs;
-    const float* src = row < R ? x + (size_t)min(r0 + row, m - 1) * k : a + (size_t)min(j0 + row - R, rank - 1) * k;
-    const uint32_t off = 4u * (uint32_t)min(4 * lane, k - 4 - 256 * seg);  // k % 4 == 0: k - 256*seg >= 4
-    dma16s(src + 256 * seg, off, lds + row * RS + 256 * seg);
-  }
-  wait_vmcnt<0>();
-  lds_barrier();
-  if (tid >= NT) return;  // wave-uniform: NT is a multiple of 64
-  const int pr = tid >> 3, i = tid & 7, r = pr / J, j = pr - r * J;
-  // Both row bases as opaque LDS addresses: the compiler would otherwise fold
-  // the constant R * RS * 4 (over 64 KB) into every read's offset and, since
-  // the offset field stops at 64 KB, rebuild each read's address on the VALU.
-  typedef __attribute__((address_space(3))) const float* lds_row;
-  lds_row xs = (lds_row)(lds + r * RS);
-  lds_row as = (lds_row)(lds + (R + j) * RS);
-  // this lane's elements i, i + 8, ...: one address step per CU chunks, the
-  // chunks within it as immediate offsets; all CU chunks' operands are read
-  // before the first is summed, so one LDS latency per CU chunks is exposed
-  // (the chain's adds hide the rest)
-  constexpr int CU = 32;
-  lds_row xp = xs + i, ap = as + i;
-  asm volatile("" : "+v"(xp), "+v"(ap));
-  const int chunks = k >> 3;
-  float acc = 0.0f;
-  int c = 0;
-  for (; c + CU <= chunks; c += CU, xp += 8 * CU, ap += 8 * CU) {
-    float xv[CU], av[CU];
+  const int chunks = k >> 3, tiles = (chunks + ST - 1) / ST;
+  if (w != 0) {
+    // row w - 1 of the block's 6 (4 of x, 2 of A), two 1 KB loads per tile
+    const int lr = w - 1;
+    const float* src = lr < R ? x + (size_t)min(r0 + lr, m - 1) * k : a + (size_t)min(j0 + lr - R, rank - 1) * k;
+    auto issue = [&](int t) {
 #pragma unroll
-    for (int u = 0; u < CU; ++u) {
-      xv[u] = xp[8 * u];
-      av[u] = ap[8 * u];
+      for (int p = 0; p < 2; ++p)
+        dma16s(src, 4u * (uint32_t)min(KT * t + 256 * p + 4 * lane, k - 4), &L.ring[t % NS][lr][256 * p]);  // k % 4 == 0
+    };
+    for (int t = 0; t < min(NS - 1, tiles); ++t) issue(t);
+    // item e of a tile's 16: 4 steps x 8 pairs x 2 halves of a step's 8 inputs;
+    // this wave's are e = w - 1 + 6u (past 15: a repeat of item 15, same values)
+    const int half = lane & 1, pr = (lane >> 1) & 7, st = lane >> 4;
+    int xo[3], ao[3], po[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const int step = 4 * min(w - 1 + 6 * u, 15) + st;
+      xo[u] = (pr / J) * (KT + 8) + 8 * step + 4 * half;
+      ao[u] = (R + pr % J) * (KT + 8) + 8 * step + 4 * half;
+      po[u] = 64 * step + 8 * pr + 4 * half;
     }
+    for (int t = 0; t < tiles; ++t) {
+      wait_tile<NS - 2>(tiles - 1 - t);
+      lds_barrier();
+      const float* slot = &L.ring[t % NS][0][0];
+      float* post = &L.prod[t & 1][0][0];
+      v4f xv[3], av[3];
 #pragma unroll
-    for (int u = 0; u < CU; ++u) acc = acc + xv[u] * av[u];
+      for (int u = 0; u < 3; ++u) {
+        xv[u] = *reinterpret_cast<const v4f*>(slot + xo[u]);
+        av[u] = *reinterpret_cast<const v4f*>(slot + ao[u]);
+      }
+      if (ST * (t + 1) <= chunks) {  // uniform
+#pragma unroll
+        for (int u = 0; u < 3; ++u) *reinterpret_cast<v4f*>(post + po[u]) = xv[u] * av[u];
+      } else {
+        const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+          const v4f pv = xv[u] * av[u];
+          *reinterpret_cast<v4f*>(post + po[u]) = ST * t + (po[u] >> 6) < chunks ? pv : zero4;
+        }
+      }
+      if (t + NS - 1 < tiles) issue(t + NS - 1);  // the slot of tile t - 1
+    }
+    lds_barrier();  // iterations tiles and tiles + 1: wave 0 alone
+    lds_barrier();
+    return;
   }
-  for (; c < chunks; ++c, xp += 8, ap += 8) acc = acc + xp[0] * ap[0];
+  float acc = 0.0f;
+  auto read = [&](float (&pv)[ST], int t) {
+#pragma unroll
+    for (int u = 0; u < ST; ++u) pv[u] = L.prod[t & 1][u][lane];
+  };
+  // (steps past the last chunk are posted as +0.0, and acc is never -0.0: it
+  // starts at +0.0, so adding them changes nothing)
+  auto add = [&](const float (&pv)[ST]) {
+#pragma unroll
+    for (int u = 0; u < ST; ++u) acc = acc + pv[u];
+    asm volatile("" : "+v"(acc));
+#pragma unroll
+    for (int u = 0; u < ST / 2; ++u) {  // the reads between the adds
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+  };
+  float pa[ST], pb[ST];
+  lds_barrier();
+  lds_barrier();
+  read(pa, 0);
+  int t = 2;  // iteration
+  for (; t <= tiles; t += 2) {
+    lds_barrier();
+    read(pb, t - 1);
+    add(pa);
+    lds_barrier();
+    read(pa, t);
+    add(pb);
+  }
+  if (t <= tiles + 1) {
+    lds_barrier();
+    add(pa);
+  }
+  const int pr = lane >> 3, i = lane & 7;
   float sum = -0.0f;
 #pragma unroll
   for (int ii = 0; ii < 8; ++ii) sum = sum + __shfl(acc, (lane & ~7) + ii);
-  const int row = r0 + r, jr = j0 + j;
+  const int row = r0 + pr / J, jr = j0 + pr % J;
   if (i == 0 && row < m && jr < rank) {
-    for (int e = 8 * chunks; e < k; ++e) sum = sum + xs[e] * as[e];
+    const float *xg = x + (size_t)row * k, *ag = a + (size_t)jr * k;
+    for (int e = 8 * chunks; e < k; ++e) sum = sum + xg[e] * ag[e];
     mid[(size_t)row * rank + jr] = sum + 0.0f;
   }
 }
-__global__ __launch_bounds__(256) void k_lora_mid_small(const float* __restrict__ x, int m, int k,
+__global__ __launch_bounds__(64 * kSmallWaves) void k_lora_mid_small(const float* __restrict__ x, int m, int k,
                                                         const float* __restrict__ a, int rank, float* __restrict__ mid) {
-  __shared__ __attribute__((aligned(16))) float lds[(kSmallR + kSmallJ) * kSmallRS];
-  lora_mid_small<kSmallR, kSmallJ, kSmallKR>(x, m, k, a, rank, mid, (int)blockIdx.x, lds);
+  __shared__ __attribute__((aligned(16))) SmallLds L;
+  lora_mid_small(x, m, k, a, rank, mid, (int)blockIdx.x, L);
+}
+// A few rows' quantization and one adapter's middle product of the same x in
+// one launch: neither needs the other, and neither fills the GPU (24 x 6144,
+// rank 16: 144 quantizer blocks beside 48 blocks of the middle product, which
+// come first).  A dq8_ffn's h: QMID_FIG.
+__global__ __launch_bounds__(64 * kSmallWaves) void k_quantize_mid(const float* __restrict__ x, int m, int k, int total,
+                                                      int8_t* __restrict__ q, float* __restrict__ scales,
+                                                      uint32_t* nonfinite, Chain* chain, Divider cdiv,
+                                                      const float* __restrict__ a, int rank, float* __restrict__ mid,
+                                                      int mid_blocks) {
+  __shared__ __attribute__((aligned(16))) SmallLds L;
+  if (chain) chain_open(chain);
+  if ((int)blockIdx.x < mid_blocks) {
+    lora_mid_small(x, m, k, a, rank, mid, (int)blockIdx.x, L);
+  } else {
+    quantize_chunks<DQ8_QUANT_LOOP>(x, k, total, q, k, scales, k >> 6, nonfinite, chain, cdiv,
+                                    ((int)blockIdx.x - mid_blocks) * kSmallWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
+                                    ((int)gridDim.x - mid_blocks) * kSmallWaves);
+  }
 }
 // Several middle products in one launch (block -> item by find_mid).
-__global__ __launch_bounds__(256) void k_lora_mid_small_batch(MidBatch bt) {
-  __shared__ __attribute__((aligned(16))) float lds[(kSmallR + kSmallJ) * kSmallRS];
+__global__ __launch_bounds__(64 * kSmallWaves) void k_lora_mid_small_batch(MidBatch bt) {
+  __shared__ __attribute__((aligned(16))) SmallLds L;
   const int b = (int)blockIdx.x;
   const MidItem I = bt.it[find_mid(bt, b)];
-  lora_mid_small<kSmallR, kSmallJ, kSmallKR>(I.x, I.m, I.k, I.a, I.rank, I.mid, b - I.block_begin, lds);
+  lora_mid_small(I.x, I.m, I.k, I.a, I.rank, I.mid, b - I.block_begin, L);
 }
 
 }  // namespace
@@ -3079,8 +3168,7 @@ hipError_t launch_linear_fp32(const FProj& p, hipStream_t s) {
 }
 
 bool lora_mid_small_ok(const float* x, int m, int k, const float* a) {
-  return k % 4 == 0 && ((size_t)x & 15) == 0 && ((size_t)a & 15) == 0 && m <= DQ8_MID_SMALL_M &&
-         ((k + 255) & ~255) <= kSmallKR;
+  return k % 4 == 0 && ((size_t)x & 15) == 0 && ((size_t)a & 15) == 0 && m <= DQ8_MID_SMALL_M;
 }
 long lora_mid_small_blocks(int m, int rank) { return (long)((m + kSmallR - 1) / kSmallR) * ((rank + kSmallJ - 1) / kSmallJ); }
 
@@ -3096,22 +3184,16 @@ hipError_t launch_lora_mid_batch(const MidBatch& b, long blocks, bool tiled, hip
   if (tiled)
     k_lora_mid_dma_batch<<<(unsigned)blocks, 256, 0, s>>>(b);
   else
-    k_lora_mid_small_batch<<<(unsigned)blocks, 256, 0, s>>>(b);
+    k_lora_mid_small_batch<<<(unsigned)blocks, 64 * kSmallWaves, 0, s>>>(b);
   return hipGetLastError();
 }
 
 hipError_t launch_lora_mid(const float* x, int m, int k, const float* a, int rank, float* mid, hipStream_t s) {
   if (m == 0 || rank == 0) return hipSuccess;
-  const bool dma = k % 4 == 0 && ((size_t)x & 15) == 0 && ((size_t)a & 15) == 0;
-  const int kr = (k + 255) & ~255;
-  if (dma && m <= DQ8_MID_SMALL_M && kr <= kSmallKR) {
-    // 4 x rows and 2 adapter rows per block (6 rows in LDS: the fewest for a
-    // wave of lane sums); measured 6.1 us at 24 x 2048 rank 16 against 8.4 for
-    // 8 x 4 blocks and 8.2 for the tiled kernel, 14.3 against 20.8 at k = 6144
-    k_lora_mid_small<<<(unsigned)lora_mid_small_blocks(m, rank), 256, 0, s>>>(x, m, k, a, rank, mid);
-  } else if (dma) {
-    const long blocks = (long)((m + kMidRows - 1) / kMidRows) * ((rank + kMidJ - 1) / kMidJ);
-    k_lora_mid_dma<<<(unsigned)blocks, 256, 0, s>>>(x, m, k, a, rank, mid);
+  if (lora_mid_small_ok(x, m, k, a)) {
+    k_lora_mid_small<<<(unsigned)lora_mid_small_blocks(m, rank), 64 * kSmallWaves, 0, s>>>(x, m, k, a, rank, mid);
+  } else if (lora_mid_tiled_ok(x, k, a)) {
+    k_lora_mid_dma<<<(unsigned)lora_mid_tiled_blocks(m, rank), 256, 0, s>>>(x, m, k, a, rank, mid);
   } else {
     const long waves = (long)((m + 3) / 4) * ((rank + 7) / 8);
     k_lora_mid_rows<<<blocks_for(waves, 4), 256, 0, s>>>(x, m, k, a, rank, mid);
@@ -3142,6 +3224,18 @@ hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, 
   const Divider wdiv = Divider::of((uint32_t)(((k + 255) / 256 + PER - 1) / PER));
   k_quantize<PER><<<blocks_for(waves, DQ8_QUANT_WPB), 64 * DQ8_QUANT_WPB, 0, s>>>(x, rows, k, q, ldq, scales, lds,
                                                                                  nonfinite, chain, wdiv);
+  return hipGetLastError();
+}
+
+bool quantize_mid_ok(const float* x, int m, int k, const int8_t* q, const float* a, int rank) {
+  return rank > 0 && k % 256 == 0 && ((uintptr_t)q & 3) == 0 && lora_mid_small_ok(x, m, k, a) && lora_mid_small_blocks(m, rank) <= 256;
+}
+hipError_t launch_quantize_mid(const float* x, int m, int k, int8_t* q, float* scales, uint32_t* nonfinite, Chain* chain,
+                               const float* a, int rank, float* mid, hipStream_t s) {
+  const int total = m * (k / 256), mids = (int)lora_mid_small_blocks(m, rank);
+  const int blocks = std::min(kQuantLoopBlocks, (total + kSmallWaves - 1) / kSmallWaves);
+  k_quantize_mid<<<mids + blocks, 64 * kSmallWaves, 0, s>>>(x, m, k, total, q, scales, nonfinite, chain,
+                                               Divider::of((uint32_t)(k / 256)), a, rank, mid, mids);
   return hipGetLastError();
 }
 

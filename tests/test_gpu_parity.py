@@ -595,8 +595,7 @@ def test_config1_single_linear_seed0_bit_exact(ctx):
 LORA_MID_SHAPES = [(1, 64, 1), (5, 131, 13), (24, 2048, 16), (67, 100, 3), (130, 2048, 16), (9, 7, 9), (4, 6144, 8),
                    (130, 2048, 40), (9, 256, 64), (300, 1000, 24), (16, 8, 17), (33, 4, 5), (8, 2052, 16),
                    (2048, 2048, 16), (17, 264, 33),
-                   # m <= 32: whole rows staged in LDS (4 x rows + 2 adapter rows per block) up to
-                   # k = 6656, beyond that the tiled kernel
+                   # m <= 32: the few-rows kernel (4 x rows + 2 adapter rows per block)
                    (32, 3328, 16), (32, 3332, 7), (20, 6656, 16), (5, 6660, 3), (31, 2048, 5), (32, 6144, 64)]
 
 
@@ -611,8 +610,8 @@ def test_lora_mid_bit_exact(ctx, m, k, rank):
 
 def test_lora_mid_batch_matches_single_calls(ctx):
     # adapters in one call: few-rows items share grouped launches (35 of them:
-    # two launches), items with more rows or k > 6656 share grouped launches of
-    # the tiled kernel, the rest (k % 4 != 0, unaligned x) run on their own and
+    # two launches), items with more rows share grouped launches of the tiled
+    # kernel, the rest (k % 4 != 0, unaligned x) run on their own and
     # rank 0 / m 0 do nothing; every result equals its single call and the oracle
     rng = np.random.default_rng(40)
     shapes = [(24, 2048, 16), (24, 6144, 16), (9, 512, 8), (32, 3332, 7), (1, 64, 1)] * 7 + \
@@ -1325,3 +1324,17 @@ def test_apply_non_finite_on_the_mid_and_wide_kernels(ctx, m, k, n):
                           (330, 256, 3100, (16, "aligned"), (16, "aligned"))])
 def test_mid_and_wide_ffn_gate_up(ctx, m, hidden, inter, gl, ul):
     test_ffn_gate_up_with_adapters(ctx, m, hidden, inter, gl, ul)
+
+
+# The few-rows middle-product kernel at its tile edges (512 inputs) and past its
+# ring of 8 tiles, and fused with h's quantization in dq8_ffn (widths of whole
+# 256-element chunks).
+@pytest.mark.parametrize("m,k,rank", [(4, 508, 2), (5, 512, 3), (3, 516, 1), (32, 1024, 16), (1, 764, 5), (2, 4096, 16),
+                                      (7, 4356, 9), (24, 8448, 16), (1, 4, 1)])
+def test_lora_mid_few_rows_edges(ctx, m, k, rank):
+    test_lora_mid_bit_exact(ctx, m, k, rank)
+
+
+@pytest.mark.parametrize("m,hidden,inter", [(1, 256, 256), (24, 256, 6144), (32, 320, 512), (40, 256, 512)])
+def test_ffn_chain_quantizes_beside_the_middle_product(ctx, m, hidden, inter):
+    test_ffn_chain_matches_the_reference_sequence(ctx, m, hidden, inter, True)
