@@ -795,6 +795,11 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
 // the device, with no synchronization.
 dq8_status apply_through(const dq8::Weights& w, const float* x, size_t m, const float* bias, const dq8_lora* lora,
                          float* out, int layout, int epilogue, const WorkInputs& in, dq8::Chain* chain, hipStream_t s) {
+  if (dq8::apply_few_ok((int)m, w.g, w.n)) {  // one launch, which quantizes in its blocks and chooses by itself
+    dq8::Proj p = {};
+    fill_proj(p, w, nullptr, 0, nullptr, 0, m, bias, out, nullptr, layout, epilogue, lora);
+    return from_hip(dq8::launch_apply_few(p, x, w.k, s));
+  }
   dq8_status st = from_hip(dq8::launch_quantize(x, (int)m, w.k, in.q, in.ldq, in.xs, in.ldxs, nullptr, chain, s));
   if (st != DQ8_OK) return st;
   const Fallback fb = {chain, x};

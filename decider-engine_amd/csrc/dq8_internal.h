@@ -190,6 +190,9 @@ hipError_t launch_lora_mid_batch(const MidBatch& b, long blocks, bool tiled, hip
 // 32, few blocks).  dots selects the debug kernel (not for kind 3).
 constexpr int kKinds = 4;
 hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s);
+// dq8_apply of a few rows x [m][k] in one launch (p's q and xs are not used).
+bool apply_few_ok(int m, int g, int n);
+hipError_t launch_apply_few(const Proj& p, const float* x, int k, hipStream_t s);
 // Columns of a skinny strip for g groups (all rows), and the waves that share
 // a strip's groups (1 or 4).
 // Skinny kernel paths: 1 segment (one wave per strip, all groups; short K) or

@@ -496,14 +496,19 @@ __device__ __forceinline__ float quant_scale_fma(float m) {
 // elements exactly.
 // FMA: u = v * rs + 128 rounded once instead of twice; u is then within 2^-16
 // + 2^-17 of Q + 128, inside the same margin.
-template <int N, bool FMA = false>
-__device__ __forceinline__ void quant_pack(const float (&v)[N], float scale, uint32_t (&w)[N / 4]) {
-  const float rs = __builtin_amdgcn_rcpf(scale);
+// (S > 1: N / S consecutive elements share a scale, so several chunks round side
+// by side.)
+template <int N, bool FMA = false, int S = 1>
+__device__ __forceinline__ void quant_pack(const float (&v)[N], const float (&scale)[S], uint32_t (&w)[N / 4]) {
+  float rs[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) rs[i] = __builtin_amdgcn_rcpf(scale[i]);
+  auto part = [](int i) { return i / (N / S); };
   float r[N];
   float fm = 0.0f;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const float u = FMA ? __builtin_fmaf(v[i], rs, 128.0f) : v[i] * rs + 128.0f;
+    const float u = FMA ? __builtin_fmaf(v[i], rs[part(i)], 128.0f) : v[i] * rs[part(i)] + 128.0f;
     r[i] = rintf(u);
     fm = fmaxf(fm, fabsf(u - r[i]));
   }
@@ -516,10 +521,10 @@ __device__ __forceinline__ void quant_pack(const float (&v)[N], float scale, uin
     asm volatile("");  // keeps the divisions inside the branch
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      const float u = FMA ? __builtin_fmaf(v[i], rs, 128.0f) : v[i] * rs + 128.0f;
+      const float u = FMA ? __builtin_fmaf(v[i], rs[part(i)], 128.0f) : v[i] * rs[part(i)] + 128.0f;
       if (__ballot(!(0.5f - fabsf(u - r[i]) > 0x1p-14f)) != 0) {
         asm volatile("");
-        r[i] = fminf(fmaxf(roundf(v[i] / scale), -127.0f), 127.0f) + 128.0f;
+        r[i] = fminf(fmaxf(roundf(v[i] / scale[part(i)]), -127.0f), 127.0f) + 128.0f;
       }
     }
   }
@@ -530,6 +535,11 @@ __device__ __forceinline__ void quant_pack(const float (&v)[N], float scale, uin
     for (int i = 0; i < 4; ++i) x = __builtin_amdgcn_cvt_pk_u8_f32(r[4 * j + i], i, x);
     w[j] = x ^ 0x80808080u;
   }
+}
+template <int N, bool FMA = false>
+__device__ __forceinline__ void quant_pack(const float (&v)[N], float scale, uint32_t (&w)[N / 4]) {
+  const float s1[1] = {scale};
+  quant_pack<N, FMA, 1>(v, s1, w);
 }
 
 // Quantization: QuantizedInputs::new (tensor.rs:321-339) and the 8-bit
@@ -2714,6 +2724,146 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
     }
   }
 }
+// ---------------------------------------------------------------------------
+// dq8_apply of at most kFewRows rows in one launch, Projection::apply_quantized
+// (tensor.rs:127-202) whole: every block quantizes all of x into its LDS (a few
+// KB; QuantizedInputs::new's arithmetic as in k_quantize_loop) while its weights
+// are in flight, so the quantizer's launch and its hand-off go.  A block covers
+// 16 columns; wave w takes groups w, w + 4, ..., every one of its weight
+// fragments loaded up front, and posts each group's t = dot * p; after one barrier
+// a thread per output adds its t's in group order.  All blocks see all of x, so
+// each knows by itself whether it is finite; if not, it computes the FP32 path.
+// GMAX bounds the groups (the posted t's are 1 KB per group), 4 * NMAX the
+// 256-input chunks of all rows.  Graph-replayed against the quantizer's launch and
+// the skinny kernel's, and submitted eagerly (a launch costs the host ~4 us): 1 x
+// 2048 -> 2048 4.7 and 6.8 us, eager 7.6 and 10.5; 2 rows 5.5 and 6.8; 4 rows 6.9
+// and 6.8, eager 7.4 and 10.5; 1 x 2048 -> 8224 7.4 and 9.1; 1 x 6144 -> 2048 10.4
+// and 12.0.  Past the bounds of few_kind the blocks' own quantization costs more:
+// 8 x 2048 -> 2048 9.7 and 6.8, 4 x 2048 -> 8224 (NMAX = 8: two blocks per CU) 13.6
+// and 9.1, 2 x 6144 -> 2048 11.9 and 12.0.
+constexpr int kFewRows = 8;
+template <int GMAX, int NMAX>
+__global__ __launch_bounds__(256) void k_apply_few(Proj P, const float* __restrict__ x, int k, Divider cdiv) {
+  constexpr int NG = GMAX / 4, QS = GMAX * kGroup + 16;  // groups per wave; LDS row stride
+  __shared__ __attribute__((aligned(16))) uint8_t qx[kFewRows * QS];
+  __shared__ float xs[kFewRows][GMAX];
+  __shared__ __attribute__((aligned(16))) float tp[GMAX][4][64];
+  static_assert(sizeof(tp) >= sizeof(F32Lds), "the FP32 tile fits");
+  const int G = P.g, m = P.m;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c0 = 16 * (int)blockIdx.x;
+  const uint8_t* pb;
+  const float* pw;
+  skinny_weights<true>(P, c0, lane, pb, pw);
+  v4i bq[NG];
+  float wq[NG];
+#pragma unroll
+  for (int i = 0; i < NG; ++i) {
+    const int g = min(4 * i + wid, G - 1);
+    bq[i] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(pb + (size_t)g * 2 * kFragBytes));
+    wq[i] = pw[(size_t)g * P.np];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // chunks of 256 inputs of a row, dealt to the waves
+  const int cpr = (G + 3) >> 2;
+  const bool vec = (k & 3) == 0 && ((uintptr_t)x & 15) == 0;
+  bool bad = false;
+  const int total = m * cpr;  // at most 4 * NMAX
+  // N chunks of a wave, every load out before the first is used and their
+  // arithmetic side by side (a wave alone on its SIMD would wait out each one)
+  auto quantize = [&](auto count) __attribute__((always_inline)) {
+    constexpr int N = decltype(count)::value;
+    float e[4 * N], ma[N], scale[N];
+    int row[N], k0[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int c = min(wid + 4 * u, total - 1);  // (past the end: the last chunk again, same bytes)
+      row[u] = cdiv.div((uint32_t)c);
+      k0[u] = (c - row[u] * cpr) * 256 + 4 * lane;
+      const float* xr = x + (size_t)row[u] * k;
+      if (vec) {  // uniform; k0 < k then holds for whole vectors
+        const v4f t = *reinterpret_cast<const v4f*>(xr + min(k0[u], k - 4));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[4 * u + i] = k0[u] < k ? t[i] : 0.0f;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float t = xr[min(k0[u] + i, k - 1)];
+          e[4 * u + i] = k0[u] + i < k ? t : 0.0f;
+        }
+      }
+    }
+    bool usual = true;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      uint32_t mb = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mb = max(mb, __builtin_bit_cast(uint32_t, e[4 * u + i]) & 0x7fffffffu);
+      bad |= mb >= 0x7f800000u;
+      ma[u] = max_row16(__builtin_bit_cast(float, mb));
+      // quant_scale_fma, its branch taken for all of them together
+      const float q0 = ma[u] * (1.0f / 127.0f);
+      scale[u] = __builtin_fmaf(__builtin_fmaf(-q0, 127.0f, ma[u]), 1.0f / 127.0f, q0);
+      usual = usual && ma[u] >= 0x1p-100f && ma[u] <= FLT_MAX;
+    }
+    if (__ballot(!usual) != 0) {
+#pragma unroll
+      for (int u = 0; u < N; ++u) scale[u] = quant_scale_fma(ma[u]);
+    }
+    uint32_t w[N];
+    quant_pack<4 * N, true, N>(e, scale, w);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int g = k0[u] >> 6;
+      if (g < G) {
+        *reinterpret_cast<uint32_t*>(qx + row[u] * QS + k0[u]) = w[u];
+        if ((lane & 15) == 0) xs[row[u]][g] = scale[u];
+      }
+    }
+  };
+  if (NMAX == 4 && total <= 8) quantize(std::integral_constant<int, 2>{});
+  else quantize(std::integral_constant<int, NMAX>{});
+  if (__syncthreads_or(bad)) {  // the FP32 path of this block's outputs
+    wait_vmcnt<0>();
+    fp32_block<1>(P, x, k, 0, m, c0, min(c0 + 16, P.n), reinterpret_cast<uint8_t*>(&tp));
+    return;
+  }
+  const v4i magic = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
+  const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  const uint8_t* qa = qx + min(lane & 15, m - 1) * QS + 16 * (lane >> 4);
+  const float* xa = xs[min(4 * (lane >> 4) + (lane & 3), m - 1)];
+#pragma unroll
+  for (int i = 0; i < NG; ++i) {
+    const int g = 4 * i + wid;
+    if (g < G) {  // wave-uniform
+      const v4i dd = mfma_i8_16(*reinterpret_cast<const v4i*>(qa + g * kGroup), bq[i], magic);
+      const v4f dv = mfma_k1_4(-kMagic, 1.0f, __builtin_bit_cast(v4f, dd));
+      const v4f pv = mfma_k1_4(xa[g], wq[i], zero4);
+      const v4f t = dv * pv;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) tp[g][v][lane] = t[v];
+    }
+  }
+  __syncthreads();
+  // thread (wid, lane): output row 4*(lane/16) + wid, column c0 + lane%16
+  const int row = 4 * (lane >> 4) + wid, col = c0 + (lane & 15);
+  if (row >= m || col >= P.n) return;
+  float s = 0.0f;
+#pragma unroll 8
+  for (int g = 0; g < G; ++g) s = s + tp[g][wid][lane];
+  float y = s + (P.bias ? P.bias[col] : 0.0f);  // tensor.rs:437
+  if (P.lora) {                                 // Adapter::combine (tensor.rs:109-117)
+    const float d =
+        (P.rank > 0 ? dot_scores_rows(P.lmid + (size_t)row * P.rank, P.lb + (size_t)col * P.rank, P.rank) : -0.0f) + 0.0f;
+    const float scaled = P.lscale * d;
+    y = y + scaled;
+  }
+  float* dst = P.layout == 1 ? P.out + (size_t)col * P.m + row : P.out + (size_t)row * P.n + col;
+  if (P.epilogue == 0 || P.layout == 1) *dst = y;
+  else if (P.epilogue == 1) *dst = *dst + y;
+  else *dst = silu(*dst) * y;
+}
 // LoRA middle product (weights.rs:480, 495): mid[r][j] = dot_scores(x_r, a_j)
 // + 0.0 for x [m][k], a [rank][k], in dot_scores' x86-64 order (tensor.rs:6-25).
 // Two kernels compute it in that order.  k_lora_mid_rows reads plain memory and
@@ -2989,10 +3139,12 @@ __global__ __launch_bounds__(256) void k_lora_mid_dma_batch(MidBatch bt) {
 // tile t - 2.  The 8 lane sums of a pair, in consecutive lanes, are then added
 // in order from -0.0, then the tail elements.  Loads past a row's end are
 // clamped to its last 16 bytes; their products are never added.
-// Requires k % 4 == 0 and 16-byte aligned x and a.  24 rows, rank 16, by
-// rocprof: MIDS_FIG (one wave reading
-// both operands, multiplying and adding, after whole rows had landed: 5.4 us at
-// K = 2048, 11.4 at 6144).
+// Requires k % 4 == 0 and 16-byte aligned x and a.  24 rows, rank 16, graph-
+// replayed: 4.7 us at K = 2048 and 8.3 at 6144 (5.3 and 11.5 with one wave
+// reading both operands, multiplying and adding after whole rows had landed).
+// A tile now moves 76 KB through LDS, ~600 of its ~970 cycles; 256-input tiles
+// (one barrier per 32 steps) took 19 us at 6144, 3 producers of two rows each the
+// same 8.4.
 constexpr int kSmallR = 4, kSmallJ = 2, kSmallSlots = 8, kSmallKT = 512, kSmallSteps = kSmallKT / 8;
 constexpr int kSmallWaves = 1 + kSmallR + kSmallJ;
 struct SmallLds {
@@ -3118,7 +3270,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_lora_mid_small(const float
 // A few rows' quantization and one adapter's middle product of the same x in
 // one launch: neither needs the other, and neither fills the GPU (24 x 6144,
 // rank 16: 144 quantizer blocks beside 48 blocks of the middle product, which
-// come first).  A dq8_ffn's h: QMID_FIG.
+// come first).  That case by
+// rocprof: 9.3 us against 4.7 + 11.4 for the two launches.
 __global__ __launch_bounds__(64 * kSmallWaves) void k_quantize_mid(const float* __restrict__ x, int m, int k, int total,
                                                       int8_t* __restrict__ q, float* __restrict__ scales,
                                                       uint32_t* nonfinite, Chain* chain, Divider cdiv,
@@ -3314,6 +3467,27 @@ int block_cols(int kind, bool pair) {
   return kind == 0 ? 32 * DQ8_WIDE_CT * DQ8_WIDE_WN / (pair ? 2 : 1) : 64;
 }
 bool wide_can_pair() { return wide_pair_shape(DQ8_WIDE_WN, DQ8_WIDE_RT, DQ8_WIDE_CT); }
+
+// The instance of k_apply_few for m rows, g groups and n outputs: 4 or 8 chunks per
+// wave (the latter's registers leave two blocks per CU: one round of 4096 outputs),
+// or 96 groups and 6 chunks (one block per CU by its LDS); 0: none.
+static int few_kind(int m, int g, int n) {
+  const int chunks = m <= kFewRows ? m * ((g + 3) / 4) : 1 << 30;
+  if (g <= 32) return chunks <= 16 ? 4 : chunks <= 32 && n <= 4096 ? 8 : 0;
+  return g <= 96 && chunks <= 24 && n <= 4096 ? 6 : 0;
+}
+bool apply_few_ok(int m, int g, int n) { return few_kind(m, g, n) != 0; }
+hipError_t launch_apply_few(const Proj& p, const float* x, int k, hipStream_t s) {
+  const unsigned blocks = (unsigned)((p.n + 15) / 16);
+  const Divider cdiv = Divider::of((uint32_t)((p.g + 3) / 4));
+  switch (few_kind(p.m, p.g, p.n)) {
+    case 4: k_apply_few<32, 4><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
+    case 8: k_apply_few<32, 8><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
+    case 6: k_apply_few<96, 6><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
 
 hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s) {
   if (b.total_waves == 0) return hipSuccess;

@@ -127,3 +127,33 @@ def test_ffn_with_a_non_finite_h_takes_the_fp32_down(ctx, m):
     assert fp32
     assert same(host(resid), want_r)
     assert int(host(flag)[0]) == 1
+
+
+# dq8_apply of a few rows in one launch (quantization and the choice of path
+# inside its blocks): the bounds of each instance (rows, chunks, groups, outputs)
+# and just past them, a partial last group, widths of no whole vector, an
+# unaligned x, the columns layout.
+@pytest.mark.parametrize("m,k,n,rank", [(1, 2048, 100, 0), (2, 2048, 33, 16), (4, 2048, 33, 16), (5, 2048, 33, 16),
+                                        (8, 512, 40, 0), (9, 64, 40, 0), (3, 1, 1, 0), (5, 67, 17, 3), (2, 2049, 16, 0),
+                                        (1, 6144, 40, 5), (1, 6145, 20, 0), (3, 1500, 4100, 0), (2, 1111, 4100, 2)])
+@pytest.mark.parametrize("bad", [False, True])
+def test_apply_few_rows(ctx, m, k, n, rank, bad):
+    rng = np.random.default_rng(m + k + n + rank)
+    x, v, s, bias, a, b = case(rng, m, k, n, rank)
+    if bad:
+        x[m - 1, k - 1] = np.nan
+    h = ctx.weights_from_quantized(dev(v), dev(s))
+    base = rng.standard_normal((m, n)).astype(np.float32)
+    store = torch.empty(m * k + 1, device="cuda")
+    for off in (0, 1):
+        xd = store[off:off + m * k].view(m, k)
+        xd.copy_(dev(x))
+        lora = dq8.Lora(ctx.lora_mid(xd, dev(a)), dev(b), 0.5) if rank else None
+        for ep in (dq8.WRITE, dq8.ADD, dq8.SWIGLU):
+            got = host(ctx.apply(h, xd, out=dev(base.copy()), bias=dev(bias), lora=lora, epilogue=ep))
+            want, fp32 = dq8o.apply(x, v, s, bias=bias, a=a, b=b, scale=0.5, result=base, epilogue=ep, threads=8)
+            assert fp32 == bad
+            assert same(got, want)
+        cols = host(ctx.apply(h, xd, bias=dev(bias), lora=lora, layout=dq8.COLUMNS))
+        want, _ = dq8o.apply(x, v, s, bias=bias, a=a, b=b, scale=0.5, result=base, epilogue=0, threads=8)
+        assert same(cols, np.ascontiguousarray(want.T))
