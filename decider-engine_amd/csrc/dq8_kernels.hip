@@ -2656,6 +2656,21 @@ __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, i
   return false;
 }
 
+// One 16-row tile per long-K block: 17-32 rows take two blocks per strip.  The
+// two blocks of a strip are 8 apart (blocks are dealt to the 8 XCDs in turn), so
+// both run on one XCD and the second read of the strip's weights is served by
+// that XCD's L2: in each run of 16 blocks, blocks 0-7 take the first row tile of
+// 8 strips and blocks 8-15 the second.  A last run of R < 8 strips pairs blocks R
+// apart.  strip: the block of the projection in, its strip out; r0: its first row.
+__device__ __forceinline__ void skinny_row_tile(const Proj& P, int& strip, int& r0) {
+  const int run = strip >> 4, in = strip & 15;
+  const int left = P.waves_n - 8 * run;  // strips from this run on
+  const int r = left >= 8 ? 8 : left;
+  const int t = r == 8 ? in >> 3 : in / r;  // the row tile (a division only in the last run)
+  strip = 8 * run + in - t * r;
+  r0 = 16 * t;
+}
+
 template <int RT, int CT, int CTL, int DBS, int DBL, bool DOTS, bool LORA>
 __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[skinny_lds_bytes(RT, CTL)];
@@ -2699,18 +2714,7 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   } else {
     int strip = local;
     if (RT == 2) {
-      // One 16-row tile per block: 17-32 rows take two blocks per strip.  The
-      // two blocks of a strip are 8 apart (blocks are dealt to the 8 XCDs in
-      // turn), so both run on one XCD and the second read of the strip's weights
-      // is served by that XCD's L2: in each run of 16 blocks, blocks 0-7 take
-      // the first row tile of 8 strips and blocks 8-15 the second.  A last run
-      // of R < 8 strips pairs blocks R apart.
-      const int run = local >> 4, in = local & 15;
-      const int left = P.waves_n - 8 * run;  // strips from this run on
-      const int r = left >= 8 ? 8 : left;
-      const int t = r == 8 ? in >> 3 : in / r;  // the row tile (a division only in the last run)
-      strip = 8 * run + in - t * r;
-      m0 = 16 * t;
+      skinny_row_tile(P, strip, m0);
       mhi = min(mhi, m0 + 16);
     }
     nlo = 16 * CTL * strip;
@@ -2724,6 +2728,120 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
     }
   }
 }
+// The long-K path for launches of few blocks, without its step-by-step hand-off:
+// a block still covers 16 columns x 16 rows, but its waves have every weight,
+// activation and scale load of their groups (w, w + 4, ...) out before the first
+// product, post all t's (1 KB per group), and after the one barrier a thread per
+// output adds its t's in group order.  GMAX bounds the groups
+// (post_groups).  Bound by latency and, at 96 groups, by the CU's load path: 196 KB
+// per block.
+template <int GMAX, bool TWO, bool LORA>
+__global__ __launch_bounds__(256) void k_linear_post(Batch b) {
+  constexpr int NG = GMAX / 4;
+  __shared__ __attribute__((aligned(16))) float xl[16][GMAX + 4];
+  __shared__ __attribute__((aligned(16))) float tp[GMAX][4][64];
+  static_assert(sizeof(tp) >= sizeof(F32Lds), "the FP32 tile fits");
+  const int pidx = find_proj<true>(b, blockIdx.x);
+  const Proj P = b.p[pidx];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = P.g;
+  int strip = blockIdx.x - P.wave_begin, r0 = 0;
+  if (TWO) skinny_row_tile(P, strip, r0);
+  const int c0 = 16 * strip;
+  // x scales: thread t takes 4-group pieces t%16, t%16 + 16, .. of row t/16
+  // (rows of 16-byte aligned multiples of 4 floats)
+  constexpr int XN = (GMAX / 4 + 15) / 16;
+  v4f xv[XN];
+  const float* xr = P.xs + (size_t)min(r0 + (int)(threadIdx.x >> 4), P.m - 1) * P.ldxs;
+  const int last_piece = (G + 3) / 4 - 1;
+#pragma unroll
+  for (int i = 0; i < XN; ++i)
+    xv[i] = *reinterpret_cast<const v4f*>(xr + 4 * min((int)(threadIdx.x & 15) + 16 * i, last_piece));
+  const uint8_t* pb;
+  const float* pw;
+  skinny_weights<true>(P, c0, lane, pb, pw);
+  const int8_t* pa = P.q + (size_t)min(r0 + (lane & 15), P.m - 1) * P.ldq + 16 * (lane >> 4);
+  v4i aq[NG], bq[NG];
+  float wq[NG];
+#pragma unroll
+  for (int i = 0; i < NG; ++i) {
+    const int g = min(4 * i + wid, G - 1);
+    bq[i] = load16(pb + (size_t)g * 2 * kFragBytes);
+    aq[i] = load16(pa + g * kGroup);
+    wq[i] = pw[(size_t)g * P.np];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (b.chain) {  // uniform; non-finite inputs: the FP32 path of this block's outputs
+    const bool hit = chain_hit(b.chain);
+    chain_close(b.chain);
+    if (hit) {
+      fp32_block<1>(P, b.fx[pidx], b.fk, r0, min(r0 + 16, P.m), c0, min(c0 + 16, P.n), reinterpret_cast<uint8_t*>(&tp));
+      return;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < XN; ++i) {
+    const int pc = (int)(threadIdx.x & 15) + 16 * i;
+    if (pc <= last_piece) *reinterpret_cast<v4f*>(&xl[threadIdx.x >> 4][4 * pc]) = xv[i];
+  }
+  lds_barrier();  // (waits for no weight load)
+  const v4i magic = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
+  const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  const float* xa = xl[4 * (lane >> 4) + (lane & 3)];
+#pragma unroll
+  for (int i = 0; i < NG; ++i) {
+    const int g = 4 * i + wid;
+    const v4i dd = mfma_i8_16(aq[i], bq[i], magic);
+    const v4f dv = mfma_k1_4(-kMagic, 1.0f, __builtin_bit_cast(v4f, dd));
+    const v4f pv = mfma_k1_4(xa[min(g, G - 1)], wq[i], zero4);
+    const v4f t = dv * pv;
+    if (g < G) {  // wave-uniform
+#pragma unroll
+      for (int v = 0; v < 4; ++v) tp[g][v][lane] = t[v];
+    }
+  }
+  // thread (wid, lane): output row r0 + 4*(lane/16) + wid, column c0 + lane%16
+  const int row = r0 + 4 * (lane >> 4) + wid, col = c0 + (lane & 15);
+  const int rc = min(row, P.m - 1), cc = min(col, P.n - 1);
+  const float bias = P.bias != nullptr ? P.bias[cc] : 0.0f;
+  // what the epilogue reads, loaded before the sums
+  const bool l16 = LORA && P.lora && P.rank == 16 && ((size_t)P.lmid & 15) == 0 && ((size_t)P.lb & 15) == 0;  // uniform
+  v4f lm[4], lb[4];
+  if (l16) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      lm[q] = *reinterpret_cast<const v4f*>(P.lmid + (size_t)rc * 16 + 4 * q);
+      lb[q] = *reinterpret_cast<const v4f*>(P.lb + (size_t)cc * 16 + 4 * q);
+    }
+  }
+  float* dst = P.layout == 1 ? P.out + (size_t)cc * P.m + rc : P.out + (size_t)rc * P.n + cc;
+  const float old = P.epilogue != 0 ? *dst : 0.0f;
+  lds_barrier();
+  float s = 0.0f;
+#pragma unroll 8
+  for (int g = 0; g < G; ++g) s = s + tp[g][wid][lane];
+  float y = s + bias;  // tensor.rs:437
+  if (LORA && P.lora) {  // Adapter::combine (tensor.rs:109-117), dot_scores' order
+    float d;
+    if (l16) {
+      d = -0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float lo = lm[i >> 2][i & 3] * lb[i >> 2][i & 3], hi = lm[2 + (i >> 2)][i & 3] * lb[2 + (i >> 2)][i & 3];
+        d = d + ((0.0f + lo) + hi);
+      }
+    } else {
+      d = P.rank > 0 ? dot_scores_rows(P.lmid + (size_t)rc * P.rank, P.lb + (size_t)cc * P.rank, P.rank) : -0.0f;
+    }
+    const float scaled = P.lscale * (d + 0.0f);
+    y = y + scaled;
+  }
+  if (P.epilogue == 1) y = old + y;
+  if (P.epilogue == 2) y = silu(old) * y;
+  if (row < P.m && col < P.n) st_out(dst, y);
+}
+
 // ---------------------------------------------------------------------------
 // dq8_apply of at most kFewRows rows in one launch, Projection::apply_quantized
 // (tensor.rs:127-202) whole: every block quantizes all of x into its LDS (a few
@@ -2733,18 +2851,18 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
 // fragments loaded up front, and posts each group's t = dot * p; after one barrier
 // a thread per output adds its t's in group order.  All blocks see all of x, so
 // each knows by itself whether it is finite; if not, it computes the FP32 path.
-// GMAX bounds the groups (the posted t's are 1 KB per group), 4 * NMAX the
-// 256-input chunks of all rows.  Graph-replayed against the quantizer's launch and
-// the skinny kernel's, and submitted eagerly (a launch costs the host ~4 us): 1 x
-// 2048 -> 2048 4.7 and 6.8 us, eager 7.6 and 10.5; 2 rows 5.5 and 6.8; 4 rows 6.9
-// and 6.8, eager 7.4 and 10.5; 1 x 2048 -> 8224 7.4 and 9.1; 1 x 6144 -> 2048 10.4
-// and 12.0.  Past the bounds of few_kind the blocks' own quantization costs more:
-// 8 x 2048 -> 2048 9.7 and 6.8, 4 x 2048 -> 8224 (NMAX = 8: two blocks per CU) 13.6
-// and 9.1, 2 x 6144 -> 2048 11.9 and 12.0.
+// At most 32 groups (the posted t's are 1 KB per group) and 4 * NMAX chunks of 256
+// inputs in all rows.  Graph-replayed against the quantizer's launch and the
+// posting kernel's, and submitted eagerly (a launch costs the host ~4 us): 1 x
+// 2048 -> 2048 4.8 and 5.8 us, eager 5.9 and 9.0; 2 rows 5.5 and 5.8, eager 5.9 and
+// 9.0; 4 rows 7.1 and 5.8, eager 6.9 and 9.0; 1 x 2048 -> 8224 7.1 and 9.0.  Past the
+// bounds of few_kind the blocks' own quantization costs more: 8 x 2048 -> 2048 9.7
+// and 5.8, 4 x 2048 -> 8224 13.6 and 9.0; 1 x 6144 -> 2048 (all 96 groups posted) 9.5
+// and 9.5.
 constexpr int kFewRows = 8;
-template <int GMAX, int NMAX>
+template <int NMAX>
 __global__ __launch_bounds__(256) void k_apply_few(Proj P, const float* __restrict__ x, int k, Divider cdiv) {
-  constexpr int NG = GMAX / 4, QS = GMAX * kGroup + 16;  // groups per wave; LDS row stride
+  constexpr int GMAX = 32, NG = GMAX / 4, QS = GMAX * kGroup + 16;  // groups, per wave; LDS row stride
   __shared__ __attribute__((aligned(16))) uint8_t qx[kFewRows * QS];
   __shared__ float xs[kFewRows][GMAX];
   __shared__ __attribute__((aligned(16))) float tp[GMAX][4][64];
@@ -3466,24 +3584,39 @@ int block_rows(int kind, bool pair) { return kind == 0 ? 32 * DQ8_WIDE_RT * DQ8_
 int block_cols(int kind, bool pair) {
   return kind == 0 ? 32 * DQ8_WIDE_CT * DQ8_WIDE_WN / (pair ? 2 : 1) : 64;
 }
+// The group bound of the posting kernel (k_linear_post) that takes a skinny launch,
+// or 0: every projection on the 4-wave path, and up to 32 groups, or 65 to 96 in at
+// most one block per CU (its LDS).  Graph-replayed, 24 rows, against the skinny
+// kernel: 2048 -> 2048 3.8 and 4.6 us, 2048 -> 4608 (576 blocks) 7.2 and 9.0, 6144
+// -> 2048 9.1 and 9.8; 4096 -> 2048 (64 groups, a third of the loads repeats) 8.6
+// and 7.3, 6144 -> 4096 (512 blocks) 16.1 and 12.3.
+static int post_groups(const Batch& b) {
+  int lo = 1 << 30, hi = 0;
+  for (int i = 0; i < b.count; ++i) {
+    if (b.p[i].nseg != 4 || b.p[i].pair) return 0;
+    lo = std::min(lo, b.p[i].g);
+    hi = std::max(hi, b.p[i].g);
+  }
+  if (hi <= 32) return 32;
+  return lo > 64 && hi <= 96 && b.total_waves <= 256 ? 96 : 0;
+}
 bool wide_can_pair() { return wide_pair_shape(DQ8_WIDE_WN, DQ8_WIDE_RT, DQ8_WIDE_CT); }
 
 // The instance of k_apply_few for m rows, g groups and n outputs: 4 or 8 chunks per
-// wave (the latter's registers leave two blocks per CU: one round of 4096 outputs),
-// or 96 groups and 6 chunks (one block per CU by its LDS); 0: none.
+// wave (the latter's registers leave two blocks per CU: one round of 4096
+// outputs); 0: none.
 static int few_kind(int m, int g, int n) {
-  const int chunks = m <= kFewRows ? m * ((g + 3) / 4) : 1 << 30;
-  if (g <= 32) return chunks <= 16 ? 4 : chunks <= 32 && n <= 4096 ? 8 : 0;
-  return g <= 96 && chunks <= 24 && n <= 4096 ? 6 : 0;
+  if (m > kFewRows || g > 32) return 0;
+  const int chunks = m * ((g + 3) / 4);
+  return chunks <= 16 ? 4 : chunks <= 32 && n <= 4096 ? 8 : 0;
 }
 bool apply_few_ok(int m, int g, int n) { return few_kind(m, g, n) != 0; }
 hipError_t launch_apply_few(const Proj& p, const float* x, int k, hipStream_t s) {
   const unsigned blocks = (unsigned)((p.n + 15) / 16);
   const Divider cdiv = Divider::of((uint32_t)((p.g + 3) / 4));
   switch (few_kind(p.m, p.g, p.n)) {
-    case 4: k_apply_few<32, 4><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
-    case 8: k_apply_few<32, 8><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
-    case 6: k_apply_few<96, 6><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
+    case 4: k_apply_few<4><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
+    case 8: k_apply_few<8><<<blocks, 256, 0, s>>>(p, x, k, cdiv); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -3549,6 +3682,18 @@ hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s) {
            : k_linear_mid<2, 2, kMidRing, false, false><<<b.total_waves, 256, 0, s>>>(b);
     return hipGetLastError();
   }
+  const int post = dots ? 0 : post_groups(b);
+#define DQ8_POST(GM, T) \
+  (lora ? k_linear_post<GM, T, true><<<b.total_waves, 256, 0, s>>>(b) : k_linear_post<GM, T, false><<<b.total_waves, 256, 0, s>>>(b))
+  if (post == 32) {
+    kind == 2 ? DQ8_POST(32, true) : DQ8_POST(32, false);
+    return hipGetLastError();
+  }
+  if (post == 96) {
+    kind == 2 ? DQ8_POST(96, true) : DQ8_POST(96, false);
+    return hipGetLastError();
+  }
+#undef DQ8_POST
   // total_waves counts blocks of 4 waves for the skinny kernel; kind 1: M <= 16, kind 2: M <= 32
   constexpr int CT = DQ8_SKINNY_CT, CL = DQ8_SKINNY_CTL;
 #define DQ8_SKINNY(R, D, L)                                                                                  \

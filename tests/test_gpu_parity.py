@@ -1289,8 +1289,8 @@ def test_mid_and_wide_kernel_edges(ctx, m, k, n, rank):
             want = dq8o.linear_lora(x, wv, ws, a, b, -0.75, bias=bias, result=base, epilogue=ep, threads=8)
             got = ctx.linear_lora(h, q, s, lora, out=dev(base.copy()), bias=dev(bias), epilogue=ep)
         assert bits_equal(host(got), want)
-    if rank is None:  # columns, from 33 rows up
-        for rows in (33, m):
+    if rank is None:  # columns
+        for rows in (min(33, m), m):
             got = host(ctx.linear(h, q[:rows], s[:rows], layout=dq8.COLUMNS))
             assert bits_equal(got, np.ascontiguousarray(dq8o.linear(x[:rows], wv, ws, threads=8).T))
 
@@ -1338,3 +1338,13 @@ def test_lora_mid_few_rows_edges(ctx, m, k, rank):
 @pytest.mark.parametrize("m,hidden,inter", [(1, 256, 256), (24, 256, 6144), (32, 320, 512), (40, 256, 512)])
 def test_ffn_chain_quantizes_beside_the_middle_product(ctx, m, hidden, inter):
     test_ffn_chain_matches_the_reference_sequence(ctx, m, hidden, inter, True)
+
+
+# The posting kernel (few strips, up to 32 groups or 65 to 96) at its bounds and
+# just past them: one group, a partial last one, 64 / 65 / 96 / 97 groups, one and
+# two row tiles, a last run of fewer than 8 strips, more than 256 blocks.
+@pytest.mark.parametrize("m,k,n,rank", [(1, 64, 16, None), (16, 2048, 33, 16), (31, 2047, 50, 5), (17, 4096, 40, 16),
+                                        (17, 4160, 200, 16), (32, 6144, 2064, None), (20, 6144, 70, 20),
+                                        (9, 6145, 48, None), (33, 1000, 100, 16)])
+def test_posting_kernel_edges(ctx, m, k, n, rank):
+    test_mid_and_wide_kernel_edges(ctx, m, k, n, rank)
