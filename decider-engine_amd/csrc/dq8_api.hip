@@ -291,10 +291,11 @@ void xcd_chunks(dq8::Proj& p, int kind, int row_tiles) {
 int kind_of(const dq8::Weights&, size_t m) { return m > 32 ? 0 : m > 16 ? 2 : 1; }
 
 // A skinny launch whose projections would run on fewer 32-column strips than
-// this takes the 4-wave path for all of them: each wave then streams a quarter
+// this takes the 4-wave path for all of them (k_linear_post where it takes the
+// groups, otherwise the skinny kernel's): each wave then streams a quarter
 // of a strip's groups, so 4x the waves keep weight loads in flight.  Measured
-// at 24 rows, graph-replayed, 4-wave path against short-K blocks of dealt
-// units: 2048x2048 (64 strips) 4.9 against 8.0 us, o + GDN out (128) 7.6
+// at 24 rows, graph-replayed, the skinny kernel's 4-wave path (k_linear_post takes
+// 3.8 for its 4.6 us) against short-K blocks of dealt units: 2048x2048 (64 strips) 4.9 against 8.0 us, o + GDN out (128) 7.6
 // against 8.3 us, 2048x6144 (192) 10.6 against 8.3 us, GDN in (257) 10.4
 // against 8.2 us.
 constexpr long kSkinnyFewStrips = 160;
@@ -920,10 +921,16 @@ dq8_status dq8_create(int device, dq8_ctx** out) {
   dq8_ctx* ctx = new (std::nothrow) dq8_ctx();
   if (!ctx) return DQ8_ERR_NOMEM;
   ctx->device = device;
-  // the chain state, then the flag
+  // the chain state, then the flag, zero before any stream's first call (cleared
+  // on a stream of its own: the NULL stream may not be used while another stream
+  // captures)
+  RelaxedCapture relaxed;
+  hipStream_t own = nullptr;
   hipError_t e = hipMalloc(&ctx->chain_state, sizeof(dq8::Chain) + sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMemset(ctx->chain_state, 0, sizeof(dq8::Chain) + sizeof(uint32_t));
-  if (e == hipSuccess) e = hipDeviceSynchronize();  // zero before any stream's first call
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipMemsetAsync(ctx->chain_state, 0, sizeof(dq8::Chain) + sizeof(uint32_t), own);
+  if (e == hipSuccess) e = hipStreamSynchronize(own);
+  if (own) (void)hipStreamDestroy(own);
   ctx->flag = reinterpret_cast<uint32_t*>(ctx->chain_state + 1);
   if (e == hipSuccess) e = hipHostMalloc(&ctx->host_flag, sizeof(uint32_t), hipHostMallocDefault);
   if (e != hipSuccess) {
@@ -1187,11 +1194,14 @@ dq8_status dq8_lora_mid_batch(dq8_ctx* ctx, const dq8_lora_mid_item* items, size
   dq8::MidBatch b[2];
   long blocks[2] = {0, 0};
   b[0].count = b[1].count = 0;
+  long few = 0;  // the few-rows kernel's blocks of every item
+  for (size_t i = 0; i < count; ++i)
+    if (items[i].m && items[i].rank) few += dq8::lora_mid_small_blocks((int)items[i].m, (int)items[i].rank);
   for (size_t i = 0; i < count; ++i) {
     const dq8_lora_mid_item& it = items[i];
     if (it.m == 0 || it.rank == 0) continue;
     const int m = (int)it.m, k = (int)it.k, rank = (int)it.rank;
-    const bool small = dq8::lora_mid_small_ok(it.x, m, k, it.a);
+    const bool small = dq8::lora_mid_small_ok(it.x, m, k, it.a, few);
     if (!small && !dq8::lora_mid_tiled_ok(it.x, k, it.a)) {  // the plain-memory kernel: a launch of its own
       hipError_t e = dq8::launch_lora_mid(it.x, m, k, it.a, rank, it.mid, s);
       if (e != hipSuccess) return from_hip(e);

@@ -181,7 +181,7 @@ hipError_t launch_chain_reset(Chain* chain, hipStream_t s);
 hipError_t launch_linear_fp32(const FProj& p, hipStream_t s);
 // LoRA middle product mid [m][rank] = dot_scores(x_r, a_j) + 0.0 (x [m][k], a [rank][k]).
 hipError_t launch_lora_mid(const float* x, int m, int k, const float* a, int rank, float* mid, hipStream_t s);
-bool lora_mid_small_ok(const float* x, int m, int k, const float* a);  // the few-rows kernel takes it
+bool lora_mid_small_ok(const float* x, int m, int k, const float* a, long blocks);  // the few-rows kernel takes it
 long lora_mid_small_blocks(int m, int rank);
 bool lora_mid_tiled_ok(const float* x, int k, const float* a);  // otherwise the LDS-tiled kernel, if this holds
 long lora_mid_tiled_blocks(int m, int rank);

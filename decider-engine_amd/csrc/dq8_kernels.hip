@@ -3246,7 +3246,7 @@ __global__ __launch_bounds__(256) void k_lora_mid_dma_batch(MidBatch bt) {
   lora_mid_tiled(I.x, I.m, I.k, I.a, I.rank, I.mid, b - I.block_begin, lds);
 }
 
-// k_lora_mid_small: few rows (m <= 32).  A block covers 4 rows of x and 2
+// k_lora_mid_small: few rows (lora_mid_small_ok).  A block covers 4 rows of x and 2
 // adapter rows: 64 lane sums, one per lane of wave 0, which only adds.  The
 // time is that chain (K/8 dependent adds of ~9.5 cycles), so everything else is
 // kept off it: waves 1-6 load 512-input tiles of the 6 rows into a ring by
@@ -3438,8 +3438,15 @@ hipError_t launch_linear_fp32(const FProj& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-bool lora_mid_small_ok(const float* x, int m, int k, const float* a) {
-  return k % 4 == 0 && ((size_t)x & 15) == 0 && ((size_t)a & 15) == 0 && m <= DQ8_MID_SMALL_M;
+// Whether the few-rows kernel takes a middle product, in a call whose products
+// would make `blocks` of its blocks (lora_mid_small_blocks): any up to 32 rows, and
+// one round of one block per CU.  The tiled kernel's few blocks take 8.9 us at K =
+// 2048 and 21.5 at 6144 whatever their number; graph-replayed at rank 16 this one
+// takes 5.3 and 9.8 at 77 rows (160 blocks), 10.6 at 128 x 6144 (256); past the
+// round 9.3 for two of 128 x 2048 (512), 10.2 at 200 x 2048 (400).
+constexpr long kSmallBlocks = 256;
+bool lora_mid_small_ok(const float* x, int m, int k, const float* a, long blocks) {
+  return k % 4 == 0 && ((size_t)x & 15) == 0 && ((size_t)a & 15) == 0 && (m <= DQ8_MID_SMALL_M || blocks <= kSmallBlocks);
 }
 long lora_mid_small_blocks(int m, int rank) { return (long)((m + kSmallR - 1) / kSmallR) * ((rank + kSmallJ - 1) / kSmallJ); }
 
@@ -3461,7 +3468,7 @@ hipError_t launch_lora_mid_batch(const MidBatch& b, long blocks, bool tiled, hip
 
 hipError_t launch_lora_mid(const float* x, int m, int k, const float* a, int rank, float* mid, hipStream_t s) {
   if (m == 0 || rank == 0) return hipSuccess;
-  if (lora_mid_small_ok(x, m, k, a)) {
+  if (lora_mid_small_ok(x, m, k, a, lora_mid_small_blocks(m, rank))) {
     k_lora_mid_small<<<(unsigned)lora_mid_small_blocks(m, rank), 64 * kSmallWaves, 0, s>>>(x, m, k, a, rank, mid);
   } else if (lora_mid_tiled_ok(x, k, a)) {
     k_lora_mid_dma<<<(unsigned)lora_mid_tiled_blocks(m, rank), 256, 0, s>>>(x, m, k, a, rank, mid);
@@ -3499,7 +3506,8 @@ hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, 
 }
 
 bool quantize_mid_ok(const float* x, int m, int k, const int8_t* q, const float* a, int rank) {
-  return rank > 0 && k % 256 == 0 && ((uintptr_t)q & 3) == 0 && lora_mid_small_ok(x, m, k, a) && lora_mid_small_blocks(m, rank) <= 256;
+  return rank > 0 && k % 256 == 0 && ((uintptr_t)q & 3) == 0 && lora_mid_small_blocks(m, rank) <= 256 &&
+         lora_mid_small_ok(x, m, k, a, 0);
 }
 hipError_t launch_quantize_mid(const float* x, int m, int k, int8_t* q, float* scales, uint32_t* nonfinite, Chain* chain,
                                const float* a, int rank, float* mid, hipStream_t s) {

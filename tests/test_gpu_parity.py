@@ -595,7 +595,7 @@ def test_config1_single_linear_seed0_bit_exact(ctx):
 LORA_MID_SHAPES = [(1, 64, 1), (5, 131, 13), (24, 2048, 16), (67, 100, 3), (130, 2048, 16), (9, 7, 9), (4, 6144, 8),
                    (130, 2048, 40), (9, 256, 64), (300, 1000, 24), (16, 8, 17), (33, 4, 5), (8, 2052, 16),
                    (2048, 2048, 16), (17, 264, 33),
-                   # m <= 32: the few-rows kernel (4 x rows + 2 adapter rows per block)
+                   # m <= 32 (or few blocks): the few-rows kernel (4 x rows + 2 adapter rows per block)
                    (32, 3328, 16), (32, 3332, 7), (20, 6656, 16), (5, 6660, 3), (31, 2048, 5), (32, 6144, 64)]
 
 
@@ -1330,9 +1330,19 @@ def test_mid_and_wide_ffn_gate_up(ctx, m, hidden, inter, gl, ul):
 # ring of 8 tiles, and fused with h's quantization in dq8_ffn (widths of whole
 # 256-element chunks).
 @pytest.mark.parametrize("m,k,rank", [(4, 508, 2), (5, 512, 3), (3, 516, 1), (32, 1024, 16), (1, 764, 5), (2, 4096, 16),
-                                      (7, 4356, 9), (24, 8448, 16), (1, 4, 1)])
+                                      (7, 4356, 9), (24, 8448, 16), (1, 4, 1), (100, 1000, 20), (128, 516, 16),
+                                      (129, 516, 16)])
 def test_lora_mid_few_rows_edges(ctx, m, k, rank):
     test_lora_mid_bit_exact(ctx, m, k, rank)
+
+
+@pytest.mark.parametrize("m", [60, 68])  # 15 and 17 row blocks x 8 x 2 items: 240 and 272 of the few-rows blocks
+def test_lora_mid_batch_past_few_rows(ctx, m):
+    rng = np.random.default_rng(m)
+    x = make_x(rng, m, 1032)
+    pairs = [(dev(x), dev((rng.standard_normal((16, 1032)) * 0.05).astype(np.float32))) for _ in range(2)]
+    for (_, a), got in zip(pairs, ctx.lora_mid_batch(pairs)):
+        assert bits_equal(host(got), dq8o.lora_mid(x, host(a), threads=4))
 
 
 @pytest.mark.parametrize("m,hidden,inter", [(1, 256, 256), (24, 256, 6144), (32, 320, 512), (40, 256, 512)])
