@@ -238,16 +238,17 @@ typedef struct dq8_ffn_weights {
 /* The FFN's gate and up projections (qwen.rs:489-490) on one shared quantized
  * input: h = silu(gate(x) + gate_bias) * (up(x) + up_bias), exactly what
  * dq8_linear(gate, DQ8_WRITE into h) followed by dq8_linear(up, DQ8_SWIGLU
- * into h) store, bit for bit (Epilogue::SwiGlu, tensor.rs:96-99).  With more
- * than 64 rows both projections run in one launch that computes a gate and an
- * up tile of the same outputs side by side, so h is stored once and the gate
- * result is never written and read back.  No reference counterpart of its own:
+ * into h) store, bit for bit (Epilogue::SwiGlu, tensor.rs:96-99).  Both
+ * projections run in one launch that computes the gate and up values of the
+ * same outputs side by side, so h is stored once and the gate result is never
+ * written and read back (two launches for inputs that need padding, and for the
+ * adapters noted below).  No reference counterpart of its own:
  * it schedules the crate's two apply calls of the FFN together.  gate and up
  * must have the same shape; h is [m][n] (rows layout).
  * h_q/h_scales (both or neither; NULL: h is only stored): h is also quantized
  * for the down projection (qwen.rs:491, QuantizedInputs::new, tensor.rs:321-339)
  * into h_q [m][n] and h_scales [m][ceil(n/64)], exactly what dq8_quantize(h)
- * writes; on the one-launch path the launch itself does it, with no second
+ * writes; above a few rows the launch itself does it, with no second
  * pass over h.  A non-finite value in h is reported as by dq8_quantize:
  * nonfinite == NULL synchronizes and returns DQ8_ERR_NONFINITE (h_q/h_scales
  * then unspecified; h is written); otherwise 1 is ORed into *nonfinite. */
@@ -260,8 +261,9 @@ dq8_status dq8_ffn_gate_up(dq8_ctx *ctx, const dq8_weights *gate, const dq8_weig
  * bias, tensor.rs:437-438), each adapter's middle product `mid` already
  * computed (dq8_lora_mid / dq8_lora_mid_batch).  The one-launch path takes
  * adapters of rank 0, and of rank 16 (the reference checkpoints' rank) with
- * 16-byte aligned mid and b: h is then still stored (and quantized) once.
- * Other adapters run as the two separate launches, with the same bits. */
+ * 16-byte aligned mid and b, at any row count, and most others at few rows: h is
+ * then still stored (and quantized) once.  Other adapters run as the two
+ * separate launches, with the same bits. */
 dq8_status dq8_ffn_gate_up_lora(dq8_ctx *ctx, const dq8_weights *gate, const dq8_weights *up, const int8_t *q,
                                 const float *scales, size_t m, const float *gate_bias, const float *up_bias,
                                 const dq8_lora *gate_lora, const dq8_lora *up_lora, float *h, int8_t *h_q,
@@ -305,8 +307,8 @@ dq8_status dq8_apply(dq8_ctx *ctx, const dq8_weights *w, const float *x, size_t 
  * example 2048 x 6144 or 4096 x 2048), else DQ8_ERR_LIMIT and nothing is
  * enqueued.  Results are those of dq8_apply, bit for bit.  All calls on one
  * GPU share that array, whatever their context: calls that overlap on one GPU
- * (two streams, or two host threads) race and give wrong results; each call's
- * flag is cleared by a kernel, so stream-ordered calls need no other care. */
+ * (two streams, or two host threads) race and give wrong results; stream-ordered
+ * calls need no care. */
 dq8_status dq8_apply_noalloc(dq8_ctx *ctx, const dq8_weights *w, const float *x, size_t m, const float *bias,
                              const dq8_lora *lora, float *out, dq8_layout layout, dq8_epilogue epilogue,
                              void *stream);
