@@ -225,6 +225,7 @@ void fill_proj(dq8::Proj& p, const dq8::Weights& w, const int8_t* q, int ldq, co
   p.np = w.np;
   p.epilogue = epilogue;
   p.layout = layout;
+  p.ldm = (int)m;
   p.wt2 = nullptr;
   p.wst2 = nullptr;
   p.bias2 = nullptr;
@@ -320,7 +321,7 @@ int units_per_block(long units, bool /*has_long*/) {
 
 // How a call's items of more than 32 rows run (measured graph-replayed, 24
 // launches over rotating weights):
-//  * small: items of at most 512 rows (rows layout) as chunks of at most 32
+//  * small: items of at most 512 rows as chunks of at most 32
 //    rows on the skinny kernel, if all the call's chunks together read at most
 //    chunk_bytes of weights (the first read comes from HBM, the rest mostly
 //    from cache).  Against the mid kernel: 128 x 2048 -> 2048 7.8 and 9.6 us,
@@ -343,14 +344,12 @@ int units_per_block(long units, bool /*has_long*/) {
 constexpr long kMidBlocks = 256, kMidMixedBlocks = 768;
 double chunk_bytes(size_t k) { return std::min(17.5e3 * (double)k, 45e6); }
 double weight_bytes(const dq8::Weights& w) { return (double)w.n * w.k + 4.0 * w.n * w.g; }
-bool may_split(const dq8::Weights& w, size_t m, int layout) {
-  return kind_of(w, m) == 0 && layout == DQ8_ROWS && m <= 512;
-}
+bool may_split(const dq8::Weights& w, size_t m) { return kind_of(w, m) == 0 && m <= 512; }
 long wide_blocks(const dq8::Weights& w, size_t m) {
   return (long)((m + dq8::block_rows(0, false) - 1) / dq8::block_rows(0, false)) * (w.np / dq8::block_cols(0, false));
 }
-size_t row_chunks(const dq8::Weights& w, size_t m, int layout, bool small) {
-  return may_split(w, m, layout) && small ? (m + 31) / 32 : 1;
+size_t row_chunks(const dq8::Weights& w, size_t m, bool small) {
+  return may_split(w, m) && small ? (m + 31) / 32 : 1;
 }
 struct CallPlan {
   bool small, mid;
@@ -365,7 +364,7 @@ CallPlan call_plan(const Item* items, size_t count, W weights_of) {
     const dq8::Weights& w = weights_of(items[i]);
     const size_t m = items[i].m;
     if (m == 0 || kind_of(w, m) != 0) continue;
-    const bool can = may_split(w, m, items[i].layout);
+    const bool can = may_split(w, m);
     (can ? blocks : fixed) += wide_blocks(w, m);
     if (can) {
       bytes += (double)((m + 31) / 32) * weight_bytes(w);
@@ -506,7 +505,7 @@ dq8::FProj make_fproj(const dq8::Weights& w, const float* x, size_t m, const flo
   p.lmid = lora ? lora->mid : nullptr;
   p.lb = lora ? lora->b : nullptr;
   p.out = out;
-  p.m = (int)m;
+  p.m = p.ldm = (int)m;
   p.k = w.k;
   p.g = w.g;
   p.n = w.n;
@@ -550,7 +549,7 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
   for (size_t i = 0; i < count; ++i) {
     const dq8_linear_item& it = items[i];
     if (it.m == 0) continue;
-    const size_t nch = row_chunks(it.w->w, it.m, it.layout, plan.small);
+    const size_t nch = row_chunks(it.w->w, it.m, plan.small);
     const int kind = item_kind(it.w->w, it.m, nch, plan);
     strips[kind] += (long)nch * short_strips(it.w->w);
     units[kind] += (long)nch * short_units(it.w->w);
@@ -590,7 +589,7 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
     // once from HBM), which beats a wide launch of half-empty row tiles whose
     // long-K blocks trail (measured 44 against 52 us for 48 rows of a layer's
     // projection set).  Rows are independent, so the results are the same bits.
-    const size_t nch = row_chunks(w, it.m, it.layout, plan.small);
+    const size_t nch = row_chunks(w, it.m, plan.small);
     const int kind = item_kind(w, it.m, nch, plan);
     const size_t half = (it.m + nch - 1) / nch;
     for (size_t r0 = 0; r0 < it.m; r0 += half) {
@@ -606,8 +605,9 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
       dq8::Proj& p = b.p[b.count++];
       // (the dots kernels read neither x scales nor out, which may be stand-ins)
       fill_proj(p, w, q + r0 * ldq, ldq, dots ? xs : xs + r0 * ldxs, ldxs, rows, it.bias,
-                dots ? it.out : it.out + r0 * w.n, dots ? dots + r0 * w.n * w.g : nullptr, it.layout, it.epilogue,
+                dots ? it.out : it.out + (it.layout == DQ8_COLUMNS ? r0 : r0 * w.n), dots ? dots + r0 * w.n * w.g : nullptr, it.layout, it.epilogue,
                 dots ? nullptr : it.lora);
+      p.ldm = (int)it.m;
       if (p.lora) {
         p.lmid += r0 * p.rank;
         b.any_lora = 1;
@@ -764,10 +764,9 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
   // (row chunks as in run_linear; at most 512 rows make at most 16 chunks)
   struct One {
     size_t m;
-    int layout;
-  } one = {m, layout};
+  } one = {m};
   const CallPlan plan = call_plan(&one, 1, [&](const One&) -> const dq8::Weights& { return w; });
-  const size_t nch = row_chunks(w, m, layout, plan.small);
+  const size_t nch = row_chunks(w, m, plan.small);
   static_assert(dq8::kMaxBatch >= 16, "512 rows in chunks of 32");
   const int kind = item_kind(w, m, nch, plan);
   const size_t half = (m + nch - 1) / nch;
@@ -777,7 +776,8 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
   for (size_t r0 = 0; r0 < m; r0 += half) {
     dq8::Proj& p = b.p[b.count++];
     fill_proj(p, w, in.q + r0 * in.ldq, in.ldq, in.xs + r0 * in.ldxs, in.ldxs, std::min(half, m - r0), bias,
-              out + r0 * w.n, nullptr, layout, epilogue, lora);
+              out + (layout == DQ8_COLUMNS ? r0 : r0 * w.n), nullptr, layout, epilogue, lora);
+    p.ldm = (int)m;
     if (p.lora) p.lmid += r0 * p.rank;
     if (fb) {
       b.fx[b.count - 1] = fb->x + r0 * w.k;

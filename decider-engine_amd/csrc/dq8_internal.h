@@ -70,7 +70,8 @@ struct Proj {
   float lscale;
   int m, ldq, ldxs, g, n, np;
   int epilogue;       // 0 write, 1 add, 2 swiglu
-  int layout;         // 0 rows [M][N], 1 columns [N][M]
+  int layout;         // 0 rows [M][N], 1 columns [N][ldm]
+  int ldm;            // columns layout: rows of the whole output (M, or more for a row chunk)
   int wave_begin;     // first block of this projection in the launch
   int waves_n;        // column strips (wide: one block tile wide; skinny long K: 16 columns wide;
                       // skinny short K: 16-column units, dealt to blocks `units` at a time)
@@ -151,7 +152,7 @@ struct FProj {
   int lora, rank;
   float lscale;
   float* out;
-  int m, k, g, n, np;
+  int m, ldm, k, g, n, np;
   int epilogue, layout;
   Chain* chain;  // if set, the launch computes only if the chain's inputs were not finite, and ends its call
 };

@@ -196,7 +196,7 @@ __device__ __forceinline__ void store_tile(const Proj& P, const int (&row)[E], c
   if (P.layout == 1) {
 #pragma unroll
     for (int e = 0; e < E; ++e)
-      if (row[e] < P.m && col[e] < P.n) st_out(P.out + (size_t)col[e] * P.m + row[e], y[e]);
+      if (row[e] < P.m && col[e] < P.n) st_out(P.out + (size_t)col[e] * P.ldm + row[e], y[e]);
     return;
   }
   if (P.epilogue == 0) {
@@ -1784,7 +1784,7 @@ __device__ __forceinline__ void fp32_tile(const FProj& P, int m0, int n0, int mh
         const float scaled = P.lscale * delta;
         y = y + scaled;
       }
-      float* dst = P.layout == 1 ? P.out + (size_t)n * P.m + row : P.out + (size_t)row * P.n + n;
+      float* dst = P.layout == 1 ? P.out + (size_t)n * P.ldm + row : P.out + (size_t)row * P.n + n;
       if (P.epilogue == 0 || P.layout == 1) *dst = y;
       else if (P.epilogue == 1) *dst = *dst + y;
       else *dst = silu(*dst) * y;
@@ -1811,7 +1811,7 @@ __global__ __launch_bounds__(256) void k_linear_fp32(FProj P) {
 // The FP32 path of an int8 block's outputs: rows [m0, mhi) (at most 16*RPT), columns [nlo, nhi).
 template <int RPT>
 __device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k, int m0, int mhi, int nlo, int nhi, uint8_t* lds) {
-  const FProj P = {x, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, k, S.g, S.n, S.np,
+  const FProj P = {x, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, S.ldm, k, S.g, S.n, S.np,
                    S.epilogue, S.layout, nullptr};
   __syncthreads();  // every wave's loads into this LDS have landed
   for (int n0 = nlo / kF32Cols * kF32Cols; n0 < nhi; n0 += kF32Cols)
@@ -2815,7 +2815,7 @@ __global__ __launch_bounds__(256) void k_linear_post(Batch b) {
       lb[q] = *reinterpret_cast<const v4f*>(P.lb + (size_t)cc * 16 + 4 * q);
     }
   }
-  float* dst = P.layout == 1 ? P.out + (size_t)cc * P.m + rc : P.out + (size_t)rc * P.n + cc;
+  float* dst = P.layout == 1 ? P.out + (size_t)cc * P.ldm + rc : P.out + (size_t)rc * P.n + cc;
   const float old = P.epilogue != 0 ? *dst : 0.0f;
   lds_barrier();
   float s = 0.0f;
@@ -2977,7 +2977,7 @@ __global__ __launch_bounds__(256) void k_apply_few(Proj P, const float* __restri
     const float scaled = P.lscale * d;
     y = y + scaled;
   }
-  float* dst = P.layout == 1 ? P.out + (size_t)col * P.m + row : P.out + (size_t)row * P.n + col;
+  float* dst = P.layout == 1 ? P.out + (size_t)col * P.ldm + row : P.out + (size_t)row * P.n + col;
   if (P.epilogue == 0 || P.layout == 1) *dst = y;
   else if (P.epilogue == 1) *dst = *dst + y;
   else *dst = silu(*dst) * y;

@@ -157,3 +157,20 @@ def test_apply_few_rows(ctx, m, k, n, rank, bad):
         cols = host(ctx.apply(h, xd, bias=dev(bias), lora=lora, layout=dq8.COLUMNS))
         want, _ = dq8o.apply(x, v, s, bias=bias, a=a, b=b, scale=0.5, result=base, epilogue=0, threads=8)
         assert same(cols, np.ascontiguousarray(want.T))
+
+
+# Columns layout as row chunks (each chunk's rows inside the whole output's columns).
+@pytest.mark.parametrize("m,k,n", [(40, 2048, 200), (333, 1000, 130), (70, 6144, 33)])
+@pytest.mark.parametrize("bad", [False, True])
+def test_apply_columns_in_row_chunks(ctx, m, k, n, bad):
+    rng = np.random.default_rng(m + k + n)
+    x, v, s, bias, a, b = case(rng, m, k, n, 16)
+    if bad:
+        x[m - 1, 0] = np.inf
+    h = ctx.weights_from_quantized(dev(v), dev(s))
+    lora = dq8.Lora(ctx.lora_mid(dev(x), dev(a)), dev(b), 0.5)
+    got = host(ctx.apply(h, dev(x), bias=dev(bias), lora=lora, layout=dq8.COLUMNS))
+    want, fp32 = dq8o.apply(x, v, s, bias=bias, a=a, b=b, scale=0.5, result=np.zeros((m, n), np.float32), epilogue=0,
+                            threads=8)
+    assert fp32 == bad
+    assert same(got, np.ascontiguousarray(want.T))

@@ -1257,7 +1257,7 @@ def test_small_call_with_adapter_and_group(ctx, m):
 
 
 # The mid kernel (more than 32 rows whose wide grid is at most 256 blocks, here
-# past the 512 rows that run as chunks, or in the columns layout): one row and
+# past the 512 rows that run as chunks): one row and
 # one column past a tile, widths of one input, of one and several groups, an odd
 # group count (the last group is paired with a clamped copy) and long K; and the
 # wide kernel's own ragged edges, in grids just past that limit.
