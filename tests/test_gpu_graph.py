@@ -263,3 +263,37 @@ def test_reserve_while_another_stream_captures_globally_keeps_that_capture():
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+@pytest.mark.parametrize("m,k,n", [(2, 512, 300), (24, 2048, 300), (24, 6144, 512), (100, 512, 300), (600, 512, 300),
+                                   (1100, 128, 2050)])
+def test_replayed_apply_follows_each_inputs_finiteness(ctx, m, k, n):
+    # the device's choice between the int8 and the FP32 path (few-rows, posting,
+    # skinny, mid and wide kernels) in replays of one captured call, with finite
+    # and non-finite inputs in turn and eager calls of the context between them
+    rng = np.random.default_rng(m + k)
+    w = ctx.weights_from_quantized(*(dev(t) for t in dq8o.quantize_weights(
+        (rng.standard_normal((n, k)) * 0.05).astype(np.float32))))
+    good = dev(rng.standard_normal((m, k)).astype(np.float32))
+    bad = good.clone()
+    bad[m - 1, k // 2] = float("inf")
+    x, out = good.clone(), torch.zeros((m, n), device="cuda")
+    want = {id(t): host(ctx.apply(w, t)) for t in (good, bad)}
+    ctx.reserve(m, k)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ctx.apply(w, x, out=out)
+    torch.cuda.current_stream().wait_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ctx.apply(w, x, out=out)
+    for i, t in enumerate((good, bad, bad, good, bad, good, good)):
+        x.copy_(t)
+        out.fill_(-1.0)
+        g.replay()
+        got = host(out)
+        nan = np.isnan(want[id(t)])
+        assert np.array_equal(np.isnan(got), nan) and got[~nan].tobytes() == want[id(t)][~nan].tobytes(), i
+        if i % 2:
+            ctx.apply(w, bad if i == 3 else good)
