@@ -93,6 +93,13 @@ dq8_status from_hip(hipError_t e) {
 
 bool aligned(const void* p, size_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
 
+// Whether an [an]-element and a [bn]-element array share a byte.
+template <class A, class B>
+bool overlap(const A* a, size_t an, const B* b, size_t bn) {
+  const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+  return p < q + bn * sizeof(B) && q < p + an * sizeof(A);
+}
+
 // Whether work on s would be recorded into a graph.  A failed query counts as
 // capturing: HIP reports an error for the legacy NULL stream while another
 // stream captures in global mode, and an allocation then would invalidate that
@@ -796,7 +803,10 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
 // the device, with no synchronization.
 dq8_status apply_through(const dq8::Weights& w, const float* x, size_t m, const float* bias, const dq8_lora* lora,
                          float* out, int layout, int epilogue, const WorkInputs& in, dq8::Chain* chain, hipStream_t s) {
-  if (dq8::apply_few_ok((int)m, w.g, w.n)) {  // one launch, which quantizes in its blocks and chooses by itself
+  // One launch, which quantizes in its blocks and chooses by itself: every block
+  // reads all of x while others store, so an out that shares memory with x (an
+  // in-place call) takes the two launches, whose quantizer has read x before.
+  if (dq8::apply_few_ok((int)m, w.g, w.n) && !overlap(x, m * w.k, out, m * w.n)) {
     dq8::Proj p = {};
     fill_proj(p, w, nullptr, 0, nullptr, 0, m, bias, out, nullptr, layout, epilogue, lora);
     return from_hip(dq8::launch_apply_few(p, x, w.k, s));

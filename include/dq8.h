@@ -294,7 +294,9 @@ dq8_status dq8_linear_fp32(dq8_ctx *ctx, const dq8_weights *w, const float *x, s
  * quantize x (QuantizedInputs::new), then the int8 projection, or the FP32
  * path of dq8_linear_fp32 if x holds a non-finite value.  Both are queued and
  * a device flag lets exactly one run: no synchronization, the crate's result
- * either way.  Uses the context workspace (calls of one context are ordered). */
+ * either way.  out may share memory with x (x is quantized before anything is
+ * stored) if x is finite; the FP32 path reads x while it stores.  Uses the
+ * context workspace (calls of one context are ordered). */
 dq8_status dq8_apply(dq8_ctx *ctx, const dq8_weights *w, const float *x, size_t m, const float *bias,
                      const dq8_lora *lora, float *out, dq8_layout layout, dq8_epilogue epilogue, void *stream);
 /* dq8_apply that allocates nothing, ever: no counterpart in the reference.  It

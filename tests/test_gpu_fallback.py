@@ -174,3 +174,28 @@ def test_apply_columns_in_row_chunks(ctx, m, k, n, bad):
                             threads=8)
     assert fp32 == bad
     assert same(got, np.ascontiguousarray(want.T))
+
+
+# out sharing memory with a finite x: in place, shifted by rows or by part of a
+# row, and reaching into x from either side, at the rows that k_apply_few would
+# otherwise take and just past them.
+@pytest.mark.parametrize("m", [1, 2, 4, 8, 9, 24])
+@pytest.mark.parametrize("k,n", [(512, 512), (2048, 2048), (256, 1024), (1024, 96)])
+def test_apply_out_overlapping_x(ctx, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    x, v, s, bias, _, _ = case(rng, m, k, n)
+    h = ctx.weights_from_quantized(dev(v), dev(s))
+    want, fp32 = dq8o.apply(x, v, s, bias=bias, result=np.zeros((m, n), np.float32), epilogue=0, threads=8)
+    assert not fp32
+    for shift in (0, k, -n, 17, -33, (m * k - 1), -(m * n - 1)):  # out starts `shift` floats after x
+        lo, hi = min(0, shift), max(m * k, shift + m * n)
+        store = torch.zeros(hi - lo, device="cuda")
+        xd = store[-lo:m * k - lo].view(m, k)
+        out = store[shift - lo:shift - lo + m * n].view(m, n)
+        xd.copy_(dev(x))
+        ctx.apply(h, xd, out=out, bias=dev(bias))
+        assert host(out).tobytes() == want.tobytes(), shift
+    if k == n:  # a residual: x + W x into x
+        xd = dev(x)
+        ctx.apply(h, xd, out=xd, bias=dev(bias), epilogue=dq8.ADD)
+        assert host(xd).tobytes() == (x + want).astype(np.float32).tobytes()
