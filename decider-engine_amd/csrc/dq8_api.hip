@@ -1169,7 +1169,19 @@ int pair_kind(const dq8::Weights& g, const int8_t* q, const float* xs, size_t m,
 dq8_status gate_up(dq8_ctx* ctx, const dq8_weights* gate, const dq8_weights* up, const int8_t* q, const float* xs,
                    size_t m, const float* gate_bias, const float* up_bias, const dq8_lora* gate_lora,
                    const dq8_lora* up_lora, float* h, const QOut* qout, hipStream_t s) {
-  const int kind = pair_kind(gate->w, q, xs, m, gate_lora, up_lora);
+  int kind = pair_kind(gate->w, q, xs, m, gate_lora, up_lora);
+  // The wide and mid pair launches store h's quantization while other blocks still
+  // read the call's inputs: buffers that hold both (one q buffer for the layer,
+  // say) take the two launches and the quantizer behind them.
+  if (qout && (kind == 0 || kind == 3)) {
+    const size_t k = (size_t)gate->w.k, n = (size_t)gate->w.n, gk = groups_of(k), gn = groups_of(n);
+    auto stored_over = [&](const auto* in, size_t count) {
+      return overlap(qout->q, m * n, in, count) || overlap(qout->scales, m * gn, in, count);
+    };
+    bool shared = stored_over(q, m * k) || stored_over(xs, m * gk);
+    for (const dq8_lora* l : {gate_lora, up_lora}) shared = shared || (l && stored_over(l->mid, m * l->rank));
+    if (shared) kind = -1;
+  }
   if (kind >= 0)
     return run_pair(gate->w, up->w, q, xs, m, gate_bias, up_bias, gate_lora, up_lora, h, qout, kind, s);
   dq8_linear_item gi = {gate, q, xs, m, gate_bias, h, DQ8_ROWS, DQ8_WRITE, gate_lora};

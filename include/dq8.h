@@ -249,7 +249,9 @@ typedef struct dq8_ffn_weights {
  * for the down projection (qwen.rs:491, QuantizedInputs::new, tensor.rs:321-339)
  * into h_q [m][n] and h_scales [m][ceil(n/64)], exactly what dq8_quantize(h)
  * writes; above a few rows the launch itself does it, with no second
- * pass over h.  A non-finite value in h is reported as by dq8_quantize:
+ * pass over h.  They may share memory with q, scales and the adapters' middle
+ * products (the quantization then runs behind the projections).  A non-finite
+ * value in h is reported as by dq8_quantize:
  * nonfinite == NULL synchronizes and returns DQ8_ERR_NONFINITE (h_q/h_scales
  * then unspecified; h is written); otherwise 1 is ORed into *nonfinite. */
 dq8_status dq8_ffn_gate_up(dq8_ctx *ctx, const dq8_weights *gate, const dq8_weights *up, const int8_t *q,

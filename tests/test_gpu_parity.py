@@ -1189,6 +1189,48 @@ def test_ffn_gate_up_with_adapters(ctx, m, hidden, inter, gl, ul):
     assert np.array_equal(host(hq), oq) and bits_equal(host(hs), os_)
 
 
+# h's quantization written over the call's own inputs (one q and one scales
+# buffer for the layer; the adapters' middle products): the skinny pair, shapes
+# of the mid pair (partial and whole blocks, one round of them) and of the wide
+# pair, and buffers that share a part only.
+@pytest.mark.parametrize("m,hidden,inter", [(24, 256, 384), (64, 2048, 6144), (600, 256, 1100), (600, 256, 2048)])
+@pytest.mark.parametrize("shared", ["q", "scales", "mid"])
+def test_ffn_gate_up_quantizes_over_its_inputs(ctx, m, hidden, inter, shared):
+    rng = np.random.default_rng(m + inter)
+    x = make_x(rng, m, hidden, "outliers")
+    gv, gs = dq8o.quantize_weights(make_w(rng, inter, hidden))
+    uv, us = dq8o.quantize_weights(make_w(rng, inter, hidden))
+    G, U = ctx.weights_from_quantized(dev(gv), dev(gs)), ctx.weights_from_quantized(dev(uv), dev(us))
+    a, b, lora = _adapter(ctx, rng, m, hidden, inter, 16, 0.5, x, "aligned")
+    q0, s0 = ctx.quantize(dev(x))
+    want, wq, ws = (host(t) for t in ctx.ffn_gate_up(G, U, q0, s0, quantize=True, loras=(lora, lora)))
+    gate = dq8o.linear_lora(x, gv, gs, a, b, 0.5, threads=8)
+    assert bits_equal(want, dq8o.linear_lora(x, uv, us, a, b, 0.5, result=gate, epilogue=2, threads=8))
+    gh = dq8.groups(inter)
+    qbuf = torch.zeros(m * (hidden + inter), dtype=torch.int8, device="cuda")
+    sbuf = torch.zeros(m * (dq8.groups(hidden) + gh + 16), dtype=torch.float32, device="cuda")
+    q, s, mid = qbuf[:m * hidden].view(m, hidden), sbuf[:m * s0.shape[1]].view(m, -1), lora.mid
+    hq = qbuf[m * hidden:].view(m, inter)
+    hs = sbuf[m * s0.shape[1]:m * (s0.shape[1] + gh)].view(m, gh)
+    if shared == "q":  # from q's last row on: a part of q, or (more outputs) all that follows too
+        hq = qbuf[(m - 1) * hidden:(m - 1) * hidden + m * inter].view(m, inter)
+    elif shared == "scales":
+        hs = sbuf[:m * gh].view(m, gh)
+    else:
+        mid = sbuf[m * s0.shape[1]:m * (s0.shape[1] + 16)].view(m, 16)
+        mid.copy_(lora.mid)
+    q.copy_(q0)
+    s.copy_(s0)
+    h = torch.empty((m, inter), dtype=torch.float32, device="cuda")
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    lo = ctx._lora(dq8.Lora(mid, lora.b, lora.scale), m, inter)
+    assert dq8.lib().dq8_ffn_gate_up_lora(ctx.handle, G.handle, U.handle, q.data_ptr(), s.data_ptr(), m, None, None,
+                                          ctypes.byref(lo), ctypes.byref(lo), h.data_ptr(), hq.data_ptr(),
+                                          hs.data_ptr(), flag.data_ptr(),
+                                          torch.cuda.current_stream().cuda_stream) == dq8.OK
+    assert bits_equal(host(h), want) and bits_equal(host(hq), wq) and bits_equal(host(hs), ws)
+
+
 # The skinny pair launch (up to 64 rows), whose 16-column tiles hold 8 gate and
 # 8 up columns: one and two row tiles and chunks, widths that end inside a unit,
 # the one-wave path (160 or more strips) and the 4-wave paths for few strips and
