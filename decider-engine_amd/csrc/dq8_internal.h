@@ -44,13 +44,24 @@ struct Divider {
 
 // Whether the inputs of a call were finite, decided on the device with no
 // clearing launch and no synchronization.  A call's quantizer stores next into
-// cur (its first block) and next + 1 into hit if it sees a non-finite value;
-// the launches after it compare hit with cur + 1, and the call's last launch
-// stores cur + 1 into next (its first block).  No launch reads a word that it
-// writes, so calls in stream order, and graph replays of them, each see their
-// own answer.  All zero at first.
+// cur (its first block) and report(next) into hit if it sees a non-finite value;
+// the launches after it ask reported(hit, cur), and the call's last launch
+// raises next to closed(hit, cur) (its first block, an atomic maximum).  No launch
+// reads a word that it writes, so calls in stream order, and graph replays of
+// them, each see their own answer.  All zero at first.
+//
+// A call that starts with hit <= next (and runs alone) sees its own reports only,
+// and every close leaves hit <= next: also after calls that overlapped, which may
+// mix up their own answers but not a later call's.  The last value stored in hit
+// is some call's report; that call's close comes after it, reads it and raises
+// next to it, and next never falls.
 struct Chain {
   uint64_t next, cur, hit;
+  __host__ __device__ static constexpr uint64_t report(uint64_t next) { return next + 1; }
+  __host__ __device__ static constexpr bool reported(uint64_t hit, uint64_t cur) { return hit == cur + 1; }
+  __host__ __device__ static constexpr uint64_t closed(uint64_t hit, uint64_t cur) {
+    return hit > cur + 1 ? hit : cur + 1;
+  }
 };
 
 // One projection of a launch.  q is [M][ldq] bytes with ldq % 16 == 0 and

@@ -427,20 +427,21 @@ __device__ __forceinline__ void load4(const float* p, float (&v)[4]) {
 __device__ __forceinline__ bool chain_hit(const Chain* c) {
   typedef const __attribute__((address_space(4))) Chain* scalar_chain;
   const scalar_chain sc = (scalar_chain)(uintptr_t)c;
-  return sc->hit == sc->cur + 1;
+  return Chain::reported(sc->hit, sc->cur);
 }
 __device__ __forceinline__ void chain_open(Chain* c) {  // by the quantizer's first block
   if (blockIdx.x == 0 && threadIdx.x == 0) c->cur = c->next;
 }
 __device__ __forceinline__ void chain_close(Chain* c) {  // by the last launch's first block
-  if (blockIdx.x == 0 && threadIdx.x == 0) c->next = c->cur + 1;
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    atomicMax(reinterpret_cast<unsigned long long*>(&c->next), Chain::closed(c->hit, c->cur));
 }
 // One report per wave with a lane that saw a non-finite element.
 __device__ __forceinline__ void report_nonfinite(bool bad, uint32_t* flag, Chain* chain) {
   const unsigned long long b = __ballot(bad);
   if (b != 0 && (int)(threadIdx.x & 63) == __builtin_ffsll((long long)b) - 1) {
     if (flag) atomicOr(flag, 1u);
-    if (chain) chain->hit = chain->next + 1;  // every reporter stores the same value
+    if (chain) chain->hit = Chain::report(chain->next);  // every reporter stores the same value
   }
 }
 

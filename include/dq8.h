@@ -312,7 +312,7 @@ dq8_status dq8_apply(dq8_ctx *ctx, const dq8_weights *w, const float *x, size_t 
  * enqueued.  Results are those of dq8_apply, bit for bit.  All calls on one
  * GPU share that array, whatever their context: calls that overlap on one GPU
  * (two streams, or two host threads) race and give wrong results; stream-ordered
- * calls need no care. */
+ * calls need no care, also after calls that overlapped. */
 dq8_status dq8_apply_noalloc(dq8_ctx *ctx, const dq8_weights *w, const float *x, size_t m, const float *bias,
                              const dq8_lora *lora, float *out, dq8_layout layout, dq8_epilogue epilogue,
                              void *stream);
