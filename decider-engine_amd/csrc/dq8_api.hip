@@ -546,7 +546,6 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
   for (dq8::Batch& b : batch) {
     b.count = b.total_waves = b.any_lora = 0;
     b.chain = fb ? fb->chain : nullptr;
-    b.fallback = 0;
   }
   CallPlan plan = call_plan(items, count, [](const dq8_linear_item& it) -> const dq8::Weights& { return it.w->w; });
   if (dots) plan.mid = false;
@@ -622,7 +621,6 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
       if (fb) {
         b.fx[b.count - 1] = fb->x + r0 * w.k;
         b.fk = w.k;
-        b.fallback = kind != 0;  // the other kernels hold the FP32 path themselves
       }
       place_proj(p, kind, b, strips[kind] < kSkinnyFewStrips, units[kind], has_long[kind]);
     }
@@ -662,7 +660,6 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
   b.total_waves = 0;
   b.any_lora = gate_lora != nullptr || up_lora != nullptr;
   b.chain = b.hchain = nullptr;
-  b.fallback = 0;
   // skinny: row chunks of at most 32 (run_linear)
   const size_t nch = kind == 0 || kind == 3 ? 1 : (m + 31) / 32, rows = (m + nch - 1) / nch;
   const long units = (long)nch * ((g.n + 7) / 8);
@@ -779,7 +776,6 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
   const size_t half = (m + nch - 1) / nch;
   b.count = 0;
   b.chain = fb ? fb->chain : nullptr;
-  b.fallback = fb && kind != 0;
   for (size_t r0 = 0; r0 < m; r0 += half) {
     dq8::Proj& p = b.p[b.count++];
     fill_proj(p, w, in.q + r0 * in.ldq, in.ldq, in.xs + r0 * in.ldxs, in.ldxs, std::min(half, m - r0), bias,
@@ -793,7 +789,7 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
     place_proj(p, kind, b, (long)nch * short_strips(w) < kSkinnyFewStrips, (long)nch * short_units(w), w.g > 32);
   }
   hipError_t e = dq8::launch_linear(b, kind, false, s);
-  if (e == hipSuccess && fb && !b.fallback)
+  if (e == hipSuccess && fb && kind == 0)  // the other kernels hold the FP32 path themselves
     e = dq8::launch_linear_fp32(make_fproj(w, fb->x, m, bias, lora, out, layout, epilogue, fb->chain), s);
   return from_hip(e);
 }

@@ -125,13 +125,12 @@ struct Batch {
   int count;
   int total_waves;  // blocks of the launch
   int any_lora;     // some projection has a LoRA adapter (selects the kernels with the LoRA epilogue)
-  // When set, and the chain says that the inputs were not finite: with
-  // `fallback` (skinny kernels) the blocks compute the FP32 path of their
-  // outputs from Proj::fx, and the launch ends the chain's call; without it the
-  // launch does nothing and k_linear_fp32 computes these outputs instead.
+  // When set, and the chain says that the inputs were not finite: the skinny,
+  // posting and mid kernels' blocks compute the FP32 path of their outputs from
+  // fx, and the launch ends the chain's call; the wide kernel does nothing and
+  // k_linear_fp32 behind it computes these outputs.
   Chain* chain;
-  int fallback;
-  int fk;                       // with fallback: fx[i] [M][fk], the FP32 inputs of p[i]
+  int fk;                       // with chain: fx[i] [M][fk], the FP32 inputs of p[i]
   const float* fx[kMaxBatch];
   Chain* hchain;                // with Proj::hq: marked if h is not finite
 };

@@ -1819,6 +1819,15 @@ __device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k,
     fp32_tile<RPT>(P, m0, n0, mhi, nlo, nhi, *reinterpret_cast<F32Lds*>(lds));
 }
 
+// What a launch of the skinny, posting or mid kernel holds besides plain
+// projections, as instances of their own (launch_mode): the FP32 path for inputs
+// that were not finite (Batch::chain), or a SwiGLU pair.  In one instance both
+// cost every dq8_linear launch registers and prologue: k_linear_post<32> 188 VGPRs
+// instead of 84, k_linear_skinny<2> 185 instead of 146, and spilled SGPRs in
+// k_linear_post<96> and k_linear_mid; graph-replayed, 33 x 2048 -> 8224 10.5 us
+// instead of 10.0, 40 x 1024 -> 4096 5.5 and 5.3, 48 x 2304 -> 1000 5.8 and 5.5.
+constexpr int kModePlain = 0, kModeChained = 1, kModePair = 2;
+
 // ---------------------------------------------------------------------------
 // Projection kernel for launches that leave the wide kernel's blocks alone on
 // their CUs.  There every wave waits out each group's whole chain (LDS reads,
@@ -1852,8 +1861,9 @@ __device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k,
 // projection's two column tiles, waves 2 and 3 the up projection's; the tiles
 // meet in LDS after the loop, where 8 threads take one row's group of h.
 constexpr int kMidRing = 3;
-template <int WM, int WN, int S, bool LORA, bool PAIR>
+template <int WM, int WN, int S, bool LORA, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_linear_mid(Batch b) {
+  constexpr bool PAIR = MODE == kModePair;
   constexpr int NW = 4, BM = 32 * WM, BN = 32 * WN, XCH = 16;
   constexpr int AS = BM / 8, BF = 4 * WN;       // 1 KB loads per step: A units, B fragments
   constexpr int KA = AS / NW, KB = BF / NW;     // ... per wave
@@ -1980,7 +1990,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     issue(ring[i], i);
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (!PAIR && b.chain) {  // uniform; non-finite inputs take the FP32 path, once the loads into LDS have landed
+  if constexpr (MODE == kModeChained) {  // non-finite inputs take the FP32 path, once the loads into LDS have landed
     const bool hit = chain_hit(b.chain);
     chain_close(b.chain);
     if (hit) {
@@ -2244,12 +2254,12 @@ __device__ __forceinline__ void issue_x_chunk(const Proj& P, int c, int wid, uin
 // host pairs adapters of one rank only; a block of 4 lanes, which forms its own
 // products, never mixes the two), then the gate lanes store h = silu(gate) * up
 // (tensor.rs:96-99, qwen.rs:489-490) with up from 8 lanes on.
-template <int RT, int CT, bool LORA>
+template <int RT, int CT, bool LORA, bool PAIR>
 __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4f (&s)[RT * CT], int r0 = 0) {
   constexpr int E = 4 * RT * CT;
   const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-  const bool up = P.pair && (lane & 8);
-  auto col_of = [&](int ct) { return P.pair ? ((c0 + 16 * ct) >> 1) + (lane & 7) : c0 + 16 * ct + (lane & 15); };
+  const bool up = PAIR && (lane & 8);
+  auto col_of = [&](int ct) { return PAIR ? ((c0 + 16 * ct) >> 1) + (lane & 7) : c0 + 16 * ct + (lane & 15); };
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int col = col_of(ct);
@@ -2272,7 +2282,7 @@ __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4
       // 16-byte loads when rank is 16 and the rows are 16-byte aligned
       float am[RT][16], bm[CT][16];
       if (P.rank == 16 && ((size_t)P.lmid & 15) == 0 && ((size_t)P.lb & 15) == 0 &&
-          (!P.pair || (((size_t)P.lmid2 & 15) == 0 && ((size_t)P.lb2 & 15) == 0))) {
+          (!PAIR || (((size_t)P.lmid2 & 15) == 0 && ((size_t)P.lb2 & 15) == 0))) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -2312,7 +2322,7 @@ __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4
                                       [&](int i) { return mfma_k1_4(lm[rt][i], lbc[ct][i], zero4); });
     }
   }
-  if (P.pair) {
+  if constexpr (PAIR) {
     const ExpTab T = exp_table(lane);
 #pragma unroll
     for (int k = 0; k < RT * CT; ++k) {
@@ -2350,12 +2360,12 @@ __device__ __forceinline__ void skinny_store(const Proj& P, int c0, int lane, v4
 // c0/2 + l%8 of the gate (l%16 < 8) or the up projection.  A pair's tile thus
 // reads 128-byte runs of both projections' fragments, and the gate and up
 // values of one output sit 8 lanes apart.
-template <bool DOTS>
+template <bool PAIR>
 __device__ __forceinline__ void skinny_weights(const Proj& P, int c0, int lane, const uint8_t*& pb, const float*& pw) {
   int col = c0 + (lane & 15);
   const uint8_t* wt = P.wt;
   const float* wst = P.wst;
-  if (!DOTS && P.pair) {  // uniform
+  if constexpr (PAIR) {
     col = (c0 >> 1) + (lane & 7);
     wt = lane & 8 ? P.wt2 : wt;
     wst = lane & 8 ? P.wst2 : wst;
@@ -2406,7 +2416,7 @@ __device__ __forceinline__ void skinny_group(const Proj& P, int c0, int lane, bo
 // groups, 2 groups per step.  Returns true, with nothing computed, if the
 // inputs were not finite (so does skinny_long).  The block's 4 waves first load its activation
 // together; a wave with no columns (live false) only helps with that.
-template <int RT, int CT, int DB, bool DOTS, bool LORA>
+template <int RT, int CT, int DB, bool DOTS, bool LORA, int MODE>
 __device__ __forceinline__ bool skinny_short(const Proj& P, int c0, bool live, int wid, int lane, uint8_t* lds,
                                              const Chain* chain) {
   constexpr int ROWS = 16 * RT;
@@ -2420,7 +2430,7 @@ __device__ __forceinline__ bool skinny_short(const Proj& P, int c0, bool live, i
   const uint8_t* pb[CT];
   const float* pw[CT];
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) skinny_weights<DOTS>(P, c0 + 16 * ct, lane, pb[ct], pw[ct]);
+  for (int ct = 0; ct < CT; ++ct) skinny_weights<MODE == kModePair>(P, c0 + 16 * ct, lane, pb[ct], pw[ct]);
   v4i bq[DB][2][CT];
   float wq[DB][2][CT];
   auto issue = [&](v4i (&bs)[2][CT], float (&ws)[2][CT], int j) {
@@ -2459,7 +2469,7 @@ __device__ __forceinline__ bool skinny_short(const Proj& P, int c0, bool live, i
   }
   // the non-finite flag is read while the first loads are in flight; the
   // whole block leaves on it (after they land: they write this block's LDS)
-  const bool skip = chain != nullptr && chain_hit(chain);
+  const bool skip = MODE == kModeChained && chain_hit(chain);
   wait_vmcnt<0>();
   if (skip) return true;
   lds_barrier();
@@ -2520,13 +2530,13 @@ __device__ __forceinline__ bool skinny_short(const Proj& P, int c0, bool live, i
     if (j0 + d < steps) step(j0 + d, d);
   wait_vmcnt<0>();  // the clamped loads past the end
   if constexpr (!DOTS)
-    if (live) skinny_store<RT, CT, LORA>(P, c0, lane, s);
+    if (live) skinny_store<RT, CT, LORA, MODE == kModePair>(P, c0, lane, s);
   return false;
 }
 
 // Long K (G > 32): one strip per block (TPB = 4/NSEG = 1), its 16*RT rows from row
 // r0, NSEG waves, one group per wave and step.
-template <int RT, int CT, int DB, int NSEG, bool DOTS, bool LORA>
+template <int RT, int CT, int DB, int NSEG, bool DOTS, bool LORA, int MODE>
 __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, int lane, uint8_t* lds, int r0,
                                             const Chain* chain) {
   constexpr int ROWS = 16 * RT, NT = RT * CT, TPB = 4 / NSEG;
@@ -2551,7 +2561,7 @@ __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, i
   const uint8_t* pb[CT];
   const float* pw[CT];
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) skinny_weights<DOTS>(P, c0 + 16 * ct, lane, pb[ct], pw[ct]);
+  for (int ct = 0; ct < CT; ++ct) skinny_weights<MODE == kModePair>(P, c0 + 16 * ct, lane, pb[ct], pw[ct]);
   v4i aq[DB][RT], bq[DB][CT];
   float wq[DB][CT];
   auto issue = [&](v4i (&as)[RT], v4i (&bs)[CT], float (&ws)[CT], int j) {
@@ -2595,7 +2605,7 @@ __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, i
   }
   // the non-finite flag, read while the first loads are in flight (the block
   // leaves after they land: the x chunk writes this block's LDS)
-  if (chain != nullptr && chain_hit(chain)) {
+  if (MODE == kModeChained && chain_hit(chain)) {
     wait_vmcnt<0>();
     return true;
   }
@@ -2653,7 +2663,7 @@ __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, i
   }
   wait_vmcnt<0>();  // the clamped loads past the end
   if constexpr (!DOTS)
-    if (live && sidx == 0) skinny_store<RT, CT, LORA>(P, c0, lane, s, r0);
+    if (live && sidx == 0) skinny_store<RT, CT, LORA, MODE == kModePair>(P, c0, lane, s, r0);
   return false;
 }
 
@@ -2672,10 +2682,10 @@ __device__ __forceinline__ void skinny_row_tile(const Proj& P, int& strip, int& 
   r0 = 16 * t;
 }
 
-template <int RT, int CT, int CTL, int DBS, int DBL, bool DOTS, bool LORA>
+template <int RT, int CT, int CTL, int DBS, int DBL, bool DOTS, bool LORA, int MODE>
 __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[skinny_lds_bytes(RT, CTL)];
-  static_assert(DOTS || skinny_lds_bytes(RT, CTL) >= (int)sizeof(F32Lds), "the FP32 tile fits");
+  static_assert(MODE != kModeChained || skinny_lds_bytes(RT, CTL) >= (int)sizeof(F32Lds), "the FP32 tile fits");
   const int pidx = find_proj<true>(b, blockIdx.x);
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2709,9 +2719,9 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
       nhi = nlo + 16 * c;
     }
     if (cnt == 2)
-      skip = skinny_short<RT, 2, DBS, DOTS, LORA>(P, 16 * u0, true, wid, lane, lds, b.chain);
+      skip = skinny_short<RT, 2, DBS, DOTS, LORA, MODE>(P, 16 * u0, true, wid, lane, lds, b.chain);
     else
-      skip = skinny_short<RT, 1, DBS, DOTS, LORA>(P, 16 * u0, cnt == 1, wid, lane, lds, b.chain);
+      skip = skinny_short<RT, 1, DBS, DOTS, LORA, MODE>(P, 16 * u0, cnt == 1, wid, lane, lds, b.chain);
   } else {
     int strip = local;
     if (RT == 2) {
@@ -2720,13 +2730,11 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
     }
     nlo = 16 * CTL * strip;
     nhi = nlo + 16 * CTL;
-    skip = skinny_long<1, CTL, DBL, 4, DOTS, LORA>(P, strip, wid, lane, lds, m0, b.chain);
+    skip = skinny_long<1, CTL, DBL, 4, DOTS, LORA, MODE>(P, strip, wid, lane, lds, m0, b.chain);
   }
-  if constexpr (!DOTS) {
-    if (b.fallback) {  // uniform over the launch
-      chain_close(b.chain);
-      if (skip) fp32_block<RT>(P, b.fx[pidx], b.fk, m0, mhi, nlo, min(nhi, P.n), lds);
-    }
+  if constexpr (MODE == kModeChained) {
+    chain_close(b.chain);
+    if (skip) fp32_block<RT>(P, b.fx[pidx], b.fk, m0, mhi, nlo, min(nhi, P.n), lds);
   }
 }
 // The long-K path for launches of few blocks, without its step-by-step hand-off:
@@ -2736,12 +2744,12 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
 // output adds its t's in group order.  GMAX bounds the groups
 // (post_groups).  Bound by latency and, at 96 groups, by the CU's load path: 196 KB
 // per block.
-template <int GMAX, bool TWO, bool LORA>
+template <int GMAX, bool TWO, bool LORA, int MODE>
 __global__ __launch_bounds__(256) void k_linear_post(Batch b) {
   constexpr int NG = GMAX / 4;
   __shared__ __attribute__((aligned(16))) float xl[16][GMAX + 4];
   __shared__ __attribute__((aligned(16))) float tp[GMAX][4][64];
-  static_assert(sizeof(tp) >= sizeof(F32Lds), "the FP32 tile fits");
+  static_assert(MODE == kModePlain || (MODE == kModeChained && sizeof(tp) >= sizeof(F32Lds)), "the FP32 tile fits");
   const int pidx = find_proj<true>(b, blockIdx.x);
   const Proj P = b.p[pidx];
   const int lane = threadIdx.x & 63;
@@ -2761,7 +2769,7 @@ __global__ __launch_bounds__(256) void k_linear_post(Batch b) {
     xv[i] = *reinterpret_cast<const v4f*>(xr + 4 * min((int)(threadIdx.x & 15) + 16 * i, last_piece));
   const uint8_t* pb;
   const float* pw;
-  skinny_weights<true>(P, c0, lane, pb, pw);
+  skinny_weights<false>(P, c0, lane, pb, pw);
   const int8_t* pa = P.q + (size_t)min(r0 + (lane & 15), P.m - 1) * P.ldq + 16 * (lane >> 4);
   v4i aq[NG], bq[NG];
   float wq[NG];
@@ -2773,7 +2781,7 @@ __global__ __launch_bounds__(256) void k_linear_post(Batch b) {
     wq[i] = pw[(size_t)g * P.np];
   }
   __builtin_amdgcn_sched_barrier(0);
-  if (b.chain) {  // uniform; non-finite inputs: the FP32 path of this block's outputs
+  if constexpr (MODE == kModeChained) {  // non-finite inputs: the FP32 path of this block's outputs
     const bool hit = chain_hit(b.chain);
     chain_close(b.chain);
     if (hit) {
@@ -2874,7 +2882,7 @@ __global__ __launch_bounds__(256) void k_apply_few(Proj P, const float* __restri
   const int c0 = 16 * (int)blockIdx.x;
   const uint8_t* pb;
   const float* pw;
-  skinny_weights<true>(P, c0, lane, pb, pw);
+  skinny_weights<false>(P, c0, lane, pb, pw);
   v4i bq[NG];
   float wq[NG];
 #pragma unroll
@@ -3631,6 +3639,21 @@ hipError_t launch_apply_few(const Proj& p, const float* x, int k, hipStream_t s)
   return hipGetLastError();
 }
 
+// The mode of a skinny, posting or mid launch, and the instance for it.
+static int launch_mode(const Batch& b) {
+  if (b.chain) return kModeChained;
+  for (int i = 0; i < b.count; ++i)
+    if (b.p[i].pair) return kModePair;
+  return kModePlain;
+}
+template <class F>
+static void by_mode(int mode, bool lora, F launch) {
+  auto with = [&](auto md) { lora ? launch(std::true_type{}, md) : launch(std::false_type{}, md); };
+  if (mode == kModeChained) with(std::integral_constant<int, kModeChained>{});
+  else if (mode == kModePair) with(std::integral_constant<int, kModePair>{});
+  else with(std::integral_constant<int, kModePlain>{});
+}
+
 hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s) {
   if (b.total_waves == 0) return hipSuccess;
   const bool lora = !dots && b.any_lora;
@@ -3680,43 +3703,38 @@ hipError_t launch_linear(const Batch& b, int kind, bool dots, hipStream_t s) {
 #undef DQ8_WIDE
     return hipGetLastError();
   }
+  const int mode = launch_mode(b);
   if (kind == 3) {
-    bool pair = false;
-    for (int i = 0; i < b.count; ++i) pair |= b.p[i].pair != 0;
-    if (pair)
-      lora ? k_linear_mid<1, 4, kMidRing, true, true><<<b.total_waves, 256, 0, s>>>(b)
-           : k_linear_mid<1, 4, kMidRing, false, true><<<b.total_waves, 256, 0, s>>>(b);
-    else
-      lora ? k_linear_mid<2, 2, kMidRing, true, false><<<b.total_waves, 256, 0, s>>>(b)
-           : k_linear_mid<2, 2, kMidRing, false, false><<<b.total_waves, 256, 0, s>>>(b);
+    by_mode(mode, lora, [&](auto l, auto md) {
+      constexpr bool PAIR = md() == kModePair;
+      k_linear_mid<PAIR ? 1 : 2, PAIR ? 4 : 2, kMidRing, l(), md()><<<b.total_waves, 256, 0, s>>>(b);
+    });
     return hipGetLastError();
   }
-  const int post = dots ? 0 : post_groups(b);
-#define DQ8_POST(GM, T) \
-  (lora ? k_linear_post<GM, T, true><<<b.total_waves, 256, 0, s>>>(b) : k_linear_post<GM, T, false><<<b.total_waves, 256, 0, s>>>(b))
-  if (post == 32) {
-    kind == 2 ? DQ8_POST(32, true) : DQ8_POST(32, false);
+  if (const int post = dots ? 0 : post_groups(b)) {
+    by_mode(mode, lora, [&](auto l, auto md) {
+      if constexpr (md() != kModePair) {  // (post_groups takes no pair)
+        if (post == 32)
+          kind == 2 ? k_linear_post<32, true, l(), md()><<<b.total_waves, 256, 0, s>>>(b)
+                    : k_linear_post<32, false, l(), md()><<<b.total_waves, 256, 0, s>>>(b);
+        else
+          kind == 2 ? k_linear_post<96, true, l(), md()><<<b.total_waves, 256, 0, s>>>(b)
+                    : k_linear_post<96, false, l(), md()><<<b.total_waves, 256, 0, s>>>(b);
+      }
+    });
     return hipGetLastError();
   }
-  if (post == 96) {
-    kind == 2 ? DQ8_POST(96, true) : DQ8_POST(96, false);
-    return hipGetLastError();
-  }
-#undef DQ8_POST
   // total_waves counts blocks of 4 waves for the skinny kernel; kind 1: M <= 16, kind 2: M <= 32
   constexpr int CT = DQ8_SKINNY_CT, CL = DQ8_SKINNY_CTL;
-#define DQ8_SKINNY(R, D, L)                                                                                  \
+#define DQ8_SKINNY(R, D, L, M)                                                                               \
   k_linear_skinny<R, CT, CL, (R == 1 ? DQ8_SKINNY_DBS : DQ8_SKINNY_DBS2), (R == 1 ? DQ8_SKINNY_DBL : DQ8_SKINNY_DBL2), \
-                  D, L><<<b.total_waves, 256, 0, s>>>(b)
-  if (kind == 1) {
-    if (dots) DQ8_SKINNY(1, true, false);
-    else if (lora) DQ8_SKINNY(1, false, true);
-    else DQ8_SKINNY(1, false, false);
-  } else {
-    if (dots) DQ8_SKINNY(2, true, false);
-    else if (lora) DQ8_SKINNY(2, false, true);
-    else DQ8_SKINNY(2, false, false);
-  }
+                  D, L, M><<<b.total_waves, 256, 0, s>>>(b)
+  if (dots)
+    kind == 1 ? DQ8_SKINNY(1, true, false, kModePlain) : DQ8_SKINNY(2, true, false, kModePlain);
+  else
+    by_mode(mode, lora, [&](auto l, auto md) {
+      kind == 1 ? DQ8_SKINNY(1, false, l(), md()) : DQ8_SKINNY(2, false, l(), md());
+    });
 #undef DQ8_SKINNY
   return hipGetLastError();
 }
