@@ -421,20 +421,24 @@ __device__ __forceinline__ void load4(const float* p, float (&v)[4]) {
   for (int j = 0; j < 4; ++j) v[j] = t[j];
 }
 
-// Chain (dq8_internal.h): whether the call's inputs were not finite; its two ends.
+// Chain (dq8_internal.h): a call's state as its later launches see it; its two ends.
 // (Read through the scalar cache: no launch writes the words that it reads, and
 // a vector load would wait for the direct loads issued before it.)
-__device__ __forceinline__ bool chain_hit(const Chain* c) {
+struct ChainView {
+  uint64_t cur, hit;
+  __device__ __forceinline__ bool reported() const { return Chain::reported(hit, cur); }
+};
+__device__ __forceinline__ ChainView chain_view(const Chain* c) {
   typedef const __attribute__((address_space(4))) Chain* scalar_chain;
   const scalar_chain sc = (scalar_chain)(uintptr_t)c;
-  return Chain::reported(sc->hit, sc->cur);
+  return {sc->cur, sc->hit};
 }
 __device__ __forceinline__ void chain_open(Chain* c) {  // by the quantizer's first block
   if (blockIdx.x == 0 && threadIdx.x == 0) c->cur = c->next;
 }
-__device__ __forceinline__ void chain_close(Chain* c) {  // by the last launch's first block
+__device__ __forceinline__ void chain_close(Chain* c, const ChainView& v) {  // by the last launch's first block
   if (blockIdx.x == 0 && threadIdx.x == 0)
-    atomicMax(reinterpret_cast<unsigned long long*>(&c->next), Chain::closed(c->hit, c->cur));
+    atomicMax(reinterpret_cast<unsigned long long*>(&c->next), Chain::closed(v.hit, v.cur));
 }
 // One report per wave with a lane that saw a non-finite element.
 __device__ __forceinline__ void report_nonfinite(bool bad, uint32_t* flag, Chain* chain) {
@@ -1279,7 +1283,7 @@ __global__ __launch_bounds__(64 * WM * WN) DQ8_WIDE_ATTR void k_linear_wide(Batc
     issue_b(ring.b[i], i);
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (b.chain && chain_hit(b.chain)) {  // uniform: the block leaves once its loads into LDS have landed
+  if (b.chain && chain_view(b.chain).reported()) {  // uniform: the block leaves once its loads into LDS have landed
     wait_vmcnt<0>();
     return;
   }
@@ -1697,82 +1701,107 @@ __device__ __forceinline__ float dequant(const FProj& P, int n, int t) {
 //   y = y + scale * (dot_scores(mid_r, B_n) + 0.0)   with an adapter (Adapter::combine)
 // stored through the epilogue.  The dot products run in dot_scores' order, so
 // NaN and infinity propagate as in the crate.  fp32_tile: a block of 256
-// threads computes 16*RPT rows x 64 columns from (m0, n0) and stores those in rows
-// [m0, mhi) x columns [nlo, nhi); for RPT = 2 thread (tr, tc) owns rows 2tr, 2tr+1 and columns tc + 16j (j < 4)
+// threads computes 16*RPT rows x 16*CJ columns from (m0, n0) and stores those below
+// mhi and nhi; thread (tr, tc) owns rows RPT*tr + i and columns tc + 16j
 // with eight lane sums each.  Per group of 64 inputs the block stages x and
 // the dequantized weights in LDS (rows padded to 68 floats: the 16 columns a
-// wave reads per step fall in distinct banks).
-constexpr int kF32Rows = 32, kF32Cols = 64, kF32Pad = 68;
+// wave reads per step fall in distinct banks), the next group's loads in flight
+// while it computes.  Bound by the VALU: two instructions per product, with one
+// wave per SIMD in an int8 block.  Non-finite dq8_apply, graph-replayed, against
+// the separate launch of 32 x 64 tiles that once followed every int8 launch (4.5
+// us on finite inputs): 24 x 2048 -> 8224 125 us and 139 (260 in blocks that each
+// computed whole 64-column tiles of the grid), 128 x 2048 -> 2048 93 and 133, 512 x
+// 6144 -> 2048 507 and 456 (796), 128 x 6144 -> 2048 495 and 398 (776: 64 blocks of 64
+// x 64, half the CUs' tiles twice as large).
+constexpr int kF32Pad = 68;
+template <int RPT, int CJ>
 struct F32Lds {
-  float xs[kF32Rows][kF32Pad], ws[kF32Cols][kF32Pad];
+  float xs[16 * RPT][kF32Pad], ws[16 * CJ][kF32Pad];
 };
-template <int RPT>
-__device__ __forceinline__ void fp32_tile(const FProj& P, int m0, int n0, int mhi, int nlo, int nhi, F32Lds& L) {
+template <int RPT, int CJ>
+__device__ __forceinline__ void fp32_tile(const FProj& P, int m0, int n0, int mhi, int nhi, F32Lds<RPT, CJ>& L) {
   auto &xs = L.xs;
   auto &ws = L.ws;
   const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
   const int chunks = P.k >> 3;  // full chunks of 8 go to the lane sums
-  float acc[RPT][4][8];
+  float acc[RPT][CJ][8];
 #pragma unroll
   for (int i = 0; i < RPT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < CJ; ++j)
 #pragma unroll
       for (int q = 0; q < 8; ++q) acc[i][j][q] = 0.0f;
+  // x: thread t stages inputs 4(t%16) .. +4 of rows t/16 + 16i (zero past m or k);
+  // w: 4*CJ bytes of one column's fragment lane (the repacked layout is zero past n
+  // and k; columns past np are read as its last and not stored)
+  constexpr int WPC = 16 / CJ;
+  const int xk = 4 * tc;
+  const bool vec = (P.k & 3) == 0 && ((uintptr_t)P.x & 15) == 0;  // uniform
+  const int wcol = tid / WPC, woff = 4 * CJ * (tid % WPC), wn = min(n0 + wcol, P.np - 1);
+  const uint8_t* wr = P.wt + ((size_t)(wn >> 5) * P.g * 2 + (woff >> 5)) * kFragBytes +
+                      ((wn & 31) + 32 * ((woff >> 4) & 1)) * 16 + (woff & 15);
+  v4f xv[RPT];
+  float sc;
+  uint32_t wv[CJ];
+  auto fetch = [&](int g) {
+    const int kk = 64 * g + xk;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      const int row = m0 + tr + 16 * i;
+      const float* xr = P.x + (size_t)min(row, P.m - 1) * P.k;
+      if (vec) {  // (kk < k then holds for whole vectors)
+        xv[i] = *reinterpret_cast<const v4f*>(xr + min(kk, P.k - 4));
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xv[i][u] = xr[min(kk + u, P.k - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) xv[i][u] = row < P.m && kk + u < P.k ? xv[i][u] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < CJ; ++u) wv[u] = reinterpret_cast<const uint32_t*>(wr + (size_t)g * 2 * kFragBytes)[u];
+    sc = P.wst[(size_t)g * P.np + wn];
+  };
+  if (chunks > 0) fetch(0);
   for (int g = 0; 8 * g < chunks; ++g) {
     const int nfull = min(8, chunks - 8 * g);  // uniform over the block
-    __syncthreads();                           // the previous group's reads are done
-    {
-      // x: thread t stages 4*RPT inputs of one row (zero past m or k)
-      constexpr int SEG = 4 * RPT, SPR = kGroup / SEG;
-      const int r = tid / SPR, seg = tid % SPR, row = m0 + r, kk = 64 * g + SEG * seg;
+    lds_barrier();                             // the previous group's reads are done
 #pragma unroll
-      for (int u = 0; u < SEG; ++u)
-        xs[r][SEG * seg + u] = (row < P.m && kk + u < P.k) ? P.x[(size_t)row * P.k + kk + u] : 0.0f;
-    }
-    {
-      // w: thread t stages column t/4, 16 inputs from one fragment lane (the
-      // repacked layout is zero past n and k, and n0 + 63 < np)
-      const int c = tid >> 2, h = (tid >> 1) & 1, part = tid & 1, n = n0 + c;
-      const uint4 raw = *reinterpret_cast<const uint4*>(
-          P.wt + ((size_t)((n >> 5) * P.g + g) * 2 + h) * kFragBytes + ((n & 31) + 32 * part) * 16);
-      const float sc = P.wst[(size_t)g * P.np + n];
-      const uint32_t word[4] = {raw.x, raw.y, raw.z, raw.w};
+    for (int i = 0; i < RPT; ++i) *reinterpret_cast<v4f*>(&xs[tr + 16 * i][xk]) = xv[i];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) ws[c][32 * h + 16 * part + u] = (float)(int8_t)(word[u >> 2] >> (8 * (u & 3))) * sc;
-    }
-    __syncthreads();
+    for (int u = 0; u < 4 * CJ; ++u) ws[wcol][woff + u] = (float)(int8_t)(wv[u >> 2] >> (8 * (u & 3))) * sc;
+    if (8 * (g + 1) < chunks) fetch(g + 1);
+    lds_barrier();
+#pragma unroll RPT * CJ >= 8 ? 1 : 2
     for (int cc = 0; cc < nfull; ++cc) {
-      float xv[RPT][8], wv[4][8];
+      float a[RPT][8], b[CJ][8];
+      auto read8 = [&](const float* src, float (&d)[8]) {
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const float4 a = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc]);
-        const float4 b = *reinterpret_cast<const float4*>(&xs[RPT * tr + i][8 * cc + 4]);
-        xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w;
-        xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
-      }
+        for (int h = 0; h < 2; ++h) {
+          const v4f t = *reinterpret_cast<const v4f*>(src + 8 * cc + 4 * h);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float4 a = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc]);
-        const float4 b = *reinterpret_cast<const float4*>(&ws[tc + 16 * j][8 * cc + 4]);
-        wv[j][0] = a.x; wv[j][1] = a.y; wv[j][2] = a.z; wv[j][3] = a.w;
-        wv[j][4] = b.x; wv[j][5] = b.y; wv[j][6] = b.z; wv[j][7] = b.w;
-      }
+          for (int u = 0; u < 4; ++u) d[4 * h + u] = t[u];
+        }
+      };
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) read8(xs[RPT * tr + i], a[i]);
+#pragma unroll
+      for (int j = 0; j < CJ; ++j) read8(ws[tc + 16 * j], b[j]);
 #pragma unroll
       for (int i = 0; i < RPT; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < CJ; ++j)
 #pragma unroll
-          for (int q = 0; q < 8; ++q) acc[i][j][q] = acc[i][j][q] + xv[i][q] * wv[j][q];
+          for (int q = 0; q < 8; ++q) acc[i][j][q] = acc[i][j][q] + a[i][q] * b[j][q];
     }
   }
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int row = m0 + RPT * tr + i;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < CJ; ++j) {
       const int n = n0 + tc + 16 * j;
-      if (row >= mhi || n < nlo || n >= nhi) continue;
+      if (row >= mhi || n >= nhi) continue;
       float y = -0.0f;
 #pragma unroll
       for (int q = 0; q < 8; ++q) y = y + acc[i][j][q];
@@ -1795,28 +1824,32 @@ __device__ __forceinline__ void fp32_tile(const FProj& P, int m0, int n0, int mh
 // The FP32 path of a whole projection: the blocks walk its tiles.  Behind a wide
 // launch (P.chain) they mostly only leave, which takes ~4.6 us by rocprof whether
 // the grid is 512 or 2048 blocks.
+constexpr int kF32Rpt = 2, kF32Cj = 4;
 __global__ __launch_bounds__(256) void k_linear_fp32(FProj P) {
-  __shared__ __attribute__((aligned(16))) F32Lds L;
+  constexpr int ROWS = 16 * kF32Rpt, COLS = 16 * kF32Cj;
+  __shared__ __attribute__((aligned(16))) F32Lds<kF32Rpt, kF32Cj> L;
   if (P.chain) {
-    const bool hit = chain_hit(P.chain);
-    chain_close(P.chain);
-    if (!hit) return;  // the inputs were finite: the int8 kernels ran
+    const ChainView v = chain_view(P.chain);
+    chain_close(P.chain, v);
+    if (!v.reported()) return;  // the inputs were finite: the int8 kernels ran
   }
-  const int col_tiles = (P.n + kF32Cols - 1) / kF32Cols;
-  const int tiles = ((P.m + kF32Rows - 1) / kF32Rows) * col_tiles;
+  const int col_tiles = (P.n + COLS - 1) / COLS;
+  const int tiles = ((P.m + ROWS - 1) / ROWS) * col_tiles;
   for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const int m0 = t / col_tiles * kF32Rows, n0 = t % col_tiles * kF32Cols;
-    fp32_tile<2>(P, m0, n0, P.m, 0, P.n, L);
+    const int m0 = t / col_tiles * ROWS, n0 = t % col_tiles * COLS;
+    fp32_tile(P, m0, n0, P.m, P.n, L);
   }
 }
-// The FP32 path of an int8 block's outputs: rows [m0, mhi) (at most 16*RPT), columns [nlo, nhi).
-template <int RPT>
-__device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k, int m0, int mhi, int nlo, int nhi, uint8_t* lds) {
+// The FP32 path of an int8 block's outputs: rows [m0, mhi) (at most 16*RPT), columns
+// [nlo, nhi) (at most 16*CJ).
+template <int RPT, int CJ, int BYTES>
+__device__ __forceinline__ void fp32_block(const Proj& S, const float* x, int k, int m0, int mhi, int nlo, int nhi,
+                                           uint8_t (&lds)[BYTES]) {
+  static_assert(sizeof(F32Lds<RPT, CJ>) <= BYTES, "the FP32 tile fits");
   const FProj P = {x, S.wt, S.wst, S.bias, S.lmid, S.lb, S.lora, S.rank, S.lscale, S.out, S.m, S.ldm, k, S.g, S.n, S.np,
                    S.epilogue, S.layout, nullptr};
   __syncthreads();  // every wave's loads into this LDS have landed
-  for (int n0 = nlo / kF32Cols * kF32Cols; n0 < nhi; n0 += kF32Cols)
-    fp32_tile<RPT>(P, m0, n0, mhi, nlo, nhi, *reinterpret_cast<F32Lds*>(lds));
+  fp32_tile(P, m0, nlo, mhi, nhi, reinterpret_cast<F32Lds<RPT, CJ>&>(lds));
 }
 
 // What a launch of the skinny, posting or mid kernel holds besides plain
@@ -1991,15 +2024,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     __builtin_amdgcn_sched_barrier(0);
   }
   if constexpr (MODE == kModeChained) {  // non-finite inputs take the FP32 path, once the loads into LDS have landed
-    const bool hit = chain_hit(b.chain);
-    chain_close(b.chain);
-    if (hit) {
+    const ChainView cv = chain_view(b.chain);
+    chain_close(b.chain, cv);
+    if (cv.reported()) {
       wait_vmcnt<0>();
       // (the fields are read again here, so that they do not stay in registers)
       int pi = __builtin_amdgcn_readfirstlane(pidx);
       asm volatile("" : "+s"(pi));
-      for (int r = m0; r < min(m0 + BM, P.m); r += 32)
-        fp32_block<2>(b.p[pi], b.fx[pi], b.fk, r, min(r + 32, P.m), n0, min(n0 + BN, P.n), reinterpret_cast<uint8_t*>(&ring));
+      fp32_block<BM / 16, BN / 16>(b.p[pi], b.fx[pi], b.fk, m0, min(m0 + BM, P.m), n0, min(n0 + BN, P.n),
+                                   reinterpret_cast<uint8_t(&)[sizeof(ring)]>(ring));
       return;
     }
   }
@@ -2469,7 +2502,7 @@ __device__ __forceinline__ bool skinny_short(const Proj& P, int c0, bool live, i
   }
   // the non-finite flag is read while the first loads are in flight; the
   // whole block leaves on it (after they land: they write this block's LDS)
-  const bool skip = MODE == kModeChained && chain_hit(chain);
+  const bool skip = MODE == kModeChained && chain_view(chain).reported();
   wait_vmcnt<0>();
   if (skip) return true;
   lds_barrier();
@@ -2605,7 +2638,7 @@ __device__ __forceinline__ bool skinny_long(const Proj& P, int local, int wid, i
   }
   // the non-finite flag, read while the first loads are in flight (the block
   // leaves after they land: the x chunk writes this block's LDS)
-  if (MODE == kModeChained && chain_hit(chain)) {
+  if (MODE == kModeChained && chain_view(chain).reported()) {
     wait_vmcnt<0>();
     return true;
   }
@@ -2685,7 +2718,6 @@ __device__ __forceinline__ void skinny_row_tile(const Proj& P, int& strip, int& 
 template <int RT, int CT, int CTL, int DBS, int DBL, bool DOTS, bool LORA, int MODE>
 __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[skinny_lds_bytes(RT, CTL)];
-  static_assert(MODE != kModeChained || skinny_lds_bytes(RT, CTL) >= (int)sizeof(F32Lds), "the FP32 tile fits");
   const int pidx = find_proj<true>(b, blockIdx.x);
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2733,8 +2765,17 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
     skip = skinny_long<1, CTL, DBL, 4, DOTS, LORA, MODE>(P, strip, wid, lane, lds, m0, b.chain);
   }
   if constexpr (MODE == kModeChained) {
-    chain_close(b.chain);
-    if (skip) fp32_block<RT>(P, b.fx[pidx], b.fk, m0, mhi, nlo, min(nhi, P.n), lds);
+    chain_close(b.chain, chain_view(b.chain));
+    if (skip) {  // (a 4-wave block's columns are one tile of CTL; a dealt block's go 64, then 32 at a time)
+      const float* x = b.fx[pidx];
+      nhi = min(nhi, P.n);
+      if (P.nseg != 1) {
+        fp32_block<1, CTL>(P, x, b.fk, m0, mhi, nlo, nhi, lds);
+      } else {
+        for (; nhi - nlo > 32; nlo += 64) fp32_block<RT, 4>(P, x, b.fk, m0, mhi, nlo, min(nhi, nlo + 64), lds);
+        if (nlo < nhi) fp32_block<RT, 2>(P, x, b.fk, m0, mhi, nlo, nhi, lds);
+      }
+    }
   }
 }
 // The long-K path for launches of few blocks, without its step-by-step hand-off:
@@ -2749,7 +2790,7 @@ __global__ __launch_bounds__(256) void k_linear_post(Batch b) {
   constexpr int NG = GMAX / 4;
   __shared__ __attribute__((aligned(16))) float xl[16][GMAX + 4];
   __shared__ __attribute__((aligned(16))) float tp[GMAX][4][64];
-  static_assert(MODE == kModePlain || (MODE == kModeChained && sizeof(tp) >= sizeof(F32Lds)), "the FP32 tile fits");
+  static_assert(MODE == kModePlain || MODE == kModeChained, "no pair");
   const int pidx = find_proj<true>(b, blockIdx.x);
   const Proj P = b.p[pidx];
   const int lane = threadIdx.x & 63;
@@ -2767,6 +2808,7 @@ __global__ __launch_bounds__(256) void k_linear_post(Batch b) {
 #pragma unroll
   for (int i = 0; i < XN; ++i)
     xv[i] = *reinterpret_cast<const v4f*>(xr + 4 * min((int)(threadIdx.x & 15) + 16 * i, last_piece));
+  __builtin_amdgcn_sched_barrier(0);  // the first loads: what the wait before the barrier needs
   const uint8_t* pb;
   const float* pw;
   skinny_weights<false>(P, c0, lane, pb, pw);
@@ -2782,10 +2824,11 @@ __global__ __launch_bounds__(256) void k_linear_post(Batch b) {
   }
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (MODE == kModeChained) {  // non-finite inputs: the FP32 path of this block's outputs
-    const bool hit = chain_hit(b.chain);
-    chain_close(b.chain);
-    if (hit) {
-      fp32_block<1>(P, b.fx[pidx], b.fk, r0, min(r0 + 16, P.m), c0, min(c0 + 16, P.n), reinterpret_cast<uint8_t*>(&tp));
+    const ChainView cv = chain_view(b.chain);
+    chain_close(b.chain, cv);
+    if (cv.reported()) {
+      fp32_block<1, 1>(P, b.fx[pidx], b.fk, r0, min(r0 + 16, P.m), c0, min(c0 + 16, P.n),
+                       reinterpret_cast<uint8_t(&)[sizeof(tp)]>(tp));
       return;
     }
   }
@@ -2875,7 +2918,6 @@ __global__ __launch_bounds__(256) void k_apply_few(Proj P, const float* __restri
   __shared__ __attribute__((aligned(16))) uint8_t qx[kFewRows * QS];
   __shared__ float xs[kFewRows][GMAX];
   __shared__ __attribute__((aligned(16))) float tp[GMAX][4][64];
-  static_assert(sizeof(tp) >= sizeof(F32Lds), "the FP32 tile fits");
   const int G = P.g, m = P.m;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2953,7 +2995,7 @@ __global__ __launch_bounds__(256) void k_apply_few(Proj P, const float* __restri
   else quantize(std::integral_constant<int, NMAX>{});
   if (__syncthreads_or(bad)) {  // the FP32 path of this block's outputs
     wait_vmcnt<0>();
-    fp32_block<1>(P, x, k, 0, m, c0, min(c0 + 16, P.n), reinterpret_cast<uint8_t*>(&tp));
+    fp32_block<1, 1>(P, x, k, 0, m, c0, min(c0 + 16, P.n), reinterpret_cast<uint8_t(&)[sizeof(tp)]>(tp));
     return;
   }
   const v4i magic = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
@@ -3441,7 +3483,7 @@ hipError_t launch_chain_reset(Chain* chain, hipStream_t s) {
 
 hipError_t launch_linear_fp32(const FProj& p, hipStream_t s) {
   if (p.m == 0 || p.n == 0) return hipSuccess;
-  const long tiles = (long)((p.m + kF32Rows - 1) / kF32Rows) * ((p.n + kF32Cols - 1) / kF32Cols);
+  const long tiles = (long)((p.m + 16 * kF32Rpt - 1) / (16 * kF32Rpt)) * ((p.n + 16 * kF32Cj - 1) / (16 * kF32Cj));
   const long blocks = std::min(tiles, 1L << 23);  // a grid under 2^32 threads
   k_linear_fp32<<<(unsigned)blocks, 256, 0, s>>>(p);
   return hipGetLastError();

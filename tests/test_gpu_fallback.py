@@ -176,6 +176,30 @@ def test_apply_columns_in_row_chunks(ctx, m, k, n, bad):
     assert same(got, np.ascontiguousarray(want.T))
 
 
+# The FP32 path inside the blocks of the skinny, posting and mid kernels, finite
+# and non-finite inputs in turn: short K with 2, 3, 5, 6 and 7 units of 16 columns
+# per block (FP32 tiles of 32 and 64 columns, partial ones and the last block's
+# included), one and two row tiles, row chunks; 4-wave blocks of one and two row
+# tiles and of 33 to 64 groups; the posting kernel's; the mid kernel's 64 x 64.
+@pytest.mark.parametrize("m,k,n,rank", [(24, 2048, 5200, 0), (12, 512, 5200, 16), (16, 70, 8230, 0), (20, 64, 17001, 0),
+                                        (17, 72, 20800, 3), (9, 64, 28011, 0), (128, 2048, 2050, 0), (65, 64, 5203, 16),
+                                        (24, 4096, 300, 5), (10, 2112, 33, 0), (33, 2304, 100, 16), (24, 512, 300, 0),
+                                        (30, 6145, 70, 16), (12, 4224, 40, 0), (100, 512, 300, 5), (513, 96, 65, 16)])
+def test_apply_non_finite_inside_the_int8_kernels(ctx, m, k, n, rank):
+    rng = np.random.default_rng(m + k + n + rank)
+    x, v, s, bias, a, b = case(rng, m, k, n, rank)
+    h = ctx.weights_from_quantized(dev(v), dev(s))
+    base = rng.standard_normal((m, n)).astype(np.float32)
+    bad = x.copy()
+    bad[m - 1, k - 1] = np.nan  # the other rows stay finite: the FP32 path's own sums
+    for inp in (x, bad, x, bad):
+        lora = dq8.Lora(ctx.lora_mid(dev(inp), dev(a)), dev(b), 0.5) if rank else None
+        got = host(ctx.apply(h, dev(inp), out=dev(base.copy()), bias=dev(bias), lora=lora, epilogue=dq8.ADD))
+        want, fp32 = dq8o.apply(inp, v, s, bias=bias, a=a, b=b, scale=0.5, result=base, epilogue=1, threads=8)
+        assert fp32 == (inp is bad)
+        assert same(got, want)
+
+
 # out sharing memory with a finite x: in place, shifted by rows or by part of a
 # row, and reaching into x from either side, at the rows that k_apply_few would
 # otherwise take and just past them.

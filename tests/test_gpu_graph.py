@@ -266,7 +266,8 @@ def test_reserve_while_another_stream_captures_globally_keeps_that_capture():
 
 
 @pytest.mark.parametrize("m,k,n", [(2, 512, 300), (24, 2048, 300), (24, 6144, 512), (100, 512, 300), (600, 512, 300),
-                                   (1100, 128, 2050)])
+                                   (1100, 128, 2050), (24, 512, 5200), (12, 512, 5200), (128, 2048, 2050),
+                                   (24, 4096, 300)])
 def test_replayed_apply_follows_each_inputs_finiteness(ctx, m, k, n):
     # the device's choice between the int8 and the FP32 path (few-rows, posting,
     # skinny, mid and wide kernels) in replays of one captured call, with finite
