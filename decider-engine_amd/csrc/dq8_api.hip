@@ -329,14 +329,19 @@ int units_per_block(long units, bool /*has_long*/) {
 // How a call's items of more than 32 rows run (measured graph-replayed, 24
 // launches over rotating weights):
 //  * small: items of at most 512 rows as chunks of at most 32
-//    rows on the skinny kernel, if all the call's chunks together read at most
-//    chunk_bytes of weights (the first read comes from HBM, the rest mostly
-//    from cache).  Against the mid kernel: 128 x 2048 -> 2048 7.8 and 9.6 us,
-//    256 x 2048 -> 2048 (36 MB) 8.1 and 9.9, 64 x 2048 -> 6144 (27 MB) 7.9 and
-//    9.9, 96 x 6144 -> 2048 (40 MB) 18.9 and 20.9; beyond the limit 96 x 2048 ->
-//    6144 (40 MB) 11.2 and 10.3, 256 x 6144 -> 1024 (53 MB) 22.0 and 21.1, 64 x
-//    6144 -> 8224 (107 MB) 45 and 21.5, 512 x 512 -> 2048 (18 MB) 8.1 and 5.7.
-//    A chunk's time is its bytes, the mid kernel's its K.
+//    rows on the skinny kernel, if all the call's chunks together read few enough
+//    weight bytes (the first read comes from HBM, the rest mostly from cache).  A
+//    chunk's time is its bytes, the mid kernel's its longest K; against the mid
+//    kernel, short K (a wave streams whole columns): 128 x 2048 -> 2048 7.8 and 9.6
+//    us, 256 x 2048 -> 2048 (36 MB) 8.1 and 9.9, 64 x 2048 -> 6144 (27 MB) 7.9 and
+//    9.9; beyond the limit 96 x 2048 -> 6144 (40 MB) 11.2 and 10.3, 512 x 512 -> 2048
+//    (18 MB) 8.1 and 5.7.  Long K (4 waves share them) up to half the bytes per input,
+//    where the two meet: 128 x 4096 -> 2048 (36 MB) 16.2 and 16.2, 192 (53 MB) 22.2 and
+//    16.4; 256 x 6144 -> 1024 (53 MB) 21.6 and 21.6, 96 x 6144 -> 2048 (40 MB) 19.1 and
+//    21.8; 256 x 8192 -> 1024 (71 MB) 27.0 and 27.7, 192 (53 MB) 23.3 and 27.5; 36 x
+//    16384 -> 2048 (71 MB) 25.8 and 50.7, 128 (143 MB) 46.9 and 50.8, 192 67.9 and 51.1.
+//    Both sorts in one call: 45 rows of two 2048 -> 6144, 8192 -> 1024 and 4096 -> 2048
+//    (54 and 36 MB) 25.2 and 30.0.
 //  * mid: the others on the mid kernel if the wide grid would leave its blocks
 //    alone on their CUs: at most kMidBlocks blocks (64 x 128; one round of the
 //    mid kernel's 64 x 64 blocks, two per CU).  Against the wide kernel: 512 x
@@ -349,7 +354,9 @@ int units_per_block(long units, bool /*has_long*/) {
 //  * the wide kernel otherwise.
 // Rows are independent, so the results are the same bits either way.
 constexpr long kMidBlocks = 256, kMidMixedBlocks = 768;
-double chunk_bytes(size_t k) { return std::min(17.5e3 * (double)k, 45e6); }
+// The inputs (K) whose time on the mid kernel equals that of `bytes` of chunks of
+// a projection of k inputs.
+double chunk_cost(size_t k, double bytes) { return bytes / (groups_of(k) <= 32 ? 17.5e3 : 8.8e3); }
 double weight_bytes(const dq8::Weights& w) { return (double)w.n * w.k + 4.0 * w.n * w.g; }
 bool may_split(const dq8::Weights& w, size_t m) { return kind_of(w, m) == 0 && m <= 512; }
 long wide_blocks(const dq8::Weights& w, size_t m) {
@@ -364,7 +371,7 @@ struct CallPlan {
 template <class Item, class W>
 CallPlan call_plan(const Item* items, size_t count, W weights_of) {
   long blocks = 0, fixed = 0;  // wide blocks of the items that may run as chunks, and of the others
-  double bytes = 0;
+  double cost = 0;
   size_t longest = 0;
   bool has_long = false, has_short = false;
   for (size_t i = 0; i < count; ++i) {
@@ -374,12 +381,12 @@ CallPlan call_plan(const Item* items, size_t count, W weights_of) {
     const bool can = may_split(w, m);
     (can ? blocks : fixed) += wide_blocks(w, m);
     if (can) {
-      bytes += (double)((m + 31) / 32) * weight_bytes(w);
+      cost += chunk_cost(w.k, (double)((m + 31) / 32) * weight_bytes(w));
       longest = std::max(longest, (size_t)w.k);
     }
     (w.g > 32 ? has_long : has_short) = true;
   }
-  const bool small = bytes <= chunk_bytes(longest);
+  const bool small = cost <= (double)longest;
   const long left = fixed + (small ? 0 : blocks);
   return {small, left <= (has_long && has_short ? kMidMixedBlocks : kMidBlocks)};
 }
@@ -1148,7 +1155,7 @@ dq8_status check_mid(const float* x, size_t m, size_t k, const float* a, size_t 
 constexpr long kMidPairBlocks = 512;
 int pair_kind(const dq8::Weights& g, const int8_t* q, const float* xs, size_t m, const dq8_lora* a, const dq8_lora* b) {
   if (needs_pad(g, q) || needs_xs_pad(g, xs)) return -1;
-  const bool skinny = m <= 32 || (m <= 512 && 2.0 * (double)((m + 31) / 32) * weight_bytes(g) <= chunk_bytes(g.k));
+  const bool skinny = m <= 32 || (m <= 512 && chunk_cost(g.k, 2.0 * (double)((m + 31) / 32) * weight_bytes(g)) <= (double)g.k);
   if (skinny && !a == !b && (!a || a->rank == b->rank)) return m > 16 ? 2 : 1;
   if (m <= 32) return -1;
   const long tiles = (long)((m + dq8::block_rows(3, true) - 1) / dq8::block_rows(3, true)) *

@@ -1254,7 +1254,8 @@ SMALL_CALLS = [(65, 2048, 300, dq8.WRITE), (96, 6144, 2048, dq8.ADD), (128, 2048
                (128, 2048, 8224, dq8.WRITE), (200, 4096, 100, dq8.ADD), (256, 2048, 512, dq8.WRITE),
                (384, 2048, 2048, dq8.SWIGLU), (512, 2048, 2048, dq8.WRITE), (512, 6144, 1024, dq8.ADD),
                (513, 2048, 256, dq8.WRITE), (192, 2048, 6144, dq8.SWIGLU), (192, 6144, 2048, dq8.ADD),
-               (256, 6144, 2048, dq8.ADD)]
+               (256, 6144, 2048, dq8.ADD), (33, 16384, 300, dq8.ADD), (64, 12288, 700, dq8.WRITE),
+               (70, 8192, 2050, dq8.WRITE), (330, 3072, 700, dq8.SWIGLU)]
 
 
 @pytest.mark.parametrize("m,k,n,ep", SMALL_CALLS)
@@ -1272,6 +1273,25 @@ def test_small_calls_bit_exact(ctx, m, k, n, ep):
     # the same rows through dq8_apply (fp32 input, quantized inside, its own launch)
     got_a = host(ctx.apply(h, dev(x), out=dev(base.copy()), bias=dev(bias), epilogue=ep))
     assert bits_equal(got_a, want)
+
+
+# Long and short K in one call, whose row chunks cost what the longest K would on
+# the mid kernel: calls on both sides of that.
+@pytest.mark.parametrize("m,shapes", [(45, [(2048, 1500), (2048, 700), (8192, 300), (4096, 500)]),
+                                      (100, [(2048, 3000), (6144, 900)]), (40, [(12288, 200), (130, 999)])])
+def test_grouped_call_of_long_and_short_k(ctx, m, shapes):
+    rng = np.random.default_rng(m)
+    items, wants = [], []
+    for k, n in shapes:
+        x = make_x(rng, m, k, "outliers")
+        wv, ws = dq8o.quantize_weights(make_w(rng, n, k))
+        q, s = ctx.quantize(dev(x))
+        items.append(dq8.Item(ctx.weights_from_quantized(dev(wv), dev(ws)), q, s,
+                              torch.zeros((m, n), dtype=torch.float32, device="cuda")))
+        wants.append(dq8o.linear(x, wv, ws, threads=8))
+    ctx.linear_batch(items)
+    for it, want in zip(items, wants):
+        assert bits_equal(host(it.out), want)
 
 
 @pytest.mark.parametrize("m", [100, 300])
