@@ -3644,11 +3644,16 @@ int block_cols(int kind, bool pair) {
   return kind == 0 ? 32 * DQ8_WIDE_CT * DQ8_WIDE_WN / (pair ? 2 : 1) : 64;
 }
 // The group bound of the posting kernel (k_linear_post) that takes a skinny launch,
-// or 0: every projection on the 4-wave path, and up to 32 groups, or 65 to 96 in at
-// most one block per CU (its LDS).  Graph-replayed, 24 rows, against the skinny
-// kernel: 2048 -> 2048 3.8 and 4.6 us, 2048 -> 4608 (576 blocks) 7.2 and 9.0, 6144
-// -> 2048 9.1 and 9.8; 4096 -> 2048 (64 groups, a third of the loads repeats) 8.6
-// and 7.3, 6144 -> 4096 (512 blocks) 16.1 and 12.3.
+// or 0: every projection on the 4-wave path, and
+//  * up to 32 groups (an instance loads all 32, repeats past the last): 13 or more,
+//    or 5 or more in at most one block per CU.  Graph-replayed against the skinny
+//    kernel: 24 x 2048 -> 2048 3.8 and 4.5 us, 24 x 1024 -> 2048 3.6 and 4.2; 40 rows -> 2048
+//    (512 blocks) of K = 1024 4.8 and 5.0, 768 4.9 and 4.7, 512 4.7 and 4.4, 256 4.7 and
+//    4.2; one block per CU or fewer, 24 rows -> 2048 of 512 3.5 and 3.7, 256 3.55 and 3.45.
+//  * 65 to 96 groups in at most one block per CU (its LDS): 24 x 6144 -> 2048 8.2 and
+//    9.6, 24 x 5120 -> 1024 7.6 and 8.2, 24 x 4352 -> 1024 7.3 and 7.2, 1 x 4352 -> 1024
+//    5.9 and 6.9; 64 groups on this instance (a third of the loads repeats), 24 x 4096 ->
+//    2048, 8.6 and 7.3; 6144 -> 4096 (512 blocks) 16.1 and 12.3.
 static int post_groups(const Batch& b) {
   int lo = 1 << 30, hi = 0;
   for (int i = 0; i < b.count; ++i) {
@@ -3656,7 +3661,7 @@ static int post_groups(const Batch& b) {
     lo = std::min(lo, b.p[i].g);
     hi = std::max(hi, b.p[i].g);
   }
-  if (hi <= 32) return 32;
+  if (hi <= 32) return hi > 12 || (hi > 4 && b.total_waves <= 256) ? 32 : 0;
   return lo > 64 && hi <= 96 && b.total_waves <= 256 ? 96 : 0;
 }
 bool wide_can_pair() { return wide_pair_shape(DQ8_WIDE_WN, DQ8_WIDE_RT, DQ8_WIDE_CT); }

@@ -1412,11 +1412,12 @@ def test_ffn_chain_quantizes_beside_the_middle_product(ctx, m, hidden, inter):
     test_ffn_chain_matches_the_reference_sequence(ctx, m, hidden, inter, True)
 
 
-# The posting kernel (few strips, up to 32 groups or 65 to 96) at its bounds and
-# just past them: one group, a partial last one, 64 / 65 / 96 / 97 groups, one and
+# The posting kernel (few strips, 5 to 32 groups or 65 to 96) at its bounds and
+# just past them: one group, 4 and 5, a partial last one, 12 and 13 in more than a block per CU, 64 / 65 / 96 / 97 groups, one and
 # two row tiles, a last run of fewer than 8 strips, more than 256 blocks.
 @pytest.mark.parametrize("m,k,n,rank", [(1, 64, 16, None), (16, 2048, 33, 16), (31, 2047, 50, 5), (17, 4096, 40, 16),
                                         (17, 4160, 200, 16), (32, 6144, 2064, None), (20, 6144, 70, 20),
-                                        (9, 6145, 48, None), (33, 1000, 100, 16)])
+                                        (9, 6145, 48, None), (33, 1000, 100, 16), (24, 256, 300, 16),
+                                        (24, 320, 300, 5), (40, 768, 2048, None), (40, 832, 2050, 16)])
 def test_posting_kernel_edges(ctx, m, k, n, rank):
     test_mid_and_wide_kernel_edges(ctx, m, k, n, rank)
