@@ -348,12 +348,18 @@ int units_per_block(long units, bool /*has_long*/) {
 //    6144 -> 2048 (128 blocks) 22.3 and 39.0 us, 1000 x 2048 -> 2048 (256) 14.4
 //    and 16.3; beyond it 400 x 2048 -> 6144 (336) 20.2 and 19.9, 2048 x 2048 ->
 //    2048 (512) 25.0 and 21.1.  In a call that mixes long and short K the wide
-//    kernel's long blocks trail, up to kMidMixedBlocks: a layer set of 9
-//    projections at 77 rows (466) 29.5 and 42.3 us, 192 (699) 42.6 and 49.4;
-//    384 (1404) 77.9 and 66.6.
+//    kernel's long blocks trail alone on their CUs, up to kMidMixedBlocks whatever
+//    they are (down + k at 1300 rows, 420 blocks, 54.1 and 54.7; down + q at 768, 384,
+//    38.2 and 42.0), and while the long ones are few, at most kMidLongBlocks, up to
+//    kMidFewLongBlocks: a layer set of 9 projections at 77 rows (468, 32 long) 29.5 and
+//    42.3 us, 192 (702, 48) 46.2 and 53.7, 256 (936) 58.6 and 55.9; down + gate at 640
+//    rows (640, 160) 48.0 and 50.9, 768 (768, 192) 55.7 and 54.9; 8192 -> 1024 + q at 1600
+//    (600, 200) 59.5 and 66.0; but 4096 -> 2048 +
+//    q at 1000 (512, 256 long) 37.7 and 33.7, down + k at 1600 (500, 400) 66.7 and 58.0, 2048
+//    (640, 512) 75.0 and 70.8.
 //  * the wide kernel otherwise.
 // Rows are independent, so the results are the same bits either way.
-constexpr long kMidBlocks = 256, kMidMixedBlocks = 768;
+constexpr long kMidBlocks = 256, kMidMixedBlocks = 400, kMidFewLongBlocks = 720, kMidLongBlocks = 208;
 // The inputs (K) whose time on the mid kernel equals that of `bytes` of chunks of
 // a projection of k inputs.
 double chunk_cost(size_t k, double bytes) { return bytes / (groups_of(k) <= 32 ? 17.5e3 : 8.8e3); }
@@ -370,7 +376,8 @@ struct CallPlan {
 };
 template <class Item, class W>
 CallPlan call_plan(const Item* items, size_t count, W weights_of) {
-  long blocks = 0, fixed = 0;  // wide blocks of the items that may run as chunks, and of the others
+  // wide blocks (all, long K) of the items that may run as chunks, and of the others
+  long blocks[2] = {0, 0}, fixed[2] = {0, 0};
   double cost = 0;
   size_t longest = 0;
   bool has_long = false, has_short = false;
@@ -379,7 +386,9 @@ CallPlan call_plan(const Item* items, size_t count, W weights_of) {
     const size_t m = items[i].m;
     if (m == 0 || kind_of(w, m) != 0) continue;
     const bool can = may_split(w, m);
-    (can ? blocks : fixed) += wide_blocks(w, m);
+    long* part = can ? blocks : fixed;
+    part[0] += wide_blocks(w, m);
+    if (w.g > 32) part[1] += wide_blocks(w, m);
     if (can) {
       cost += chunk_cost(w.k, (double)((m + 31) / 32) * weight_bytes(w));
       longest = std::max(longest, (size_t)w.k);
@@ -387,8 +396,9 @@ CallPlan call_plan(const Item* items, size_t count, W weights_of) {
     (w.g > 32 ? has_long : has_short) = true;
   }
   const bool small = cost <= (double)longest;
-  const long left = fixed + (small ? 0 : blocks);
-  return {small, left <= (has_long && has_short ? kMidMixedBlocks : kMidBlocks)};
+  const long left = fixed[0] + (small ? 0 : blocks[0]), left_long = fixed[1] + (small ? 0 : blocks[1]);
+  const long mixed = left_long <= kMidLongBlocks ? kMidFewLongBlocks : kMidMixedBlocks;
+  return {small, left <= (has_long && has_short ? mixed : kMidBlocks)};
 }
 // Kernel kind of an item in nch row chunks.
 int item_kind(const dq8::Weights& w, size_t m, size_t nch, const CallPlan& plan) {

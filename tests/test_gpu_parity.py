@@ -1275,10 +1275,13 @@ def test_small_calls_bit_exact(ctx, m, k, n, ep):
     assert bits_equal(got_a, want)
 
 
-# Long and short K in one call, whose row chunks cost what the longest K would on
-# the mid kernel: calls on both sides of that.
+# Long and short K in one call: calls on both sides of the rule by which row chunks
+# cost what the longest K would on the mid kernel, and of the mid kernel's block limits
+# (many and few long-K blocks).
 @pytest.mark.parametrize("m,shapes", [(45, [(2048, 1500), (2048, 700), (8192, 300), (4096, 500)]),
-                                      (100, [(2048, 3000), (6144, 900)]), (40, [(12288, 200), (130, 999)])])
+                                      (100, [(2048, 3000), (6144, 900)]), (40, [(12288, 200), (130, 999)]),
+                                      (520, [(2112, 2700), (130, 3000)]), (520, [(2112, 3000), (130, 2600)]),
+                                      (600, [(2112, 640), (65, 8200)]), (700, [(2112, 640), (65, 7700)])])
 def test_grouped_call_of_long_and_short_k(ctx, m, shapes):
     rng = np.random.default_rng(m)
     items, wants = [], []
