@@ -3310,7 +3310,11 @@ __global__ __launch_bounds__(256) void k_lora_mid_dma_batch(MidBatch bt) {
 // clamped to its last 16 bytes; their products are never added.
 // Requires k % 4 == 0 and 16-byte aligned x and a.  24 rows, rank 16, graph-
 // replayed: 4.7 us at K = 2048 and 8.3 at 6144 (5.3 and 11.5 with one wave
-// reading both operands, multiplying and adding after whole rows had landed).
+// reading both operands, multiplying and adding after whole rows had landed).  Below
+// ~1100 inputs the hand-off is not won back: 3.0 and 2.6 us at 256, 3.1 and 3.0 at 512,
+// 3.85 and 3.3 at 524 (two tiles), 3.85 and 3.7 at 1024; a single tile adds
+// its own steps only (24 x 256: 3.4 us with all 64), and the tail elements are loaded up
+// front (524: 4.3 with their loads behind the sums).
 // A tile now moves 76 KB through LDS, ~600 of its ~970 cycles; 256-input tiles
 // (one barrier per 32 steps) took 19 us at 6144, 3 producers of two rows each the
 // same 8.4.
@@ -3386,6 +3390,14 @@ __device__ __forceinline__ void lora_mid_small(const float* __restrict__ x, int 
     lds_barrier();
     return;
   }
+  const int pr = lane >> 3, i = lane & 7;
+  const int row = r0 + pr / J, jr = j0 + pr % J;
+  // the tail elements (k % 4 == 0: none or four), loaded before the sums
+  v4f xt = {0.0f, 0.0f, 0.0f, 0.0f}, at = xt;
+  if (k & 4) {  // uniform
+    xt = *reinterpret_cast<const v4f*>(x + (size_t)min(row, m - 1) * k + 8 * chunks);
+    at = *reinterpret_cast<const v4f*>(a + (size_t)min(jr, rank - 1) * k + 8 * chunks);
+  }
   float acc = 0.0f;
   auto read = [&](float (&pv)[ST], int t) {
 #pragma unroll
@@ -3406,28 +3418,45 @@ __device__ __forceinline__ void lora_mid_small(const float* __restrict__ x, int 
   float pa[ST], pb[ST];
   lds_barrier();
   lds_barrier();
-  read(pa, 0);
-  int t = 2;  // iteration
-  for (; t <= tiles; t += 2) {
-    lds_barrier();
-    read(pb, t - 1);
-    add(pa);
-    lds_barrier();
-    read(pa, t);
-    add(pb);
+  if (tiles <= 1) {  // up to 512 inputs: their steps only, 16 at a time
+    if (tiles == 1) lds_barrier();
+    constexpr int PC = 16;
+#pragma unroll
+    for (int p = 0; p < ST; p += PC)
+      if (p < chunks) {  // uniform
+#pragma unroll
+        for (int u = p; u < p + PC; ++u) pa[u] = L.prod[0][u][lane];
+      }
+#pragma unroll
+    for (int p = 0; p < ST; p += PC)
+      if (p < chunks) {
+#pragma unroll
+        for (int u = p; u < p + PC; ++u) acc = acc + pa[u];
+      }
+  } else {
+    read(pa, 0);
+    int t = 2;  // iteration
+    for (; t <= tiles; t += 2) {
+      lds_barrier();
+      read(pb, t - 1);
+      add(pa);
+      lds_barrier();
+      read(pa, t);
+      add(pb);
+    }
+    if (t <= tiles + 1) {
+      lds_barrier();
+      add(pa);
+    }
   }
-  if (t <= tiles + 1) {
-    lds_barrier();
-    add(pa);
-  }
-  const int pr = lane >> 3, i = lane & 7;
   float sum = -0.0f;
 #pragma unroll
   for (int ii = 0; ii < 8; ++ii) sum = sum + __shfl(acc, (lane & ~7) + ii);
-  const int row = r0 + pr / J, jr = j0 + pr % J;
   if (i == 0 && row < m && jr < rank) {
-    const float *xg = x + (size_t)row * k, *ag = a + (size_t)jr * k;
-    for (int e = 8 * chunks; e < k; ++e) sum = sum + xg[e] * ag[e];
+    if (k & 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum = sum + xt[e] * at[e];
+    }
     mid[(size_t)row * rank + jr] = sum + 0.0f;
   }
 }
