@@ -87,12 +87,12 @@ def check_overflow_cases(want):
     assert np.isfinite(want).any()
 
 
-# m = 9 and 24: the skinny kernel (16- and 32-row); 48: two skinny row chunks;
-# 96 and 200: the wide kernel.  n = 100 columns run on the 4-wave strips (few
-# strips); k = 6144 is long K.
-@pytest.mark.parametrize("m", [9, 24, 48, 96, 200])
+# m = 9 and 24: the posting kernel (one and two row tiles; k = 2048 and 6144) and
+# the skinny kernel's long path (2112); 48 to 200: row chunks on them; 600: the mid
+# kernel (at k = 2112 with an odd last group); 1700 and n = 2500: the wide kernel.
+@pytest.mark.parametrize("m", [9, 24, 48, 96, 200, 600])
 @pytest.mark.parametrize("ep", [dq8.WRITE, dq8.ADD, dq8.SWIGLU])
-@pytest.mark.parametrize("k", [2048, 6144])
+@pytest.mark.parametrize("k", [2048, 6144, 2112])
 def test_overflowing_scale_products(ctx, m, ep, k):
     rng = np.random.default_rng(31 * m + 7 * ep + k)
     n = 100
@@ -118,6 +118,20 @@ def test_overflowing_scale_products(ctx, m, ep, k):
     h.free()
 
 
+def test_overflowing_scale_products_on_the_wide_kernel(ctx):
+    rng = np.random.default_rng(1700)
+    m, n, k = 1700, 2500, 192
+    x = overflow_x(rng, m, k)
+    wv, ws = dq8o.quantize_weights(overflow_w(rng, n, k))
+    h = ctx.weights_from_quantized(dev(wv), dev(ws))
+    q, s = ctx.quantize(dev(x))
+    got = host(ctx.linear(h, q, s))
+    want = dq8o.linear(x, wv, ws, threads=8)
+    check_overflow_cases(want)
+    assert same_bits(got, want)
+    h.free()
+
+
 @pytest.mark.parametrize("m", [9, 24])
 def test_overflowing_scale_products_on_dealt_short_k_units(ctx, m):
     # 6144 columns at short K: 192 strips, so the skinny launch deals its
@@ -135,12 +149,13 @@ def test_overflowing_scale_products_on_dealt_short_k_units(ctx, m):
     h.free()
 
 
-def test_overflowing_scale_products_through_the_pair_launch(ctx):
-    # gate and up of one FFN in one wide launch (h = silu(gate) * up), with
+# skinny pair in chunks, mid pair, wide pair
+@pytest.mark.parametrize("m,k,n", [(130, 2048, 320), (600, 2112, 330), (600, 256, 2000)])
+def test_overflowing_scale_products_through_the_pair_launch(ctx, m, k, n):
+    # gate and up of one FFN in one launch (h = silu(gate) * up), with
     # the overflowing groups in both projections; h's quantization reports
     # the non-finite h through the device flag.
     rng = np.random.default_rng(4242)
-    m, k, n = 130, 2048, 320
     x = overflow_x(rng, m, k)
     gv, gs = dq8o.quantize_weights(overflow_w(rng, n, k))
     wu = overflow_w(rng, n, k)[::-1].copy()

@@ -100,11 +100,13 @@ def test_apply_takes_the_path_the_crate_takes(ctx, m, k, n, rank, bad, ep):
     assert got2.tobytes() == got.tobytes()
 
 
-@pytest.mark.parametrize("m", [24, 130])
-def test_ffn_with_a_non_finite_h_takes_the_fp32_down(ctx, m):
+# h from the skinny pair (24 and 130 rows), the mid pair and the wide pair; each
+# call twice, with finite calls before and between
+@pytest.mark.parametrize("m,inter", [(24, 384), (130, 384), (600, 384), (600, 2048)])
+def test_ffn_with_a_non_finite_h_takes_the_fp32_down(ctx, m, inter):
     # qwen.rs:486-492 with h overflowing to infinity: the crate's down
     # projection finds QuantizedInputs::new(h) = None and runs columns_tiled.
-    hidden, inter = 256, 384
+    hidden = 256
     rng = np.random.default_rng(m)
     x = rng.standard_normal((m, hidden)).astype(np.float32)
     gv, gs = dq8o.quantize_weights((rng.standard_normal((inter, hidden)) * 0.05).astype(np.float32))
@@ -127,6 +129,14 @@ def test_ffn_with_a_non_finite_h_takes_the_fp32_down(ctx, m):
     assert fp32
     assert same(host(resid), want_r)
     assert int(host(flag)[0]) == 1
+    # finite and non-finite calls after it: each follows its own h
+    fh = dq8o.linear(x, uv, us, result=dq8o.linear(x, gv, gs, threads=4), epilogue=2, threads=4)
+    fr, fp32 = dq8o.apply(fh, dv, ds, result=resid0, epilogue=1, threads=8)
+    assert not fp32
+    for bad in (False, True, True, False):
+        resid, flag = dev(resid0.copy()), torch.zeros(1, dtype=torch.int32, device="cuda")
+        ctx.ffn(G, U, D, q, s, resid, biases=(dev(gb), dev(ub), None) if bad else (None, None, None), nonfinite=flag)
+        assert same(host(resid), want_r if bad else fr) and int(host(flag)[0]) == bad
 
 
 # dq8_apply of a few rows in one launch (quantization and the choice of path

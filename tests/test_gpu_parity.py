@@ -928,8 +928,8 @@ def test_ffn_chain_matches_the_reference_sequence(ctx, m, hidden, inter, lora):
 def test_ffn_gate_up_equals_write_then_swiglu(ctx, m, hidden, inter):
     # dq8_ffn_gate_up stores what the crate's gate Write and up SwiGlu apply
     # calls store (qwen.rs:489-490): the same bits as two dq8_linear calls and as
-    # the oracle, with and without biases; more than 64 rows take the wide pair
-    # launch, fewer the skinny one.  With quantize=True, h is also
+    # the oracle, with and without biases, on the skinny pair (few rows or few weight
+    # bytes) and the mid one.  With quantize=True, h is also
     # quantized (qwen.rs:491): the same bytes and scales as dq8_quantize(h) and
     # as the oracle's QuantizedInputs::new(h), for widths that end in a partial
     # group and widths that are not a multiple of 16 (byte stores).
@@ -958,13 +958,15 @@ def test_ffn_gate_up_equals_write_then_swiglu(ctx, m, hidden, inter):
         assert np.array_equal(host(hq), oq) and bits_equal(host(hs), os_)
 
 
-@pytest.mark.parametrize("m", [200, 24])
+# the skinny pair and the quantizer behind it (200 and 24 rows), the mid pair (114
+# blocks) and the wide pair (608 of the mid pair's blocks)
+@pytest.mark.parametrize("m,inter", [(200, 384), (24, 384), (600, 384), (600, 2048)])
 @pytest.mark.parametrize("given", [False, True])
-def test_ffn_gate_up_quantize_reports_a_non_finite_h(ctx, m, given):
+def test_ffn_gate_up_quantize_reports_a_non_finite_h(ctx, m, inter, given):
     # h overflowing to infinity in one column: QuantizedInputs::new(h) is None
     # (tensor.rs:321-339), reported as dq8_quantize reports it: NonFinite
     # without a flag, 1 ORed into the flag with one; h itself is still stored.
-    hidden, inter = 256, 384
+    hidden = 256
     rng = np.random.default_rng(m + given)
     x = rng.standard_normal((m, hidden)).astype(np.float32)
     gv, gs = dq8o.quantize_weights((rng.standard_normal((inter, hidden)) * 0.05).astype(np.float32))
@@ -1042,15 +1044,17 @@ def test_full_size_gdn_in_projection_properties(ctx):
     assert bits_equal(np.concatenate([host(ctx.linear(h1, q, s)), host(ctx.linear(h2, q, s))], axis=1), full)
 
 
-def test_ffn_gate_up_quantize_edge_groups(ctx):
-    # The pair launch's quantization of h on edge groups.  Weight rows 0-191 are
+# skinny pair, mid pair (76 blocks) and wide pair (912 of the mid pair's blocks)
+@pytest.mark.parametrize("m,inter", [(130, 256), (600, 256), (900, 2048)])
+def test_ffn_gate_up_quantize_edge_groups(ctx, m, inter):
+    # The pair launches' quantization of h on edge groups.  Weight rows 0-191 are
     # zero, so those columns of h come from the biases alone: columns 0-63 give
     # silu(-1000) * 0 = -0 (an all-zero group, scale 1); 64-127 silu(-80) ~
     # -1.5e-33 times up biases from 1e-10 to 8e-6 (subnormal h only, scale
     # FLT_MIN, bytes 0 and -1); 128-191 1e18 * 1e18..2e18 (h near 1e36);
-    # 192-255 ordinary values.  h, its bytes and scales must equal the
+    # 192 and up ordinary values.  h, its bytes and scales must equal the
     # oracle's h and QuantizedInputs::new(h).
-    m, hidden, inter = 130, 256, 256
+    hidden = 256
     rng = np.random.default_rng(4242)
     x = rng.standard_normal((m, hidden)).astype(np.float32)
     wg = (rng.standard_normal((inter, hidden)) * 0.01).astype(np.float32)
@@ -1101,9 +1105,9 @@ def _adapter(ctx, rng, m, k, n, rank, scale, x, placed):
 
 
 # (rows, hidden, intermediate, gate adapter, up adapter); an adapter is (rank,
-# placement) or None.  Rank 16 with aligned buffers (the reference checkpoints'
-# rank) and rank 0 run in the one-launch pair path; other ranks and offset
-# buffers go to separate gate and up launches.
+# placement) or None.  The wide pair takes rank 16 with aligned buffers (the
+# reference checkpoints' rank) and rank 0, the skinny one two adapters of one
+# rank, the mid one any; the others are separate gate and up launches.
 PAIR_LORA_CASES = [(130, 256, 384, (16, "aligned"), (16, "aligned")),
                    (130, 256, 384, (16, "aligned"), None),
                    (130, 256, 384, None, (16, "aligned")),
@@ -1231,8 +1235,8 @@ def test_ffn_gate_up_quantizes_over_its_inputs(ctx, m, hidden, inter, shared):
     assert bits_equal(host(h), want) and bits_equal(host(hq), wq) and bits_equal(host(hs), ws)
 
 
-# The skinny pair launch (up to 64 rows), whose 16-column tiles hold 8 gate and
-# 8 up columns: one and two row tiles and chunks, widths that end inside a unit,
+# The skinny pair launch (few rows or few weight bytes), whose 16-column tiles hold
+# 8 gate and 8 up columns: one and two row tiles and chunks, widths that end inside a unit,
 # the one-wave path (160 or more strips) and the 4-wave paths for few strips and
 # for long K, adapters of one rank, and the two-launch form they exclude.
 SKINNY_PAIR_CASES = [(1, 256, 5, None, None), (16, 256, 264, (16, "aligned"), (16, "aligned")),
@@ -1247,8 +1251,8 @@ def test_skinny_ffn_gate_up(ctx, m, hidden, inter, gl, ul):
     test_ffn_gate_up_with_adapters(ctx, m, hidden, inter, gl, ul)
 
 
-# 65-512 rows whose wide launch would be small run as 32-row chunks on the
-# skinny kernel (dq8_linear and grouped calls through run_linear, dq8_apply
+# 33-512 rows whose chunks read few weight bytes run as 32-row chunks on the
+# skinny and posting kernels (dq8_linear and grouped calls through run_linear, dq8_apply
 # through its own launch); shapes on both sides of the rule's limits.
 SMALL_CALLS = [(65, 2048, 300, dq8.WRITE), (96, 6144, 2048, dq8.ADD), (128, 2048, 2048, dq8.SWIGLU),
                (128, 2048, 8224, dq8.WRITE), (200, 4096, 100, dq8.ADD), (256, 2048, 512, dq8.WRITE),
@@ -1379,14 +1383,18 @@ def test_apply_non_finite_on_the_mid_and_wide_kernels(ctx, m, k, n):
         assert np.array_equal(np.isnan(got), nan) and got[~nan].tobytes() == want[~nan].tobytes()
 
 
-# The mid kernel's SwiGLU pair (at most 512 blocks of 32 x 64 outputs): partial
-# row and column blocks, long K, adapters of any two ranks or on one projection only; and the wide pair's
-# ragged edges just past that limit.
+# The mid kernel's SwiGLU pair (at most 512 blocks of 32 x 64 outputs, and more
+# weight bytes than the skinny pair's chunks may read): partial row and column
+# blocks, long K, adapters of any two ranks or on one projection only, and none; the
+# wide pair's ragged edges just past that limit.  (The first and the third run as
+# skinny chunks.)
 @pytest.mark.parametrize("m,hidden,inter,gl,ul",
                          [(100, 2304, 1000, None, None), (65, 6400, 136, (16, "aligned"), (5, "aligned")),
                           (97, 2048, 1300, (16, "offset"), (16, "aligned")), (130, 2048, 1001, None, (16, "aligned")),
                           (600, 256, 1100, (0, "aligned"), (20, "aligned")), (300, 256, 3300, None, None),
-                          (330, 256, 3100, (16, "aligned"), (16, "aligned"))])
+                          (330, 256, 3100, (16, "aligned"), (16, "aligned")), (600, 256, 1100, None, None),
+                          (77, 2048, 6144, None, None), (600, 256, 1100, (16, "offset"), (16, "aligned")),
+                          (577, 320, 1025, (16, "aligned"), (16, "aligned"))])
 def test_mid_and_wide_ffn_gate_up(ctx, m, hidden, inter, gl, ul):
     test_ffn_gate_up_with_adapters(ctx, m, hidden, inter, gl, ul)
 
@@ -1396,7 +1404,8 @@ def test_mid_and_wide_ffn_gate_up(ctx, m, hidden, inter, gl, ul):
 # 256-element chunks).
 @pytest.mark.parametrize("m,k,rank", [(4, 508, 2), (5, 512, 3), (3, 516, 1), (32, 1024, 16), (1, 764, 5), (2, 4096, 16),
                                       (7, 4356, 9), (24, 8448, 16), (1, 4, 1), (100, 1000, 20), (128, 516, 16),
-                                      (129, 516, 16)])
+                                      (129, 516, 16), (3, 100, 2), (24, 128, 16), (5, 132, 3), (24, 256, 16),
+                                      (6, 260, 5), (4, 388, 5), (1, 8, 1)])
 def test_lora_mid_few_rows_edges(ctx, m, k, rank):
     test_lora_mid_bit_exact(ctx, m, k, rank)
 
