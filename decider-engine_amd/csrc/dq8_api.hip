@@ -317,14 +317,8 @@ long short_units(const dq8::Weights& w) { return w.g <= 32 ? (w.n + 15) / 16 : 0
 // 8.3 us, gate+up 11.0 -> 8.8 us against 8-unit blocks of 4 whole strips on
 // fewer CUs).  Launches with long-K projections deal them the same way: the
 // 24-row 9-projection layer set went 3.42 -> 3.51 TB/s per question
-// (graph-replayed, 5 rotating weight copies).  (8 would select blocks of 4
-// whole 32-column strips, one per wave.)
-#ifndef DQ8_SKINNY_UNITS_MAX
-#define DQ8_SKINNY_UNITS_MAX 7
-#endif
-int units_per_block(long units, bool /*has_long*/) {
-  return (int)std::min((long)DQ8_SKINNY_UNITS_MAX, std::max(2L, (units + 255) / 256));
-}
+// (graph-replayed, 5 rotating weight copies).
+int units_per_block(long units) { return (int)std::min(7L, std::max(2L, (units + 255) / 256)); }
 
 // How a call's items of more than 32 rows run (measured graph-replayed, 24
 // launches over rotating weights):
@@ -408,7 +402,7 @@ int item_kind(const dq8::Weights& w, size_t m, size_t nch, const CallPlan& plan)
 
 // Place a filled projection in a launch of the given kernel kind: its first
 // wave/block, column strips, XCD split and the launch's running total.
-void place_proj(dq8::Proj& p, int kind, dq8::Batch& b, bool few_strips, long launch_units, bool launch_has_long) {
+void place_proj(dq8::Proj& p, int kind, dq8::Batch& b, bool few_strips, long launch_units) {
   p.wave_begin = b.total_waves;
   b.wave_begin[&p - b.p] = p.wave_begin;
   p.xcd_gm = 0;
@@ -435,8 +429,7 @@ void place_proj(dq8::Proj& p, int kind, dq8::Batch& b, bool few_strips, long lau
     if (p.nseg == 1) {
       // short K: 16-column units dealt to blocks, units_per_block at a time
       p.waves_n = p.pair ? (p.n + 7) / 8 : (p.n + 15) / 16;  // a pair's unit holds 8 outputs of each projection
-      p.units = units_per_block(launch_units, launch_has_long);
-      const int blocks = (p.waves_n + p.units - 1) / p.units;
+      const int units = units_per_block(launch_units), blocks = (p.waves_n + units - 1) / units;
       p.deal_q = p.waves_n / blocks;
       p.deal_r = p.waves_n % blocks;
       b.total_waves += blocks;
@@ -568,7 +561,6 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
   if (dots) plan.mid = false;
   // one-wave strips each skinny launch would have (see kSkinnyFewStrips)
   long strips[dq8::kKinds] = {}, units[dq8::kKinds] = {};
-  bool has_long[dq8::kKinds] = {};
   for (size_t i = 0; i < count; ++i) {
     const dq8_linear_item& it = items[i];
     if (it.m == 0) continue;
@@ -576,7 +568,6 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
     const int kind = item_kind(it.w->w, it.m, nch, plan);
     strips[kind] += (long)nch * short_strips(it.w->w);
     units[kind] += (long)nch * short_units(it.w->w);
-    has_long[kind] = has_long[kind] || it.w->w.g > 32;
   }
   size_t offset = 0;
   // Two passes: projections with long K (more than 32 groups) first, so their
@@ -639,7 +630,7 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
         b.fx[b.count - 1] = fb->x + r0 * w.k;
         b.fk = w.k;
       }
-      place_proj(p, kind, b, strips[kind] < kSkinnyFewStrips, units[kind], has_long[kind]);
+      place_proj(p, kind, b, strips[kind] < kSkinnyFewStrips, units[kind]);
     }
   }
   for (int kind = 0; kind < dq8::kKinds; ++kind) {
@@ -701,7 +692,7 @@ dq8_status run_pair(const dq8::Weights& g, const dq8::Weights& u, const int8_t* 
       b.hchain = qout->chain;
     }
     p.pair = 1;
-    place_proj(p, kind, b, units / 2 < kSkinnyFewStrips, units, g.g > 32);
+    place_proj(p, kind, b, units / 2 < kSkinnyFewStrips, units);
   }
   hipError_t e = dq8::launch_linear(b, kind, false, s);
   if (e == hipSuccess && qout) {
@@ -803,7 +794,7 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
       b.fx[b.count - 1] = fb->x + r0 * w.k;
       b.fk = w.k;
     }
-    place_proj(p, kind, b, (long)nch * short_strips(w) < kSkinnyFewStrips, (long)nch * short_units(w), w.g > 32);
+    place_proj(p, kind, b, (long)nch * short_strips(w) < kSkinnyFewStrips, (long)nch * short_units(w));
   }
   hipError_t e = dq8::launch_linear(b, kind, false, s);
   if (e == hipSuccess && fb && kind == 0)  // the other kernels hold the FP32 path themselves

@@ -85,8 +85,7 @@ struct Proj {
   int ldm;            // columns layout: rows of the whole output (M, or more for a row chunk)
   int wave_begin;     // first block of this projection in the launch
   int waves_n;        // column strips (wide: one block tile wide; skinny long K: 16 columns wide;
-                      // skinny short K: 16-column units, dealt to blocks `units` at a time)
-  int units;          // skinny short K: at most this many 16-column units per block (2..8)
+                      // skinny short K: 16-column units, dealt to blocks)
   int deal_q, deal_r; // skinny short K: the waves_n units over B = ceil(waves_n / units) blocks,
                       // deal_q = waves_n / B each and one more for the first deal_r = waves_n % B
   int xcd_gm;         // wide: row bands of the per-XCD tile regions (1, 2, 4, 8), 0 = row-major order

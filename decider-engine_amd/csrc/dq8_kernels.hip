@@ -2730,26 +2730,15 @@ __global__ __launch_bounds__(256) void k_linear_skinny(Batch b) {
   int m0 = 0, mhi = P.m, nlo, nhi;
   if (P.nseg == 1) {
     static_assert(CT == 2, "short-K waves take at most two 16-column units");
-    const int H = P.waves_n;  // units of 16 columns
-    int u0, cnt;
-    if (P.units == 8) {
-      // 4 strips of two units per block, one per wave, from unit 8*local
-      u0 = 2 * (4 * local + wid);
-      cnt = u0 < H ? 2 : 0;
-      nlo = 128 * local;
-      nhi = nlo + 128;
-    } else {
-      // The units are dealt to B = ceil(H / units) blocks, deal_q to each and
-      // one more to the first deal_r (at most 7; the host divides), so blocks
-      // carry equal byte counts to within one unit, and a block's c units to
-      // its waves as evenly as they go (w*c/4 .. (w+1)*c/4): as many waves
-      // stream as the block has units, up to 4, and none takes more than two.
-      const int h0 = local * P.deal_q + min(local, P.deal_r), c = P.deal_q + (local < P.deal_r ? 1 : 0);
-      u0 = h0 + wid * c / 4;
-      cnt = h0 + (wid + 1) * c / 4 - u0;
-      nlo = 16 * h0;
-      nhi = nlo + 16 * c;
-    }
+    // The units of 16 columns are dealt to B = ceil(waves_n / units) blocks, deal_q
+    // to each and one more to the first deal_r (at most 7; the host divides), so
+    // blocks carry equal byte counts to within one unit, and a block's c units to
+    // its waves as evenly as they go (w*c/4 .. (w+1)*c/4): as many waves
+    // stream as the block has units, up to 4, and none takes more than two.
+    const int h0 = local * P.deal_q + min(local, P.deal_r), c = P.deal_q + (local < P.deal_r ? 1 : 0);
+    const int u0 = h0 + wid * c / 4, cnt = h0 + (wid + 1) * c / 4 - u0;
+    nlo = 16 * h0;
+    nhi = nlo + 16 * c;
     if (cnt == 2)
       skip = skinny_short<RT, 2, DBS, DOTS, LORA, MODE>(P, 16 * u0, true, wid, lane, lds, b.chain);
     else
