@@ -335,13 +335,18 @@ int units_per_block(long units) { return (int)std::min(7L, std::max(2L, (units +
 //    21.8; 256 x 8192 -> 1024 (71 MB) 27.0 and 27.7, 192 (53 MB) 23.3 and 27.5; 36 x
 //    16384 -> 2048 (71 MB) 25.8 and 50.7, 128 (143 MB) 46.9 and 50.8, 192 67.9 and 51.1.
 //    Both sorts in one call: 45 rows of two 2048 -> 6144, 8192 -> 1024 and 4096 -> 2048
-//    (54 and 36 MB) 25.2 and 30.0.
+//    (54 and 36 MB) 25.2 and 30.0.  The columns layout costs the larger tiles more
+//    (each of a wave's stores takes 4 bytes of 32 or 64 lines), so its line for short K is
+//    twice as far out: 81 x 256 -> 8192 (1.5 of the rows' limit) 9.3 us as chunks, 14.2 mid and 11.4
+//    wide, 319 x 512 -> 3072 (1.9) 14.2, 22.9 and 18.7, 128 x 2048 -> 8192 (2.0) 22.7, 21.9
+//    and 26.3; long K 81 x 4096 -> 3072 (1.1) 20.2, 18.6 and 31.3.
 //  * mid: the others on the mid kernel if the wide grid would leave its blocks
 //    alone on their CUs: at most kMidBlocks blocks (64 x 128; one round of the
 //    mid kernel's 64 x 64 blocks, two per CU).  Against the wide kernel: 512 x
 //    6144 -> 2048 (128 blocks) 22.3 and 39.0 us, 1000 x 2048 -> 2048 (256) 14.4
 //    and 16.3; beyond it 400 x 2048 -> 6144 (336) 20.2 and 19.9, 2048 x 2048 ->
-//    2048 (512) 25.0 and 21.1.  In a call that mixes long and short K the wide
+//    2048 (512) 25.0 and 21.1.  One or two groups have no chain to hide (rows layout):
+//    256 x 64 -> 8192 8.4 and 6.8, 600 x 64 -> 512 6.8 and 6.4.  In a call that mixes long and short K the wide
 //    kernel's long blocks trail alone on their CUs, up to kMidMixedBlocks whatever
 //    they are (down + k at 1300 rows, 420 blocks, 54.1 and 54.7; down + q at 768, 384,
 //    38.2 and 42.0), and while the long ones are few, at most kMidLongBlocks, up to
@@ -356,7 +361,9 @@ int units_per_block(long units) { return (int)std::min(7L, std::max(2L, (units +
 constexpr long kMidBlocks = 256, kMidMixedBlocks = 400, kMidFewLongBlocks = 720, kMidLongBlocks = 208;
 // The inputs (K) whose time on the mid kernel equals that of `bytes` of chunks of
 // a projection of k inputs.
-double chunk_cost(size_t k, double bytes) { return bytes / (groups_of(k) <= 32 ? 17.5e3 : 8.8e3); }
+double chunk_cost(size_t k, double bytes, bool columns) {
+  return bytes / (groups_of(k) > 32 ? 8.8e3 : columns ? 35e3 : 17.5e3);
+}
 double weight_bytes(const dq8::Weights& w) { return (double)w.n * w.k + 4.0 * w.n * w.g; }
 bool may_split(const dq8::Weights& w, size_t m) { return kind_of(w, m) == 0 && m <= 512; }
 long wide_blocks(const dq8::Weights& w, size_t m) {
@@ -374,7 +381,7 @@ CallPlan call_plan(const Item* items, size_t count, W weights_of) {
   long blocks[2] = {0, 0}, fixed[2] = {0, 0};
   double cost = 0;
   size_t longest = 0;
-  bool has_long = false, has_short = false;
+  bool has_long = false, has_short = false, tiny = true;
   for (size_t i = 0; i < count; ++i) {
     const dq8::Weights& w = weights_of(items[i]);
     const size_t m = items[i].m;
@@ -384,15 +391,16 @@ CallPlan call_plan(const Item* items, size_t count, W weights_of) {
     part[0] += wide_blocks(w, m);
     if (w.g > 32) part[1] += wide_blocks(w, m);
     if (can) {
-      cost += chunk_cost(w.k, (double)((m + 31) / 32) * weight_bytes(w));
+      cost += chunk_cost(w.k, (double)((m + 31) / 32) * weight_bytes(w), items[i].layout == DQ8_COLUMNS);
       longest = std::max(longest, (size_t)w.k);
     }
     (w.g > 32 ? has_long : has_short) = true;
+    tiny = tiny && w.g <= 2 && items[i].layout == DQ8_ROWS;
   }
   const bool small = cost <= (double)longest;
   const long left = fixed[0] + (small ? 0 : blocks[0]), left_long = fixed[1] + (small ? 0 : blocks[1]);
   const long mixed = left_long <= kMidLongBlocks ? kMidFewLongBlocks : kMidMixedBlocks;
-  return {small, left <= (has_long && has_short ? mixed : kMidBlocks)};
+  return {small, left <= (has_long && has_short ? mixed : kMidBlocks) && !tiny};
 }
 // Kernel kind of an item in nch row chunks.
 int item_kind(const dq8::Weights& w, size_t m, size_t nch, const CallPlan& plan) {
@@ -776,7 +784,8 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
   // (row chunks as in run_linear; at most 512 rows make at most 16 chunks)
   struct One {
     size_t m;
-  } one = {m};
+    int layout;
+  } one = {m, layout};
   const CallPlan plan = call_plan(&one, 1, [&](const One&) -> const dq8::Weights& { return w; });
   const size_t nch = row_chunks(w, m, plan.small);
   static_assert(dq8::kMaxBatch >= 16, "512 rows in chunks of 32");
@@ -1156,7 +1165,7 @@ dq8_status check_mid(const float* x, size_t m, size_t k, const float* a, size_t 
 constexpr long kMidPairBlocks = 512;
 int pair_kind(const dq8::Weights& g, const int8_t* q, const float* xs, size_t m, const dq8_lora* a, const dq8_lora* b) {
   if (needs_pad(g, q) || needs_xs_pad(g, xs)) return -1;
-  const bool skinny = m <= 32 || (m <= 512 && chunk_cost(g.k, 2.0 * (double)((m + 31) / 32) * weight_bytes(g)) <= (double)g.k);
+  const bool skinny = m <= 32 || (m <= 512 && chunk_cost(g.k, 2.0 * (double)((m + 31) / 32) * weight_bytes(g), false) <= (double)g.k);
   if (skinny && !a == !b && (!a || a->rank == b->rank)) return m > 16 ? 2 : 1;
   if (m <= 32) return -1;
   const long tiles = (long)((m + dq8::block_rows(3, true) - 1) / dq8::block_rows(3, true)) *

@@ -169,8 +169,10 @@ def test_apply_few_rows(ctx, m, k, n, rank, bad):
         assert same(cols, np.ascontiguousarray(want.T))
 
 
-# Columns layout as row chunks (each chunk's rows inside the whole output's columns).
-@pytest.mark.parametrize("m,k,n", [(40, 2048, 200), (333, 1000, 130), (70, 6144, 33)])
+# Columns layout as row chunks (each chunk's rows inside the whole output's columns),
+# up to their limit and past it.
+@pytest.mark.parametrize("m,k,n", [(40, 2048, 200), (333, 1000, 130), (70, 6144, 33), (81, 256, 7000),
+                                   (81, 256, 11100), (319, 130, 2700), (40, 4096, 2300)])
 @pytest.mark.parametrize("bad", [False, True])
 def test_apply_columns_in_row_chunks(ctx, m, k, n, bad):
     rng = np.random.default_rng(m + k + n)

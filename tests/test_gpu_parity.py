@@ -1325,12 +1325,12 @@ def test_small_call_with_adapter_and_group(ctx, m):
     assert bits_equal(host(o2), dq8o.linear(x, w2v, w2s, threads=8))
 
 
-# The mid kernel (more than 32 rows whose wide grid is at most 256 blocks, here
-# past the 512 rows that run as chunks): one row and
+# The mid kernel (more than 32 rows of more than two groups, or in the columns layout,
+# whose wide grid is at most 256 blocks, here past the 512 rows that run as chunks): one row and
 # one column past a tile, widths of one input, of one and several groups, an odd
 # group count (the last group is paired with a clamped copy) and long K; and the
 # wide kernel's own ragged edges, in grids just past that limit.
-MID_CASES = [(513, 1, 1, None), (513, 64, 65, 16), (577, 100, 63, None), (600, 192, 200, 5), (540, 1088, 130, 16),
+MID_CASES = [(513, 1, 1, None), (513, 130, 70, 16), (513, 128, 65, None), (513, 64, 65, 16), (577, 100, 63, None), (600, 192, 200, 5), (540, 1088, 130, 16),
              (520, 2112, 64, 20), (520, 6200, 70, 0), (1100, 100, 2050, None), (1090, 320, 2100, 16),
              (1100, 192, 2050, 5)]
 
