@@ -8,7 +8,7 @@ the projection kernels.
     step (grouped q/k/v, o, GDN in/out, FFN gate Write, up SwiGlu, the
     re-quantized h and down Add into the residual);
   - zero, denormal-only and 127*FLT_MIN groups of x (tensor.rs:766-803) and of
-    the weights through the wide and skinny kernels, so that x-scale * w-scale
+    the weights through every projection kernel, so that x-scale * w-scale
     products are subnormal or underflow;
   - non-finite weights rejected by every weight entry point (weights.rs:170-187).
 
@@ -127,14 +127,14 @@ def edge_w(rng, n, k):
     return w
 
 
-# m = 9 and 24: the skinny kernel (16- and 32-row); 48: two skinny row chunks;
-# 96 and 200: the wide kernel
-@pytest.mark.parametrize("m", [9, 24, 48, 96, 200])
+# m = 9 and 24: the posting kernel (one and two row tiles), or at k = 2112 the
+# skinny kernel's long path; 48 to 200: row chunks on them; 600: the mid kernel; 1030:
+# the wide kernel (n = 2050); 24 with n = 5200: the skinny kernel's short path
+@pytest.mark.parametrize("m,k,n", [(m, k, 96) for m in (9, 24, 48, 96, 200, 600) for k in (2048, 6144)] +
+                         [(24, 2112, 96), (600, 2112, 96), (24, 256, 5200), (1030, 256, 2050)])
 @pytest.mark.parametrize("ep", [dq8.WRITE, dq8.ADD, dq8.SWIGLU])
-@pytest.mark.parametrize("k", [2048, 6144])
-def test_edge_groups_through_projection_kernels(ctx, m, ep, k):
+def test_edge_groups_through_projection_kernels(ctx, m, ep, k, n):
     rng = np.random.default_rng(m * 10 + ep + k)
-    n = 96
     x = edge_x(rng, m, k)
     wv, ws = dq8o.quantize_weights(edge_w(rng, n, k))
     assert ws[1, 0] == FLT_MIN  # the denormal row's scale is the floor

@@ -4,10 +4,10 @@
     x-scale * w-scale product exceeds FLT_MAX, so p = +inf and t = dot * p is
     +-inf, or NaN where the group's dot is 0; groups whose p is finite but
     dot * p overflows; and rows where two such groups of opposite sign meet
-    (inf - inf = NaN).  They run through every projection path: the wide
-    kernel, the 16- and 32-row skinny kernels, the two-chunk split, the
-    dealt short-K units and the 4-wave long-K strips, and the SwiGLU pair
-    launch, with the Write, Add and SwiGlu stores.
+    (inf - inf = NaN).  They run through every projection path: the wide, mid,
+    posting and skinny kernels (dealt short-K units and 4-wave long-K strips, 16-
+    and 32-row), row chunks, and the SwiGLU pair launches, with the Write, Add
+    and SwiGlu stores.
   - silu (qwen.rs:194-199) on every one of the 2^32 binary32 inputs, through
     the SwiGlu store of the wide kernel and through the pair launch, against
     the oracle's silu (libm expf, as the reference's f32::exp): 0 mismatches.

@@ -1,6 +1,6 @@
 """HIP graph capture of the library's asynchronous calls.
 
-A step of quantize / linear (wide and skinny) / grouped launch / SwiGlu / Add /
+A step of quantize / linear (many rows and few) / grouped launch / SwiGlu / Add /
 LoRA (single and grouped middle products) / FFN chain / apply (device-side path
 choice) is captured once on a side stream and replayed several times, with eager
 work and synchronizations in between.  Every replay must reproduce the eager results bit for bit (NaN
@@ -29,9 +29,11 @@ def bits_equal(a, b):
     return a.shape == b.shape and a.tobytes() == b.tobytes()
 
 
-def test_captured_step_replays_bit_exact(ctx):
+# row chunks and skinny pair; mid kernel and mid pair; wide kernel, its FP32 launch
+# behind apply and down, mid pair
+@pytest.mark.parametrize("M,H,F", [(130, 256, 384), (600, 256, 384), (1100, 2112, 128)])
+def test_captured_step_replays_bit_exact(ctx, M, H, F):
     rng = np.random.default_rng(77)
-    M, H, F = 130, 256, 384
     mk = lambda n, k: ctx.weights_from_quantized(*(dev(t) for t in dq8o.quantize_weights(
         (rng.standard_normal((n, k)) * 0.05).astype(np.float32))))
     wq, wg, wu, wd = mk(H, H), mk(F, H), mk(F, H), mk(H, F)
@@ -58,8 +60,8 @@ def test_captured_step_replays_bit_exact(ctx):
         o["res"].copy_(res_init)
         ctx.quantize(x, q, s, nonfinite=flag)
         ctx.quantize(xs, qs, ss, nonfinite=flag)
-        ctx.linear(wq, q, s, out=o["wide"])
-        ctx.linear(wq, qs, ss, out=o["skinny"])
+        ctx.linear(wq, q, s, out=o["many"])
+        ctx.linear(wq, qs, ss, out=o["few"])
         ctx.linear_batch([dq8.Item(wg, q, s, o["g1"]), dq8.Item(wg, qs, ss, o["g2"])])
         ctx.lora_mid(x, A, mid=mid)
         ctx.lora_mid_batch([(x, A), (x24, A), (xs, A)], mids=[o["mb0"], o["mb1"], o["mb2"]])
@@ -69,7 +71,7 @@ def test_captured_step_replays_bit_exact(ctx):
 
     def buffers():
         z = lambda *shape: torch.zeros(shape, dtype=torch.float32, device="cuda")
-        return {"res": z(M, H), "wide": z(M, H), "skinny": z(24, H), "g1": z(M, F), "g2": z(24, F),
+        return {"res": z(M, H), "many": z(M, H), "few": z(24, H), "g1": z(M, F), "g2": z(24, F),
                 "lora": z(M, F), "h": z(M, F), "apply": z(M, H), "mb0": z(M, 8), "mb1": z(24, 8), "mb2": z(24, 8)}
 
     stream = torch.cuda.Stream()

@@ -277,11 +277,12 @@ def test_linear_add_epilogue_bit_exact(ctx, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n,ep", [(130, 16384, 200, dq8.WRITE), (300, 12288, 130, dq8.ADD),
-                                      (24, 16384, 100, dq8.WRITE), (20, 32768, 48, dq8.ADD), (9, 20480, 40, dq8.WRITE)])
+                                      (24, 16384, 100, dq8.WRITE), (20, 32768, 48, dq8.ADD), (9, 20480, 40, dq8.WRITE),
+                                      (520, 16384, 70, dq8.WRITE), (530, 12345, 65, dq8.ADD)])
 def test_linear_long_k_bit_exact(ctx, m, k, n, ep):
-    # K far beyond the model's 6144 (192 to 512 groups): the wide kernel's operand
-    # rings and x-scale chunk buffers, and the skinny long-K ring and in-order
-    # hand-off, wrap many times; the group offsets reach the largest values tested
+    # K far beyond the model's 6144 (192 to 512 groups): the skinny long-K ring and in-order
+    # hand-off (in row chunks from 33 rows on), and the mid kernel's rings and x-scale chunks (520 rows on),
+    # wrap many times; the group offsets reach the largest values tested
     rng = np.random.default_rng(m + k + 7 * n)
     x = make_x(rng, m, k, "student")
     w = make_w(rng, n, k)
@@ -392,6 +393,20 @@ def test_linear_batch_mixed_kinds_matches_single_calls(ctx):
     ctx.linear_batch(items)
     for it, want in zip(items, wants):
         assert bits_equal(host(it.out), want)
+
+
+@pytest.mark.parametrize("k", [12288, 13000])
+def test_linear_long_k_on_the_wide_kernel(ctx, k):
+    # 289 wide blocks of 192 and 204 groups: the operand rings and x-scale chunk
+    # buffers wrap many times.  Rows are independent: the oracle takes one in every tile.
+    rng = np.random.default_rng(k)
+    m, n = 1030, 2050
+    x = make_x(rng, m, k, "student")
+    wv, ws = dq8o.quantize_weights(make_w(rng, n, k))
+    h = ctx.weights_from_quantized(dev(wv), dev(ws))
+    q, s = ctx.quantize(dev(x))
+    rows = tile_rows(rng, m)
+    assert bits_equal(host(ctx.linear(h, q, s))[rows], dq8o.linear(x[rows], wv, ws, threads=8))
 
 
 def test_linear_batch_question_layer_set(ctx):
@@ -701,8 +716,8 @@ def test_lora_mid_unaligned_buffers(ctx, m, k, rank):
     assert bits_equal(host(ctx.lora_mid(dev(x), dev(a))), want)
 
 
-# (m, k, n, rank): skinny (m <= 32, short and long K) and wide kernels; ranks
-# with full chunks of 8, tails, both, and rank 0.
+# (m, k, n, rank): posting and skinny kernels (m <= 32, short and long K) and row
+# chunks on them; ranks with full chunks of 8, tails, both, and rank 0.
 LORA_SHAPES = [(1, 64, 4, 3), (5, 131, 31, 13), (24, 2048, 96, 16), (17, 6144, 40, 8), (32, 256, 70, 1),
                (67, 131, 31, 13), (130, 2048, 100, 16), (64, 192, 65, 24), (19, 128, 9, 0), (48, 2048, 96, 16),
                (37, 6144, 40, 8), (130, 16384, 100, 16), (24, 12288, 64, 16), (300, 20480, 40, 8)]
@@ -738,16 +753,17 @@ def test_linear_lora_bit_exact(ctx, m, k, n, rank):
     assert bits_equal(cols, np.ascontiguousarray(want.T))
 
 
-@pytest.mark.parametrize("m", [130, 24])
+@pytest.mark.parametrize("m,n", [(130, 200), (24, 200), (24, 5200), (600, 200), (1030, 2050)])
 @pytest.mark.parametrize("rank", [16, 15, 5, 1])
 @pytest.mark.parametrize("aligned", [True, False])
-def test_linear_lora_operand_staging(ctx, m, rank, aligned):
-    # Both kernels load the adapter operands (mid and lora_B rows) before the
+def test_linear_lora_operand_staging(ctx, m, n, rank, aligned):
+    # Every kernel loads the adapter operands (mid and lora_B rows) before the
     # products: 16-byte loads when rank == 16 and both buffers are 16-byte
-    # aligned, element loads otherwise; ragged m and n clamp the rows.  130
-    # rows take the wide kernel (operands staged in LDS), 24 the skinny one.
+    # aligned, element loads otherwise; ragged m and n clamp the rows.  1030
+    # rows take the wide kernel and 600 the mid one (operands staged in LDS), 24 and 130
+    # (chunks) the posting and, at 5200 outputs, the skinny one.
     rng = np.random.default_rng(rank * 2 + aligned + m)
-    k, n = 256, 200
+    k = 512
     x, wv, ws, a, b, bias = _lora_case(rng, m, k, n, rank)
     h = ctx.weights_from_quantized(dev(wv), dev(ws))
     q, s = ctx.quantize(dev(x))

@@ -42,8 +42,10 @@ def test_apply_noalloc_matches_apply_on_consecutive_calls(ctx):
     rng = np.random.default_rng(707)
     cases = [
         # (m, k, n, epilogue, non-finite input, adapter rank)
-        (1024, 2048, 512, dq8.ADD, False, 0),   # wide kernel, 1024 x 2048 quantized into the scratch
-        (24, 6144, 96, dq8.SWIGLU, False, 8),   # smaller: skinny kernel, long K, with an adapter
+        (1024, 2048, 512, dq8.ADD, False, 0),   # mid kernel, 1024 x 2048 quantized into the scratch
+        (24, 6144, 96, dq8.SWIGLU, False, 8),   # smaller: posting kernel, long K, with an adapter
+        (1100, 128, 2050, dq8.ADD, True, 0),    # wide kernel, and the FP32 launch behind it
+        (1100, 128, 2050, dq8.ADD, False, 0),
         (70, 300, 40, dq8.WRITE, True, 0),      # a NaN: the device flag picks the FP32 path
     ]
     for m, k, n, ep, bad, rank in cases:
@@ -99,11 +101,11 @@ def test_apply_noalloc_captures_on_a_fresh_context_and_replays_bit_exact():
     # allocate (and refuses under capture); dq8_apply_noalloc captures as it
     # is and its replays equal the oracle.  Shapes: a 128-row small call whose
     # int8 path runs as skinny row chunks over the scratch-held inputs, a
-    # 2048-row wide launch, and a 24-row skinny call.
+    # 2048-row mid launch, a wide one, and a 24-row posting call.
     rng = np.random.default_rng(909)
     c = dq8.Context(0)
     try:
-        cases = [(128, 2048, 2048), (2048, 2048, 512), (24, 6144, 256)]
+        cases = [(128, 2048, 2048), (2048, 2048, 512), (1100, 128, 2050), (24, 6144, 256)]
         stream = torch.cuda.Stream()
         for m, k, n in cases:
             x0 = rng.standard_normal((m, k)).astype(np.float32)
