@@ -302,10 +302,13 @@ int kind_of(const dq8::Weights&, size_t m) { return m > 32 ? 0 : m > 16 ? 2 : 1;
 // this takes the 4-wave path for all of them (k_linear_post where it takes the
 // groups, otherwise the skinny kernel's): each wave then streams a quarter
 // of a strip's groups, so 4x the waves keep weight loads in flight.  Measured
-// at 24 rows, graph-replayed, the skinny kernel's 4-wave path (k_linear_post takes
-// 3.8 for its 4.6 us) against short-K blocks of dealt units: 2048x2048 (64 strips) 4.9 against 8.0 us, o + GDN out (128) 7.6
-// against 8.3 us, 2048x6144 (192) 10.6 against 8.3 us, GDN in (257) 10.4
-// against 8.2 us.
+// at 24 rows, graph-replayed, that path (k_linear_post from 13 groups on) against
+// short-K blocks of dealt units, us at K = 512, 1024 and 2048: 64 strips 3.5/3.8,
+// 3.6/5.2, 3.7/7.6; 128 4.4/4.2, 4.7/5.3, 5.2/8.0; 144 5.9/4.3, 5.9/5.4, 6.5/8.0; 160
+// 6.0/4.2, 5.9/5.4, 6.7/8.1; 192 6.1/4.3, 6.0/5.4, 6.7/8.2; 224 6.8/4.3, 7.3/5.8,
+// 7.9/8.3; 257 8.2/4.4, 8.6/6.0, 9.0/8.4.  At one row the 4-wave path is ahead at
+// every one of these, by 3 to 45%.  The line is one for all K and rows: what K = 2048 would
+// gain by a later one, short K would lose.
 constexpr long kSkinnyFewStrips = 160;
 long short_strips(const dq8::Weights& w) { return (w.n + dq8::skinny_cols(1) - 1) / dq8::skinny_cols(1); }
 // 16-column units of a short-K projection (one-wave strips hold two).
@@ -606,11 +609,9 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
       xs = dst;
       offset += xs_pad_bytes(w, it.m);
     }
-    // Row chunks of at most 32 rows on the skinny kernel (row_chunks): for 33-64
-    // rows the weights are read twice (the chunks run side by side, so mostly
-    // once from HBM), which beats a wide launch of half-empty row tiles whose
-    // long-K blocks trail (measured 44 against 52 us for 48 rows of a layer's
-    // projection set).  Rows are independent, so the results are the same bits.
+    // Row chunks of at most 32 rows on the skinny kernel where call_plan has them:
+    // each chunk reads the weights (side by side, so mostly once from HBM).  Rows are
+    // independent, so the results are the same bits.
     const size_t nch = row_chunks(w, it.m, plan.small);
     const int kind = item_kind(w, it.m, nch, plan);
     const size_t half = (it.m + nch - 1) / nch;
@@ -1417,8 +1418,8 @@ dq8_status dq8_ffn(dq8_ctx* ctx, const dq8_ffn_weights* f, const int8_t* q, cons
   float* sh = (float*)((char*)ctx->chain + qbytes);
   float* mid = (float*)((char*)ctx->chain + qbytes + sbytes);
   // gate: Write into h (qwen.rs:489); up: SwiGlu into h (qwen.rs:490); h is
-  // then quantized for down (qwen.rs:491).  Without adapters, on the wide
-  // kernel, both projections run in one launch that stores h directly.
+  // then quantized for down (qwen.rs:491).  Where pair_kind has a kernel for
+  // them, both projections run in one launch that stores h directly.
   dq8::Chain* chain = ctx->chain_state;
   QOut qo = {qh, sh, nonfinite, chain, f->down_lora_a, rank, mid};  // (down's middle product from h)
   st = gate_up(ctx, f->gate, f->up, q, scales, m, f->gate_bias, f->up_bias, f->gate_lora, f->up_lora, h, &qo, s);

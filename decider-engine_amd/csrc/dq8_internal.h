@@ -99,7 +99,7 @@ struct Proj {
   // Fused SwiGLU pair: wt/wst/bias are the gate weights,
   // wt2/wst2/bias2 the up weights of the same shape; the launch stores
   // h = silu(gate(x) + bias) * (up(x) + bias2) into out [M][N].  With hq
-  // set (wide kernel only) it also quantizes h as k_quantize does: hq [M][N] int8, hs [M][G_h]
+  // set (wide and mid kernels only) it also quantizes h as k_quantize does: hq [M][N] int8, hs [M][G_h]
   // scales (G_h = ceil(N / 64)); if h is not finite, 1 is ORed into *hflag
   // (when set) and Batch::hchain (when set) is marked.
   const uint8_t* wt2;
@@ -172,7 +172,8 @@ struct FProj {
 hipError_t launch_quantize(const float* x, int rows, int k, int8_t* q, int ldq, float* scales, int lds,
                            uint32_t* nonfinite, Chain* chain, hipStream_t s);
 // launch_quantize (q [m][k], scales [m][k/64]) and the middle product of x and a
-// [rank][k] in one launch, where quantize_mid_ok: few rows (m <= 32).
+// [rank][k] in one launch, where quantize_mid_ok: at most 256 blocks of the few-rows
+// middle product (128 rows at rank 16), k % 256 == 0.
 bool quantize_mid_ok(const float* x, int m, int k, const int8_t* q, const float* a, int rank);
 hipError_t launch_quantize_mid(const float* x, int m, int k, int8_t* q, float* scales, uint32_t* nonfinite, Chain* chain,
                                const float* a, int rank, float* mid, hipStream_t s);

@@ -496,9 +496,9 @@ __device__ __forceinline__ float quant_scale_fma(float m) {
 // u = a + 128 is within 2^-17 of the exact sum, so when u lies more than 2^-14
 // from every half-integer, rint(u) = round(Q) + 128, an integer in [1, 255]
 // (|a| < 127.0001, no clamp needed), converted and packed by v_cvt_pk_u8_f32;
-// the XOR with 0x80 turns it into the two's complement byte.  A wave with an
-// element closer than that (about 1 in 8000 elements) divides all its
-// elements exactly.
+// the XOR with 0x80 turns it into the two's complement byte.  Where an
+// element of a wave is closer (about 1 in 8000 is), the lanes divide their elements of that
+// index exactly.
 // FMA: u = v * rs + 128 rounded once instead of twice; u is then within 2^-16
 // + 2^-17 of Q + 128, inside the same margin.
 // (S > 1: N / S consecutive elements share a scale, so several chunks round side
@@ -1890,6 +1890,8 @@ constexpr int kModePlain = 0, kModeChained = 1, kModePair = 2;
 // us for the first; a ring of 4 steps 22.1 (and one block per CU for the pair:
 // 22.2 for the last); one MFMA per 8 VALU instructions forced by
 // sched_group_barrier 23.2.
+// Every instance is at the 256 VGPRs of two waves per SIMD, 1 to 3 of them in
+// scratch (8 to 16 bytes a lane).
 // PAIR: a SwiGLU pair block owns 32 rows x 64 outputs, waves 0 and 1 the gate
 // projection's two column tiles, waves 2 and 3 the up projection's; the tiles
 // meet in LDS after the loop, where 8 threads take one row's group of h.
@@ -3135,7 +3137,7 @@ constexpr int kMidRows = 8, kMidJ = 16, kMidKT = 256, kMidStride = kMidKT + 8;
 #define DQ8_MID_PIPE 1
 #endif
 #ifndef DQ8_MID_SMALL_M
-#define DQ8_MID_SMALL_M 32  // rows up to which k_lora_mid_small runs (0: never)
+#define DQ8_MID_SMALL_M 32  // rows up to which k_lora_mid_small runs whatever its blocks (lora_mid_small_ok)
 #endif
 constexpr int kMidSlots = DQ8_MID_SLOTS, kMidLoads = 6;  // DMA loads per wave per tile
 constexpr int kMidBatch = DQ8_MID_BATCH;

@@ -192,7 +192,8 @@ dq8_status dq8_lora_mid(dq8_ctx *ctx, const float *x, size_t m, size_t k, const 
  * possible: the projections of a question that carry adapters, each with its
  * own input x [m][k], lora_A [rank][k] and output mid [m][rank].  Items with
  * k % 4 == 0 and 16-byte aligned x and a share grouped launches of up to 32
- * items (one for items of at most 32 rows and k <= 6656, one for the others);
+ * items (one for items of at most 32 rows, or of calls with few rows and ranks
+ * in all, one for the others);
  * the rest run one launch each.  Every item is
  * checked as dq8_lora_mid checks it before anything is enqueued; the results
  * are those of dq8_lora_mid, bit for bit.  Items run concurrently: no item's
@@ -241,8 +242,8 @@ typedef struct dq8_ffn_weights {
  * into h) store, bit for bit (Epilogue::SwiGlu, tensor.rs:96-99).  Both
  * projections run in one launch that computes the gate and up values of the
  * same outputs side by side, so h is stored once and the gate result is never
- * written and read back (two launches for inputs that need padding, and for the
- * adapters noted below).  No reference counterpart of its own:
+ * written and read back (two launches for inputs that need padding, for the
+ * adapters noted below, and for outputs that share memory with inputs).  No reference counterpart of its own:
  * it schedules the crate's two apply calls of the FFN together.  gate and up
  * must have the same shape; h is [m][n] (rows layout).
  * h_q/h_scales (both or neither; NULL: h is only stored): h is also quantized
@@ -261,11 +262,12 @@ dq8_status dq8_ffn_gate_up(dq8_ctx *ctx, const dq8_weights *gate, const dq8_weig
  * the gate Write and up SwiGlu apply calls of Linear::apply_into_shared with
  * adapters (weights.rs:492-520; Adapter::combine, tensor.rs:109-117, after the
  * bias, tensor.rs:437-438), each adapter's middle product `mid` already
- * computed (dq8_lora_mid / dq8_lora_mid_batch).  The one-launch path takes
- * adapters of rank 0, and of rank 16 (the reference checkpoints' rank) with
- * 16-byte aligned mid and b, at any row count, and most others at few rows: h is
- * then still stored (and quantized) once.  Other adapters run as the two
- * separate launches, with the same bits. */
+ * computed (dq8_lora_mid / dq8_lora_mid_batch).  The one-launch path takes, up
+ * to 32 rows, adapters of one rank on both projections; in launches of some
+ * hundreds of small blocks (about 33 to 150 rows of a 2048 -> 6144 FFN) any; and
+ * beyond them rank 0 and rank 16 (the reference checkpoints' rank) with 16-byte
+ * aligned mid and b: h is then still stored (and quantized) once.  Other adapters run
+ * as the two separate launches, with the same bits. */
 dq8_status dq8_ffn_gate_up_lora(dq8_ctx *ctx, const dq8_weights *gate, const dq8_weights *up, const int8_t *q,
                                 const float *scales, size_t m, const float *gate_bias, const float *up_bias,
                                 const dq8_lora *gate_lora, const dq8_lora *up_lora, float *h, int8_t *h_q,
