@@ -325,47 +325,54 @@ int units_per_block(long units) { return (int)std::min(7L, std::max(2L, (units +
 
 // How a call's items of more than 32 rows run (measured graph-replayed, 24
 // launches over rotating weights):
-//  * small: items of at most 512 rows as chunks of at most 32
-//    rows on the skinny kernel, if all the call's chunks together read few enough
-//    weight bytes (the first read comes from HBM, the rest mostly from cache).  A
-//    chunk's time is its bytes, the mid kernel's its longest K; against the mid
-//    kernel, short K (a wave streams whole columns): 128 x 2048 -> 2048 7.8 and 9.6
-//    us, 256 x 2048 -> 2048 (36 MB) 8.1 and 9.9, 64 x 2048 -> 6144 (27 MB) 7.9 and
-//    9.9; beyond the limit 96 x 2048 -> 6144 (40 MB) 11.2 and 10.3, 512 x 512 -> 2048
-//    (18 MB) 8.1 and 5.7.  Long K (4 waves share them) up to half the bytes per input,
-//    where the two meet: 128 x 4096 -> 2048 (36 MB) 16.2 and 16.2, 192 (53 MB) 22.2 and
-//    16.4; 256 x 6144 -> 1024 (53 MB) 21.6 and 21.6, 96 x 6144 -> 2048 (40 MB) 19.1 and
-//    21.8; 256 x 8192 -> 1024 (71 MB) 27.0 and 27.7, 192 (53 MB) 23.3 and 27.5; 36 x
-//    16384 -> 2048 (71 MB) 25.8 and 50.7, 128 (143 MB) 46.9 and 50.8, 192 67.9 and 51.1.
-//    Both sorts in one call: 45 rows of two 2048 -> 6144, 8192 -> 1024 and 4096 -> 2048
-//    (54 and 36 MB) 25.2 and 30.0.  The columns layout costs the larger tiles more
-//    (each of a wave's stores takes 4 bytes of 32 or 64 lines), so its line for short K is
-//    twice as far out: 81 x 256 -> 8192 (1.5 of the rows' limit) 9.3 us as chunks, 14.2 mid and 11.4
-//    wide, 319 x 512 -> 3072 (1.9) 14.2, 22.9 and 18.7, 128 x 2048 -> 8192 (2.0) 22.7, 21.9
-//    and 26.3; long K 81 x 4096 -> 3072 (1.1) 20.2, 18.6 and 31.3.
+//  * small: items of at most 512 rows as chunks of at most 32 rows on the skinny
+//    kernel, if all the call's chunks together read few enough weight bytes (the
+//    first read comes from HBM, the rest mostly from cache).  A chunk's time is its
+//    bytes, the mid kernel's its longest K.  Against the mid kernel, in us:
+//    - short K (a wave streams whole columns): 128 x 2048 -> 2048 7.8 and 9.6, 256 x
+//      2048 -> 2048 (36 MB) 8.1 and 9.9, 64 x 2048 -> 6144 (27 MB) 7.9 and 9.9; beyond
+//      the limit 96 x 2048 -> 6144 (40 MB) 11.2 and 10.3, 512 x 512 -> 2048 (18 MB) 8.1
+//      and 5.7;
+//    - long K (4 waves share them) up to about half the bytes per input, where the
+//      two meet: 128 x 4096 -> 2048 (36 MB) 16.2 and 16.2, 192 (53 MB) 22.2 and 16.4; 96
+//      x 6144 -> 2048 (40 MB) 19.1 and 21.8, 128 (53 MB) 21.9 and 21.8, Add 23.7 and
+//      21.4; 256 x 8192 -> 1024 (71 MB) 27.0 and 27.7, 192 (53 MB) 23.3 and 27.5; 36 x
+//      16384 -> 2048 (71 MB) 25.8 and 50.7, 128 (143 MB) 46.9 and 50.8, 192 67.9 and 51.1;
+//    - both in one call, where long K costs a quarter more: 45 rows of two 2048 ->
+//      6144, 8192 -> 1024 and 4096 -> 2048 (54 and 36 MB) 25.2 and 30.0; 56 rows of 4096 ->
+//      2048, 6144 -> 2048, two 512 -> 2048 and 2048 -> 2048 (13 and 45 MB) 27.4 and 23.1;
+//    - the columns layout, which costs the larger tiles more (each of a wave's stores
+//      takes 4 bytes of 32 or 64 lines), at short K twice as far: 81 x 256 -> 8192 (1.5
+//      of the rows' limit) 9.3, 14.2 and 11.4 wide, 319 x 512 -> 3072 (1.9) 14.2, 22.9
+//      and 18.7, 128 x 2048 -> 8192 (2.0) 22.7, 21.9 and 26.3; long K as in rows, 81 x 4096
+//      -> 3072 (1.1) 20.2, 18.6 and 31.3.
 //  * mid: the others on the mid kernel if the wide grid would leave its blocks
 //    alone on their CUs: at most kMidBlocks blocks (64 x 128; one round of the
 //    mid kernel's 64 x 64 blocks, two per CU).  Against the wide kernel: 512 x
 //    6144 -> 2048 (128 blocks) 22.3 and 39.0 us, 1000 x 2048 -> 2048 (256) 14.4
 //    and 16.3; beyond it 400 x 2048 -> 6144 (336) 20.2 and 19.9, 2048 x 2048 ->
-//    2048 (512) 25.0 and 21.1.  One or two groups have no chain to hide (rows layout):
-//    256 x 64 -> 8192 8.4 and 6.8, 600 x 64 -> 512 6.8 and 6.4.  In a call that mixes long and short K the wide
-//    kernel's long blocks trail alone on their CUs, up to kMidMixedBlocks whatever
-//    they are (down + k at 1300 rows, 420 blocks, 54.1 and 54.7; down + q at 768, 384,
-//    38.2 and 42.0), and while the long ones are few, at most kMidLongBlocks, up to
-//    kMidFewLongBlocks: a layer set of 9 projections at 77 rows (468, 32 long) 29.5 and
-//    42.3 us, 192 (702, 48) 46.2 and 53.7, 256 (936) 58.6 and 55.9; down + gate at 640
-//    rows (640, 160) 48.0 and 50.9, 768 (768, 192) 55.7 and 54.9; 8192 -> 1024 + q at 1600
-//    (600, 200) 59.5 and 66.0; but 4096 -> 2048 +
-//    q at 1000 (512, 256 long) 37.7 and 33.7, down + k at 1600 (500, 400) 66.7 and 58.0, 2048
-//    (640, 512) 75.0 and 70.8.
+//    2048 (512) 25.0 and 21.1.
+//    - In a call that mixes long and short K the wide kernel's longest blocks trail
+//      alone on their CUs while all the call's blocks, each counted by its groups,
+//      would make at most kMidMixedBlocks of the longest: a layer set of 9 projections
+//      at 128 rows (177 such blocks) 33.8 and 48.1, 192 (266) 46.2 and 53.7, 256 (355)
+//      58.6 and 55.9; down + gate at 640 rows (320) 48.0 and 50.9, 768 (384) 55.7 and 54.9;
+//      down + q at 768 (256) 38.2 and 42.0, 1000 (341) 49.7 and 49.3; 4096 -> 2048 + q at
+//      768 (288) 31.0 and 30.7, 1000 (384) 37.7 and 33.7; 8192 -> 1024 + q at 1600 (300)
+//      61.2 and 67.2, 2048 (384) 73.7 and 72.1.
+//    - One or two groups have no chain to hide (plain stores): 256 x 64 -> 8192 8.4
+//      and 6.8, 600 x 64 -> 512 6.8 and 6.4.
+//    - Short-K results in the columns layout of about one L2 (2.4 or 2.8 to 5.6 MB),
+//      whose lines fewer blocks at a time complete before they leave it: 1063 x 256 ->
+//      1020 17.2 and 12.1, 520 x 512 -> 2048 19.3 and 15.3, 666 x 512 -> 1020 13.9 and 11.1;
+//      but 520 x 512 -> 1020 9.0 and 12.4, 777 x 512 -> 2048 29.7 and 31.9.
 //  * the wide kernel otherwise.
 // Rows are independent, so the results are the same bits either way.
-constexpr long kMidBlocks = 256, kMidMixedBlocks = 400, kMidFewLongBlocks = 720, kMidLongBlocks = 208;
+constexpr long kMidBlocks = 256, kMidMixedBlocks = 330;
 // The inputs (K) whose time on the mid kernel equals that of `bytes` of chunks of
 // a projection of k inputs.
 double chunk_cost(size_t k, double bytes, bool columns) {
-  return bytes / (groups_of(k) > 32 ? 8.8e3 : columns ? 35e3 : 17.5e3);
+  return bytes / (groups_of(k) > 32 ? 9.3e3 - 4e6 / (double)k : columns ? 35e3 : 17.5e3);
 }
 double weight_bytes(const dq8::Weights& w) { return (double)w.n * w.k + 4.0 * w.n * w.g; }
 bool may_split(const dq8::Weights& w, size_t m) { return kind_of(w, m) == 0 && m <= 512; }
@@ -378,13 +385,16 @@ size_t row_chunks(const dq8::Weights& w, size_t m, bool small) {
 struct CallPlan {
   bool small, mid;
 };
+// chained: inputs that may be non-finite (the wide kernel then has the FP32 launch behind it).
 template <class Item, class W>
-CallPlan call_plan(const Item* items, size_t count, W weights_of) {
-  // wide blocks (all, long K) of the items that may run as chunks, and of the others
+CallPlan call_plan(const Item* items, size_t count, bool chained, W weights_of) {
+  // wide blocks (all; times their groups) of the items that may run as chunks, and of the others
   long blocks[2] = {0, 0}, fixed[2] = {0, 0};
-  double cost = 0;
+  double cost[2] = {0, 0};  // of chunks, short and long K
   size_t longest = 0;
-  bool has_long = false, has_short = false, tiny = true;
+  long groups = 0;
+  bool has_long = false, has_short = false, tiny = !chained, columns = true;
+  double col_out = 0;
   for (size_t i = 0; i < count; ++i) {
     const dq8::Weights& w = weights_of(items[i]);
     const size_t m = items[i].m;
@@ -392,18 +402,21 @@ CallPlan call_plan(const Item* items, size_t count, W weights_of) {
     const bool can = may_split(w, m);
     long* part = can ? blocks : fixed;
     part[0] += wide_blocks(w, m);
-    if (w.g > 32) part[1] += wide_blocks(w, m);
+    part[1] += wide_blocks(w, m) * w.g;
+    groups = std::max(groups, (long)w.g);
     if (can) {
-      cost += chunk_cost(w.k, (double)((m + 31) / 32) * weight_bytes(w), items[i].layout == DQ8_COLUMNS);
+      cost[w.g > 32] += chunk_cost(w.k, (double)((m + 31) / 32) * weight_bytes(w), items[i].layout == DQ8_COLUMNS);
       longest = std::max(longest, (size_t)w.k);
     }
     (w.g > 32 ? has_long : has_short) = true;
-    tiny = tiny && w.g <= 2 && items[i].layout == DQ8_ROWS;
+    if (w.g <= 16 && items[i].layout == DQ8_COLUMNS) col_out += (double)m * w.n;
+    else columns = false;
+    tiny = tiny && w.g <= 2 && items[i].layout == DQ8_ROWS && items[i].epilogue == DQ8_WRITE && !items[i].lora;
   }
-  const bool small = cost <= (double)longest;
-  const long left = fixed[0] + (small ? 0 : blocks[0]), left_long = fixed[1] + (small ? 0 : blocks[1]);
-  const long mixed = left_long <= kMidLongBlocks ? kMidFewLongBlocks : kMidMixedBlocks;
-  return {small, left <= (has_long && has_short ? mixed : kMidBlocks) && !tiny};
+  const bool small = cost[0] + (cost[0] > 0 ? 1.25 : 1.0) * cost[1] <= (double)longest;
+  const long left = fixed[0] + (small ? 0 : blocks[0]), work = fixed[1] + (small ? 0 : blocks[1]);
+  const bool burst = columns && col_out > (groups > 4 ? 0.6e6 : 0.7e6) && col_out < 1.4e6;
+  return {small, (has_long && has_short ? work <= kMidMixedBlocks * groups : left <= kMidBlocks) && !tiny && !burst};
 }
 // Kernel kind of an item in nch row chunks.
 int item_kind(const dq8::Weights& w, size_t m, size_t nch, const CallPlan& plan) {
@@ -568,7 +581,7 @@ dq8_status run_linear(dq8_ctx* ctx, const dq8_linear_item* items, size_t count, 
     b.count = b.total_waves = b.any_lora = 0;
     b.chain = fb ? fb->chain : nullptr;
   }
-  CallPlan plan = call_plan(items, count, [](const dq8_linear_item& it) -> const dq8::Weights& { return it.w->w; });
+  CallPlan plan = call_plan(items, count, fb != nullptr, [](const dq8_linear_item& it) -> const dq8::Weights& { return it.w->w; });
   if (dots) plan.mid = false;
   // one-wave strips each skinny launch would have (see kSkinnyFewStrips)
   long strips[dq8::kKinds] = {}, units[dq8::kKinds] = {};
@@ -785,9 +798,10 @@ dq8_status launch_one(const dq8::Weights& w, const WorkInputs& in, size_t m, con
   // (row chunks as in run_linear; at most 512 rows make at most 16 chunks)
   struct One {
     size_t m;
-    int layout;
-  } one = {m, layout};
-  const CallPlan plan = call_plan(&one, 1, [&](const One&) -> const dq8::Weights& { return w; });
+    int layout, epilogue;
+    const dq8_lora* lora;
+  } one = {m, layout, epilogue, lora};
+  const CallPlan plan = call_plan(&one, 1, fb != nullptr, [&](const One&) -> const dq8::Weights& { return w; });
   const size_t nch = row_chunks(w, m, plan.small);
   static_assert(dq8::kMaxBatch >= 16, "512 rows in chunks of 32");
   const int kind = item_kind(w, m, nch, plan);

@@ -3665,23 +3665,28 @@ int block_cols(int kind, bool pair) {
 }
 // The group bound of the posting kernel (k_linear_post) that takes a skinny launch,
 // or 0: every projection on the 4-wave path, and
-//  * up to 32 groups (an instance loads all 32, repeats past the last): 13 or more,
-//    or 5 or more in at most one block per CU.  Graph-replayed against the skinny
+//  * up to 32 groups (an instance loads all 32, repeats past the last): 13 or more (5
+//    with an adapter or an Add or SwiGlu store, whose operands it loads beside the
+//    weights), or at most one block per CU.  Graph-replayed against the skinny
 //    kernel: 24 x 2048 -> 2048 3.8 and 4.5 us, 24 x 1024 -> 2048 3.6 and 4.2; 40 rows -> 2048
 //    (512 blocks) of K = 1024 4.8 and 5.0, 768 4.9 and 4.7, 512 4.7 and 4.4, 256 4.7 and
-//    4.2; one block per CU or fewer, 24 rows -> 2048 of 512 3.5 and 3.7, 256 3.55 and 3.45.
+//    4.2; Add 768 5.0 and 5.55, 512 5.0 and 5.25, 256 4.9 and 5.0; 466 x 512 -> 256 with a
+//    rank-32 adapter 6.6 and 7.6, 24 x 512 -> 4096 with rank 16 5.3 and 5.2; one block per CU or fewer, 24 rows -> 2048 of 512 3.5 and 3.7, 256 3.55 and 3.45,
+//    but 3 x 256 -> 256 Add 3.3 and 3.7, 3 x 256 -> 4096 with a rank-32 adapter 4.6 and 6.3.
 //  * 65 to 96 groups in at most one block per CU (its LDS): 24 x 6144 -> 2048 8.2 and
 //    9.6, 24 x 5120 -> 1024 7.6 and 8.2, 24 x 4352 -> 1024 7.3 and 7.2, 1 x 4352 -> 1024
 //    5.9 and 6.9; 64 groups on this instance (a third of the loads repeats), 24 x 4096 ->
 //    2048, 8.6 and 7.3; 6144 -> 4096 (512 blocks) 16.1 and 12.3.
 static int post_groups(const Batch& b) {
   int lo = 1 << 30, hi = 0;
+  bool writes = true;
   for (int i = 0; i < b.count; ++i) {
     if (b.p[i].nseg != 4 || b.p[i].pair) return 0;
+    writes = writes && b.p[i].epilogue == 0 && !b.p[i].lora;
     lo = std::min(lo, b.p[i].g);
     hi = std::max(hi, b.p[i].g);
   }
-  if (hi <= 32) return hi > 12 || (hi > 4 && b.total_waves <= 256) ? 32 : 0;
+  if (hi <= 32) return hi > (writes ? 12 : 4) || b.total_waves <= 256 ? 32 : 0;
   return lo > 64 && hi <= 96 && b.total_waves <= 256 ? 96 : 0;
 }
 bool wide_can_pair() { return wide_pair_shape(DQ8_WIDE_WN, DQ8_WIDE_RT, DQ8_WIDE_CT); }

@@ -1296,12 +1296,13 @@ def test_small_calls_bit_exact(ctx, m, k, n, ep):
 
 
 # Long and short K in one call: calls on both sides of the rule by which row chunks
-# cost what the longest K would on the mid kernel, and of the mid kernel's block limits
-# (many and few long-K blocks).
+# cost what the longest K would on the mid kernel, and of the mid kernel's limit of 330
+# blocks of the longest.
 @pytest.mark.parametrize("m,shapes", [(45, [(2048, 1500), (2048, 700), (8192, 300), (4096, 500)]),
                                       (100, [(2048, 3000), (6144, 900)]), (40, [(12288, 200), (130, 999)]),
-                                      (520, [(2112, 2700), (130, 3000)]), (520, [(2112, 3000), (130, 2600)]),
-                                      (600, [(2112, 640), (65, 8200)]), (700, [(2112, 640), (65, 7700)])])
+                                      (520, [(2112, 2700), (130, 3000)]), (700, [(2112, 3500), (130, 2600)]),
+                                      (600, [(2112, 640), (65, 8200)]), (1100, [(2112, 2200), (65, 2000)]),
+                                      (56, [(4096, 700), (130, 999)]), (172, [(8192, 300), (1024, 1024)])])
 def test_grouped_call_of_long_and_short_k(ctx, m, shapes):
     rng = np.random.default_rng(m)
     items, wants = [], []
@@ -1346,7 +1347,8 @@ def test_small_call_with_adapter_and_group(ctx, m):
 # one column past a tile, widths of one input, of one and several groups, an odd
 # group count (the last group is paired with a clamped copy) and long K; and the
 # wide kernel's own ragged edges, in grids just past that limit.
-MID_CASES = [(513, 1, 1, None), (513, 130, 70, 16), (513, 128, 65, None), (513, 64, 65, 16), (577, 100, 63, None), (600, 192, 200, 5), (540, 1088, 130, 16),
+MID_CASES = [(513, 1, 1, None), (513, 130, 70, 16), (513, 128, 65, None),
+             (520, 100, 1020, None), (701, 200, 1020, None), (513, 64, 65, 16), (577, 100, 63, None), (600, 192, 200, 5), (540, 1088, 130, 16),
              (520, 2112, 64, 20), (520, 6200, 70, 0), (1100, 100, 2050, None), (1090, 320, 2100, 16),
              (1100, 192, 2050, 5)]
 
@@ -1441,11 +1443,12 @@ def test_ffn_chain_quantizes_beside_the_middle_product(ctx, m, hidden, inter):
 
 
 # The posting kernel (few strips, 5 to 32 groups or 65 to 96) at its bounds and
-# just past them: one group, 4 and 5, a partial last one, 12 and 13 in more than a block per CU, 64 / 65 / 96 / 97 groups, one and
+# just past them: one group, a partial last one, 4 / 5 / 12 / 13 in more than a block per CU, 64 / 65 / 96 / 97 groups, one and
 # two row tiles, a last run of fewer than 8 strips, more than 256 blocks.
 @pytest.mark.parametrize("m,k,n,rank", [(1, 64, 16, None), (16, 2048, 33, 16), (31, 2047, 50, 5), (17, 4096, 40, 16),
                                         (17, 4160, 200, 16), (32, 6144, 2064, None), (20, 6144, 70, 20),
                                         (9, 6145, 48, None), (33, 1000, 100, 16), (24, 256, 300, 16),
-                                        (24, 320, 300, 5), (40, 768, 2048, None), (40, 832, 2050, 16)])
+                                        (24, 320, 300, 5), (40, 768, 2048, None), (40, 832, 2050, 16),
+                                        (40, 256, 2050, None), (40, 300, 2048, 16)])
 def test_posting_kernel_edges(ctx, m, k, n, rank):
     test_mid_and_wide_kernel_edges(ctx, m, k, n, rank)
